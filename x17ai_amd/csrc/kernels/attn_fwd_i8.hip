@@ -760,7 +760,7 @@ void kernel(
 					f32 resc = 1.0f;
 					if (__any(tmax > m)) {
 						f32 new_m = __builtin_fmaxf(tmax, m);
-						resc = sfu::ex2(m - new_m);      // exactly 1 for rows whose max did not move
+						resc = strict::ex2<true>(m - new_m);      // exactly 1 for rows whose max did not move
 						m = new_m;
 						if constexpr (STRICT) {
 							X17_UNROLL for (u32 db = 0; db < D_BLOCKS; ++db) {
@@ -786,7 +786,7 @@ void kernel(
 					// :265-290 -- p = ex2(s - max) * 255; partial sums over key quads; P = rne(p)
 					f32 p[8];
 					if constexpr (STRICT) {
-						X17_UNROLL for (u32 r = 0; r < 8; ++r) p[r] = sfu::ex2(s[r] - m) * PROB_SCALE;
+						X17_UNROLL for (u32 r = 0; r < 8; ++r) p[r] = strict::ex2<true>(s[r] - m) * PROB_SCALE;
 					} else {
 						f32 const shift = m - LOG2_PROB_SCALE;        // 255 * 2^(s - m) = 2^(s - (m - lg2 255))
 						if (int_path) {

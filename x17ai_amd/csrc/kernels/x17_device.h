@@ -156,12 +156,18 @@ template<int STORE> X17_DEV u32 store_convert(f32 v) {
 // Same algorithms, constants and operation order as the CPU checker uses; see the header note.
 
 namespace strict {
-	// 2^x; results below 2^-125 flush to zero
+	// 2^x; results below 2^-125 flush to zero.  NONPOSITIVE: the caller guarantees x <= 0 (or NaN), the upper clamp goes.
+	// No branch: an early return for the flushed arguments makes the compiler guard every call with an execution
+	// mask of its own, and the calls of a softmax row (or of a writer's row) then run one behind the other instead of
+	// interleaved.  Adding 1.5 * 2^23 rounds to an integer exactly like rint (ties to even) and leaves that integer in
+	// the low bits of the sum: two plain additions in place of a rounding and a conversion, which issue more slowly.
+	template <bool NONPOSITIVE = false>
 	X17_DEV f32 ex2(f32 x) {
-		if (!(x >= -125.0f)) return 0.0f;
-		x = __builtin_fminf(x, 126.0f);
-		f32 n = __builtin_rintf(x);
-		f32 f = x - n;
+		constexpr f32 MAGIC = 12582912.0f;
+		bool const kept = x >= -125.0f;
+		if constexpr (!NONPOSITIVE) x = __builtin_fminf(x, 126.0f);
+		f32 const t = x + MAGIC;
+		f32 f = x - (t - MAGIC);
 		f32 p = 0.00015453163359779865f;
 		p = fmaf32(p, f, 0.0013390863314270973f);
 		p = fmaf32(p, f, 0.009618083015084267f);
@@ -169,8 +175,8 @@ namespace strict {
 		p = fmaf32(p, f, 0.24022650718688965f);
 		p = fmaf32(p, f, 0.6931471824645996f);
 		p = fmaf32(p, f, 1.0f);
-		i32 ni = (i32)n;
-		return u2f(f2u(p) + ((u32)ni << 23));
+		f32 const r = u2f(f2u(p) + (f2u(t) << 23));      // (the bits of MAGIC above the integer leave in the shift)
+		return kept ? r : 0.0f;
 	}
 
 	// log2(x), x positive normal finite
