@@ -1,8 +1,7 @@
 // Host-side audit of the attention kernel's K/V tile requests.  Compiled with the kernel's own common.h and
 // attn_tile.h -- the index arithmetic below IS the kernel's (attn_fwd_i8.hip calls the same functions) -- it walks, on
-// the CPU, every workgroup of a launch (sequence, head, query block) through the request schedule of its build (the
-// speed build asks for a tile in every step, past the end the last one again; the strict build stops asking) and
-// checks that every 16-byte request, every 4-byte scale request of the row-scaled build and every query load stays
+// the CPU, every workgroup of a launch (sequence, head, query block) through the request schedule (a tile in every
+// step, past the end the last one again) and checks that every 16-byte request, every 4-byte scale request of the row-scaled build and every query load stays
 // inside its operand and inside the workgroup's own sequence, and that the requests of a tile cover its chunks once.
 //
 //     attn_requests_audit <seq_len> <batch> <window_size> [rows q / kv really have, default seq_len * batch]
@@ -31,7 +30,6 @@ int main(int argc, char **argv) {
 	unsigned const window_size = (unsigned)std::strtoull(argv[3], nullptr, 10);
 	constexpr unsigned HD = X17_HEAD_DIM, H = X17_N_HEADS, Q_STRIDE = X17_Q_STRIDE, KV_STRIDE = X17_KV_STRIDE;
 	constexpr unsigned CPR = at::CHUNKS_PER_ROW;
-	constexpr bool SPEED = X17_STRICT_MATH == 0;
 	if (seq_len_arg % 64 != 0 || seq_len_arg < at::Q_PER_BLOCK || batch == 0 || seq_len_arg * batch > 0xFFFFFFFFull
 	    || (window_size != 0 && window_size % 16 != 0)) {
 		return fail("the launcher rejects this shape (seq_len % 64, at least one query block, window % 16)", seq_len_arg, at::Q_PER_BLOCK);
@@ -84,21 +82,16 @@ int main(int argc, char **argv) {
 				requests += 2ull * stagers;
 				return 0;
 			};
-			if (SPEED) {
-				// prologue: raw V tile 0, then K tiles 0..2 with V tiles 1..3; the source then stands at tile 3
-				for (unsigned j = 0; j <= at::PREFETCH; ++j) if (int rc = tile(j)) return rc;
-				unsigned src_tile = at::PREFETCH;
-				for (unsigned s = 0; s < n_steps; ++s) {
-					bool const more = at::further_tile_exists(s, n_steps);
-					if (int rc = tile(src_tile)) return rc;                         // K (and the scales of the row-scaled build)
-					if (int rc = tile(src_tile + (more ? 1 : 0))) return rc;        // raw V, one tile further while there is one
-					src_tile += more ? 1 : 0;
-				}
-				if (src_tile != last) return fail("the source pointer does not end on the last tile", src_tile, last);
-			} else {
-				for (unsigned j = 0; j < at::PREFETCH && j < n_steps; ++j) if (int rc = tile(j)) return rc;
-				for (unsigned i = 0; i + at::PREFETCH < n_steps; ++i) if (int rc = tile(i + at::PREFETCH)) return rc;
+			// prologue: raw V tile 0, then K tiles 0..2 with V tiles 1..3; the source then stands at tile 3
+			for (unsigned j = 0; j <= at::PREFETCH; ++j) if (int rc = tile(j)) return rc;
+			unsigned src_tile = at::PREFETCH;
+			for (unsigned s = 0; s < n_steps; ++s) {
+				bool const more = at::further_tile_exists(s, n_steps);
+				if (int rc = tile(src_tile)) return rc;                         // K (and the scales of the row-scaled build)
+				if (int rc = tile(src_tile + (more ? 1 : 0))) return rc;        // raw V, one tile further while there is one
+				src_tile += more ? 1 : 0;
 			}
+			if (src_tile != last) return fail("the source pointer does not end on the last tile", src_tile, last);
 			// the block's query rows (16-byte loads, 32 bytes of head_dim per lane and slice)
 			unsigned long long const q_end = (row_base + q0 + at::Q_PER_BLOCK - 1) * Q_STRIDE + (unsigned long long)(H - 1) * HD + HD;
 			if (q_end > q_bytes) return fail("query load past the end of q", q_end, q_bytes);

@@ -28,7 +28,8 @@ constexpr unsigned RING = PREFETCH + 1;
 // Register budget: this many wavefronts (= workgroups) share a SIMD, so that one workgroup's waits for
 // its K/V tiles and its barrier are covered by the others' arithmetic.
 #ifndef X17_ATTN_WAVES_PER_SIMD
-#define X17_ATTN_WAVES_PER_SIMD (X17_STRICT_MATH ? 2 : 3)   // the deterministic transcendentals need more registers
+// (the deterministic transcendentals need more registers; with smaller heads the accumulators leave room again)
+#define X17_ATTN_WAVES_PER_SIMD (!(X17_STRICT_MATH) || X17_HEAD_DIM == 64 ? 3 : X17_HEAD_DIM == 32 ? (X17_ATTN_ROW_SCALES ? 4 : 5) : 2)
 #endif
 constexpr unsigned WAVES_PER_SIMD = X17_ATTN_WAVES_PER_SIMD;
 
@@ -72,7 +73,7 @@ constexpr unsigned stage_k_offset(unsigned tid, unsigned kv_stride) {
 constexpr unsigned stage_v_offset(unsigned tid, unsigned kv_stride) {
 	return (tid / CHUNKS_PER_ROW) * kv_stride + HEAD_DIM + (tid % CHUNKS_PER_ROW) * 16;
 }
-// Speed build: step s requests K tile min(s + PREFETCH, last) and raw V tile min(s + PREFETCH + 1, last); its source
+// Step s requests K tile min(s + PREFETCH, last) and raw V tile min(s + PREFETCH + 1, last); its source
 // pointer moves on to the next tile exactly when that further tile exists.
 constexpr bool further_tile_exists(unsigned s, unsigned n_steps) { return s + PREFETCH + 1 < n_steps; }
 
