@@ -1221,7 +1221,7 @@ Status AttnKernel::launch(AttnKernelArgs const &a) {
 	// the plain kernel takes the first nine arguments only
 	void *raw_args[14] = {&seq_len_arg, &q_ptr, &kv_ptr, &sk, &sv, &tp, &out_ptr, &l_ptr, &window_arg,
 	                      &scale_ptrs[0], &scale_ptrs[1], &scale_ptrs[2], &scale_ptrs[3], &scale_ptrs[4]};
-	size_t grid[3] = {(seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK, config.head_group_cnt(), a.batch};
+	size_t grid[3] = {(seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK, config.n_heads, a.batch};
 	size_t block[3] = {metadata.THREADS_PER_BLOCK, 1, 1};
 	return kernel->launch(*device->stream, grid, block, metadata.SMEM_BYTES, raw_args);
 }
@@ -1278,7 +1278,7 @@ Status AttnKernel::launch_d_q(AttnKernelArgs const &a) {
 	void *out_ptr = a.out->ptr, *do_ptr = a.d_out->ptr, *dq_ptr = a.d_q->ptr, *l_ptr = a.l->ptr;
 	void *d_ptr = a.d != nullptr ? a.d->ptr : nullptr;
 	void *raw_args[12] = {&seq_len_arg, &q_ptr, &kv_ptr, &sk, &sv, &tp, &out_ptr, &do_ptr, &dq_ptr, &l_ptr, &d_ptr, &window_arg};
-	size_t grid[3] = {(seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK, config.head_group_cnt(), a.batch};
+	size_t grid[3] = {(seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK, config.n_heads, a.batch};
 	size_t block[3] = {metadata.THREADS_PER_BLOCK, 1, 1};
 	return kernel->launch(*device->stream, grid, block, metadata.SMEM_BYTES, raw_args);
 }
@@ -1327,7 +1327,7 @@ Status AttnKernel::launch_d_kv(AttnKernelArgs const &a) {
 	void *q_ptr = a.q->ptr, *kv_ptr = a.kv->ptr, *tp = a.attn_temperature->ptr, *do_ptr = a.d_out->ptr, *l_ptr = a.l->ptr, *d_ptr = a.d->ptr;
 	void *dkv_ptr = a.d_kv->ptr;
 	void *raw_args[9] = {&seq_len_arg, &q_ptr, &kv_ptr, &tp, &do_ptr, &l_ptr, &d_ptr, &dkv_ptr, &window_arg};
-	size_t grid[3] = {(seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK, config.head_group_cnt(), a.batch};
+	size_t grid[3] = {(seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK, config.n_heads, a.batch};
 	size_t block[3] = {metadata.THREADS_PER_BLOCK, 1, 1};
 	return kernel->launch(*device->stream, grid, block, metadata.SMEM_BYTES, raw_args);
 }

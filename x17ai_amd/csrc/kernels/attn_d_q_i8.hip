@@ -142,6 +142,9 @@ void kernel(
 	u32 const lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
 	u32 const pair = lin % pairs;
 	u32 const q_block_index = gridDim.x - 1 - lin / pairs;
+	// heads of this workgroup, one behind the other: the grid says how many groups they were cut into (one group per head
+	// by this library's launchers, groups of 128 / head_dim heads by src/device/cuda/attn.rs:60-66)
+	u32 const heads_here = HPK == 1 ? 1 : N_HEADS / gridDim.y;
 	u32 const head_group = pair % gridDim.y;
 	u32 const seq = pair / gridDim.y;
 	size_t const row_base = (size_t)seq * seq_len;
@@ -157,8 +160,8 @@ void kernel(
 	u32 const wave_kb_last = q_wave0 / at::KV_PER_STEP;
 	u32 const n_steps = kb_end - kb_begin;
 
-	for (u32 hh = 0; hh < HPK; ++hh) {
-		u32 const head = head_group * HPK + hh;
+	for (u32 hh = 0; hh < heads_here; ++hh) {
+		u32 const head = head_group * heads_here + hh;
 		i8 const *q_head = q + row_base * Q_STRIDE + (size_t)head * HD;
 		i8 const *kv_head = kv + row_base * KV_STRIDE + (size_t)head * 2 * HD;
 

@@ -101,6 +101,6 @@ int main(int argc, char **argv) {
 	if (scale_extent > rows) return fail("scale request past the end of a [H, rows] scale matrix", scale_extent, rows);
 	std::printf("{\"ok\": true, \"workgroups\": %llu, \"requests\": %llu, \"kv_extent\": %llu, \"kv_bytes\": %llu, \"q_extent\": %llu, "
 	            "\"q_bytes\": %llu, \"scale_extent_rows\": %llu, \"rows\": %llu}\n",
-	            batch * q_blocks * (H / at::HEADS_PER_KERNEL), requests * H, kv_extent, kv_bytes, q_extent, q_bytes, scale_extent, rows);
+	            batch * q_blocks * H, requests * H, kv_extent, kv_bytes, q_extent, q_bytes, scale_extent, rows);
 	return 0;
 }
