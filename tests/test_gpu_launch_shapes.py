@@ -55,3 +55,45 @@ def test_head_groups_in_the_grid(shim, h, hd, seq, batch, window):  # noqa: F811
 	for name, pair in (("out", out), ("l", l), ("d_q", d_q), ("d", d), ("d_kv", d_kv)):
 		a, b = (x.download() for x in pair)
 		assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), name
+
+
+@pytest.mark.parametrize("n,window,row_scales", [
+	(8, 256, False), (8, 4096, True),                                        # at most one workgroup per compute unit: 256 / 1024 threads
+	(9, 1040, False), (9, 1024, True), (32, 512, False), (32, 1024, False),    # more: 512 / 256 / 256 / 256 threads
+	(33, 512, True), (33, 528, False), (33, 2048, False),                     # ... than four per compute unit: 128 / 256 / 512
+])
+def test_decode_workgroup_widths(n, window, row_scales):
+	"""Every width the launcher picks (32 heads of 128, capacity 4096), ragged lengths including 0, 1 and the capacity:
+	bit-equal to the oracle on sampled (sequence, head) slices."""
+	from oracle import strict as S
+	dev = X.Device(0)
+	h, hd, cap = 32, 128, 4096
+	rng = rng_for("decode widths", n, window, row_scales)
+	lens = rng.integers(2, cap, n).astype(np.uint32)
+	lens[:3] = 0, 1, cap
+	q, sk, sv = i8_codes(rng, (n, h * hd)), i8_codes(rng, (h, hd)), i8_codes(rng, (h, hd))
+	one = i8_codes(rng, (2, cap, 2 * h * hd))
+	cache = one[np.arange(n) % 2]
+	temp = (0.5 + rng.random(h)).astype(np.float32)
+	t = lambda a, dtype: X.Tensor.from_numpy(dev, np.ascontiguousarray(a), dtype)
+	out, l = X.Tensor(dev, (n, h * hd), X.BF16 if row_scales else X.INT8), X.Tensor(dev, (n, h), X.F32)
+	args = (t(q, X.INT8), t(cache, X.INT8), t(lens.view(np.float32), X.F32), t(sk, X.INT8), t(sv, X.INT8), t(temp, X.F32), out, l, window)
+	if row_scales:
+		qs, ks, vs = (0.125 * (0.75 + 0.5 * rng.random(s)).astype(np.float32) for s in ((n, h), (n, h, cap), (n, h, cap)))
+		vw, sw, osc = recipes.attn_row_scale_operands(vs, X.BF16)
+		recipes.attn_decode_row_scaled_kernel(dev, h, hd, cap, X.BF16, True).launch_row_scaled(*args, *(t(a, X.F32) for a in (qs, ks, vw, sw, osc)))
+	else:
+		recipes.attn_decode_kernel(dev, h, hd, cap, True).launch(*args)
+	got, got_l = out.download(), l.download()
+	seqs, heads = np.array([0, 1, 2, n - 1]), np.array([0, h - 1])
+	cols = np.concatenate([np.arange(x * hd, (x + 1) * hd) for x in heads])
+	kv_cols = np.concatenate([np.arange(x * 2 * hd, (x + 1) * 2 * hd) for x in heads])
+	sub = (q[seqs][:, cols], cache[seqs][:, :, kv_cols], lens[seqs], sk[heads], sv[heads], temp[heads], len(heads), hd, window)
+	sub = tuple(np.ascontiguousarray(a) if isinstance(a, np.ndarray) else a for a in sub)
+	if row_scales:
+		pick = lambda a: np.ascontiguousarray(a[seqs][:, heads])
+		want, want_l = S.attn_decode_i8_row_scaled(*sub, pick(qs), pick(ks), pick(vw), sw[heads], osc[heads], out_bf16=True)
+	else:
+		want, want_l = S.attn_decode_i8(*sub)
+	assert np.array_equal(got[seqs][:, cols], want)
+	assert np.array_equal(got_l[seqs][:, heads].view(np.uint32), want_l.view(np.uint32))

@@ -743,6 +743,10 @@ static std::string one_line(std::string s) {
 	return s;
 }
 
+// MI355X
+static constexpr size_t COMPUTE_UNITS = 256;
+static constexpr size_t LDS_BYTES = 160 * 1024;
+
 static bool is_pow2(size_t v) { return v != 0 && (v & (v - 1)) == 0; }
 static unsigned ctz(size_t v) { unsigned n = 0; while ((v & 1) == 0) { v >>= 1; ++n; } return n; }
 
@@ -1414,25 +1418,46 @@ std::unique_ptr<AttnDecodeKernel> AttnDecodeKernel::create(std::shared_ptr<HipDe
 	if (config.row_scales) {
 		common << "#define X17_ATTN_ROW_SCALES 1\n#define X17_ATTN_OUT_BF16 " << (config.out_dtype == DType::Bf16 ? 1 : 0) << "\n";
 	}
-	auto built = kernel_build::build(kernel_name, common.str(), "attn_decode_i8.hip", "decode_meta.cpp", diag);
-	if (!built) return nullptr;
-	auto meta = kernel_build::read_metadata_json(built->meta_json_path, diag);
-	if (!meta) return nullptr;
 	auto out = std::make_unique<AttnDecodeKernel>();
-	auto get = [&](char const *k) { auto v = kernel_build::meta_get(*meta, k); return v ? *v : size_t(0); };
-	out->metadata = AttnDecodeMetadata{get("THREADS_PER_BLOCK"), get("SMEM_BYTES"), get("HEADS_PER_BLOCK")};
-	if (out->metadata.THREADS_PER_BLOCK == 0 || out->metadata.HEADS_PER_BLOCK == 0 || config.n_heads % out->metadata.HEADS_PER_BLOCK != 0) {
-		diag.add_error("Invalid JSON metadata in " + built->meta_json_path);
+	// one code object: the default (threads == 0) or one with `threads` per workgroup
+	struct Built { kernel_build::BuiltKernel files; AttnDecodeMetadata metadata; std::unique_ptr<HipKernel> kernel; };
+	auto build_one = [&](size_t threads) -> std::optional<Built> {
+		std::string const suffix = threads == 0 ? "" : "-t" + std::to_string(threads);
+		std::string const define = threads == 0 ? "" : "#define X17_DECODE_THREADS " + std::to_string(threads) + "\n";
+		auto built = kernel_build::build(kernel_name + suffix, common.str() + define, "attn_decode_i8.hip", "decode_meta.cpp", diag);
+		if (!built) return std::nullopt;
+		auto meta = kernel_build::read_metadata_json(built->meta_json_path, diag);
+		if (!meta) return std::nullopt;
+		auto get = [&](char const *k) { auto v = kernel_build::meta_get(*meta, k); return v ? *v : size_t(0); };
+		Built b{*built, AttnDecodeMetadata{get("THREADS_PER_BLOCK"), get("SMEM_BYTES"), get("HEADS_PER_BLOCK")}, nullptr};
+		if (b.metadata.THREADS_PER_BLOCK == 0 || b.metadata.HEADS_PER_BLOCK == 0 || config.n_heads % b.metadata.HEADS_PER_BLOCK != 0) {
+			diag.add_error("Invalid JSON metadata in " + built->meta_json_path);
+			return std::nullopt;
+		}
+		if (device && b.metadata.SMEM_BYTES <= LDS_BYTES) {
+			b.kernel = kernel_build::load_kernel(*device->stream, built->code_object_path, "kernel", b.metadata.SMEM_BYTES, diag);
+			if (!b.kernel) return std::nullopt;
+		}
+		return b;
+	};
+	auto base = build_one(0);
+	if (!base) return nullptr;
+	out->files = base->files;
+	out->metadata = base->metadata;
+	out->kernel = std::move(base->kernel);
+	if (device && !out->kernel) {
+		diag.add_error("decode kernel needs " + std::to_string(out->metadata.SMEM_BYTES) + " bytes of LDS for this cache capacity");
 		return nullptr;
 	}
-	out->name = kernel_name;
-	out->files = *built;
-	out->config = config;
-	if (device) {
-		out->kernel = kernel_build::load_kernel(*device->stream, built->code_object_path, "kernel", out->metadata.SMEM_BYTES, diag);
-		if (!out->kernel) return nullptr;
-		out->device = std::move(device);
+	for (size_t threads : {1024, 512, 256}) {
+		auto b = build_one(threads);
+		if (!b) return nullptr;
+		// (a wide workgroup stages more of the P.V partials: with a long cache it may not fit)
+		if (b->kernel) out->wide.push_back(Wide{b->metadata, std::move(b->kernel)});
 	}
+	out->name = kernel_name;
+	out->config = config;
+	out->device = std::move(device);
 	return out;
 }
 
@@ -1502,9 +1527,28 @@ Status AttnDecodeKernel::launch(AttnDecodeArgs const &a) {
 	// the plain kernel takes the first nine arguments only
 	void *raw_args[14] = {&q_ptr, &cache_ptr, &len_ptr, &sk, &sv, &tp, &out_ptr, &l_ptr, &window_arg,
 	                      &scale_ptrs[0], &scale_ptrs[1], &scale_ptrs[2], &scale_ptrs[3], &scale_ptrs[4]};
-	size_t grid[3] = {config.n_heads / metadata.HEADS_PER_BLOCK, seqs, 1};
-	size_t block[3] = {metadata.THREADS_PER_BLOCK, 1, 1};
-	return kernel->launch(*device->stream, grid, block, metadata.SMEM_BYTES, raw_args);
+	// Threads per workgroup, by the number of workgroups and by the key bytes each may have to stream (the figures behind
+	// the lines are in attn_decode_i8.hip).  At most one workgroup per compute unit: sixteen wavefronts each, unless the
+	// window is so short that a workgroup's set-up outweighs it.  More: a long window streams best from 512 threads; below
+	// that the width that keeps all workgroups resident, two wavefronts for the shortest.
+	size_t const workgroups = seqs * (config.n_heads / metadata.HEADS_PER_BLOCK);
+	size_t const keys = a.window_size == 0 || a.window_size > config.cache_capacity ? config.cache_capacity : a.window_size;
+	size_t const key_bytes = keys * config.head_dim;
+	size_t const threads = workgroups <= COMPUTE_UNITS ? (key_bytes <= 32 * 1024 ? 256 : 1024)
+	                     : key_bytes > 128 * 1024 ? 512
+	                     : workgroups <= 4 * COMPUTE_UNITS || key_bytes > 64 * 1024 ? 256 : 128;
+	AttnDecodeMetadata const *meta = &metadata;
+	HipKernel *chosen = kernel.get();
+	for (Wide const &w : wide) {
+		if (w.metadata.THREADS_PER_BLOCK <= threads) {
+			meta = &w.metadata;
+			chosen = w.kernel.get();
+			break;
+		}
+	}
+	size_t grid[3] = {config.n_heads / meta->HEADS_PER_BLOCK, seqs, 1};
+	size_t block[3] = {meta->THREADS_PER_BLOCK, 1, 1};
+	return chosen->launch(*device->stream, grid, block, meta->SMEM_BYTES, raw_args);
 }
 
 } // namespace x17

@@ -341,6 +341,9 @@ struct AttnDecodeKernel {
 	AttnDecodeMetadata metadata{};
 	std::shared_ptr<HipDevice> device;
 	std::unique_ptr<HipKernel> kernel;
+	// the same kernel with more wavefronts per (sequence, head), widest first; launch() picks by the size of the launch
+	struct Wide { AttnDecodeMetadata metadata; std::unique_ptr<HipKernel> kernel; };
+	std::vector<Wide> wide;
 	static std::unique_ptr<AttnDecodeKernel> create(std::shared_ptr<HipDevice> device, std::string const &kernel_name,
 	                                                 AttnDecodeConfig const &config, bool strict_math, Diagnostics &diag);
 	Status launch(AttnDecodeArgs const &args);

@@ -11,10 +11,13 @@
 //
 // The work is bandwidth: every cached K byte is read exactly once, and so is every V row whose
 // 8-bit probability is not zero (rows with probability 0 contribute nothing and are not fetched).  One workgroup
-// of two wavefronts per (sequence, head), small enough in registers and LDS that eight share a compute unit:
-// all workgroups of 64 sequences x 32 heads are then resident together and the key stream runs without a
-// second, half-empty round.  The recurrence is cut into phases so that only two cheap scans remain
-// sequential:
+// per (sequence, head); its width is chosen at launch (X17_DECODE_THREADS, decode_tile.h) by how many workgroups there
+// are and how many key bytes each streams: few workgroups have to keep enough loads in flight by themselves, many
+// short ones want to be resident together.  Measured at 32 heads of 128 (us, 128 / 256 / 512 / 1024 threads):
+//   1 sequence x 4096 keys   63 / 37 / 23 / 19     8 x 4096   100 / 58 / 37 / 34    1 x 256   9.3 / 8.2 / 7.8 / 8.3
+//   24 x 512                 20 / 15 / 20 / 26    24 x 4096   106 / 82 / 76 / 85
+//   64 x 512                 33 / 33 / 41 / 68    64 x 4096   197 / 187 / 171 / 199
+// The recurrence is cut into phases so that only two cheap scans remain sequential:
 //   1  scores: HD/16 lanes per key row (16-byte coalesced loads), v_dot4 + lane reduction
 //   2  per-tile max, prefix max over tiles (exact), rescale factors, probabilities, quad sums
 //   3  four partial-sum chains (4 lanes)
@@ -89,8 +92,8 @@ void kernel(
 	f32 *s_mrun = reinterpret_cast<f32 *>(smem + dt::TILE_STATE_OFFSET);         // [MAX_TILES] tile max, then running max
 	f32 *s_tmax = s_mrun;
 	f32 *s_resc = s_mrun + dt::MAX_TILES;                                        // [MAX_TILES]
-	f32 *s_bmax = s_resc + dt::MAX_TILES;                                        // [4] one per wavefront
-	f32 *s_sum = s_bmax + 4;                                                     // [4]
+	f32 *s_bmax = s_resc + dt::MAX_TILES;                                        // [MAX_SLOTS] one per wavefront
+	f32 *s_sum = s_bmax + dt::MAX_SLOTS;                                                     // [4]
 	u32 *s_nact = reinterpret_cast<u32 *>(s_sum + 4);                            // [4] (one used)
 	u16 *s_act = reinterpret_cast<u16 *>(s_nact + 4);                            // [MAX_TILES] tiles that move O
 
@@ -132,10 +135,11 @@ void kernel(
 	// ---- phase 1: scores of all keys of the walked tiles.  A thread keeps BATCH independent 16-byte
 	// loads in flight (a load per pass would leave the kernel waiting on memory latency).
 	u32 const n_keys = n_tiles * 16;
-	// Few loads per thread and many resident workgroups: the workgroups of one sequence then walk its rows nearly
-	// in step, which the DRAM pages like (measured: 2 loads in flight per thread beat 1, 4, 8 and 16).
+	// Loads in flight per thread: four, except for the 512-thread workgroups, which long windows of many sequences take
+	// and which stream best with sixteen (64 sequences x 4096 keys: 171 us with 16, 182 with 4, 196 with 2; 24
+	// sequences x 128 keys on 256 threads: 8.3 us with 4, 10.7 with 16).
 #ifndef X17_DECODE_BATCH
-#define X17_DECODE_BATCH 2
+#define X17_DECODE_BATCH (X17_DECODE_THREADS == 512 ? 16 : 4)
 #endif
 	constexpr u32 BATCH = X17_DECODE_BATCH;
 	for (u32 base = 0; base < n_keys; base += KEYS_PER_PASS * BATCH) {
