@@ -2,6 +2,7 @@
 shim: attention grids with groups of heads per workgroup (src/device/cuda/attn.rs:60-66, 413-415: grid.y counts groups of
 128 / head_dim heads) give the bytes of the one-head-per-workgroup launch, forward and backward."""
 import ctypes
+import json
 import os
 
 import numpy as np
@@ -9,18 +10,17 @@ import pytest
 
 import x17ai_amd as X
 from x17ai_amd import _ffi, recipes
-from tests.gpu_common import i8_codes, rng_for
+from tests.gpu_common import e4m3_bytes, e4m3_compare, i8_codes, rng_for
 from tests.test_gpu_shim import P, SZ, _ok, _value, shim  # noqa: F401  (shim is a fixture)
 
 pytestmark = pytest.mark.gpu
 
 
-def _launch_groups(shim, kernel, grid, slots):
-	"""One launch of a built kernel's code object with `grid`, on a stream of its own."""
-	meta = kernel.metadata
+def _launch(shim, directory, meta, grid, slots):
+	"""One launch of a built code object with `grid`, on a stream of its own."""
 	ctx = _value(shim, shim.x17ai_hip_open_context(0))
 	stream = _value(shim, shim.x17ai_hip_open_stream(ctx))
-	module = _value(shim, shim.x17ai_hip_load_module(ctx, os.path.join(_ffi.kernel_cache_dir(), kernel.name, "kernel.hsaco").encode()))
+	module = _value(shim, shim.x17ai_hip_load_module(ctx, os.path.join(directory, "kernel.hsaco").encode()))
 	function = _value(shim, shim.x17ai_hip_get_kernel(module, b"kernel", meta["SMEM_BYTES"]))
 	values = [ctypes.c_uint64(s.device_ptr() if isinstance(s, X.Tensor) else s) for s in slots]
 	args = (P * len(values))(*[ctypes.cast(ctypes.byref(v), P) for v in values])
@@ -29,6 +29,10 @@ def _launch_groups(shim, kernel, grid, slots):
 	_ok(shim, shim.x17ai_hip_del_module(module))
 	_ok(shim, shim.x17ai_hip_close_stream(stream))
 	_ok(shim, shim.x17ai_hip_close_context(ctx))
+
+
+def _launch_groups(shim, kernel, grid, slots):
+	_launch(shim, os.path.join(_ffi.kernel_cache_dir(), kernel.name), kernel.metadata, grid, slots)
 
 
 @pytest.mark.parametrize("h,hd,seq,batch,window", [(4, 32, 192, 2, 48), (2, 64, 256, 1, 0)])
@@ -97,3 +101,83 @@ def test_decode_workgroup_widths(n, window, row_scales):
 		want, want_l = S.attn_decode_i8(*sub)
 	assert np.array_equal(got[seqs][:, cols], want)
 	assert np.array_equal(got_l[seqs][:, heads].view(np.uint32), want_l.view(np.uint32))
+
+
+# (kernel, K, raw columns, result per row, operand types): every writer, each operand mix
+GEMM_FORMS = [
+	("scale", lambda: recipes.attn_q_kernel(None, 512, 384), 512, 384),
+	("geglu", lambda: recipes.ffn_f_kernel(None, 512, 384, True, X.E4M3), 512, 384),
+	("geglu_i8_fast", lambda: recipes.ffn_f_kernel(None, 2048, 1024, False, X.INT8), 2048, 1024),
+	("residual", lambda: recipes.attn_y_kernel(None, 192, 512, True, X.E4M3), 512, 384),
+	("l2norm_32", lambda: recipes.attn_kv_kernel(None, 512, 384, 32), 512, 384),
+	("l2norm_64", lambda: recipes.attn_kv_kernel(None, 512, 384, 64), 512, 384),
+	("l2norm_128", lambda: recipes.attn_kv_kernel(None, 512, 512, 128), 512, 512),
+	("dequant", lambda: recipes.dequant_gemm_kernel(None, 512, 384, X.INT8, X.INT8, False, True), 512, 384),
+	("dequant_geglu", lambda: recipes.dequant_gemm_kernel(None, 512, 384, X.INT8, X.INT8, True, True), 512, 384),
+	("qnorm", lambda: recipes.attn_q_norm_kernel(None, 512, 384, 64, 0.0), 512, 384),
+	("qkv", lambda: recipes.attn_qkv_kernel(None, 512, 256, 384, 64), 512, 640),
+	("mixed", lambda: recipes.mixed_gemm_kernel(None, 512, 384, False), 512, 384),
+	("mixed_residual", lambda: recipes.ffn_y_kernel(None, 128, 512, True, X.E4M3, X.INT8), 512, 256),
+	("e4m3", lambda: recipes.ffn_f_f8_kernel(None, 512, 256, True), 512, 256),
+	("one_step", lambda: recipes.attn_q_kernel(None, 128, 256), 128, 256),
+]
+
+
+@pytest.mark.parametrize("name,make,k,n", GEMM_FORMS, ids=[f[0] for f in GEMM_FORMS])
+@pytest.mark.parametrize("rows", [256, 320, 448])
+def test_every_tile_size_gives_the_same_product(shim, name, make, k, n, rows):  # noqa: F811
+	"""The 64 x 64 and 128 x 128 forms of a GEMM against its 256 x 256 kernel (which the oracle pins): the same bytes for
+	int8 operands; with e4m3 operands the float32 sums are added in another order -- a result may fall on the other side
+	of a rounding boundary of its 8-bit format, in at most 0.5 % of the elements and by one step."""
+	dev = X.Device(0)
+	rng = rng_for("tile sizes", name, rows)
+	e4 = name in ("mixed", "mixed_residual", "e4m3")
+	t = lambda a, dtype: X.Tensor.from_numpy(dev, np.ascontiguousarray(a), dtype)
+	a = t(e4m3_bytes(rng, (rows, k)), X.E4M3) if e4 else t(i8_codes(rng, (rows, k)), X.INT8)
+	weights = lambda r: t(e4m3_bytes(rng, (r, k)), X.E4M3) if name == "e4m3" else t(i8_codes(rng, (r, k)), X.INT8)
+	kernel = make()
+	pairs = "geglu" in name or "residual" in name or name == "e4m3"
+	out_cols, out_type = n // 2 if pairs else n, X.BF16 if "dequant" in name else X.E4M3 if pairs and name != "geglu_i8_fast" else X.INT8
+	residual = t(i8_codes(rng, (rows, out_cols)), X.INT8)
+	scales = t((0.01 + 0.01 * rng.random(rows)).astype(np.float32), X.F32), t((0.01 + 0.01 * rng.random(n)).astype(np.float32), X.F32)
+	learned = t((rng.standard_normal(n).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16), X.BF16)
+	q_cols = 256 if name == "qkv" else n
+	b, b_kv = weights(q_cols), weights(max(n - q_cols, 128))
+	heads = (n - q_cols if name == "qkv" else n) // (2 * int(name.split("_")[1]) if name.startswith("l2norm") else 128)
+	results = {}
+	base = os.path.join(_ffi.kernel_cache_dir(), kernel.name)
+	for form in ("", "-s64x4", "-s128x4", "-s128x2"):
+		if form == "-s64x4" and k % 256 != 0:
+			continue
+		with open(os.path.join(base + form, "meta.json")) as f:
+			meta = json.load(f)
+		c = X.Tensor(dev, (rows, q_cols if name == "qkv" else out_cols), out_type)
+		c_kv, rrms = X.Tensor(dev, (rows, max(n - q_cols, 128)), X.INT8), X.Tensor(dev, (rows, max(heads, 1)), X.F32)
+		outputs = [c]
+		slots = [a, rows, b, n, c]
+		if name.startswith("l2norm"):
+			slots.append(rrms)
+			outputs.append(rrms)
+		elif "residual" in name:
+			slots.append(residual)
+		elif "dequant" in name:
+			slots.extend(scales)
+		elif name == "qnorm":
+			slots.append(learned)
+		elif name == "qkv":
+			slots.extend([rrms, b_kv, c_kv])
+			outputs.extend([rrms, c_kv])
+		dev.synchronize()
+		tiles = -(-rows // meta["M_PER_BLOCK"]) * -(-n // meta["N_PER_BLOCK"])
+		_launch(shim, base + form, meta, (tiles, 1, 1), slots)
+		results[form] = [x.download() for x in outputs]
+	for form, got in results.items():
+		for x, y in zip(got, results[""]):
+			if not e4:
+				assert np.array_equal(x.view(np.uint8), y.view(np.uint8)), (form, name)
+			elif out_type == X.E4M3:
+				differ, beyond = e4m3_compare(x, y)
+				assert differ < 0.005 and beyond == 0.0, (form, name, differ, beyond)
+			else:
+				d = np.abs(x.astype(np.int32) - y.astype(np.int32))
+				assert d.max() <= 1 and np.mean(d != 0) < 0.005, (form, name)

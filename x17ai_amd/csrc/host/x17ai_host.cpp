@@ -909,6 +909,27 @@ std::unique_ptr<GemmKernel> GemmKernel::create(std::shared_ptr<HipDevice> device
 			+ std::to_string(out->metadata.N_PER_BLOCK));
 		return nullptr;
 	}
+	struct SmallForm { size_t tile, stages; };
+	for (SmallForm f : {SmallForm{64, 4}, SmallForm{128, 4}, SmallForm{128, 2}}) {
+		if (g.a.cols % (f.tile == 64 ? 256 : 128) != 0) continue;       // whole K steps (gemm_small_tile.h)
+		std::string const defines = "#define X17_SMALL_TILE " + std::to_string(f.tile) + "\n#define X17_SMALL_STAGES " + std::to_string(f.stages) + "\n";
+		auto small_built = kernel_build::build(kernel_name + "-s" + std::to_string(f.tile) + "x" + std::to_string(f.stages), common.str() + defines,
+		                                       "gemm_b8_small.hip", "gemm_small_meta.cpp", diag);
+		if (!small_built) return nullptr;
+		auto small_meta = kernel_build::read_metadata_json(small_built->meta_json_path, diag);
+		if (!small_meta) return nullptr;
+		auto get_small = [&](char const *k) { auto v = kernel_build::meta_get(*small_meta, k); return v ? *v : size_t(0); };
+		GemmKernel::Small s{f.tile, f.stages, {get_small("THREADS_PER_BLOCK"), get_small("SMEM_BYTES"), get_small("M_PER_BLOCK"), get_small("N_PER_BLOCK"), 0}, nullptr};
+		if (s.metadata.THREADS_PER_BLOCK == 0 || !is_pow2(s.metadata.M_PER_BLOCK) || !is_pow2(s.metadata.N_PER_BLOCK)) {
+			diag.add_error("Invalid JSON metadata in " + small_built->meta_json_path);
+			return nullptr;
+		}
+		if (device) {
+			s.kernel = kernel_build::load_kernel(*device->stream, small_built->code_object_path, "kernel", s.metadata.SMEM_BYTES, diag);
+			if (!s.kernel) return nullptr;
+		}
+		out->small.push_back(std::move(s));
+	}
 	out->name = kernel_name;
 	out->files = *built;
 	out->epilogue_kind = kind;
@@ -997,8 +1018,6 @@ Status GemmKernel::launch(GemmArgs const &args) {
 	if (a_rows > 0xFFFFFFFFull || b_rows_v > 0xFFFFFFFFull) {
 		return Status::err(TensorOpError::Other, std::string(op) + " sizes exceed 32 bits (the kernel's row counts are u32)");
 	}
-	size_t grid_x = (a_rows + metadata.M_PER_BLOCK - 1) >> ctz(metadata.M_PER_BLOCK);
-	size_t grid_y = (b_rows_v + metadata.N_PER_BLOCK - 1) >> ctz(metadata.N_PER_BLOCK);
 	// 8-byte slots passed by address, exactly as gemm.rs:618-631 does; the kernel's u32 parameters
 	// read the low halves.
 	void *a_ptr = args.a->ptr;
@@ -1009,12 +1028,77 @@ Status GemmKernel::launch(GemmArgs const &args) {
 	void *extra_ptr = args.extra != nullptr ? args.extra->ptr : nullptr;
 	void *extra2_ptr = args.extra2 != nullptr ? args.extra2->ptr : nullptr;
 	void *raw_args[7] = {&a_ptr, &a_rows_arg, &b_ptr, &b_rows_arg, &c_ptr, &extra_ptr, &extra2_ptr};
-	size_t grid[3] = {grid_x, grid_y, 1};
-	if (metadata.MAX_BLOCKS != 0 && grid_x * grid_y > metadata.MAX_BLOCKS) {
-		// persistent kernel: the workgroups share the tiles out among themselves
-		grid[0] = metadata.MAX_BLOCKS;
-		grid[1] = 1;
+	return launch_tiles(a_rows, b_rows_v, raw_args);
+}
+
+// ---- which tile size a GEMM launch takes.
+// Estimated microseconds of a launch as rounds of workgroups over the 256 compute units, each round fixed + per_k * K
+// (K in bytes), fitted to launches of 256 .. 4096 token rows on an MI355X (K = 2048 / 8192 int8, 4096 / 16384 e4m3,
+// 8192 e4m3 x int8; us measured at 4096 columns, K = 2048, int8, 256 / 512 / 1024 / 2048 / 4096 rows:
+// 64 x 64 tiles 6.2 / 10.9 / 19.9 / 51 / 103, 128 x 128 four stages 9.9 / 10.3 / 11.3 / 25 / 45, two stages
+// 9.7 / 10.1 / 11.4 / 20 / 39, 256 x 256 23 / 23 / 24 / 26 / 35).  The estimates hold within about 10 %; where two
+// forms are that close either will do.
+namespace gemm_cost {
+	struct Line { double fixed, per_k; double at(double k) const { return fixed + per_k * k; } };
+	struct Rates {
+		Line tile64;                // a round of 64 x 64 tiles, one workgroup per compute unit
+		Line tile128_deep;          // a round of 128 x 128 tiles with four stages, one workgroup per compute unit
+		Line tile128_first;         // 256 of the two-stage 128 x 128 tiles (two workgroups share a compute unit) alone ...
+		Line tile128;               // ... and each 256 of them in a larger launch
+		Line tile256_latency;       // a round of the persistent 256 x 256 kernel: bound by one tile's walk over K ...
+		Line tile256_full;          // ... or, times the round's fill, by the clock the full chip holds
+	};
+	static Rates const RATES[3] = {
+		{{1.6, 1.53e-3}, {2.7, 3.3e-3}, {0.0, 4.75e-3}, {0.6, 4.1e-3}, {9.0, 7.0e-3}, {2.0, 12.8e-3}},       // int8
+		{{1.6, 1.53e-3}, {2.0, 3.8e-3}, {0.0, 4.6e-3}, {0.8, 3.65e-3}, {15.0, 6.6e-3}, {4.0, 10.4e-3}},     // e4m3
+		{{0.0, 2.9e-3}, {0.0, 6.8e-3}, {0.0, 6.4e-3}, {0.0, 7.0e-3}, {4.0, 15.9e-3}, {0.0, 23.0e-3}},      // e4m3 x int8
+	};
+	static constexpr double LAUNCH = 1.5;
+	static double rounds_of(size_t tiles) { return double((tiles + COMPUTE_UNITS - 1) / COMPUTE_UNITS); }
+	static double small(Rates const &r, size_t tile, size_t stages, bool natural, size_t tiles, double k) {
+		double const n = rounds_of(tiles);
+		// the head-normalising writers' wavefronts of 32 x 128 read more per product (64: 32 x 128 tiles load more as well)
+		double const shape = !natural ? 1.0 : tile == 64 ? 1.25 : 1.1;
+		if (tile == 64) return LAUNCH + shape * n * r.tile64.at(k);
+		if (stages == 4) return LAUNCH + shape * n * r.tile128_deep.at(k) * (n > 1.0 ? 1.1 : 1.0);
+		if (n == 1.0) return LAUNCH + shape * r.tile128_first.at(k);
+		// (of two workgroups' worth, the second shortens with its fill)
+		double const fill = n == 2.0 ? 0.73 + 0.27 * (double(tiles) / COMPUTE_UNITS - 1.0) : 1.0;
+		return LAUNCH + shape * n * r.tile128.at(k) * fill;
 	}
+	static double large(Rates const &r, size_t tiles, double k) {
+		double const full = double(tiles / COMPUTE_UNITS), rest = double(tiles % COMPUTE_UNITS) / COMPUTE_UNITS;
+		double us = full * std::max(r.tile256_latency.at(k), r.tile256_full.at(k));
+		// (a last, partly filled round starts with its first tiles already in LDS)
+		if (rest > 0.0) us += std::max(r.tile256_latency.at(k) - (full > 0.0 ? 2.0 : 0.0), rest * r.tile256_full.at(k));
+		return us;
+	}
+}
+
+Status GemmKernel::launch_tiles(size_t a_rows, size_t n_raw, void **raw_args) {
+	auto tiles_of = [&](GemmLauncherMetadata const &m) {
+		return ((a_rows + m.M_PER_BLOCK - 1) >> ctz(m.M_PER_BLOCK)) * ((n_raw + m.N_PER_BLOCK - 1) >> ctz(m.N_PER_BLOCK));
+	};
+	bool const e4m3 = a_dtype == DType::E4m3, e4m3_weights = b_dtype == DType::E4m3;
+	gemm_cost::Rates const &rates = gemm_cost::RATES[e4m3 != e4m3_weights ? 2 : e4m3 ? 1 : 0];
+	bool const natural = epilogue_kind == 3 || epilogue_kind == 5 || epilogue_kind == 6;
+	size_t const tiles = tiles_of(metadata);
+	double best = gemm_cost::large(rates, tiles, double(a_cols));
+	Small const *chosen = nullptr;
+	for (Small const &s : small) {
+		double const us = gemm_cost::small(rates, s.tile, s.stages, natural, tiles_of(s.metadata), double(a_cols));
+		if (us < best) {
+			best = us;
+			chosen = &s;
+		}
+	}
+	if (chosen != nullptr) {
+		size_t grid[3] = {tiles_of(chosen->metadata), 1, 1};
+		size_t block[3] = {chosen->metadata.THREADS_PER_BLOCK, 1, 1};
+		return chosen->kernel->launch(*device->stream, grid, block, chosen->metadata.SMEM_BYTES, raw_args);
+	}
+	// persistent kernel: the workgroups share the tiles out among themselves
+	size_t grid[3] = {metadata.MAX_BLOCKS != 0 && tiles > metadata.MAX_BLOCKS ? metadata.MAX_BLOCKS : tiles, 1, 1};
 	size_t block[3] = {metadata.THREADS_PER_BLOCK, 1, 1};
 	return kernel->launch(*device->stream, grid, block, metadata.SMEM_BYTES, raw_args);
 }
@@ -1056,10 +1140,7 @@ Status GemmKernel::launch_qkv(GemmArgs const &args, size_t a_rows) {
 	void *b2_ptr = args.b2->ptr;
 	void *c2_ptr = args.c2->ptr;
 	void *raw_args[8] = {&a_ptr, &a_rows_arg, &b_ptr, &b_rows_arg, &c_ptr, &rrms_ptr, &b2_ptr, &c2_ptr};
-	size_t tiles = ((a_rows + metadata.M_PER_BLOCK - 1) >> ctz(metadata.M_PER_BLOCK)) * ((*b_rows + metadata.N_PER_BLOCK - 1) >> ctz(metadata.N_PER_BLOCK));
-	size_t grid[3] = {metadata.MAX_BLOCKS != 0 && tiles > metadata.MAX_BLOCKS ? metadata.MAX_BLOCKS : tiles, 1, 1};
-	size_t block[3] = {metadata.THREADS_PER_BLOCK, 1, 1};
-	return kernel->launch(*device->stream, grid, block, metadata.SMEM_BYTES, raw_args);
+	return launch_tiles(a_rows, *b_rows, raw_args);
 }
 
 // ================================================================ attention (src/device/cuda/attn.rs)

@@ -236,6 +236,9 @@ struct GemmKernel {
 	GemmLauncherMetadata metadata{};
 	std::shared_ptr<HipDevice> device;    // null for a build-only kernel
 	std::unique_ptr<HipKernel> kernel;
+	// the same product over small tiles (gemm_b8_small.hip), smallest first: launches with too few 256 x 256 tiles take one
+	struct Small { size_t tile, stages; GemmLauncherMetadata metadata; std::unique_ptr<HipKernel> kernel; };
+	std::vector<Small> small;
 
 	// device == nullptr: generate + compile only (what a build step without a GPU does)
 	static std::unique_ptr<GemmKernel> create(std::shared_ptr<HipDevice> device, std::string const &kernel_name,
@@ -243,6 +246,7 @@ struct GemmKernel {
 	                                           bool strict_math, Diagnostics &diag);
 	Status launch(GemmArgs const &args);
 	Status launch_qkv(GemmArgs const &args, size_t a_rows);   // epilogue_kind 6, reached through launch()
+	Status launch_tiles(size_t a_rows, size_t n_raw, void **raw_args);   // picks the tile size and launches
 	double n_ops(Tensor const &a, Tensor const &b) const;     // 2*M*K*N_raw, gemm.rs:445-449
 };
 

@@ -1,0 +1,210 @@
+// gemm_b8_small.hip -- the GEMM of gemm_b8.hip (same operands, writers and module ABI) over small tiles, for launches
+// whose output has too few 256 x 256 tiles to fill the chip.
+//
+// With 256 token rows a 4096-column product is sixteen 256 x 256 tiles: sixteen of 256 compute units work, each through
+// the whole of K.  Here a workgroup owns 64 x 64 outputs (or 128 x 128: X17_SMALL_TILE) and its wavefronts split K:
+// every wavefront computes the whole 64 x 64 block over its part of each K step, so that the operand fragments it reads
+// from LDS are used as often as in a large tile (16 bytes of fragment per lane and matrix instruction), and the partial
+// sums are exchanged through LDS once at the end, each wavefront finishing and writing a part of the block.
+// What bounds it is the stream of tiles from L2 / HBM into LDS: three K steps of requests are kept in flight per
+// workgroup, one barrier per step.
+// The int32 sums are exact in any order; the float32 sums of e4m3 operands are added as WAVES_K partial sums.
+
+#include "common.h"
+#include "x17_device.h"
+#include "gemm_small_tile.h"
+
+#include <type_traits>
+
+using namespace x17;
+namespace gt = x17::gemm_small_tile;
+namespace {
+// after the exchange a wavefront writes 32-column blocks one at a time; the head-normalising writers need all 128 columns
+constexpr int LANE_COLS = gt::NATURAL ? 64 : 16;
+}
+#include "gemm_parts.h"
+
+namespace {
+
+constexpr u32 K_STEPS = K_TOTAL / gt::K_STEP;
+constexpr u32 X_TILE_BYTES = gt::M_PER_BLOCK * ROW_BYTES;
+constexpr u32 LOADS_PER_STAGE = gt::X_UNITS + gt::W_UNITS;
+constexpr u32 SLICES_PER_WAVE = SLICES / gt::WAVES_K;
+static_assert(SLICES_PER_WAVE * gt::WAVES_K == SLICES, "K steps divide evenly over the wavefronts that share a block");
+static_assert(N_RAW % gt::N_PER_BLOCK == 0, "raw output columns are whole tiles");
+
+// the exchange: blocks of 32 x 32 outputs, 16 registers per lane; block j belongs to wavefront owner(j) of the WAVES_K
+constexpr int BLOCKS = BN * BM;
+constexpr u32 BLOCK_BYTES = 64 * 64;
+constexpr u32 owner(int j) { return gt::NATURAL ? 0 : (u32)j * gt::WAVES_K / BLOCKS; }
+// where wavefront `from` leaves its sums of block j, which it does not own
+constexpr u32 GROUP_BYTES = BLOCKS * (gt::WAVES_K - 1) * BLOCK_BYTES;
+X17_DEV u32 exchange_offset(int j, u32 from) { return (j * (gt::WAVES_K - 1) + (from < owner(j) ? from : from - 1)) * BLOCK_BYTES; }
+static_assert(gt::WAVES / gt::WAVES_K * GROUP_BYTES <= gt::SMEM_BYTES, "the exchange fits the ring");
+
+} // namespace
+
+extern "C" __global__ __launch_bounds__(gt::THREADS_PER_BLOCK)
+__attribute__((amdgpu_waves_per_eu(gt::WAVES_PER_SIMD)))
+void kernel(
+	u8 const *a, u32 a_rows,
+	u8 const *b, u32 b_rows,
+	u8 *c
+#if X17_EPILOGUE == 3
+	, f32 *rrms
+#elif X17_EPILOGUE == 2
+	, i8 const *residual
+#elif X17_EPILOGUE == 4
+	, f32 const *row_scale, f32 const *col_scale
+#elif X17_EPILOGUE == 5
+	, u16 const *q_norm_scales
+#elif X17_EPILOGUE == 6
+	, f32 *rrms, u8 const *b_kv, u8 *c_kv
+#endif
+) {
+	extern __shared__ __attribute__((aligned(1024))) u8 smem[];
+	(void)b_rows;
+
+	u32 const tiles = ((a_rows + gt::M_PER_BLOCK - 1) / gt::M_PER_BLOCK) * (N_RAW / gt::N_PER_BLOCK);
+	u32 const group = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+	if (group >= tiles) return;
+	gt::TileOrigin const tile = gt::tile_origin(group, a_rows, N_RAW);
+
+	u32 const tid = threadIdx.x;
+	u32 const lane = tid % 64;
+	u32 const wave = __builtin_amdgcn_readfirstlane(tid / 64);
+	u32 const half = lane / 32;
+	u32 const wk = wave % gt::WAVES_K;
+	u32 const wn = (wave / gt::WAVES_K) % gt::WAVES_N;
+	u32 const wm = wave / (gt::WAVES_K * gt::WAVES_N);
+
+	u8 const *a_tile = a + (size_t)tile.m * K_TOTAL;
+#if X17_EPILOGUE == 6
+	static_assert(X17_Q_COLS % gt::N_PER_BLOCK == 0, "the q part is whole tiles");
+	u8 const *b_tile = tile.n < X17_Q_COLS ? b + (size_t)tile.n * K_TOTAL : b_kv + (size_t)(tile.n - X17_Q_COLS) * K_TOTAL;
+#else
+	u8 const *b_tile = b + (size_t)tile.n * K_TOTAL;
+#endif
+
+	// ---- requests: this wavefront's units of the token tile and of the weight tile
+	u32 x_src[gt::X_UNITS], w_src[gt::W_UNITS];
+	X17_UNROLL for (u32 u = 0; u < gt::X_UNITS; ++u) {
+		u32 const unit = wave * gt::X_UNITS + u;
+		x_src[u] = gt::unit_row(unit, lane) * K_TOTAL + 16 * gt::unit_chunk(unit, lane);
+	}
+	X17_UNROLL for (u32 u = 0; u < gt::W_UNITS; ++u) {
+		u32 const unit = wave * gt::W_UNITS + u;
+		w_src[u] = gt::w_source_row(gt::unit_row(unit, lane)) * K_TOTAL + 16 * gt::unit_chunk(unit, lane);
+	}
+	u8 *const x_dst = smem + wave * gt::X_UNITS * 1024;
+	u8 *const w_dst = smem + X_TILE_BYTES + wave * gt::W_UNITS * 1024;
+	// past the end the last step is requested again, into a slot nobody reads any more: the waits stay constant
+	auto request = [&](u32 step, u32 slot) __attribute__((always_inline)) {
+		u32 const k0 = (step < K_STEPS ? step : K_STEPS - 1) * gt::K_STEP;
+		X17_UNROLL for (u32 u = 0; u < gt::X_UNITS; ++u) load_to_lds_16(x_dst + slot * gt::STAGE_BYTES + u * 1024, a_tile + k0, x_src[u]);
+		X17_UNROLL for (u32 u = 0; u < gt::W_UNITS; ++u) load_to_lds_16(w_dst + slot * gt::STAGE_BYTES + u * 1024, b_tile + k0, w_src[u]);
+	};
+	X17_UNROLL for (u32 s = 0; s + 1 < gt::STAGES; ++s) request(s, s);
+
+	Acc acc[BN][BM];
+	X17_UNROLL for (int bn = 0; bn < BN; ++bn) {
+		X17_UNROLL for (int bm = 0; bm < BM; ++bm) {
+			X17_UNROLL for (int r = 0; r < 16; ++r) acc[bn][bm][r] = 0;
+		}
+	}
+	u32 const swz = gt::swizzle(lane % 32);
+	u32 const x_off = (wm * gt::WAVE_M + lane % 32) * ROW_BYTES;
+	u32 const w_off = X_TILE_BYTES + (wn * gt::WAVE_N + lane % 32) * ROW_BYTES;
+
+	u32 slot = 0;
+	for (u32 ks = 0; ks < K_STEPS; ++ks) {
+		// this wavefront's requests of step ks have landed and its reads of step ks - 1 are done; behind the barrier so
+		// are everybody's, and the slot of step ks - 1 takes the requests of step ks + STAGES - 1
+		wait_vmcnt<(gt::STAGES - 2) * LOADS_PER_STAGE>();
+		__builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0)
+		__builtin_amdgcn_s_barrier();
+		request(ks + gt::STAGES - 1, slot == 0 ? gt::STAGES - 1 : slot - 1);
+		u8 const *stage = smem + slot * gt::STAGE_BYTES;
+		Frags frags[SLICES_PER_WAVE];
+		X17_UNROLL for (u32 s = 0; s < SLICES_PER_WAVE; ++s) {
+			load_frags(frags[s], stage + w_off, stage + x_off, wk * SLICES_PER_WAVE + s, half, swz);
+		}
+		X17_UNROLL for (u32 s = 0; s < SLICES_PER_WAVE; ++s) mma_slice(frags[s], acc);
+		slot = slot + 1 == gt::STAGES ? 0 : slot + 1;
+	}
+
+	// ---- the wavefronts that share a block add up their partial sums: each writes the blocks it does not own, the
+	// owner reads them back.  (The last requests write the ring too: they must have landed, everywhere.)
+	wait_vmcnt<0>();
+	__builtin_amdgcn_s_waitcnt(0xC07F);
+	__builtin_amdgcn_s_barrier();
+	u8 *const exchange = smem + (wave / gt::WAVES_K) * GROUP_BYTES + lane * 16;
+	X17_UNROLL for (int j = 0; j < BLOCKS; ++j) {
+		if (owner(j) != wk) {
+			v16i const v = __builtin_bit_cast(v16i, acc[j / BM][j % BM]);
+			X17_UNROLL for (int q = 0; q < 4; ++q) {
+				*reinterpret_cast<v4i *>(exchange + exchange_offset(j, wk) + q * 1024) = v4i{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+			}
+		}
+	}
+	__syncthreads();
+
+	u32 const row0 = tile.m + wm * gt::WAVE_M + lane % 32;
+	u32 const col0 = tile.n + wn * gt::WAVE_N;                 // the wavefront's first raw column
+	using Sum = __attribute__((ext_vector_type(16))) std::conditional_t<ACC_F32, float, int>;
+	using Part = __attribute__((ext_vector_type(4))) std::conditional_t<ACC_F32, float, int>;
+	auto total_of = [&](int j, f32 (&x)[16]) __attribute__((always_inline)) {
+		Sum sum = __builtin_bit_cast(Sum, acc[j / BM][j % BM]);
+		X17_UNROLL for (u32 other = 0; other < gt::WAVES_K; ++other) {
+			if (other != owner(j)) {
+				X17_UNROLL for (int q = 0; q < 4; ++q) {
+					Part const part = *reinterpret_cast<Part const *>(exchange + exchange_offset(j, other) + q * 1024);
+					X17_UNROLL for (int i = 0; i < 4; ++i) sum[4 * q + i] = sum[4 * q + i] + part[i];
+				}
+			}
+		}
+		X17_UNROLL for (int r = 0; r < 16; ++r) x[r] = f32(sum[r]);
+	};
+	if constexpr (gt::NATURAL) {
+		static_assert(!gt::NATURAL || BM == 1, "a wavefront of the head-normalising writers has 32 tokens");
+		if (wk == 0) {
+			f32 x[64];
+			X17_UNROLL for (int bn = 0; bn < BN; ++bn) {
+				f32 part[16];
+				total_of(bn, part);
+				X17_UNROLL for (int r = 0; r < 16; ++r) x[16 * bn + r] = part[r];
+			}
+#if X17_EPILOGUE == 3
+			NaturalWriters::l2norm_row(x, c, rrms, row0, col0, N_RAW, half);
+#elif X17_EPILOGUE == 5
+			NaturalWriters::qnorm_row(x, c, q_norm_scales, row0, col0, half);
+#elif X17_EPILOGUE == 6
+			constexpr u32 Q_COLS = X17_Q_COLS;
+			if (col0 < Q_COLS) {
+				NaturalWriters::scale_row(x, c, row0, col0, Q_COLS, half);
+			} else {
+				NaturalWriters::l2norm_row(x, c_kv, rrms, row0, col0 - Q_COLS, N_RAW - Q_COLS, half);
+			}
+#endif
+		}
+	} else {
+		X17_UNROLL for (int j = 0; j < BLOCKS; ++j) {
+			if (owner(j) == wk) {
+				f32 x[16];
+				total_of(j, x);
+				u32 const row = row0 + 32 * (j % BM);
+				// a lane of a 64-column wavefront holds 32 consecutive columns, 16 per block
+				u32 const n = col0 + (gt::WAVE_N / 2) * half + 16 * (j / BM);
+#if X17_EPILOGUE == 0
+				ScaleEpilogue::run(x, c, row, n, nullptr);
+#elif X17_EPILOGUE == 1
+				GeGluEpilogue::run(x, c, row, n, nullptr);
+#elif X17_EPILOGUE == 2
+				ResidualEpilogue::run(x, c, row, n, residual);
+#elif X17_EPILOGUE == 4
+				DequantEpilogue::run(x, c, row, n, row_scale, col_scale);
+#endif
+			}
+		}
+	}
+}

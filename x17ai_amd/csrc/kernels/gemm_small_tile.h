@@ -1,0 +1,66 @@
+// gemm_small_tile.h -- tile geometry and request index arithmetic of the small-tile GEMM kernel (gemm_b8_small.hip) as
+// plain constexprs, shared with the host program that prints its meta.json.  Needs X17_A_COLS, X17_A_KIND, X17_B_KIND,
+// X17_EPILOGUE, X17_SMALL_TILE and X17_SMALL_STAGES from common.h:
+//   X17_SMALL_TILE 64   64 x 64 raw columns per workgroup, K split over its four wavefronts
+//   X17_SMALL_TILE 128  128 x 128, eight wavefronts, K split in two
+//   X17_SMALL_STAGES    depth of the LDS ring of K steps: 2 (of 128 x 128, two workgroups share a compute unit) or 4
+// The writers that normalise heads of up to 128 columns need a wavefront that owns 128 of them: with those the
+// wavefront is 32 tokens x 128 columns instead of 64 x 64, the workgroup 32 x 128 or 128 x 128.
+#pragma once
+
+namespace x17 { namespace gemm_small_tile {
+
+constexpr bool NATURAL = X17_EPILOGUE == 3 || X17_EPILOGUE == 5 || X17_EPILOGUE == 6;   // weight rows in their natural order
+constexpr bool MID = X17_SMALL_TILE == 128;
+static_assert(X17_SMALL_TILE == 64 || X17_SMALL_TILE == 128, "tiles of 64 or of 128");
+
+constexpr unsigned WAVE_M = NATURAL ? 32 : 64;              // tokens per wavefront
+constexpr unsigned WAVE_N = NATURAL ? 128 : 64;             // raw output columns per wavefront
+constexpr unsigned WAVES_M = MID ? 128 / WAVE_M : 1;
+constexpr unsigned WAVES_N = MID ? 128 / WAVE_N : 1;
+constexpr unsigned WAVES_K = MID ? 2 : 4;   // wavefronts that share an output block, each a part of every K step
+constexpr unsigned WAVES = WAVES_M * WAVES_N * WAVES_K;
+constexpr unsigned THREADS_PER_BLOCK = 64 * WAVES;
+constexpr unsigned M_PER_BLOCK = WAVE_M * WAVES_M;
+constexpr unsigned N_PER_BLOCK = WAVE_N * WAVES_N;
+
+// bytes of K per pipeline step: four e4m3 slices of 64 need 256
+constexpr unsigned K_STEP = MID ? 128 : 256;
+constexpr unsigned STAGES = X17_SMALL_STAGES;               // LDS ring depth
+constexpr unsigned STAGE_BYTES = (M_PER_BLOCK + N_PER_BLOCK) * K_STEP;
+constexpr unsigned SMEM_BYTES = STAGES * STAGE_BYTES;
+constexpr unsigned WAVES_PER_SIMD = 160 * 1024 / SMEM_BYTES * WAVES / 4;      // as many workgroups as the LDS holds
+static_assert(X17_A_COLS % K_STEP == 0, "K must be whole steps");
+static_assert(SMEM_BYTES <= 160 * 1024, "LDS ring does not fit");
+
+// ---- requests (global -> LDS, 16 bytes per lane).  An LDS row is K_STEP bytes = CHUNKS chunks of 16; a 64-lane request
+// fills UNIT_ROWS rows; chunk c of row r is stored at position c ^ swizzle(r), so that the sixteen consecutive rows a
+// ds_read_b128 serves at a time land in sixteen different 16-byte columns of the 256-byte bank line.
+constexpr unsigned CHUNKS = K_STEP / 16;
+constexpr unsigned UNIT_ROWS = 64 / CHUNKS;
+constexpr unsigned X_UNITS = M_PER_BLOCK / UNIT_ROWS / WAVES;       // requests per wavefront and step
+constexpr unsigned W_UNITS = N_PER_BLOCK / UNIT_ROWS / WAVES;
+static_assert(X_UNITS * UNIT_ROWS * WAVES == M_PER_BLOCK && W_UNITS * UNIT_ROWS * WAVES == N_PER_BLOCK, "whole requests");
+constexpr unsigned swizzle(unsigned row) { return (K_STEP == 256 ? row : row >> 1) & (CHUNKS - 1); }
+constexpr unsigned unit_row(unsigned unit, unsigned lane) { return unit * UNIT_ROWS + lane / CHUNKS; }            // LDS row
+constexpr unsigned unit_chunk(unsigned unit, unsigned lane) { return (lane % CHUNKS) ^ swizzle(unit_row(unit, lane)); }
+// The weight row LDS weight row r holds (gemm_tile.h: a lane then collects consecutive output columns)
+constexpr unsigned w_source_row(unsigned r) {
+	unsigned const i = r % 32, bn = (r % WAVE_N) / 32;
+	return NATURAL ? r : WAVE_N * (r / WAVE_N) + (WAVE_N / 2) * ((i / 4) % 2) + 16 * bn + 4 * (i / 8) + i % 4;
+}
+// First token row and raw column of workgroup `lin`: each XCD (workgroups are dealt round-robin to 8 of them) gets a
+// contiguous run of tiles, column tiles slowest inside bands of BAND token tiles, so that an XCD reads its weight
+// columns once.  A last token tile that would overhang is moved back to end at the matrix edge.
+struct TileOrigin { unsigned m, n; };
+constexpr unsigned BAND = 2048 / M_PER_BLOCK;
+constexpr TileOrigin tile_origin(unsigned lin, unsigned a_rows, unsigned n_raw) {
+	unsigned const tiles_m = (a_rows + M_PER_BLOCK - 1) / M_PER_BLOCK, tiles_n = n_raw / N_PER_BLOCK, total = tiles_m * tiles_n;
+	if (total % 8 == 0) lin = (lin % 8) * (total / 8) + lin / 8;
+	unsigned const band_tiles = BAND * tiles_n, b = lin / band_tiles, in_band = lin % band_tiles;
+	unsigned const rows_in_band = tiles_m - b * BAND < BAND ? tiles_m - b * BAND : BAND;
+	unsigned const m = (b * BAND + in_band % rows_in_band) * M_PER_BLOCK;
+	return TileOrigin{m + M_PER_BLOCK > a_rows ? a_rows - M_PER_BLOCK : m, (in_band / rows_in_band) * N_PER_BLOCK};
+}
+
+}} // namespace x17::gemm_small_tile
