@@ -3,6 +3,7 @@
 // (include/x17ai_host.h).
 
 #include "x17ai_host.hpp"
+#include <atomic>
 #include <filesystem>
 #include "../../../include/x17ai_host.h"
 
@@ -494,8 +495,14 @@ namespace kernel_build {
 		return true;
 	}
 
+	// No two builds share a temporary file: threads of one process may build the same kernel at once.
+	static std::string unique_suffix() {
+		static std::atomic<unsigned> count{0};
+		return "." + std::to_string(getpid()) + "." + std::to_string(count++);
+	}
+
 	static bool write_file(std::string const &path, std::string const &text, Diagnostics &diag) {
-		std::string tmp = path + ".tmp." + std::to_string(getpid());
+		std::string tmp = path + ".tmp" + unique_suffix();
 		{
 			std::ofstream f(tmp, std::ios::binary | std::ios::trunc);
 			if (!f) { diag.add_error("failed to write generated file " + path); return false; }
@@ -627,7 +634,7 @@ namespace kernel_build {
 		char const *hipcc_env = std::getenv("X17AI_HIPCC");
 		std::string hipcc = hipcc_env != nullptr ? hipcc_env : "/opt/rocm/bin/hipcc";
 		std::string log;
-		std::string tmp_obj = out.code_object_path + ".tmp." + std::to_string(getpid());
+		std::string tmp_obj = out.code_object_path + ".tmp" + unique_suffix();
 		std::string cmd = shell_quote(hipcc) + " " + device_flags() + " --genco -I" + shell_quote(out.dir_path) + " -I" + shell_quote(kdir)
 			+ " " + shell_quote(kdir + "/" + source_file) + " -o " + shell_quote(tmp_obj);
 		int rc = run_command(cmd, log);
@@ -642,7 +649,7 @@ namespace kernel_build {
 		}
 
 		// kernel_build.rs:88-134 -- a host program prints the launch geometry the C++ constants imply
-		std::string meta_exe = out.dir_path + "/meta." + std::to_string(getpid());
+		std::string meta_exe = out.dir_path + "/meta" + unique_suffix();
 		cmd = "g++ -std=c++17 -O0 -I" + shell_quote(out.dir_path) + " -I" + shell_quote(kdir) + " "
 			+ shell_quote(kdir + "/" + meta_source_file) + " -o " + shell_quote(meta_exe);
 		rc = run_command(cmd, log);

@@ -202,7 +202,7 @@ def build_host_libraries() -> None:
 
 def build_all(workers: int = 8) -> list:
 	build_host_libraries()
-	specs = _specs()
+	specs = list(dict.fromkeys(_specs()))
 	names = []
 	with concurrent.futures.ThreadPoolExecutor(max_workers=workers) as pool:
 		for name in pool.map(_build_one, specs):
