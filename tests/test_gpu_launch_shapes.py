@@ -146,10 +146,10 @@ def test_every_tile_size_gives_the_same_product(shim, name, make, k, n, rows):  
 	heads = (n - q_cols if name == "qkv" else n) // (2 * int(name.split("_")[1]) if name.startswith("l2norm") else 128)
 	results = {}
 	base = os.path.join(_ffi.kernel_cache_dir(), kernel.name)
-	for form in ("", "-s64x4", "-s128x4", "-s128x2"):
-		if form == "-s64x4" and k % 256 != 0:
+	for form in ("", "s64x4", "s128x4", "s128x2"):
+		if form == "s64x4" and k % 256 != 0:
 			continue
-		with open(os.path.join(base + form, "meta.json")) as f:
+		with open(os.path.join(base, form, "meta.json")) as f:
 			meta = json.load(f)
 		c = X.Tensor(dev, (rows, q_cols if name == "qkv" else out_cols), out_type)
 		c_kv, rrms = X.Tensor(dev, (rows, max(n - q_cols, 128)), X.INT8), X.Tensor(dev, (rows, max(heads, 1)), X.F32)
@@ -169,7 +169,7 @@ def test_every_tile_size_gives_the_same_product(shim, name, make, k, n, rows):  
 			outputs.extend([rrms, c_kv])
 		dev.synchronize()
 		tiles = -(-rows // meta["M_PER_BLOCK"]) * -(-n // meta["N_PER_BLOCK"])
-		_launch(shim, base + form, meta, (tiles, 1, 1), slots)
+		_launch(shim, os.path.join(base, form), meta, (tiles, 1, 1), slots)
 		results[form] = [x.download() for x in outputs]
 	for form, got in results.items():
 		for x, y in zip(got, results[""]):

@@ -565,7 +565,7 @@ namespace kernel_build {
 
 	std::optional<BuiltKernel> build(std::string const &kernel_name, std::string const &common_text,
 	                                 std::string const &source_file, std::string const &meta_source_file,
-	                                 Diagnostics &diag) {
+	                                 Diagnostics &diag, std::string const &form) {
 		// gemm.rs:377-387 -- the name becomes a directory name
 		if (kernel_name.empty() || kernel_name == "." || kernel_name == ".."
 			|| kernel_name.find('/') != std::string::npos || kernel_name.find('\\') != std::string::npos) {
@@ -574,7 +574,8 @@ namespace kernel_build {
 		}
 		std::string kdir = kernels_dir();
 		BuiltKernel out;
-		out.dir_path = cache_dir() + "/" + kernel_name;
+		// (further forms of a kernel live inside its directory: one cache entry per kernel)
+		out.dir_path = cache_dir() + "/" + kernel_name + (form.empty() ? "" : "/" + form);
 		out.common_path = out.dir_path + "/common.h";
 		out.code_object_path = out.dir_path + "/kernel.hsaco";
 		out.meta_json_path = out.dir_path + "/meta.json";
@@ -920,8 +921,8 @@ std::unique_ptr<GemmKernel> GemmKernel::create(std::shared_ptr<HipDevice> device
 	for (SmallForm f : {SmallForm{64, 4}, SmallForm{128, 4}, SmallForm{128, 2}}) {
 		if (g.a.cols % (f.tile == 64 ? 256 : 128) != 0) continue;       // whole K steps (gemm_small_tile.h)
 		std::string const defines = "#define X17_SMALL_TILE " + std::to_string(f.tile) + "\n#define X17_SMALL_STAGES " + std::to_string(f.stages) + "\n";
-		auto small_built = kernel_build::build(kernel_name + "-s" + std::to_string(f.tile) + "x" + std::to_string(f.stages), common.str() + defines,
-		                                       "gemm_b8_small.hip", "gemm_small_meta.cpp", diag);
+		auto small_built = kernel_build::build(kernel_name, common.str() + defines, "gemm_b8_small.hip", "gemm_small_meta.cpp", diag,
+		                                       "s" + std::to_string(f.tile) + "x" + std::to_string(f.stages));
 		if (!small_built) return nullptr;
 		auto small_meta = kernel_build::read_metadata_json(small_built->meta_json_path, diag);
 		if (!small_meta) return nullptr;
@@ -1510,9 +1511,9 @@ std::unique_ptr<AttnDecodeKernel> AttnDecodeKernel::create(std::shared_ptr<HipDe
 	// one code object: the default (threads == 0) or one with `threads` per workgroup
 	struct Built { kernel_build::BuiltKernel files; AttnDecodeMetadata metadata; std::unique_ptr<HipKernel> kernel; };
 	auto build_one = [&](size_t threads) -> std::optional<Built> {
-		std::string const suffix = threads == 0 ? "" : "-t" + std::to_string(threads);
+		std::string const form = threads == 0 ? "" : "t" + std::to_string(threads);
 		std::string const define = threads == 0 ? "" : "#define X17_DECODE_THREADS " + std::to_string(threads) + "\n";
-		auto built = kernel_build::build(kernel_name + suffix, common.str() + define, "attn_decode_i8.hip", "decode_meta.cpp", diag);
+		auto built = kernel_build::build(kernel_name, common.str() + define, "attn_decode_i8.hip", "decode_meta.cpp", diag, form);
 		if (!built) return std::nullopt;
 		auto meta = kernel_build::read_metadata_json(built->meta_json_path, diag);
 		if (!meta) return std::nullopt;

@@ -176,10 +176,11 @@ namespace kernel_build {
 		bool cache_hit = false;
 	};
 	// Renders common.h, compiles <source> (a file of csrc/kernels) for gfx950 and runs the meta
-	// program, unless an identical build is already cached under <cache>/<name>/.
+	// program, unless an identical build is already cached under <cache>/<name>/, or
+	// <cache>/<name>/<form>/ for a further form of the same kernel.
 	std::optional<BuiltKernel> build(std::string const &kernel_name, std::string const &common_text,
 	                                 std::string const &source_file, std::string const &meta_source_file,
-	                                 Diagnostics &diag);
+	                                 Diagnostics &diag, std::string const &form = "");
 	std::optional<std::vector<std::pair<std::string, size_t>>> read_metadata_json(std::string const &path, Diagnostics &diag);
 	std::string kernels_dir();
 	std::string cache_dir();
