@@ -2,19 +2,19 @@
 // whose output has too few 256 x 256 tiles to fill the chip.
 //
 // With 256 token rows a 4096-column product is sixteen 256 x 256 tiles: sixteen of 256 compute units work, each through
-// the whole of K.  Here a workgroup owns 64 x 64 outputs (or 128 x 128: X17_SMALL_TILE) and its wavefronts split K:
-// every wavefront computes the whole 64 x 64 block over its part of each K step, so that the operand fragments it reads
-// from LDS are used as often as in a large tile (16 bytes of fragment per lane and matrix instruction), and the partial
-// sums are exchanged through LDS once at the end, each wavefront finishing and writing a part of the block.
-// What bounds it is the stream of tiles from L2 / HBM into LDS: three K steps of requests are kept in flight per
-// workgroup, one barrier per step.
-// The int32 sums are exact in any order; the float32 sums of e4m3 operands are added as WAVES_K partial sums.
+// the whole of K.  Here a workgroup owns 64 x 64 outputs (or 128 x 128: X17_SMALL_TILE).  With int8 operands its
+// wavefronts split K: every wavefront computes the whole 64 x 64 block over its part of each K step, so that the operand
+// fragments it reads from LDS are used as often as in a large tile (16 bytes of fragment per lane and matrix
+// instruction), and the partial sums are exchanged through LDS once at the end, each wavefront finishing and writing a
+// part of the block.  Sums of e4m3 operands are float32 and depend on their order: there a wavefront walks all of K for
+// a block of its own (32 x 32 of the 64 x 64, 64 x 64 of the 128 x 128), in the 256 x 256 kernel's order, and every form
+// gives that kernel's bytes.
+// What bounds it is the stream of tiles from L2 / HBM into LDS: X17_SMALL_STAGES - 1 K steps of requests are kept in
+// flight per workgroup, one barrier per step.
 
 #include "common.h"
 #include "x17_device.h"
 #include "gemm_small_tile.h"
-
-#include <type_traits>
 
 using namespace x17;
 namespace gt = x17::gemm_small_tile;
@@ -136,34 +136,39 @@ void kernel(
 	// ---- the wavefronts that share a block add up their partial sums: each writes the blocks it does not own, the
 	// owner reads them back.  (The last requests write the ring too: they must have landed, everywhere.)
 	wait_vmcnt<0>();
-	__builtin_amdgcn_s_waitcnt(0xC07F);
-	__builtin_amdgcn_s_barrier();
 	u8 *const exchange = smem + (wave / gt::WAVES_K) * GROUP_BYTES + lane * 16;
-	X17_UNROLL for (int j = 0; j < BLOCKS; ++j) {
-		if (owner(j) != wk) {
-			v16i const v = __builtin_bit_cast(v16i, acc[j / BM][j % BM]);
-			X17_UNROLL for (int q = 0; q < 4; ++q) {
-				*reinterpret_cast<v4i *>(exchange + exchange_offset(j, wk) + q * 1024) = v4i{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
-			}
-		}
-	}
-	__syncthreads();
-
-	u32 const row0 = tile.m + wm * gt::WAVE_M + lane % 32;
-	u32 const col0 = tile.n + wn * gt::WAVE_N;                 // the wavefront's first raw column
-	using Sum = __attribute__((ext_vector_type(16))) std::conditional_t<ACC_F32, float, int>;
-	using Part = __attribute__((ext_vector_type(4))) std::conditional_t<ACC_F32, float, int>;
-	auto total_of = [&](int j, f32 (&x)[16]) __attribute__((always_inline)) {
-		Sum sum = __builtin_bit_cast(Sum, acc[j / BM][j % BM]);
-		X17_UNROLL for (u32 other = 0; other < gt::WAVES_K; ++other) {
-			if (other != owner(j)) {
+	if constexpr (gt::WAVES_K > 1) {
+		__builtin_amdgcn_s_waitcnt(0xC07F);
+		__builtin_amdgcn_s_barrier();
+		X17_UNROLL for (int j = 0; j < BLOCKS; ++j) {
+			if (owner(j) != wk) {
 				X17_UNROLL for (int q = 0; q < 4; ++q) {
-					Part const part = *reinterpret_cast<Part const *>(exchange + exchange_offset(j, other) + q * 1024);
-					X17_UNROLL for (int i = 0; i < 4; ++i) sum[4 * q + i] = sum[4 * q + i] + part[i];
+					Acc const v = acc[j / BM][j % BM];
+					*reinterpret_cast<v4i *>(exchange + exchange_offset(j, wk) + q * 1024) = v4i{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
 				}
 			}
 		}
-		X17_UNROLL for (int r = 0; r < 16; ++r) x[r] = f32(sum[r]);
+		__syncthreads();
+	}
+
+	u32 const row0 = tile.m + wm * gt::WAVE_M + lane % 32;
+	u32 const col0 = tile.n + wn * gt::WAVE_N;                 // the wavefront's first raw column
+	auto total_of = [&](int j, f32 (&x)[16]) __attribute__((always_inline)) {
+		if constexpr (ACC_F32) {
+			v16f const sum = __builtin_bit_cast(v16f, acc[j / BM][j % BM]);
+			X17_UNROLL for (int r = 0; r < 16; ++r) x[r] = sum[r];
+		} else {
+			Acc sum = acc[j / BM][j % BM];
+			X17_UNROLL for (u32 other = 0; other < gt::WAVES_K; ++other) {
+				if (other != owner(j)) {
+					X17_UNROLL for (int q = 0; q < 4; ++q) {
+						v4i const part = *reinterpret_cast<v4i const *>(exchange + exchange_offset(j, other) + q * 1024);
+						X17_UNROLL for (int i = 0; i < 4; ++i) sum[4 * q + i] = sum[4 * q + i] + part[i];
+					}
+				}
+			}
+			X17_UNROLL for (int r = 0; r < 16; ++r) x[r] = f32(sum[r]);
+		}
 	};
 	if constexpr (gt::NATURAL) {
 		static_assert(!gt::NATURAL || BM == 1, "a wavefront of the head-normalising writers has 32 tokens");

@@ -1,8 +1,8 @@
 // gemm_small_tile.h -- tile geometry and request index arithmetic of the small-tile GEMM kernel (gemm_b8_small.hip) as
 // plain constexprs, shared with the host program that prints its meta.json.  Needs X17_A_COLS, X17_A_KIND, X17_B_KIND,
 // X17_EPILOGUE, X17_SMALL_TILE and X17_SMALL_STAGES from common.h:
-//   X17_SMALL_TILE 64   64 x 64 raw columns per workgroup, K split over its four wavefronts
-//   X17_SMALL_TILE 128  128 x 128, eight wavefronts, K split in two
+//   X17_SMALL_TILE 64   64 x 64 raw columns per workgroup, four wavefronts
+//   X17_SMALL_TILE 128  128 x 128, eight wavefronts (e4m3 x int8: four)
 //   X17_SMALL_STAGES    depth of the LDS ring of K steps: 2 (of 128 x 128, two workgroups share a compute unit) or 4
 // The writers that normalise heads of up to 128 columns need a wavefront that owns 128 of them: with those the
 // wavefront is 32 tokens x 128 columns instead of 64 x 64, the workgroup 32 x 128 or 128 x 128.
@@ -14,11 +14,19 @@ constexpr bool NATURAL = X17_EPILOGUE == 3 || X17_EPILOGUE == 5 || X17_EPILOGUE 
 constexpr bool MID = X17_SMALL_TILE == 128;
 static_assert(X17_SMALL_TILE == 64 || X17_SMALL_TILE == 128, "tiles of 64 or of 128");
 
-constexpr unsigned WAVE_M = NATURAL ? 32 : 64;              // tokens per wavefront
-constexpr unsigned WAVE_N = NATURAL ? 128 : 64;             // raw output columns per wavefront
-constexpr unsigned WAVES_M = MID ? 128 / WAVE_M : 1;
-constexpr unsigned WAVES_N = MID ? 128 / WAVE_N : 1;
-constexpr unsigned WAVES_K = MID ? 2 : 4;   // wavefronts that share an output block, each a part of every K step
+// int32 sums are exact in any order: there several wavefronts share an output block, each a part of every K step, and
+// add up their sums.  A float32 sum depends on its order, which is that of the 256 x 256 kernel -- one wavefront through
+// the whole of K -- so that a row's result does not depend on how many rows are launched with it.
+constexpr bool SPLIT_K = X17_A_KIND == 0 && X17_B_KIND == 0;
+// Of the 128 x 128 forms e4m3 x e4m3 takes eight wavefronts of 64 x 32 (1024 rows x 4096 columns, two stages, K = 1024:
+// 8.0 us, four of 64 x 64 10.3, eight of 32 x 64 9.0); e4m3 x int8, which widens every fragment it reads to f16, four of
+// 64 x 64 (4096 rows, K = 2048: 62 us, 66 and 77).
+constexpr bool WIDENS = X17_A_KIND != X17_B_KIND;
+constexpr unsigned WAVE_M = NATURAL || (!SPLIT_K && !MID) ? 32 : 64;                  // tokens per wavefront
+constexpr unsigned WAVE_N = NATURAL ? 128 : SPLIT_K || (MID && WIDENS) ? 64 : 32;     // raw output columns per wavefront
+constexpr unsigned WAVES_M = MID ? 128 / WAVE_M : SPLIT_K ? 1 : 64 / WAVE_M;
+constexpr unsigned WAVES_N = MID ? 128 / WAVE_N : SPLIT_K ? 1 : 64 / WAVE_N;
+constexpr unsigned WAVES_K = !SPLIT_K ? 1 : MID ? 2 : 4;                              // wavefronts that share an output block
 constexpr unsigned WAVES = WAVES_M * WAVES_N * WAVES_K;
 constexpr unsigned THREADS_PER_BLOCK = 64 * WAVES;
 constexpr unsigned M_PER_BLOCK = WAVE_M * WAVES_M;

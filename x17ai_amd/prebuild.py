@@ -129,6 +129,10 @@ def _specs():
 	for strict in (True, False):                             # the speed builds are bench.py's
 		add(("dequant", 2048, 16384, INT8, INT8, True, strict))
 		add(("dequant", 8192, 2048, INT8, INT8, False, strict))
+	# ---- tests/test_gpu_launch_shapes.py: e4m3 products with inexact float32 sums
+	add(("dequant", 4096, 384, E4M3, E4M3, False, True))
+	add(("dequant", 4096, 384, E4M3, INT8, False, True))
+	add(("ffn_y", 256, 4096, True, E4M3, INT8))
 	# ---- x17ai_amd.block: benchmark config 4 (bench.py, tests/config4_chain.py) and the reference's own configuration
 	for strict in (True, False):
 		add(("block", 2048, 16, 128, 8192, BF16, strict))
