@@ -119,6 +119,9 @@ int x17h_gemm_kernel_launch_qkv(X17hGemmKernel *k, X17hTensor *x, X17hTensor *q_
 double x17h_gemm_kernel_n_ops(X17hGemmKernel *k, X17hTensor *a, X17hTensor *b);
 /* launch geometry read back from meta.json: THREADS_PER_BLOCK, SMEM_BYTES, M_PER_BLOCK, N_PER_BLOCK */
 int x17h_gemm_kernel_metadata(X17hGemmKernel *k, size_t out[4]);
+/* the form a launch with a_rows token rows takes: {256, 0} the persistent 256 x 256 kernel, {64 or 128, LDS stages} a
+ * small-tile form (kernel cache directory s<tile>x<stages>); all forms give the same bytes */
+int x17h_gemm_kernel_form(X17hGemmKernel *k, size_t a_rows, size_t out[2]);
 /* resources of the loaded kernel: x17ai_hip_read_kernel_attrs (9 x int32) */
 int x17h_gemm_kernel_attrs(X17hGemmKernel *k, int32_t out[9]);
 

@@ -105,6 +105,7 @@ def host() -> ctypes.CDLL:
 	h.x17h_gemm_kernel_launch_qkv.argtypes = [P, P, P, P, P, P, P]
 	h.x17h_gemm_kernel_n_ops.argtypes = [P, P, P]
 	h.x17h_gemm_kernel_n_ops.restype = ctypes.c_double
+	h.x17h_gemm_kernel_form.argtypes = [P, SZ, ctypes.POINTER(SZ)]
 	h.x17h_gemm_kernel_metadata.argtypes = [P, ctypes.POINTER(SZ)]
 	h.x17h_gemm_kernel_attrs.argtypes = [P, ctypes.POINTER(ctypes.c_int32)]
 	h.x17h_attn_kernel_new.argtypes = [P, ctypes.c_char_p, ctypes.POINTER(AttnConfigC), PP]

@@ -317,6 +317,13 @@ class GemmKernel:
 	def n_ops(self, a: Tensor, b: Tensor) -> float:
 		return float(_ffi.host().x17h_gemm_kernel_n_ops(self._h, a._h, b._h))
 
+	def form(self, a_rows: int) -> str:
+		"""The form a launch of `a_rows` token rows takes: "" the 256 x 256 kernel, else a small-tile form (the name of its
+		directory inside the kernel's cache directory)."""
+		out = (ctypes.c_size_t * 2)()
+		check(_ffi.host().x17h_gemm_kernel_form(self._h, a_rows, out))
+		return f"s{out[0]}x{out[1]}" if out[1] else ""
+
 	@property
 	def metadata(self) -> dict:
 		out = (ctypes.c_size_t * 4)()

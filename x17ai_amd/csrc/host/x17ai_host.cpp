@@ -1040,75 +1040,94 @@ Status GemmKernel::launch(GemmArgs const &args) {
 }
 
 // ---- which tile size a GEMM launch takes.
-// Estimated microseconds of a launch as rounds of workgroups over the 256 compute units, each round fixed + per_k * K
-// (K in bytes), fitted to launches of 256 .. 4096 token rows on an MI355X (K = 2048 / 8192 int8, 4096 / 16384 e4m3,
-// 8192 e4m3 x int8; us measured at 4096 columns, K = 2048, int8, 256 / 512 / 1024 / 2048 / 4096 rows:
-// 64 x 64 tiles 6.2 / 10.9 / 19.9 / 51 / 103, 128 x 128 four stages 9.9 / 10.3 / 11.3 / 25 / 45, two stages
-// 9.7 / 10.1 / 11.4 / 20 / 39, 256 x 256 23 / 23 / 24 / 26 / 35).  The estimates hold within about 10 %; where two
-// forms are that close either will do.
+// Estimated microseconds of a launch: measured curves over the number of its tiles, in units of the 256 compute units,
+// each point fixed + per_k * K / 1024 (K in bytes) and straight lines between them.  Fitted on an MI355X to 689 launches of
+// 256 .. 65536 token rows, 1024 .. 16384 columns and K = 128 .. 16384; a fit is 3-9 % off in the mean of a curve and up to
+// 40 % at single points (the two-stage form at 512 tiles of K = 512).  Over those and 255 launches of other widths the
+// form taken is 1 % slower than the best one in the mean.  us measured at 4096 columns:
+//                        rows:  256    512   1024   2048   4096  16384
+//   int8, K = 2048   64 x 64    6.1   10.3   19.3   44.3   89.3    348
+//           128 x 128, 4 / 2  8.7/8.4 8.9/8.6 10.3/10.1 23.3/19.6 43.4/36.8 166/143
+//                   256 x 256  19.5   19.6   20.4   24.3   34.1    118
+//   int8, K = 256     64 x 64   4.4    6.7   11.3   21.4   40.4    165
+//           128 x 128, 4 / 2  4.5/4.4 4.7/4.4 5.1/4.9 8.3/6.4 14.8/10.9 52.8/38.3
+//                   256 x 256   7.3    7.6    8.2    9.2   12.4   34.9
 namespace gemm_cost {
-	struct Line { double fixed, per_k; double at(double k) const { return fixed + per_k * k; } };
-	struct Rates {
-		Line tile64;                // a round of 64 x 64 tiles, one workgroup per compute unit
-		Line tile128_deep;          // a round of 128 x 128 tiles with four stages, one workgroup per compute unit
-		Line tile128_first;         // 256 of the two-stage 128 x 128 tiles (two workgroups share a compute unit) alone ...
-		Line tile128;               // ... and each 256 of them in a larger launch
-		Line tile256_latency;       // a round of the persistent 256 x 256 kernel: bound by one tile's walk over K ...
-		Line tile256_full;          // ... or, times the round's fill, by the clock the full chip holds
+	struct Point { double tiles, fixed, per_k; };          // tiles / 256
+	struct Curve {
+		Point points[6];                                    // (unused ones at the end are zero)
+		double us(size_t tiles, double k) const {
+			double const n = double(tiles) / double(COMPUTE_UNITS);
+			auto at = [&](Point const &p) { return p.fixed + p.per_k * (k / 1024.0); };
+			if (n <= points[0].tiles) return at(points[0]);
+			size_t i = 1;
+			for (; i < 6 && points[i].tiles != 0.0; ++i) {
+				Point const &a = points[i - 1], &b = points[i];
+				if (n <= b.tiles) return at(a) + (at(b) - at(a)) * (n - a.tiles) / (b.tiles - a.tiles);
+			}
+			return at(points[i - 1]) * n / points[i - 1].tiles;      // whole rounds behind each other
+		}
 	};
-	static Rates const RATES[3] = {
-		{{1.6, 1.53e-3}, {2.7, 3.3e-3}, {0.0, 4.75e-3}, {0.6, 4.1e-3}, {9.0, 7.0e-3}, {2.0, 12.8e-3}},       // int8
-		{{1.6, 1.53e-3}, {2.0, 3.8e-3}, {0.0, 4.6e-3}, {0.8, 3.65e-3}, {15.0, 6.6e-3}, {4.0, 10.4e-3}},     // e4m3
-		{{0.0, 2.9e-3}, {0.0, 6.8e-3}, {0.0, 6.4e-3}, {0.0, 7.0e-3}, {4.0, 15.9e-3}, {0.0, 23.0e-3}},      // e4m3 x int8
+	struct Curves { Curve large, tile64, tile128_deep, tile128; };   // 256 x 256 | 64 x 64 | 128 x 128, four stages | two
+	static Curves const CURVES[4] = {
+		{   // int8
+			{{{0.125, 4.7, 7.3}, {0.5, 6.4, 8.8}, {1, 8.7, 12.6}, {1.25, 11.2, 19.1}, {2, 14.8, 24.9}, {4, 22.8, 46.7}}},
+			{{{0.25, 3.8, 1.0}, {1, 3.9, 1.2}, {1.25, 5.7, 2.3}, {2, 4.2, 3.5}}},
+			{{{0.25, 3.6, 2.5}, {1, 3.9, 3.8}, {1.25, 5.8, 7.4}, {2, 6.6, 8.7}, {4, 9.7, 15.9}}},
+			{{{0.25, 3.3, 2.6}, {1, 3.3, 4.8}, {1.25, 4.2, 5.6}, {2, 4.6, 7.4}, {2.5, 6.2, 11.4}, {4, 6.2, 14.7}}},
+		},
+		{   // int8, head-normalising writers (wavefronts of 32 x 128)
+			{{{0.125, 5.4, 7.0}, {0.5, 6.4, 7.8}, {1, 7.9, 11.9}, {1.25, 10.8, 18.4}, {2, 13.7, 23.0}, {4, 17.4, 47.0}}},
+			{{{0.25, 4.5, 1.4}, {1, 4.9, 1.4}, {1.25, 7.5, 3.0}, {2, 6.4, 3.4}}},
+			{{{0.25, 4.8, 2.6}, {1, 5.1, 3.5}, {1.25, 7.7, 6.4}, {2, 8.4, 9.1}, {4, 12.7, 17.2}}},
+			{{{0.25, 4.5, 2.5}, {1, 4.7, 3.8}, {1.25, 5.3, 5.8}, {2, 6.2, 7.3}, {2.5, 8.1, 11.4}, {4, 8.4, 15.0}}},
+		},
+		{   // e4m3 x e4m3
+			{{{0.125, 9.9, 7.1}, {0.5, 12.6, 7.8}, {1, 18.3, 10.5}, {1.25, 25.3, 17.6}, {2, 33.1, 21.1}, {4, 47.1, 43.6}}},
+			{{{0.25, 3.2, 1.2}, {1, 3.0, 1.7}, {1.25, 4.6, 2.9}, {2, 3.3, 4.0}}},
+			{{{0.25, 3.7, 2.9}, {1, 4.4, 4.0}, {1.25, 7.0, 6.8}, {2, 8.1, 8.2}, {4, 11.8, 16.2}}},
+			{{{0.25, 3.3, 3.1}, {1, 3.6, 5.0}, {1.25, 5.4, 5.7}, {2, 6.5, 7.3}, {2.5, 7.9, 11.2}, {4, 8.6, 15.2}}},
+		},
+		{   // e4m3 x int8
+			{{{0.125, 6.0, 15.3}, {0.5, 8.0, 15.4}, {1, 11.3, 21.6}, {1.25, 13.7, 35.9}, {2, 19.5, 44.4}, {4, 24.2, 89.5}}},
+			{{{0.25, 2.5, 3.2}, {1, 2.6, 3.7}, {1.25, 3.8, 6.8}, {2, 2.7, 7.0}}},
+			{{{0.25, 3.0, 7.1}, {1, 3.2, 7.9}, {1.25, 5.0, 14.6}, {2, 5.3, 16.3}, {4, 7.5, 32.6}}},
+			{{{0.25, 2.8, 7.1}, {1, 3.2, 7.7}, {1.25, 3.7, 12.0}, {2, 3.7, 14.4}, {2.5, 5.3, 19.8}, {4, 4.3, 28.7}}},
+		},
 	};
-	static constexpr double LAUNCH = 1.5;
-	static double rounds_of(size_t tiles) { return double((tiles + COMPUTE_UNITS - 1) / COMPUTE_UNITS); }
-	static double small(Rates const &r, size_t tile, size_t stages, bool natural, size_t tiles, double k) {
-		double const n = rounds_of(tiles);
-		// the head-normalising writers' wavefronts of 32 x 128 read more per product (64: 32 x 128 tiles load more as well)
-		double const shape = !natural ? 1.0 : tile == 64 ? 1.25 : 1.1;
-		if (tile == 64) return LAUNCH + shape * n * r.tile64.at(k);
-		if (stages == 4) return LAUNCH + shape * n * r.tile128_deep.at(k) * (n > 1.0 ? 1.1 : 1.0);
-		if (n == 1.0) return LAUNCH + shape * r.tile128_first.at(k);
-		// (of two workgroups' worth, the second shortens with its fill)
-		double const fill = n == 2.0 ? 0.73 + 0.27 * (double(tiles) / COMPUTE_UNITS - 1.0) : 1.0;
-		return LAUNCH + shape * n * r.tile128.at(k) * fill;
-	}
-	static double large(Rates const &r, size_t tiles, double k) {
-		double const full = double(tiles / COMPUTE_UNITS), rest = double(tiles % COMPUTE_UNITS) / COMPUTE_UNITS;
-		double us = full * std::max(r.tile256_latency.at(k), r.tile256_full.at(k));
-		// (a last, partly filled round starts with its first tiles already in LDS)
-		if (rest > 0.0) us += std::max(r.tile256_latency.at(k) - (full > 0.0 ? 2.0 : 0.0), rest * r.tile256_full.at(k));
-		return us;
-	}
+	// What a small form has to gain by the estimate: the curves' spread.  Without it 10 of the 689 launches took a form
+	// slower than the 256 x 256 kernel, one by half; with it three do, by 6 % at most.
+	static constexpr double MARGIN = 1.06;
 }
 
-Status GemmKernel::launch_tiles(size_t a_rows, size_t n_raw, void **raw_args) {
+GemmKernel::Small const *GemmKernel::form_for(size_t a_rows) const {
+	size_t const n_raw = *b_rows;
 	auto tiles_of = [&](GemmLauncherMetadata const &m) {
 		return ((a_rows + m.M_PER_BLOCK - 1) >> ctz(m.M_PER_BLOCK)) * ((n_raw + m.N_PER_BLOCK - 1) >> ctz(m.N_PER_BLOCK));
 	};
-	bool const e4m3 = a_dtype == DType::E4m3, e4m3_weights = b_dtype == DType::E4m3;
-	gemm_cost::Rates const &rates = gemm_cost::RATES[e4m3 != e4m3_weights ? 2 : e4m3 ? 1 : 0];
 	bool const natural = epilogue_kind == 3 || epilogue_kind == 5 || epilogue_kind == 6;
-	size_t const tiles = tiles_of(metadata);
-	double best = gemm_cost::large(rates, tiles, double(a_cols));
+	gemm_cost::Curves const &c = gemm_cost::CURVES[a_dtype != b_dtype ? 3 : a_dtype == DType::E4m3 ? 2 : natural ? 1 : 0];
+	double best = c.large.us(tiles_of(metadata), double(a_cols));
 	Small const *chosen = nullptr;
 	for (Small const &s : small) {
-		double const us = gemm_cost::small(rates, s.tile, s.stages, natural, tiles_of(s.metadata), double(a_cols));
+		gemm_cost::Curve const &curve = s.tile == 64 ? c.tile64 : s.stages == 4 ? c.tile128_deep : c.tile128;
+		double const us = gemm_cost::MARGIN * curve.us(tiles_of(s.metadata), double(a_cols));
 		if (us < best) {
 			best = us;
 			chosen = &s;
 		}
 	}
-	if (chosen != nullptr) {
-		size_t grid[3] = {tiles_of(chosen->metadata), 1, 1};
-		size_t block[3] = {chosen->metadata.THREADS_PER_BLOCK, 1, 1};
-		return chosen->kernel->launch(*device->stream, grid, block, chosen->metadata.SMEM_BYTES, raw_args);
-	}
-	// persistent kernel: the workgroups share the tiles out among themselves
-	size_t grid[3] = {metadata.MAX_BLOCKS != 0 && tiles > metadata.MAX_BLOCKS ? metadata.MAX_BLOCKS : tiles, 1, 1};
-	size_t block[3] = {metadata.THREADS_PER_BLOCK, 1, 1};
-	return kernel->launch(*device->stream, grid, block, metadata.SMEM_BYTES, raw_args);
+	return chosen;
+}
+
+Status GemmKernel::launch_tiles(size_t a_rows, size_t n_raw, void **raw_args) {
+	Small const *chosen = form_for(a_rows);
+	GemmLauncherMetadata const &m = chosen != nullptr ? chosen->metadata : metadata;
+	size_t const tiles = ((a_rows + m.M_PER_BLOCK - 1) >> ctz(m.M_PER_BLOCK)) * ((n_raw + m.N_PER_BLOCK - 1) >> ctz(m.N_PER_BLOCK));
+	// (the 256 x 256 kernel is persistent: the workgroups share the tiles out among themselves)
+	size_t grid[3] = {m.MAX_BLOCKS != 0 && tiles > m.MAX_BLOCKS ? m.MAX_BLOCKS : tiles, 1, 1};
+	size_t block[3] = {m.THREADS_PER_BLOCK, 1, 1};
+	return (chosen != nullptr ? chosen->kernel : kernel)->launch(*device->stream, grid, block, m.SMEM_BYTES, raw_args);
 }
 
 // The fused q + kv launch: the checks of gemm.rs:591-641 for the q part and of :860-918 for the kv part.
@@ -1826,6 +1845,12 @@ int x17h_gemm_kernel_launch_qkv(X17hGemmKernel *k, X17hTensor *x, X17hTensor *q_
 	return from_status(k->k->launch(args));
 }
 double x17h_gemm_kernel_n_ops(X17hGemmKernel *k, X17hTensor *a, X17hTensor *b) { return k->k->n_ops(*a->t, *b->t); }
+int x17h_gemm_kernel_form(X17hGemmKernel *k, size_t a_rows, size_t out[2]) {
+	GemmKernel::Small const *s = k->k->form_for(a_rows);
+	out[0] = s != nullptr ? s->tile : k->k->metadata.M_PER_BLOCK;
+	out[1] = s != nullptr ? s->stages : 0;
+	return 0;
+}
 int x17h_gemm_kernel_metadata(X17hGemmKernel *k, size_t out[4]) {
 	out[0] = k->k->metadata.THREADS_PER_BLOCK; out[1] = k->k->metadata.SMEM_BYTES;
 	out[2] = k->k->metadata.M_PER_BLOCK; out[3] = k->k->metadata.N_PER_BLOCK;

@@ -247,7 +247,8 @@ struct GemmKernel {
 	                                           bool strict_math, Diagnostics &diag);
 	Status launch(GemmArgs const &args);
 	Status launch_qkv(GemmArgs const &args, size_t a_rows);   // epilogue_kind 6, reached through launch()
-	Status launch_tiles(size_t a_rows, size_t n_raw, void **raw_args);   // picks the tile size and launches
+	Small const *form_for(size_t a_rows) const;               // the tile size a launch of a_rows takes (null: 256 x 256)
+	Status launch_tiles(size_t a_rows, size_t n_raw, void **raw_args);
 	double n_ops(Tensor const &a, Tensor const &b) const;     // 2*M*K*N_raw, gemm.rs:445-449
 };
 
