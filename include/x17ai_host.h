@@ -146,8 +146,6 @@ typedef struct X17hAttnConfig {
 /* AttnKernel::new, attn.rs:170-232 */
 int x17h_attn_kernel_new(X17hDevice *dev, char const *kernel_name, X17hAttnConfig const *config, X17hAttnKernel **out);
 void x17h_attn_kernel_free(X17hAttnKernel *k);
-/* heads a workgroup of a launch takes one behind the other (1 .. 128 / head_dim; every choice gives the same bytes) */
-size_t x17h_attn_kernel_heads_per_workgroup(X17hAttnKernel *k, size_t seq_len, size_t batch, size_t window_size);
 /* AttnKernel::launch, attn.rs:234-236 / 353-447.  l may be NULL.  batch > 1 is an extension:
  * the rows of q/kv/out are `batch` independent sequences of equal length. */
 int x17h_attn_kernel_launch(X17hAttnKernel *k, X17hTensor *q, X17hTensor *kv, X17hTensor *sink_k,
@@ -192,8 +190,6 @@ int x17h_rms_norm_kernel_launch(X17hRmsNormKernel *k, X17hTensor *inp, X17hTenso
  * of attn_fwd_i8 for one query per sequence at position cache_len[s]. */
 int x17h_decode_kernel_new(X17hDevice *dev, char const *kernel_name, size_t n_heads, size_t head_dim,
                            size_t cache_capacity, int strict_math, X17hDecodeKernel **out);
-/* threads per (sequence, head) a launch takes: 128, 256, 512 or 1024 */
-size_t x17h_decode_kernel_threads(X17hDecodeKernel *k, size_t sequences, size_t window_size);
 void x17h_decode_kernel_free(X17hDecodeKernel *k);
 int x17h_decode_kernel_launch(X17hDecodeKernel *k, X17hTensor *q, X17hTensor *cache, X17hTensor *cache_len,
                               X17hTensor *sink_k, X17hTensor *sink_v, X17hTensor *attn_temperature,

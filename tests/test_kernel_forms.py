@@ -45,33 +45,3 @@ def test_forms_of_a_kernel_pass_the_code_object_scans(tmp_path):
 def test_the_form_a_launch_takes(make, picks):
 	kernel = make()
 	assert {rows: kernel.form(rows) for rows in picks} == picks
-
-
-@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
-@pytest.mark.parametrize("make,picks", [
-	(lambda: recipes.attn_decode_kernel(None, 32, 128, 4096), {
-		(1, 256): 256, (8, 256): 256, (8, 512): 512, (8, 4096): 1024,          # at most one workgroup per compute unit
-		(9, 256): 256, (16, 1024): 512, (9, 0): 512,                           # up to two
-		(32, 128): 256, (32, 1024): 256, (64, 128): 128, (48, 1024): 256, (64, 2048): 512, (64, 4096): 512}),
-	# two wavefronts already stream at the memory's rate: 48 sequences 35 us, 37 on 256 threads
-	(lambda: recipes.attn_decode_kernel(None, 2, 64, 4096), {(1, 4096): 1024, (384, 1024): 128, (384, 256): 256, (384, 4096): 512, (512, 4096): 128}),
-], ids=["head_dim 128", "head_dim 64"])
-def test_the_width_a_decode_launch_takes(make, picks):
-	kernel = make()
-	assert {key: kernel.threads(*key) for key in picks} == picks
-
-
-@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
-@pytest.mark.parametrize("make,picks", [
-	# small launches: a head per workgroup fills the chip; large ones with short walks: the group saves its workgroup's start
-	(lambda: recipes.attn_kernel(None, 8, 64, False), {(1024, 1, 256): 1, (4096, 8, 512): 1, (128, 128, 128): 2}),
-	(lambda: recipes.attn_kernel(None, 64, 32), {(256, 1, 0): 1, (2048, 1, 0): 1, (128, 512, 128): 4}),
-	(lambda: recipes.attn_d_q_kernel(None, 4, 32), {(1024, 1, 0): 1, (1024, 128, 64): 4}),
-	# dK / dV, one workgroup per compute unit: 64 heads of 32, 16384 rows in sequences of 128 193 and 178 us
-	(lambda: recipes.attn_d_kv_kernel(None, 4, 32), {(1024, 1, 0): 1, (128, 2048, 128): 4}),
-	(lambda: recipes.attn_d_kv_kernel(None, 8, 64, False), {(1856, 2, 512): 1, (128, 512, 128): 2}),
-	(lambda: recipes.attn_kernel(None, 16, 128, False), {(8192, 4, 512): 1}),
-], ids=["forward 64", "forward 32", "dQ 32", "dK/dV 32", "dK/dV 64", "head_dim 128"])
-def test_the_heads_a_workgroup_takes(make, picks):
-	kernel = make()
-	assert {key: kernel.heads_per_workgroup(*key) for key in picks} == picks

@@ -414,10 +414,6 @@ class AttnKernel:
 		check(_ffi.host().x17h_attn_kernel_launch_d_kv(
 			self._h, q._h, kv._h, attn_temperature._h, d_out._h, l._h, d._h, d_kv._h, window_size, batch))
 
-	def heads_per_workgroup(self, seq_len: int, batch: int, window_size: int) -> int:
-		"""Heads a workgroup of such a launch takes one behind the other; every choice gives the same bytes."""
-		return int(_ffi.host().x17h_attn_kernel_heads_per_workgroup(self._h, seq_len, batch, window_size))
-
 	def n_ops(self, seq_len: int, window_size: int) -> float:
 		return float(_ffi.host().x17h_attn_kernel_n_ops(self._h, seq_len, window_size))
 
@@ -485,10 +481,6 @@ class AttnDecodeKernel:
 			check(_ffi.host().x17h_decode_kernel_new(dev_h, kernel_name.encode(), n_heads, head_dim, cache_capacity,
 			                                         int(strict_math), ctypes.byref(self._h)))
 		self.diagnostics = _ffi.last_diagnostics()
-
-	def threads(self, sequences: int, window_size: int) -> int:
-		"""Threads per (sequence, head) of a launch over `sequences` with this window."""
-		return int(_ffi.host().x17h_decode_kernel_threads(self._h, sequences, window_size))
 
 	def launch_row_scaled(self, q: Tensor, cache: Tensor, cache_len: Tensor, sink_k: Tensor, sink_v: Tensor,
 	                      attn_temperature: Tensor, out: Tensor, l: Optional[Tensor], window_size: int, q_scale: Tensor,

@@ -267,6 +267,7 @@ struct AttnKernelConfig {
 	// through AttnKernel::launch_d_kv.
 	bool backward_kv = false;
 	size_t heads_per_kernel() const;
+	size_t head_group_cnt() const;
 	size_t head_group_dim() const;
 	double n_ops(size_t seq_len, size_t window_size) const;   // attn.rs:72-84
 	bool validate(Diagnostics &diag) const;
@@ -296,7 +297,6 @@ struct AttnKernel {
 	AttnLauncherMetadata metadata{};
 	std::shared_ptr<HipDevice> device;
 	std::unique_ptr<HipKernel> kernel;
-	size_t heads_per_workgroup(size_t seq_len, size_t batch, size_t window) const;     // what a launch takes
 	static std::unique_ptr<AttnKernel> create(std::shared_ptr<HipDevice> device, std::string const &kernel_name,
 	                                           AttnKernelConfig const &config, bool strict_math, Diagnostics &diag);
 	Status launch(AttnKernelArgs const &args);
@@ -350,7 +350,6 @@ struct AttnDecodeKernel {
 	// the same kernel with more wavefronts per (sequence, head), widest first; launch() picks by the size of the launch
 	struct Wide { AttnDecodeMetadata metadata; std::unique_ptr<HipKernel> kernel; };
 	std::vector<Wide> wide;
-	size_t threads_for(size_t seqs, size_t keys) const;      // the width a launch over `seqs` sequences takes, `keys` = its window
 	static std::unique_ptr<AttnDecodeKernel> create(std::shared_ptr<HipDevice> device, std::string const &kernel_name,
 	                                                 AttnDecodeConfig const &config, bool strict_math, Diagnostics &diag);
 	Status launch(AttnDecodeArgs const &args);
