@@ -45,3 +45,19 @@ def test_forms_of_a_kernel_pass_the_code_object_scans(tmp_path):
 def test_the_form_a_launch_takes(make, picks):
 	kernel = make()
 	assert {rows: kernel.form(rows) for rows in picks} == picks
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+@pytest.mark.parametrize("make,picks", [
+	# small launches: a head per workgroup fills the chip; large ones with short walks: the group saves its workgroup's start
+	(lambda: recipes.attn_kernel(None, 8, 64, False), {(1024, 1, 256): 1, (4096, 8, 512): 1, (128, 128, 128): 2}),
+	(lambda: recipes.attn_kernel(None, 64, 32), {(256, 1, 0): 1, (2048, 1, 0): 1, (128, 512, 128): 4}),
+	(lambda: recipes.attn_d_q_kernel(None, 4, 32), {(1024, 1, 0): 1, (1024, 128, 64): 4}),
+	# dK / dV, one workgroup per compute unit: 64 heads of 32, 16384 rows in sequences of 128 193 and 178 us
+	(lambda: recipes.attn_d_kv_kernel(None, 4, 32), {(1024, 1, 0): 1, (128, 2048, 128): 4}),
+	(lambda: recipes.attn_d_kv_kernel(None, 8, 64, False), {(1856, 2, 512): 1, (128, 512, 128): 2}),
+	(lambda: recipes.attn_kernel(None, 16, 128, False), {(8192, 4, 512): 1}),
+], ids=["forward 64", "forward 32", "dQ 32", "dK/dV 32", "dK/dV 64", "head_dim 128"])
+def test_the_heads_a_workgroup_takes(make, picks):
+	kernel = make()
+	assert {key: kernel.heads_per_workgroup(*key) for key in picks} == picks

@@ -414,6 +414,10 @@ class AttnKernel:
 		check(_ffi.host().x17h_attn_kernel_launch_d_kv(
 			self._h, q._h, kv._h, attn_temperature._h, d_out._h, l._h, d._h, d_kv._h, window_size, batch))
 
+	def heads_per_workgroup(self, seq_len: int, batch: int, window_size: int) -> int:
+		"""Heads a workgroup of such a launch takes one behind the other; every choice gives the same bytes."""
+		return int(_ffi.host().x17h_attn_kernel_heads_per_workgroup(self._h, seq_len, batch, window_size))
+
 	def n_ops(self, seq_len: int, window_size: int) -> float:
 		return float(_ffi.host().x17h_attn_kernel_n_ops(self._h, seq_len, window_size))
 

@@ -1173,7 +1173,6 @@ Status GemmKernel::launch_qkv(GemmArgs const &args, size_t a_rows) {
 // ================================================================ attention (src/device/cuda/attn.rs)
 
 size_t AttnKernelConfig::heads_per_kernel() const { return head_dim == 0 ? 1 : std::max<size_t>(128 / head_dim, 1); }
-size_t AttnKernelConfig::head_group_cnt() const { return n_heads / heads_per_kernel(); }
 size_t AttnKernelConfig::head_group_dim() const { return heads_per_kernel() * head_dim; }
 
 double AttnKernelConfig::n_ops(size_t seq_len, size_t window_size) const {
@@ -1257,6 +1256,43 @@ std::unique_ptr<AttnKernel> AttnKernel::create(std::shared_ptr<HipDevice> device
 	return out;
 }
 
+// Heads a workgroup takes one behind the other (a power of two up to 128 / head_dim, the reference's group,
+// src/device/cuda/attn.rs:60-66).  One head each fills the chip in a small launch; in a large launch of short walks a
+// group saves its workgroup's start.  Estimated per choice, in key steps (32 keys; dK / dV: query tiles): rounds of the
+// workgroups a compute unit holds, a partly filled last round counting more than its share, each round `start` plus the
+// group's walks, plus the tail of the longest walk.  Fitted to 870 launches of 8 .. 64 heads of 32 and 64, 1024 .. 32768
+// rows, windows of 64 .. 4096 and none: 0.1-0.8 % behind the best choice in the mean.  us, one head / the whole group:
+//   forward, 8 heads of 64:    1024 rows, no window 23 / 42    16384 rows in sequences of 128 16.2 / 14.7
+//   dQ, 64 heads of 32:        8192 rows, window 64, 8 sequences 73 / 66
+//   dK / dV, 64 heads of 32:   1024 rows, no window 36 / 104   16384 rows in sequences of 128 193 / 178
+size_t AttnKernel::heads_per_workgroup(size_t seq_len, size_t batch, size_t window) const {
+	struct Fit { double resident, start, last_round, tail; };
+	static constexpr Fit FITS[3][2] = {       // forward, dQ, dK / dV; head_dim 32 and 64
+		{{3, 2.5, 0, 0.5}, {3, 1.5, 0.5, 0.25}}, {{3, 8, 0, 0.75}, {3, 4, 0, 0.75}}, {{1, 2.5, 0, 0.1}, {1, 1, 0, 0.1}},
+	};
+	Fit const &f = FITS[config.backward_q ? 1 : config.backward_kv ? 2 : 0][config.head_dim == 32 ? 0 : 1];
+	size_t const blocks = (seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK;
+	size_t const w = window == 0 || window > seq_len ? seq_len : window;
+	// key steps of a block: its own, and those of the min(w, rows before it) keys it sees further back
+	size_t const growing = std::min(blocks, (w + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK);
+	double const own = double(metadata.Q_PER_BLOCK);
+	double const mean = (own + (own * double(growing) * double(growing - 1) / 2.0 + double(blocks - growing) * double(w)) / double(blocks)) / 32.0;
+	double const longest = (own + std::min(own * double(blocks - 1), double(w))) / 32.0;
+	size_t best = 1;
+	double best_cost = 0.0;
+	for (size_t heads = 1; heads * config.head_dim <= 128 && config.n_heads % heads == 0; heads *= 2) {
+		double const rounds = double(blocks * batch * (config.n_heads / heads)) / (f.resident * double(COMPUTE_UNITS));
+		double const walk = f.start + double(heads) * longest;
+		double const cost = rounds <= 1.0 ? walk
+			: std::max(walk, (rounds + f.last_round * (std::ceil(rounds) - rounds)) * (f.start + double(heads) * mean) + f.tail * double(heads) * longest);
+		if (heads == 1 || cost < best_cost) {
+			best = heads;
+			best_cost = cost;
+		}
+	}
+	return best;
+}
+
 // attn.rs:353-447
 Status AttnKernel::launch(AttnKernelArgs const &a) {
 	if (!device || !kernel) return Status::err(TensorOpError::Other, "attention kernel " + name + " was built without a device");
@@ -1333,7 +1369,7 @@ Status AttnKernel::launch(AttnKernelArgs const &a) {
 	// the plain kernel takes the first nine arguments only
 	void *raw_args[14] = {&seq_len_arg, &q_ptr, &kv_ptr, &sk, &sv, &tp, &out_ptr, &l_ptr, &window_arg,
 	                      &scale_ptrs[0], &scale_ptrs[1], &scale_ptrs[2], &scale_ptrs[3], &scale_ptrs[4]};
-	size_t grid[3] = {(seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK, config.n_heads, a.batch};
+	size_t grid[3] = {(seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK, config.n_heads / heads_per_workgroup(seq_len, a.batch, a.window_size), a.batch};
 	size_t block[3] = {metadata.THREADS_PER_BLOCK, 1, 1};
 	return kernel->launch(*device->stream, grid, block, metadata.SMEM_BYTES, raw_args);
 }
@@ -1390,7 +1426,7 @@ Status AttnKernel::launch_d_q(AttnKernelArgs const &a) {
 	void *out_ptr = a.out->ptr, *do_ptr = a.d_out->ptr, *dq_ptr = a.d_q->ptr, *l_ptr = a.l->ptr;
 	void *d_ptr = a.d != nullptr ? a.d->ptr : nullptr;
 	void *raw_args[12] = {&seq_len_arg, &q_ptr, &kv_ptr, &sk, &sv, &tp, &out_ptr, &do_ptr, &dq_ptr, &l_ptr, &d_ptr, &window_arg};
-	size_t grid[3] = {(seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK, config.n_heads, a.batch};
+	size_t grid[3] = {(seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK, config.n_heads / heads_per_workgroup(seq_len, a.batch, a.window_size), a.batch};
 	size_t block[3] = {metadata.THREADS_PER_BLOCK, 1, 1};
 	return kernel->launch(*device->stream, grid, block, metadata.SMEM_BYTES, raw_args);
 }
@@ -1439,7 +1475,7 @@ Status AttnKernel::launch_d_kv(AttnKernelArgs const &a) {
 	void *q_ptr = a.q->ptr, *kv_ptr = a.kv->ptr, *tp = a.attn_temperature->ptr, *do_ptr = a.d_out->ptr, *l_ptr = a.l->ptr, *d_ptr = a.d->ptr;
 	void *dkv_ptr = a.d_kv->ptr;
 	void *raw_args[9] = {&seq_len_arg, &q_ptr, &kv_ptr, &tp, &do_ptr, &l_ptr, &d_ptr, &dkv_ptr, &window_arg};
-	size_t grid[3] = {(seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK, config.n_heads, a.batch};
+	size_t grid[3] = {(seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK, config.n_heads / heads_per_workgroup(seq_len, a.batch, a.window_size), a.batch};
 	size_t block[3] = {metadata.THREADS_PER_BLOCK, 1, 1};
 	return kernel->launch(*device->stream, grid, block, metadata.SMEM_BYTES, raw_args);
 }
@@ -1923,6 +1959,9 @@ int x17h_attn_kernel_launch_d_kv(X17hAttnKernel *k, X17hTensor *q, X17hTensor *k
 	return from_status(k->k->launch_d_kv(args));
 }
 double x17h_attn_kernel_n_ops(X17hAttnKernel *k, size_t seq_len, size_t window_size) { return k->k->config.n_ops(seq_len, window_size); }
+size_t x17h_attn_kernel_heads_per_workgroup(X17hAttnKernel *k, size_t seq_len, size_t batch, size_t window_size) {
+	return k->k->heads_per_workgroup(seq_len, batch, window_size);
+}
 int x17h_attn_kernel_metadata(X17hAttnKernel *k, size_t out[3]) {
 	out[0] = k->k->metadata.THREADS_PER_BLOCK; out[1] = k->k->metadata.SMEM_BYTES; out[2] = k->k->metadata.Q_PER_BLOCK;
 	return 0;

@@ -267,7 +267,6 @@ struct AttnKernelConfig {
 	// through AttnKernel::launch_d_kv.
 	bool backward_kv = false;
 	size_t heads_per_kernel() const;
-	size_t head_group_cnt() const;
 	size_t head_group_dim() const;
 	double n_ops(size_t seq_len, size_t window_size) const;   // attn.rs:72-84
 	bool validate(Diagnostics &diag) const;
@@ -297,6 +296,7 @@ struct AttnKernel {
 	AttnLauncherMetadata metadata{};
 	std::shared_ptr<HipDevice> device;
 	std::unique_ptr<HipKernel> kernel;
+	size_t heads_per_workgroup(size_t seq_len, size_t batch, size_t window) const;     // what a launch takes
 	static std::unique_ptr<AttnKernel> create(std::shared_ptr<HipDevice> device, std::string const &kernel_name,
 	                                           AttnKernelConfig const &config, bool strict_math, Diagnostics &diag);
 	Status launch(AttnKernelArgs const &args);
