@@ -192,6 +192,8 @@ int x17h_rms_norm_kernel_launch(X17hRmsNormKernel *k, X17hTensor *inp, X17hTenso
  * of attn_fwd_i8 for one query per sequence at position cache_len[s]. */
 int x17h_decode_kernel_new(X17hDevice *dev, char const *kernel_name, size_t n_heads, size_t head_dim,
                            size_t cache_capacity, int strict_math, X17hDecodeKernel **out);
+/* threads per (sequence, head) a launch takes: 128, 256, 512 or 1024 */
+size_t x17h_decode_kernel_threads(X17hDecodeKernel *k, size_t sequences, size_t window_size);
 void x17h_decode_kernel_free(X17hDecodeKernel *k);
 int x17h_decode_kernel_launch(X17hDecodeKernel *k, X17hTensor *q, X17hTensor *cache, X17hTensor *cache_len,
                               X17hTensor *sink_k, X17hTensor *sink_v, X17hTensor *attn_temperature,

@@ -61,12 +61,12 @@ def test_head_groups_in_the_grid(shim, h, hd, seq, batch, window):  # noqa: F811
 		assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), name
 
 
-@pytest.mark.parametrize("n,window,row_scales", [
-	(8, 256, False), (8, 4096, True),                                        # at most one workgroup per compute unit: 256 / 1024 threads
-	(9, 1040, False), (9, 1024, True), (32, 512, False), (32, 1024, False),    # more: 512 / 256 / 256 / 256 threads
-	(33, 512, True), (33, 528, False), (33, 2048, False),                     # ... than four per compute unit: 128 / 256 / 512
+@pytest.mark.parametrize("n,window,row_scales,threads", [
+	(8, 256, False, 256), (8, 512, False, 512), (8, 4096, True, 1024),        # at most one workgroup per compute unit
+	(9, 1040, False, 512), (9, 1024, True, 512), (32, 128, False, 256), (32, 1024, False, 256),
+	(33, 128, True, 128), (33, 256, False, 128), (33, 528, False, 256), (33, 2048, False, 512),      # more than four
 ])
-def test_decode_workgroup_widths(n, window, row_scales):
+def test_decode_workgroup_widths(n, window, row_scales, threads):
 	"""Every width the launcher picks (32 heads of 128, capacity 4096), ragged lengths including 0, 1 and the capacity:
 	bit-equal to the oracle on sampled (sequence, head) slices."""
 	from oracle import strict as S
@@ -85,9 +85,12 @@ def test_decode_workgroup_widths(n, window, row_scales):
 	if row_scales:
 		qs, ks, vs = (0.125 * (0.75 + 0.5 * rng.random(s)).astype(np.float32) for s in ((n, h), (n, h, cap), (n, h, cap)))
 		vw, sw, osc = recipes.attn_row_scale_operands(vs, X.BF16)
-		recipes.attn_decode_row_scaled_kernel(dev, h, hd, cap, X.BF16, True).launch_row_scaled(*args, *(t(a, X.F32) for a in (qs, ks, vw, sw, osc)))
+		kernel = recipes.attn_decode_row_scaled_kernel(dev, h, hd, cap, X.BF16, True)
+		kernel.launch_row_scaled(*args, *(t(a, X.F32) for a in (qs, ks, vw, sw, osc)))
 	else:
-		recipes.attn_decode_kernel(dev, h, hd, cap, True).launch(*args)
+		kernel = recipes.attn_decode_kernel(dev, h, hd, cap, True)
+		kernel.launch(*args)
+	assert kernel.threads(n, window) == threads
 	got, got_l = out.download(), l.download()
 	seqs, heads = np.array([0, 1, 2, n - 1]), np.array([0, h - 1])
 	cols = np.concatenate([np.arange(x * hd, (x + 1) * hd) for x in heads])

@@ -49,6 +49,20 @@ def test_the_form_a_launch_takes(make, picks):
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
 @pytest.mark.parametrize("make,picks", [
+	(lambda: recipes.attn_decode_kernel(None, 32, 128, 4096), {
+		(1, 256): 256, (8, 256): 256, (8, 512): 512, (8, 4096): 1024,          # at most one workgroup per compute unit
+		(9, 256): 256, (16, 1024): 512, (9, 0): 512,                           # up to two
+		(32, 128): 256, (32, 1024): 256, (64, 128): 128, (48, 1024): 256, (64, 2048): 512, (64, 4096): 512}),
+	# two wavefronts already stream at the memory's rate: 48 sequences 35 us, 37 on 256 threads
+	(lambda: recipes.attn_decode_kernel(None, 2, 64, 4096), {(1, 4096): 1024, (384, 1024): 128, (384, 256): 256, (384, 4096): 512, (512, 4096): 128}),
+], ids=["head_dim 128", "head_dim 64"])
+def test_the_width_a_decode_launch_takes(make, picks):
+	kernel = make()
+	assert {key: kernel.threads(*key) for key in picks} == picks
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+@pytest.mark.parametrize("make,picks", [
 	# small launches: a head per workgroup fills the chip; large ones with short walks: the group saves its workgroup's start
 	(lambda: recipes.attn_kernel(None, 8, 64, False), {(1024, 1, 256): 1, (4096, 8, 512): 1, (128, 128, 128): 2}),
 	(lambda: recipes.attn_kernel(None, 64, 32), {(256, 1, 0): 1, (2048, 1, 0): 1, (128, 512, 128): 4}),

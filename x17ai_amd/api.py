@@ -486,6 +486,10 @@ class AttnDecodeKernel:
 			                                         int(strict_math), ctypes.byref(self._h)))
 		self.diagnostics = _ffi.last_diagnostics()
 
+	def threads(self, sequences: int, window_size: int) -> int:
+		"""Threads per (sequence, head) of a launch over `sequences` with this window."""
+		return int(_ffi.host().x17h_decode_kernel_threads(self._h, sequences, window_size))
+
 	def launch_row_scaled(self, q: Tensor, cache: Tensor, cache_len: Tensor, sink_k: Tensor, sink_v: Tensor,
 	                      attn_temperature: Tensor, out: Tensor, l: Optional[Tensor], window_size: int, q_scale: Tensor,
 	                      k_scale: Tensor, v_weight: Tensor, sink_v_weight: Tensor, out_scale: Tensor) -> None:

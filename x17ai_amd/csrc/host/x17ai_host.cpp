@@ -1597,12 +1597,49 @@ std::unique_ptr<AttnDecodeKernel> AttnDecodeKernel::create(std::shared_ptr<HipDe
 		auto b = build_one(threads);
 		if (!b) return nullptr;
 		// (a wide workgroup stages more of the P.V partials: with a long cache it may not fit)
-		if (b->kernel) out->wide.push_back(Wide{b->metadata, std::move(b->kernel)});
+		if (b->metadata.SMEM_BYTES <= LDS_BYTES) out->wide.push_back(Wide{b->metadata, std::move(b->kernel)});
 	}
 	out->name = kernel_name;
 	out->config = config;
 	out->device = std::move(device);
 	return out;
+}
+
+// Threads per workgroup, by the number of workgroups and by the key bytes each may have to stream (figures in
+// attn_decode_i8.hip; 1062 launches of 8 .. 64 heads of 32, 64 and 128, windows 128 .. 16384, full and ragged caches: 1-2 %
+// behind the best width in the mean).  At most one workgroup per compute unit: as many wavefronts as the window keeps
+// busy.  More: a long window streams best from 512 threads whatever their number; below that the width that keeps the
+// workgroups resident, two wavefronts for many short windows.  At head_dim 64 two wavefronts already stream at the
+// memory's rate from three workgroups per compute unit on (48 sequences x 16 heads x 1024 keys, every probability
+// counting: 35 us, 37 with 256 threads), with long windows from four (64 x 16 heads x 4096, every probability counting:
+// 177 us, 189 with 512 threads; normal keys 98 and 98; ragged 77 and 71.  48 sequences: 133 and 142, 80 and 76, 71 and 55).
+size_t AttnDecodeKernel::threads_for(size_t seqs, size_t keys) const {
+	size_t const workgroups = seqs * (config.n_heads / metadata.HEADS_PER_BLOCK);
+	size_t const key_bytes = keys * config.head_dim;
+	size_t threads;
+	if (workgroups <= COMPUTE_UNITS) {
+		threads = key_bytes <= 32 * 1024 ? 256 : key_bytes <= 64 * 1024 ? 512 : 1024;
+	} else if ((key_bytes > 128 * 1024 && !(config.head_dim == 64 && workgroups > 3 * COMPUTE_UNITS)) || (workgroups <= 2 * COMPUTE_UNITS && config.head_dim == 128 && key_bytes > 32 * 1024)) {
+		threads = 512;
+	} else if (workgroups > 4 * COMPUTE_UNITS && key_bytes <= 32 * 1024) {
+		threads = 128;
+	} else {
+		threads = config.head_dim == 64 && workgroups > 2 * COMPUTE_UNITS && key_bytes > 16 * 1024 ? 128 : 256;
+	}
+	// workgroups of one width a compute unit holds: 16 wavefronts by their registers, and by the LDS a cache capacity takes
+	auto resident = [&](size_t t) -> size_t {
+		size_t lds = t == metadata.THREADS_PER_BLOCK ? metadata.SMEM_BYTES : 0;
+		for (Wide const &w : wide) if (w.metadata.THREADS_PER_BLOCK == t) lds = w.metadata.SMEM_BYTES;
+		return lds == 0 ? 0 : std::min(1024 / t, LDS_BYTES / lds);
+	};
+	// (a long capacity: the next width keeps more wavefronts per compute unit; 24 sequences of 32 heads against 16384
+	// cached keys each, window 1024: 256 threads 33 us, 512 27 us)
+	while (workgroups > COMPUTE_UNITS && threads < 512 && workgroups > resident(threads) * COMPUTE_UNITS
+	       && resident(threads) * threads < resident(2 * threads) * 2 * threads) {
+		threads *= 2;
+	}
+	while (threads > metadata.THREADS_PER_BLOCK && resident(threads) == 0) threads /= 2;
+	return threads;
 }
 
 Status AttnDecodeKernel::launch(AttnDecodeArgs const &a) {
@@ -1671,20 +1708,12 @@ Status AttnDecodeKernel::launch(AttnDecodeArgs const &a) {
 	// the plain kernel takes the first nine arguments only
 	void *raw_args[14] = {&q_ptr, &cache_ptr, &len_ptr, &sk, &sv, &tp, &out_ptr, &l_ptr, &window_arg,
 	                      &scale_ptrs[0], &scale_ptrs[1], &scale_ptrs[2], &scale_ptrs[3], &scale_ptrs[4]};
-	// Threads per workgroup, by the number of workgroups and by the key bytes each may have to stream (the figures behind
-	// the lines are in attn_decode_i8.hip).  At most one workgroup per compute unit: sixteen wavefronts each, unless the
-	// window is so short that a workgroup's set-up outweighs it.  More: a long window streams best from 512 threads; below
-	// that the width that keeps all workgroups resident, two wavefronts for the shortest.
-	size_t const workgroups = seqs * (config.n_heads / metadata.HEADS_PER_BLOCK);
 	size_t const keys = a.window_size == 0 || a.window_size > config.cache_capacity ? config.cache_capacity : a.window_size;
-	size_t const key_bytes = keys * config.head_dim;
-	size_t const threads = workgroups <= COMPUTE_UNITS ? (key_bytes <= 32 * 1024 ? 256 : 1024)
-	                     : key_bytes > 128 * 1024 ? 512
-	                     : workgroups <= 4 * COMPUTE_UNITS || key_bytes > 64 * 1024 ? 256 : 128;
+	size_t const threads = threads_for(seqs, keys);
 	AttnDecodeMetadata const *meta = &metadata;
 	HipKernel *chosen = kernel.get();
 	for (Wide const &w : wide) {
-		if (w.metadata.THREADS_PER_BLOCK <= threads) {
+		if (w.metadata.THREADS_PER_BLOCK == threads) {
 			meta = &w.metadata;
 			chosen = w.kernel.get();
 			break;
@@ -2020,6 +2049,10 @@ int x17h_decode_kernel_launch_row_scaled(X17hDecodeKernel *k, X17hTensor *q, X17
 	                 l != nullptr ? l->t.get() : nullptr, window_size,
 	                 q_scale->t.get(), k_scale->t.get(), v_weight->t.get(), sink_v_weight->t.get(), out_scale->t.get()};
 	return from_status(k->k->launch(a));
+}
+size_t x17h_decode_kernel_threads(X17hDecodeKernel *k, size_t sequences, size_t window_size) {
+	size_t const capacity = k->k->config.cache_capacity;
+	return k->k->threads_for(sequences, window_size == 0 || window_size > capacity ? capacity : window_size);
 }
 void x17h_decode_kernel_free(X17hDecodeKernel *k) { delete k; }
 int x17h_decode_kernel_launch(X17hDecodeKernel *k, X17hTensor *q, X17hTensor *cache, X17hTensor *cache_len, X17hTensor *sink_k,

@@ -350,6 +350,7 @@ struct AttnDecodeKernel {
 	// the same kernel with more wavefronts per (sequence, head), widest first; launch() picks by the size of the launch
 	struct Wide { AttnDecodeMetadata metadata; std::unique_ptr<HipKernel> kernel; };
 	std::vector<Wide> wide;
+	size_t threads_for(size_t seqs, size_t keys) const;      // the width a launch over `seqs` sequences takes, `keys` = its window
 	static std::unique_ptr<AttnDecodeKernel> create(std::shared_ptr<HipDevice> device, std::string const &kernel_name,
 	                                                 AttnDecodeConfig const &config, bool strict_math, Diagnostics &diag);
 	Status launch(AttnDecodeArgs const &args);

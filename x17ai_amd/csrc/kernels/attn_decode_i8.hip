@@ -13,10 +13,12 @@
 // 8-bit probability is not zero (rows with probability 0 contribute nothing and are not fetched).  One workgroup
 // per (sequence, head); its width is chosen at launch (X17_DECODE_THREADS, decode_tile.h) by how many workgroups there
 // are and how many key bytes each streams: few workgroups have to keep enough loads in flight by themselves, many
-// short ones want to be resident together.  Measured at 32 heads of 128 (us, 128 / 256 / 512 / 1024 threads):
-//   1 sequence x 4096 keys   63 / 37 / 23 / 19     8 x 4096   100 / 58 / 37 / 34    1 x 256   9.3 / 8.2 / 7.8 / 8.3
-//   24 x 512                 20 / 15 / 20 / 26    24 x 4096   106 / 82 / 76 / 85
-//   64 x 512                 33 / 33 / 41 / 68    64 x 4096   197 / 187 / 171 / 199
+// short ones want to be resident together.  Measured at 32 heads of 128, capacity 4096, normal keys and queries (us,
+// 128 / 256 / 512 / 1024 threads; in parentheses 512 threads and 128 where every probability counts):
+//    3 sequences x 4096 keys  112 / 41 / 27 / 24    16 x 4096  126 / 60 / 55 / 62    16 x 512   21 / 12 / 11 / 17
+//   32 x 1024                  43 / 31 / 32 / 46    32 x 4096  141 / 103 / 97 / 109  32 x 128  9.1 / 8.7 / 16 / 28
+//   48 x 1024                  50 / 46 / 46 / 67    48 x 4096  158 / 148 / 137 / 157 (266, 271)
+//   64 x 128                 10.9 / 17 / 31 / 57    64 x 4096  193 / 192 / 184 / 206 (349, 343)
 // The recurrence is cut into phases so that only two cheap scans remain sequential:
 //   1  scores: HD/16 lanes per key row (16-byte coalesced loads), v_dot4 + lane reduction
 //   2  per-tile max, prefix max over tiles (exact), rescale factors, probabilities, quad sums
@@ -135,37 +137,44 @@ void kernel(
 	// ---- phase 1: scores of all keys of the walked tiles.  A thread keeps BATCH independent 16-byte
 	// loads in flight (a load per pass would leave the kernel waiting on memory latency).
 	u32 const n_keys = n_tiles * 16;
-	// Loads in flight per thread: four, except for the 512-thread workgroups, which long windows of many sequences take
-	// and which stream best with sixteen (64 sequences x 4096 keys: 171 us with 16, 182 with 4, 196 with 2; 24
-	// sequences x 128 keys on 256 threads: 8.3 us with 4, 10.7 with 16).
-#ifndef X17_DECODE_BATCH
-#define X17_DECODE_BATCH (X17_DECODE_THREADS == 512 ? 16 : 4)
-#endif
-	constexpr u32 BATCH = X17_DECODE_BATCH;
-	for (u32 base = 0; base < n_keys; base += KEYS_PER_PASS * BATCH) {
-		v4i kc[BATCH];
-		X17_UNROLL for (u32 bb = 0; bb < BATCH; ++bb) {
-			u32 kidx = base + bb * KEYS_PER_PASS + tid / CPR;
-			u32 j = t0 * 16 + kidx;
-			bool vis = kidx < n_keys && j >= j_lo && j < pos;
-			u32 j_safe = vis ? j : pos - 1;                   // a row that exists (n_tiles > 0 means pos >= 1)
-			// every cache byte is read once: streaming (non-temporal) loads
-			kc[bb] = __builtin_nontemporal_load(reinterpret_cast<v4i const *>(kv_head + (size_t)j_safe * ROW + 16 * c));
-		}
-		X17_UNROLL for (u32 bb = 0; bb < BATCH; ++bb) {
-			u32 kidx = base + bb * KEYS_PER_PASS + tid / CPR;
-			u32 j = t0 * 16 + kidx;
-			bool in_range = kidx < n_keys;
-			bool vis = in_range && j >= j_lo && j < pos;
-			i32 dot = 0;
-			X17_UNROLL for (int w = 0; w < 4; ++w) dot = __builtin_amdgcn_sdot4(qc[w], kc[bb][w], dot, false);
-			X17_UNROLL for (u32 mask = 1; mask < CPR; mask <<= 1) dot += __shfl_xor(dot, (int)mask, 64);
-			if (in_range && c == 0) {
-				// (row-scaled build: the key's scale and the temperature are applied in a pass of their own below)
-				f32 const score = ROW_SCALES ? f32(dot) : f32(dot) * temperature;
-				s_score[kidx] = vis ? score : -__builtin_inff();
+	auto score_keys = [&]<u32 BATCH>() __attribute__((always_inline)) {
+		for (u32 base = 0; base < n_keys; base += KEYS_PER_PASS * BATCH) {
+			v4i kc[BATCH];
+			X17_UNROLL for (u32 bb = 0; bb < BATCH; ++bb) {
+				u32 kidx = base + bb * KEYS_PER_PASS + tid / CPR;
+				u32 j = t0 * 16 + kidx;
+				bool vis = kidx < n_keys && j >= j_lo && j < pos;
+				u32 j_safe = vis ? j : pos - 1;                   // a row that exists (n_tiles > 0 means pos >= 1)
+				// every cache byte is read once: streaming (non-temporal) loads
+				kc[bb] = __builtin_nontemporal_load(reinterpret_cast<v4i const *>(kv_head + (size_t)j_safe * ROW + 16 * c));
+			}
+			X17_UNROLL for (u32 bb = 0; bb < BATCH; ++bb) {
+				u32 kidx = base + bb * KEYS_PER_PASS + tid / CPR;
+				u32 j = t0 * 16 + kidx;
+				bool in_range = kidx < n_keys;
+				bool vis = in_range && j >= j_lo && j < pos;
+				i32 dot = 0;
+				X17_UNROLL for (int w = 0; w < 4; ++w) dot = __builtin_amdgcn_sdot4(qc[w], kc[bb][w], dot, false);
+				X17_UNROLL for (u32 mask = 1; mask < CPR; mask <<= 1) dot += __shfl_xor(dot, (int)mask, 64);
+				if (in_range && c == 0) {
+					// (row-scaled build: the key's scale and the temperature are applied in a pass of their own below)
+					f32 const score = ROW_SCALES ? f32(dot) : f32(dot) * temperature;
+					s_score[kidx] = vis ? score : -__builtin_inff();
+				}
 			}
 		}
+	};
+	// Loads in flight per thread.  128 threads: two where the window is long -- eight such workgroups per compute unit
+	// then walk a sequence's rows nearly in step, which the DRAM pages like (64 sequences x 1024 keys: 57 us with 2, 60
+	// with 4; x 4096: 193 and 205) -- four where it is short (64 x 128: 11.9 and 10.9).  256 threads: eight, unless that
+	// reaches past a short window (128 x 1024: 98 us with 8, 106 with 4; 64 x 128: 17.5 and 16.5).  512 threads: eight
+	// (16 x 512: 10.9 us with 8, 11.2 with 4, 12.5 with 16).  1024: four.
+	constexpr u32 MANY = dt::THREADS_PER_BLOCK == 128 ? 2 : dt::THREADS_PER_BLOCK <= 512 ? 8 : 4;
+	constexpr u32 SHORT_BYTES = dt::THREADS_PER_BLOCK == 128 ? 32 * 1024 : dt::THREADS_PER_BLOCK == 256 ? 16 * 1024 : 0;
+	if (n_keys * HD <= SHORT_BYTES) {
+		score_keys.template operator()<4>();
+	} else {
+		score_keys.template operator()<MANY>();
 	}
 	__syncthreads();
 #if X17_ATTN_ROW_SCALES
