@@ -4,6 +4,7 @@ scratch memory, no spilled registers."""
 import glob
 import os
 import shutil
+import stat
 
 import pytest
 
@@ -75,3 +76,40 @@ def test_the_width_a_decode_launch_takes(make, picks):
 def test_the_heads_a_workgroup_takes(make, picks):
 	kernel = make()
 	assert {key: kernel.heads_per_workgroup(*key) for key in picks} == picks
+
+
+def _decode(): return recipes.attn_decode_kernel(None, 2, 64, 256)
+def _gemm(): return recipes.attn_q_kernel(None, 512, 384)
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+@pytest.mark.parametrize("make", [_gemm, _decode])
+def test_the_forms_of_a_kernel_are_compiled_side_by_side(make, tmp_path, monkeypatch):
+	"""A kernel is four compiler runs; a compiler that only notes when it starts and ends and sleeps in between."""
+	script = tmp_path / "cc"
+	script.write_text(f"#!/bin/bash\necho start >> {tmp_path}/log\nsleep 0.7\necho end >> {tmp_path}/log\n"
+	                  "while [ $# -gt 0 ]; do [ \"$1\" = -o ] && touch \"$2\"; shift; done\n")
+	script.chmod(script.stat().st_mode | stat.S_IXUSR)
+	monkeypatch.setenv("X17AI_HIPCC", str(script))
+	monkeypatch.setenv("X17AI_KERNEL_CACHE", str(tmp_path / "cache"))
+	make()
+	log = (tmp_path / "log").read_text().split()
+	assert len(log) == 8 and log[:4] == ["start"] * 4, log
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+@pytest.mark.parametrize("make,source,marker,forms", [
+	(_gemm, "gemm_b8_small.hip", '#include "common.h"', ("s64x4", "s128x4", "s128x2")),
+	(_decode, "attn_decode_i8.hip", '#include "decode_tile.h"', ("t1024", "t512", "t256")),
+])
+def test_a_form_that_cannot_be_built_does_not_refuse_the_kernel(make, source, marker, forms, tmp_path, monkeypatch):
+	"""Only the kernel itself has to compile: launches then take it at every size."""
+	shutil.copytree(os.path.join(os.path.dirname(os.path.abspath(recipes.__file__)), "csrc", "kernels"), tmp_path / "kernels")
+	path = tmp_path / "kernels" / source
+	broken = "#if defined(X17_SMALL_TILE) || defined(X17_DECODE_THREADS) && X17_DECODE_THREADS > 128\n#error not this form\n#endif\n"
+	path.write_text(path.read_text().replace(marker, marker + "\n" + broken, 1))
+	monkeypatch.setenv("X17AI_KERNELS_DIR", str(tmp_path / "kernels"))
+	monkeypatch.setenv("X17AI_KERNEL_CACHE", str(tmp_path / "cache"))
+	kernel = make()
+	assert all(f"form {f} is left out" in kernel.diagnostics for f in forms) and "not this form" in kernel.diagnostics
+	assert kernel.form(256) == "" if make is _gemm else kernel.threads(1, 0) == 128

@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <functional>
+#include <future>
 #include <cstdlib>
 #include <cstring>
 #include <fstream>
@@ -670,6 +671,25 @@ namespace kernel_build {
 		return out;
 	}
 
+	std::vector<BuiltForm> build_forms(std::string const &kernel_name, std::string const &common_text, std::vector<Form> const &forms) {
+		auto one = [&](Form const &f) {
+			BuiltForm b;
+			b.files = build(kernel_name, common_text + f.defines, f.source_file, f.meta_source_file, b.diag, f.name);
+			return b;
+		};
+		std::vector<std::future<BuiltForm>> running;
+		for (size_t i = 1; i < forms.size(); ++i) running.push_back(std::async(std::launch::async, one, std::cref(forms[i])));
+		std::vector<BuiltForm> out;
+		out.push_back(one(forms[0]));
+		for (auto &r : running) out.push_back(r.get());
+		return out;
+	}
+
+	void leave_out(std::string const &kernel_name, std::string const &form, Diagnostics const &of_form, Diagnostics &diag) {
+		diag.add_warning("kernel " + kernel_name + ": form " + form + " is left out");
+		for (Diagnostic const &d : of_form.list) diag.add_warning(d.message);
+	}
+
 	// Flat {"KEY": unsigned, ...} objects only -- all the metadata programs print.
 	std::optional<std::vector<std::pair<std::string, size_t>>> read_metadata_json(std::string const &path, Diagnostics &diag) {
 		std::string text;
@@ -897,7 +917,19 @@ std::unique_ptr<GemmKernel> GemmKernel::create(std::shared_ptr<HipDevice> device
 	if (b_rows % 128 != 0) { diag.add_error("GEMM raw output columns must be a multiple of 128, got " + std::to_string(b_rows)); return nullptr; }
 	if (b_rows < 256) { diag.add_error("GEMM raw output columns must be at least one tile (256), got " + std::to_string(b_rows)); return nullptr; }
 
-	auto built = kernel_build::build(kernel_name, common.str(), "gemm_b8.hip", "gemm_meta.cpp", diag);
+	std::vector<kernel_build::Form> forms{{"", "", "gemm_b8.hip", "gemm_meta.cpp"}};
+	struct SmallForm { size_t tile, stages; };
+	std::vector<SmallForm> small_forms;
+	for (SmallForm f : {SmallForm{64, 4}, SmallForm{128, 4}, SmallForm{128, 2}}) {
+		if (g.a.cols % (f.tile == 64 ? 256 : 128) != 0) continue;       // whole K steps (gemm_small_tile.h)
+		small_forms.push_back(f);
+		forms.push_back({"s" + std::to_string(f.tile) + "x" + std::to_string(f.stages),
+		                 "#define X17_SMALL_TILE " + std::to_string(f.tile) + "\n#define X17_SMALL_STAGES " + std::to_string(f.stages) + "\n",
+		                 "gemm_b8_small.hip", "gemm_small_meta.cpp"});
+	}
+	std::vector<kernel_build::BuiltForm> built_forms = kernel_build::build_forms(kernel_name, common.str(), forms);
+	for (Diagnostic const &d : built_forms[0].diag.list) d.is_error ? diag.add_error(d.message) : diag.add_warning(d.message);
+	std::optional<kernel_build::BuiltKernel> const &built = built_forms[0].files;
 	if (!built) return nullptr;
 
 	auto meta = kernel_build::read_metadata_json(built->meta_json_path, diag);
@@ -917,26 +949,31 @@ std::unique_ptr<GemmKernel> GemmKernel::create(std::shared_ptr<HipDevice> device
 			+ std::to_string(out->metadata.N_PER_BLOCK));
 		return nullptr;
 	}
-	struct SmallForm { size_t tile, stages; };
-	for (SmallForm f : {SmallForm{64, 4}, SmallForm{128, 4}, SmallForm{128, 2}}) {
-		if (g.a.cols % (f.tile == 64 ? 256 : 128) != 0) continue;       // whole K steps (gemm_small_tile.h)
-		std::string const defines = "#define X17_SMALL_TILE " + std::to_string(f.tile) + "\n#define X17_SMALL_STAGES " + std::to_string(f.stages) + "\n";
-		auto small_built = kernel_build::build(kernel_name, common.str() + defines, "gemm_b8_small.hip", "gemm_small_meta.cpp", diag,
-		                                       "s" + std::to_string(f.tile) + "x" + std::to_string(f.stages));
-		if (!small_built) return nullptr;
-		auto small_meta = kernel_build::read_metadata_json(small_built->meta_json_path, diag);
-		if (!small_meta) return nullptr;
-		auto get_small = [&](char const *k) { auto v = kernel_build::meta_get(*small_meta, k); return v ? *v : size_t(0); };
-		GemmKernel::Small s{f.tile, f.stages, {get_small("THREADS_PER_BLOCK"), get_small("SMEM_BYTES"), get_small("M_PER_BLOCK"), get_small("N_PER_BLOCK"), 0}, nullptr};
-		if (s.metadata.THREADS_PER_BLOCK == 0 || !is_pow2(s.metadata.M_PER_BLOCK) || !is_pow2(s.metadata.N_PER_BLOCK)) {
-			diag.add_error("Invalid JSON metadata in " + small_built->meta_json_path);
-			return nullptr;
+	for (size_t i = 0; i < small_forms.size(); ++i) {
+		SmallForm const &f = small_forms[i];
+		kernel_build::BuiltForm &b = built_forms[i + 1];
+		auto load = [&]() -> std::optional<GemmKernel::Small> {
+			if (!b.files) return std::nullopt;
+			auto small_meta = kernel_build::read_metadata_json(b.files->meta_json_path, b.diag);
+			if (!small_meta) return std::nullopt;
+			auto get_small = [&](char const *k) { auto v = kernel_build::meta_get(*small_meta, k); return v ? *v : size_t(0); };
+			GemmKernel::Small s{f.tile, f.stages, {get_small("THREADS_PER_BLOCK"), get_small("SMEM_BYTES"), get_small("M_PER_BLOCK"), get_small("N_PER_BLOCK"), 0}, nullptr};
+			if (s.metadata.THREADS_PER_BLOCK == 0 || !is_pow2(s.metadata.M_PER_BLOCK) || !is_pow2(s.metadata.N_PER_BLOCK)) {
+				b.diag.add_error("Invalid JSON metadata in " + b.files->meta_json_path);
+				return std::nullopt;
+			}
+			if (device) {
+				s.kernel = kernel_build::load_kernel(*device->stream, b.files->code_object_path, "kernel", s.metadata.SMEM_BYTES, b.diag);
+				if (!s.kernel) return std::nullopt;
+			}
+			return s;
+		};
+		if (auto s = load()) {
+			out->small.push_back(std::move(*s));
+			for (Diagnostic const &d : b.diag.list) diag.add_warning(d.message);
+		} else {
+			kernel_build::leave_out(kernel_name, forms[i + 1].name, b.diag, diag);
 		}
-		if (device) {
-			s.kernel = kernel_build::load_kernel(*device->stream, small_built->code_object_path, "kernel", s.metadata.SMEM_BYTES, diag);
-			if (!s.kernel) return nullptr;
-		}
-		out->small.push_back(std::move(s));
 	}
 	out->name = kernel_name;
 	out->files = *built;
@@ -1563,41 +1600,49 @@ std::unique_ptr<AttnDecodeKernel> AttnDecodeKernel::create(std::shared_ptr<HipDe
 		common << "#define X17_ATTN_ROW_SCALES 1\n#define X17_ATTN_OUT_BF16 " << (config.out_dtype == DType::Bf16 ? 1 : 0) << "\n";
 	}
 	auto out = std::make_unique<AttnDecodeKernel>();
-	// one code object: the default (threads == 0) or one with `threads` per workgroup
-	struct Built { kernel_build::BuiltKernel files; AttnDecodeMetadata metadata; std::unique_ptr<HipKernel> kernel; };
-	auto build_one = [&](size_t threads) -> std::optional<Built> {
-		std::string const form = threads == 0 ? "" : "t" + std::to_string(threads);
-		std::string const define = threads == 0 ? "" : "#define X17_DECODE_THREADS " + std::to_string(threads) + "\n";
-		auto built = kernel_build::build(kernel_name, common.str() + define, "attn_decode_i8.hip", "decode_meta.cpp", diag, form);
-		if (!built) return std::nullopt;
-		auto meta = kernel_build::read_metadata_json(built->meta_json_path, diag);
+	// one code object per width, the narrowest as the kernel itself
+	static constexpr size_t WIDTHS[] = {1024, 512, 256};
+	std::vector<kernel_build::Form> forms{{"", "", "attn_decode_i8.hip", "decode_meta.cpp"}};
+	for (size_t t : WIDTHS) {
+		forms.push_back({"t" + std::to_string(t), "#define X17_DECODE_THREADS " + std::to_string(t) + "\n", "attn_decode_i8.hip", "decode_meta.cpp"});
+	}
+	std::vector<kernel_build::BuiltForm> built = kernel_build::build_forms(kernel_name, common.str(), forms);
+	struct Loaded { AttnDecodeMetadata metadata; std::unique_ptr<HipKernel> kernel; };
+	auto load = [&](kernel_build::BuiltForm &b) -> std::optional<Loaded> {
+		if (!b.files) return std::nullopt;
+		auto meta = kernel_build::read_metadata_json(b.files->meta_json_path, b.diag);
 		if (!meta) return std::nullopt;
 		auto get = [&](char const *k) { auto v = kernel_build::meta_get(*meta, k); return v ? *v : size_t(0); };
-		Built b{*built, AttnDecodeMetadata{get("THREADS_PER_BLOCK"), get("SMEM_BYTES"), get("HEADS_PER_BLOCK")}, nullptr};
-		if (b.metadata.THREADS_PER_BLOCK == 0 || b.metadata.HEADS_PER_BLOCK == 0 || config.n_heads % b.metadata.HEADS_PER_BLOCK != 0) {
-			diag.add_error("Invalid JSON metadata in " + built->meta_json_path);
+		Loaded l{AttnDecodeMetadata{get("THREADS_PER_BLOCK"), get("SMEM_BYTES"), get("HEADS_PER_BLOCK")}, nullptr};
+		if (l.metadata.THREADS_PER_BLOCK == 0 || l.metadata.HEADS_PER_BLOCK == 0 || config.n_heads % l.metadata.HEADS_PER_BLOCK != 0) {
+			b.diag.add_error("Invalid JSON metadata in " + b.files->meta_json_path);
 			return std::nullopt;
 		}
-		if (device && b.metadata.SMEM_BYTES <= LDS_BYTES) {
-			b.kernel = kernel_build::load_kernel(*device->stream, built->code_object_path, "kernel", b.metadata.SMEM_BYTES, diag);
-			if (!b.kernel) return std::nullopt;
+		if (device && l.metadata.SMEM_BYTES <= LDS_BYTES) {
+			l.kernel = kernel_build::load_kernel(*device->stream, b.files->code_object_path, "kernel", l.metadata.SMEM_BYTES, b.diag);
+			if (!l.kernel) return std::nullopt;
 		}
-		return b;
+		return l;
 	};
-	auto base = build_one(0);
+	auto base = load(built[0]);
+	for (Diagnostic const &d : built[0].diag.list) d.is_error ? diag.add_error(d.message) : diag.add_warning(d.message);
 	if (!base) return nullptr;
-	out->files = base->files;
+	out->files = *built[0].files;
 	out->metadata = base->metadata;
 	out->kernel = std::move(base->kernel);
 	if (device && !out->kernel) {
 		diag.add_error("decode kernel needs " + std::to_string(out->metadata.SMEM_BYTES) + " bytes of LDS for this cache capacity");
 		return nullptr;
 	}
-	for (size_t threads : {1024, 512, 256}) {
-		auto b = build_one(threads);
-		if (!b) return nullptr;
+	for (size_t i = 1; i < forms.size(); ++i) {
+		auto l = load(built[i]);
+		if (!l) {
+			kernel_build::leave_out(kernel_name, forms[i].name, built[i].diag, diag);
+			continue;
+		}
+		for (Diagnostic const &d : built[i].diag.list) diag.add_warning(d.message);
 		// (a wide workgroup stages more of the P.V partials: with a long cache it may not fit)
-		if (b->metadata.SMEM_BYTES <= LDS_BYTES) out->wide.push_back(Wide{b->metadata, std::move(b->kernel)});
+		if (l->metadata.SMEM_BYTES <= LDS_BYTES) out->wide.push_back(Wide{l->metadata, std::move(l->kernel)});
 	}
 	out->name = kernel_name;
 	out->config = config;

@@ -181,6 +181,13 @@ namespace kernel_build {
 	std::optional<BuiltKernel> build(std::string const &kernel_name, std::string const &common_text,
 	                                 std::string const &source_file, std::string const &meta_source_file,
 	                                 Diagnostics &diag, std::string const &form = "");
+	// Builds a kernel (the first entry) and further forms of it side by side: each is a compiler run of its own.  The
+	// results are in the order of `forms`; what a form had to say is in its own diagnostics.
+	struct Form { std::string name, defines, source_file, meta_source_file; };
+	struct BuiltForm { std::optional<BuiltKernel> files; Diagnostics diag; };
+	std::vector<BuiltForm> build_forms(std::string const &kernel_name, std::string const &common_text, std::vector<Form> const &forms);
+	// A further form that cannot be built or loaded is left out: its errors become warnings of the kernel.
+	void leave_out(std::string const &kernel_name, std::string const &form, Diagnostics const &of_form, Diagnostics &diag);
 	std::optional<std::vector<std::pair<std::string, size_t>>> read_metadata_json(std::string const &path, Diagnostics &diag);
 	std::string kernels_dir();
 	std::string cache_dir();
