@@ -317,3 +317,45 @@ def test_safetensors_header_that_overflows_is_rejected_before_anything_is_alloca
 		X.Tensor(None, (2 ** 62,), X.F32)
 	ok = write("ok_i8.safetensors", {"t": {"dtype": "I8", "shape": [2, 8], "data_offsets": [0, 16]}}, bytes(range(16)))
 	assert X.Tensor.from_safetensors_file(ok, None).download().ravel().tolist() == list(range(16))
+
+
+def test_the_build_key_covers_every_header_a_kernel_includes():
+	"""The key of a cached kernel, recomputed: FNV-1a over common.h, the device flags and both sources with every header of
+	the kernels directory they include, depth first.  The Rust side of the cache (integration/rust/kernel_build_hip.rs)
+	walks the same way and keeps no list of headers of its own."""
+	rust = open(os.path.join(ROOT, "integration", "rust", "kernel_build_hip.rs")).read()
+	assert rust.count("hash_with_includes(") == 3 and not re.search(r'for \w+ in \["[a-z0-9_]+\.h"', rust)
+	flags = re.search(r"DEVICE_FLAGS: &\[&str\] = &\[(.*?)\];", rust, re.S).group(1)
+	flags = " ".join(re.findall(r'"([^"]*)"', flags))
+	kernels = os.path.join(ROOT, "x17ai_amd", "csrc", "kernels")
+
+	def key(directory, sources):
+		h, seen = 0xCBF29CE484222325, []
+
+		def write(data):
+			nonlocal h
+			for b in data:
+				h = ((h ^ b) * 0x100000001B3) & 0xFFFFFFFFFFFFFFFF
+
+		def walk(name):
+			path = os.path.join(kernels, name)
+			if name in seen or not os.path.exists(path):
+				return
+			seen.append(name)
+			body = open(path, "rb").read()
+			write(name.encode())
+			write(body)
+			for included in re.findall(rb'#include "([^"]*)"', body):
+				walk(included.decode())
+
+		write(open(os.path.join(directory, "common.h"), "rb").read())
+		write(flags.encode())
+		for source in sources:
+			walk(source)
+		return f"{h:016x}", seen
+
+	base = os.path.join(_ffi.kernel_cache_dir(), recipes.attn_q_kernel(None, 512, 384).name)
+	for form, sources in (("", ("gemm_b8.hip", "gemm_meta.cpp")), ("s64x4", ("gemm_b8_small.hip", "gemm_small_meta.cpp"))):
+		want, seen = key(os.path.join(base, form), sources)
+		assert open(os.path.join(base, form, "build.key")).read() == want
+		assert "gemm_parts.h" in seen and "x17_device.h" in seen
