@@ -1,7 +1,7 @@
 """The kernels' hand-written tile requests (global -> LDS, 16 bytes per lane, addresses formed from scalar bases and
 lane offsets outside the compiler's view) are audited on the CPU: the index arithmetic lives in gemm_tile.h /
-attn_tile.h, the kernels call it, and the audit programs beside them (gemm_requests_audit.cpp,
-attn_requests_audit.cpp) are compiled here with a kernel's own generated common.h and enumerate every request of a
+gemm_small_tile.h / attn_tile.h, the kernels call it, and the audit programs beside them (gemm_requests_audit.cpp,
+gemm_small_requests_audit.cpp, attn_requests_audit.cpp) are compiled here with a kernel's own generated common.h and enumerate every request of a
 launch -- every tile of the persistent walk and K step, every (sequence, head, query block) and step of the request
 schedule, overhanging tiles and past-the-end repeats included.  Each must stay inside its operand and each tile's
 chunks must be requested exactly once.  No GPU is involved."""
@@ -19,11 +19,12 @@ KERNELS = os.path.join(os.path.dirname(os.path.abspath(recipes.__file__)), "csrc
 pytestmark = pytest.mark.skipif(shutil.which("g++") is None or shutil.which("hipcc") is None, reason="needs g++ and hipcc")
 
 
-def _audit(tmp_path, kernel, source, *args):
-	"""Compiles `source` against the configuration of `kernel` (a kernel object built without a device) and runs it."""
-	exe = os.path.join(str(tmp_path), kernel.name + "." + source.split(".")[0])
+def _audit(tmp_path, kernel, source, *args, form=""):
+	"""Compiles `source` against the configuration of `kernel` (a kernel object built without a device), or of a further
+	form of it, and runs it."""
+	exe = os.path.join(str(tmp_path), kernel.name + form + "." + source.split(".")[0])
 	if not os.path.exists(exe):
-		subprocess.run(["g++", "-std=c++17", "-O2", "-I" + os.path.join(_ffi.kernel_cache_dir(), kernel.name), "-I" + KERNELS,
+		subprocess.run(["g++", "-std=c++17", "-O2", "-I" + os.path.join(_ffi.kernel_cache_dir(), kernel.name, form), "-I" + KERNELS,
 		                os.path.join(KERNELS, source), "-o", exe], check=True)
 	out = subprocess.run([exe] + [str(a) for a in args], capture_output=True, text=True)
 	return json.loads(out.stdout), out.returncode
@@ -57,6 +58,22 @@ def test_gemm_tile_requests_stay_inside_their_operands(tmp_path, label, make, ro
 	# shapes the launcher rejects are not audited as if they could run
 	rep, rc = _audit(tmp_path, kern, "gemm_requests_audit.cpp", 192)
 	assert rc != 0 and not rep["ok"]
+
+
+@pytest.mark.parametrize("form", ["s64x4", "s128x4", "s128x2"])
+@pytest.mark.parametrize("label,make,row_counts", GEMMS, ids=[g[0] for g in GEMMS])
+def test_small_tile_gemm_requests_stay_inside_their_operands(tmp_path, label, make, row_counts, form):
+	"""gemm_small_tile.h, every form of the same kernels; 2368 and 4416 rows: a partly filled band, an overhanging tile."""
+	kern = make()
+	if form == "s64x4" and not os.path.exists(os.path.join(_ffi.kernel_cache_dir(), kern.name, form)):
+		assert "K = 128" in label or "K = 384" in label          # (K in steps of 256: the kernel has no such form)
+		return
+	for rows in row_counts + (2368, 4416):
+		rep, rc = _audit(tmp_path, kern, "gemm_small_requests_audit.cpp", rows, form=form)
+		assert rc == 0 and rep["ok"], (label, rows, rep)
+		assert rep["a_extent"] == rep["a_bytes"] and rep["b_extent"] == rep["b_bytes"] and rep["b_kv_extent"] == rep["b_kv_bytes"], (label, rows, rep)
+	rep, rc = _audit(tmp_path, kern, "gemm_small_requests_audit.cpp", row_counts[0], row_counts[0] - 1, form=form)
+	assert rc != 0 and not rep["ok"] and "past the end of a" in rep["error"], rep
 
 
 ATTNS = [
