@@ -3,6 +3,7 @@ shim: attention grids with groups of heads per workgroup (src/device/cuda/attn.r
 128 / head_dim heads) give the bytes of the one-head-per-workgroup launch, forward and backward."""
 import ctypes
 import json
+import math
 import os
 
 import numpy as np
@@ -10,7 +11,7 @@ import pytest
 
 import x17ai_amd as X
 from x17ai_amd import _ffi, recipes
-from tests.gpu_common import e4m3_bytes, i8_codes, rng_for
+from tests.gpu_common import e4m3_bytes, e4m3_compare, i8_codes, rng_for
 from tests.test_gpu_shim import P, SZ, _ok, _value, shim  # noqa: F401  (shim is a fixture)
 
 pytestmark = pytest.mark.gpu
@@ -126,56 +127,138 @@ GEMM_FORMS = [
 ]
 
 
+def _oracle(name, k, n, q_cols, a, b, b_kv, residual, scales, learned):
+	"""What the oracle gives for a launch of GEMM_FORMS, in the order of the launch's outputs."""
+	from oracle import strict as S
+	inp = 1.0 / math.sqrt(k) / 64.0
+	if name in ("mixed", "mixed_residual", "e4m3"):
+		acc = S.gemm_f32_seq(a, True, b, name == "e4m3")
+		if name == "mixed":
+			return [S.epilogue_scale(acc, 1.0 / math.sqrt(k) / 8.0, 8.0)]
+		if name == "e4m3":
+			return [S.epilogue_geglu(acc, 1.0 / math.sqrt(k), 1.0, S.STORE_E4M3)]
+		return [S.epilogue_residual(acc, residual, math.sqrt(recipes.GELU_VAR_FIX_2 / k) / 8.0, 1.0, S.STORE_E4M3)]
+	acc = S.gemm_i32(a, b)
+	if name in ("scale", "one_step"):
+		return [S.epilogue_scale(acc, inp, 8.0)]
+	if name.startswith("geglu"):
+		return [S.epilogue_geglu(acc, inp, 8.0 if name == "geglu_i8_fast" else 1.0, S.STORE_I8 if name == "geglu_i8_fast" else S.STORE_E4M3)]
+	if name == "residual":
+		return [S.epilogue_residual(acc, residual, inp, 1.0, S.STORE_E4M3)]
+	if name.startswith("l2norm"):
+		return list(S.epilogue_l2norm(acc, int(name.split("_")[1]), recipes.L2_NORM_EPS, inp, 8.0))
+	if name.startswith("dequant"):
+		return [S.epilogue_dequant(acc, *scales, name == "dequant_geglu")]
+	if name == "qnorm":
+		return [S.epilogue_qnorm(acc, 64, 0.0, 8.0, learned)]
+	kv, rrms = S.epilogue_l2norm(S.gemm_i32(a, b_kv), 64, recipes.L2_NORM_EPS, inp, 8.0)
+	return [S.epilogue_scale(acc, inp, 8.0), rrms, kv]
+
+
 @pytest.mark.parametrize("name,make,k,n", GEMM_FORMS, ids=[f[0] for f in GEMM_FORMS])
-@pytest.mark.parametrize("rows", [256, 320, 448])
+@pytest.mark.parametrize("rows", [256, 320, 448, 2368])
 def test_every_tile_size_gives_the_same_product(shim, name, make, k, n, rows):  # noqa: F811
-	"""The 64 x 64 and 128 x 128 forms of a GEMM against its 256 x 256 kernel (which the oracle pins): the same bytes, also
-	with e4m3 operands, whose float32 sums every form adds in the same order."""
+	"""The 256 x 256 kernel against the oracle -- overhanging rows and columns moved back, every writer; launch() takes
+	small tiles at these sizes -- and the 64 x 64 and 128 x 128 forms against it: the same bytes, also with e4m3
+	operands, whose float32 sums every form adds in the same order.  (2368 rows: a partly filled band of tiles.)  The
+	outputs hold another byte pattern before each launch."""
 	dev = X.Device(0)
 	rng = rng_for("tile sizes", name, rows)
 	e4 = name in ("mixed", "mixed_residual", "e4m3")
 	t = lambda a, dtype: X.Tensor.from_numpy(dev, np.ascontiguousarray(a), dtype)
-	a = t(e4m3_bytes(rng, (rows, k)), X.E4M3) if e4 else t(i8_codes(rng, (rows, k)), X.INT8)
-	weights = lambda r: t(e4m3_bytes(rng, (r, k)), X.E4M3) if name == "e4m3" else t(i8_codes(rng, (r, k)), X.INT8)
+	a = e4m3_bytes(rng, (rows, k)) if e4 else i8_codes(rng, (rows, k))
+	weights = lambda r: e4m3_bytes(rng, (r, k)) if name == "e4m3" else i8_codes(rng, (r, k))
 	kernel = make()
 	pairs = "geglu" in name or "residual" in name or name == "e4m3"
 	out_cols, out_type = n // 2 if pairs else n, X.BF16 if "dequant" in name else X.E4M3 if pairs and name != "geglu_i8_fast" else X.INT8
-	residual = t(i8_codes(rng, (rows, out_cols)), X.INT8)
-	scales = t((0.01 + 0.01 * rng.random(rows)).astype(np.float32), X.F32), t((0.01 + 0.01 * rng.random(n)).astype(np.float32), X.F32)
-	learned = t((rng.standard_normal(n).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16), X.BF16)
+	residual = i8_codes(rng, (rows, out_cols))
+	scales = (0.01 + 0.01 * rng.random(rows)).astype(np.float32), (0.01 + 0.01 * rng.random(n)).astype(np.float32)
+	learned = (rng.standard_normal(n).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
 	q_cols = 256 if name == "qkv" else n
 	b, b_kv = weights(q_cols), weights(max(n - q_cols, 128))
 	heads = (n - q_cols if name == "qkv" else n) // (2 * int(name.split("_")[1]) if name.startswith("l2norm") else 128)
+	ta, tb, tb_kv = t(a, X.E4M3 if e4 else X.INT8), *(t(w, X.E4M3 if name == "e4m3" else X.INT8) for w in (b, b_kv))
+	extras = t(residual, X.INT8), [t(v, X.F32) for v in scales], t(learned, X.BF16)
 	results = {}
 	base = os.path.join(_ffi.kernel_cache_dir(), kernel.name)
-	for form in ("", "s64x4", "s128x4", "s128x2"):
+	for pattern, form in ((0x5A, ""), (0x3C, "s64x4"), (0xA7, "s128x4"), (0xC9, "s128x2")):
 		if form == "s64x4" and k % 256 != 0:
 			continue
 		with open(os.path.join(base, form, "meta.json")) as f:
 			meta = json.load(f)
-		c = X.Tensor(dev, (rows, q_cols if name == "qkv" else out_cols), out_type)
-		c_kv, rrms = X.Tensor(dev, (rows, max(n - q_cols, 128)), X.INT8), X.Tensor(dev, (rows, max(heads, 1)), X.F32)
+
+		def poisoned(shape, dtype):
+			size = {X.INT8: 1, X.E4M3: 1, X.BF16: 2, X.F32: 4}[dtype]
+			return t(np.full(shape[:-1] + (shape[-1] * size,), pattern, np.uint8).view({1: np.uint8, 2: np.uint16, 4: np.float32}[size]), dtype)
+		c = poisoned((rows, q_cols if name == "qkv" else out_cols), out_type)
+		c_kv, rrms = poisoned((rows, max(n - q_cols, 128)), X.INT8), poisoned((rows, max(heads, 1)), X.F32)
 		outputs = [c]
-		slots = [a, rows, b, n, c]
+		slots = [ta, rows, tb, n, c]
 		if name.startswith("l2norm"):
 			slots.append(rrms)
 			outputs.append(rrms)
 		elif "residual" in name:
-			slots.append(residual)
+			slots.append(extras[0])
 		elif "dequant" in name:
-			slots.extend(scales)
+			slots.extend(extras[1])
 		elif name == "qnorm":
-			slots.append(learned)
+			slots.append(extras[2])
 		elif name == "qkv":
-			slots.extend([rrms, b_kv, c_kv])
+			slots.extend([rrms, tb_kv, c_kv])
 			outputs.extend([rrms, c_kv])
 		dev.synchronize()
 		tiles = -(-rows // meta["M_PER_BLOCK"]) * -(-n // meta["N_PER_BLOCK"])
 		_launch(shim, os.path.join(base, form), meta, (tiles, 1, 1), slots)
 		results[form] = [x.download() for x in outputs]
+	for got, want in zip(results[""], _oracle(name, k, n, q_cols, a, b, b_kv, residual, scales, learned)):
+		if not e4 and name != "geglu_i8_fast":
+			assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), name
+		elif out_type == X.E4M3:           # (the oracle adds f32 products one by one: another order, one step at most)
+			differ, beyond = e4m3_compare(got, want)
+			assert differ < 0.005 and beyond == 0.0, (name, differ, beyond)
+		else:                              # likewise; hardware transcendentals: one code
+			d = np.abs(got.astype(np.int32) - want.astype(np.int32))
+			assert d.max() <= 1 and np.mean(d != 0) < 0.005, name
 	for form, got in results.items():
 		for x, y in zip(got, results[""]):
 			assert np.array_equal(x.view(np.uint8), y.view(np.uint8)), (form, name)
+
+
+def test_the_persistent_walk_over_more_tiles_than_workgroups(shim):  # noqa: F811
+	"""The 256 x 256 kernel alone, whatever launch() takes at these sizes: 256 workgroups walk 260 tiles of K = 384 (three
+	steps: every request of a tile's last two belongs to the workgroup's next tile), int8 and in the four-wavefront e4m3
+	form, and 264 tiles through the L2-norm writer, whose rrms stores are in flight next to the next tile's loads."""
+	from oracle import strict as S
+	dev = X.Device(0)
+	t = lambda a, dtype: X.Tensor.from_numpy(dev, np.ascontiguousarray(a), dtype)
+
+	def launch(kernel, rows, n, slots):
+		dev.synchronize()
+		assert -(-rows // 256) * (n // 256) > 256
+		_launch(shim, os.path.join(_ffi.kernel_cache_dir(), kernel.name), kernel.metadata, (256, 1, 1), slots)
+
+	rng = rng_for("persistent walk")
+	m, k, n = 256 * 65, 384, 1024
+	a, b = i8_codes(rng, (m, k)), i8_codes(rng, (n, k))
+	c = t(np.full((m, n), 0x5A, np.int8), X.INT8)
+	launch(recipes.attn_q_kernel(None, k, n), m, n, [t(a, X.INT8), m, t(b, X.INT8), n, c])
+	assert np.array_equal(c.download(), S.epilogue_scale(S.gemm_i32(a, b), 1.0 / math.sqrt(k) / 64.0, 8.0))
+
+	m, n = 256 * 130, 512
+	a8, b8 = e4m3_bytes(rng, (m, k)), e4m3_bytes(rng, (n, k))
+	c = t(np.full((m, n // 2), 0x5A, np.uint8), X.E4M3)
+	launch(recipes.ffn_f_f8_kernel(None, k, n, True), m, n, [t(a8, X.E4M3), m, t(b8, X.E4M3), n, c])
+	want = S.epilogue_geglu(S.gemm_f32_seq(a8, True, b8, True), 1.0 / math.sqrt(k), 1.0, S.STORE_E4M3)
+	differ, beyond = e4m3_compare(c.download(), want)
+	assert differ < 5e-3 and beyond == 0.0, (differ, beyond)
+
+	m, k, n = 256 * 33, 256, 2048
+	a, b = i8_codes(rng, (m, k)), i8_codes(rng, (n, k))
+	for hd in (64, 128):
+		c, rrms = t(np.full((m, n), 0x5A, np.int8), X.INT8), t(np.full((m, n // (2 * hd)), 7.5, np.float32), X.F32)
+		launch(recipes.attn_kv_kernel(None, k, n, hd), m, n, [t(a, X.INT8), m, t(b, X.INT8), n, c, rrms])
+		want_c, want_r = S.epilogue_l2norm(S.gemm_i32(a, b), hd, recipes.L2_NORM_EPS, 1.0 / math.sqrt(k) / 64.0, 8.0)
+		assert np.array_equal(c.download(), want_c) and np.array_equal(rrms.download().view(np.uint32), want_r.view(np.uint32)), hd
 
 
 @pytest.mark.parametrize("name,make,out_type", [
