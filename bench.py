@@ -495,16 +495,17 @@ def single(dev, X, recipes, name, iters):
 		c = X.Tensor(dev, (M, F3), X.E4M3)
 		k = recipes.ffn_f_f8_kernel(dev, D3, 2 * F3, False)
 		fn, work, unit = (lambda: k.launch(a, b, c)), k.n_ops(a, b) / 1e12, "TFLOP/s"
-	elif name == "ffn_y_f8_config4":
-		M = 32768
+	elif name in ("ffn_y_f8_config4", "ffn_y_f8_256_rows"):
+		M = 32768 if name == "ffn_y_f8_config4" else 256
 		a = X.Tensor.from_numpy(dev, rng.integers(0x20, 0x50, (M, F), dtype=np.uint8), X.E4M3)
 		b = X.Tensor.from_numpy(dev, _rand_codes(rng, (2 * D, F)), X.INT8)
 		r = X.Tensor.from_numpy(dev, _rand_codes(rng, (M, D)), X.INT8)
 		c = X.Tensor(dev, (M, D), X.E4M3)
 		k = recipes.ffn_y_kernel(dev, D, F, False)
 		fn, work, unit = (lambda: k.launch(a, b, c, r)), k.n_ops(a, b) / 1e12, "TFLOP/s"
-	elif name in ("attn_config4", "attn_config5"):
-		T, B, H, HD, W = (8192, 4, 16, 128, 512) if name == "attn_config4" else (65536, 1, 32, 128, 4096)
+	elif name in ("attn_config4", "attn_config5", "attn_strict_64x32"):
+		# (the last: the attention of the reference's own configuration, 64 heads of 32, no window, deterministic build)
+		T, B, H, HD, W = {"attn_config4": (8192, 4, 16, 128, 512), "attn_config5": (65536, 1, 32, 128, 4096), "attn_strict_64x32": (16384, 1, 64, 32, 0)}[name]
 		rows = T * B
 		q = X.Tensor.from_numpy(dev, _rand_codes(rng, (rows, H * HD)), X.INT8)
 		kv = X.Tensor.from_numpy(dev, _rand_codes(rng, (rows, 2 * H * HD)), X.INT8)
@@ -513,8 +514,8 @@ def single(dev, X, recipes, name, iters):
 		tp = X.Tensor.from_numpy(dev, (0.5 + rng.random(H)).astype(np.float32), X.F32)
 		o = X.Tensor(dev, (rows, H * HD), X.INT8)
 		l = X.Tensor(dev, (H, rows), X.F32)
-		k = recipes.attn_kernel(dev, H, HD, False)
-		pairs = W * (W - 1) // 2 + (T - W) * W
+		k = recipes.attn_kernel(dev, H, HD, name == "attn_strict_64x32")
+		pairs = W * (W - 1) // 2 + (T - W) * W if W else T * (T - 1) // 2
 		fn, work, unit = (lambda: k.launch(q, kv, sk, sv, tp, o, l, W, B)), 4.0 * HD * H * B * pairs / 1e12, "TOPS"
 	elif name == "attn_row_scaled_config5":
 		T, H, HD, W = 65536, 32, 128, 4096
@@ -632,7 +633,8 @@ def single(dev, X, recipes, name, iters):
 	                  "rate": work / med, "unit": unit}))
 
 
-ONLY_TARGETS = ("ffn_f_config2", "ffn_f_f8_config3", "ffn_y_f8_config4", "attn_config4", "attn_config5", "attn_row_scaled_config5",
+ONLY_TARGETS = ("ffn_f_config2", "ffn_f_f8_config3", "ffn_y_f8_config4", "ffn_y_f8_256_rows", "attn_config4", "attn_config5",
+                "attn_strict_64x32", "attn_row_scaled_config5",
                 "attn_d_q_config4", "attn_d_kv_config4", "decode_config5",
                 "decode_dense_config5", "attn_kv_config4", "attn_qkv_config4", "ffn_f_config4", "attn_y_config4", "rms_norm_config4")
 

@@ -709,7 +709,6 @@ void kernel(
 		// takes them as if that were the maximum (sgn * ext_ref - 12582912 is that extreme's dot product, exactly)
 		if constexpr (!STRICT) {
 			m = ROW_SCALES ? fmaf32(ext_ref * sgn, temperature, HEADROOM) : fmaf32(fmaf32(ext_ref, sgn, -DOT_BIAS), temperature, HEADROOM);
-			lift = 1.0f;
 		}
 
 		// ---- finish (cuda/attn_fwd_i8.cuh:293-351): the lane pair holds partial sums (s0, s2) and (s1, s3)
@@ -724,9 +723,6 @@ void kernel(
 			l_out[(size_t)head * ((size_t)gridDim.z * seq_len) + row_base + qi] = sfu::lg2(total) + m;
 		}
 		f32 inv = sfu::rcp(total);
-		if constexpr (!STRICT) {
-			inv = inv * sfu::rcp(lift);
-		}
 #if X17_ATTN_ROW_SCALES
 		f32 const head_out_scale = out_scale[head];
 		if constexpr (OUT_BF16) {
