@@ -34,6 +34,8 @@ def test_forms_of_a_kernel_pass_the_code_object_scans(tmp_path):
 @pytest.mark.parametrize("make,picks", [
 	# few tiles: the smallest form that covers the chip ...
 	(lambda: recipes.attn_q_kernel(None, 2048, 2048), {256: "s64x4", 512: "s64x4", 4096: "s128x2", 32768: ""}),
+	# (a tile more than a round of 256 x 256 begins another: 8192 rows fill one)
+	(lambda: recipes.attn_q_kernel(None, 2048, 2048), {8192: "", 8320: "s128x2", 12288: ""}),
 	(lambda: recipes.ffn_y_kernel(None, 2048, 8192, False), {256: "s64x4", 1024: "s128x2", 4096: "", 32768: ""}),
 	(lambda: recipes.ffn_y_kernel(None, 4096, 16384, False, X.E4M3, X.E4M3), {320: "s128x4", 16384: ""}),
 	# ... and with many of them the 256 x 256 kernel also where K is short: 131072 rows x 4096 columns, K = 512: 310 us and
@@ -42,7 +44,7 @@ def test_forms_of_a_kernel_pass_the_code_object_scans(tmp_path):
 	(lambda: recipes.attn_kv_kernel(None, 256, 2048, 64), {256: "s64x4", 8192: "", 262144: ""}),
 	# (a short product of e4m3 operands is faster in small tiles at any size: 16384 x 4096, K = 256: 46 us and 63)
 	(lambda: recipes.ffn_f_f8_kernel(None, 384, 512, True), {256: "s128x2", 131072: "s128x2"}),
-], ids=["int8", "e4m3 x int8", "e4m3", "int8, short K", "L2 norm, short K", "e4m3, short K"])
+], ids=["int8", "int8, past a round", "e4m3 x int8", "e4m3", "int8, short K", "L2 norm, short K", "e4m3, short K"])
 def test_the_form_a_launch_takes(make, picks):
 	kernel = make()
 	assert {rows: kernel.form(rows) for rows in picks} == picks

@@ -1078,63 +1078,68 @@ Status GemmKernel::launch(GemmArgs const &args) {
 
 // ---- which tile size a GEMM launch takes.
 // Estimated microseconds of a launch: measured curves over the number of its tiles, in units of the 256 compute units,
-// each point fixed + per_k * K / 1024 (K in bytes) and straight lines between them.  Fitted on an MI355X to 689 launches of
-// 256 .. 65536 token rows, 1024 .. 16384 columns and K = 128 .. 16384; a fit is 3-9 % off in the mean of a curve and up to
-// 40 % at single points (the two-stage form at 512 tiles of K = 512).  Over those and 255 launches of other widths the
-// form taken is 1 % slower than the best one in the mean.  us measured at 4096 columns:
-//                        rows:  256    512   1024   2048   4096  16384
-//   int8, K = 2048   64 x 64    6.1   10.3   19.3   44.3   89.3    348
-//           128 x 128, 4 / 2  8.7/8.4 8.9/8.6 10.3/10.1 23.3/19.6 43.4/36.8 166/143
-//                   256 x 256  19.5   19.6   20.4   24.3   34.1    118
-//   int8, K = 256     64 x 64   4.4    6.7   11.3   21.4   40.4    165
-//           128 x 128, 4 / 2  4.5/4.4 4.7/4.4 5.1/4.9 8.3/6.4 14.8/10.9 52.8/38.3
-//                   256 x 256   7.3    7.6    8.2    9.2   12.4   34.9
+// each point fixed + per_k * K / 1024 (K in bytes) and straight lines between them.  Two points close behind each other
+// (1 and 1.02 rounds) are the step where one tile more begins another round: the 256 x 256 kernel at K = 2048 and 4096
+// columns takes 35 us at 4096 rows and 48 at 4160, the two-stage 128 x 128 one 41 and 48.  Fitted on an MI355X to 1721
+// launches of 256 .. 65536 token rows, 1024 .. 32768 columns and K = 128 .. 16384, row counts just past a round among them,
+// below 4096 rows with weights that no cache holds (the next layer's: the two-stage 128 x 128 form, ahead with weights in
+// L2, loses to four stages there: 256 rows, K = 2048, 8.4 / 8.7 us and 16 / 12).  A fit is 3-10 % off in the mean of a curve
+// and up to 40 % at single points; over those launches the form taken is 0.3 % slower than the best one in the mean (16 % at
+// most), over 460 of other widths 0.6 % (36 %).  us measured at 4096 columns:
+//                        rows:  256    512   1024   2048   4096   8192
+//   int8, K = 2048   64 x 64    8.1   14.1   27.1   56.2    107    215
+//           128 x 128, 4 / 2   12/16  12/16  13/16  26/22  48/41  95/78
+//                   256 x 256  21.5   21.4   22.0   24.5   35.0   63.9
+//   int8, K = 256     64 x 64   4.0    6.7   11.8   22.4   42.9   83.8
+//           128 x 128, 4 / 2  4.3/4.3 4.4/4.4 5.0/4.9 8.6/6.5 15.3/11.2 27.7/19.5
+//                   256 x 256   7.6    7.9    8.4    9.5   12.6   20.3
 namespace gemm_cost {
 	struct Point { double tiles, fixed, per_k; };          // tiles / 256
 	struct Curve {
-		Point points[6];                                    // (unused ones at the end are zero)
+		Point points[8];                                    // (unused ones at the end are zero)
+		double rounds = 0.0;                                      // past the last point: the share of the time that goes with rounds begun
 		double us(size_t tiles, double k) const {
 			double const n = double(tiles) / double(COMPUTE_UNITS);
 			auto at = [&](Point const &p) { return p.fixed + p.per_k * (k / 1024.0); };
 			if (n <= points[0].tiles) return at(points[0]);
 			size_t i = 1;
-			for (; i < 6 && points[i].tiles != 0.0; ++i) {
+			for (; i < 8 && points[i].tiles != 0.0; ++i) {
 				Point const &a = points[i - 1], &b = points[i];
 				if (n <= b.tiles) return at(a) + (at(b) - at(a)) * (n - a.tiles) / (b.tiles - a.tiles);
 			}
-			return at(points[i - 1]) * n / points[i - 1].tiles;      // whole rounds behind each other
+			return at(points[i - 1]) * (rounds * std::ceil(n) + (1.0 - rounds) * n) / points[i - 1].tiles;
 		}
 	};
 	struct Curves { Curve large, tile64, tile128_deep, tile128; };   // 256 x 256 | 64 x 64 | 128 x 128, four stages | two
 	static Curves const CURVES[4] = {
 		{   // int8
-			{{{0.125, 4.7, 7.3}, {0.5, 6.4, 8.8}, {1, 8.7, 12.6}, {1.25, 11.2, 19.1}, {2, 14.8, 24.9}, {4, 22.8, 46.7}}},
-			{{{0.25, 3.8, 1.0}, {1, 3.9, 1.2}, {1.25, 5.7, 2.3}, {2, 4.2, 3.5}}},
-			{{{0.25, 3.6, 2.5}, {1, 3.9, 3.8}, {1.25, 5.8, 7.4}, {2, 6.6, 8.7}, {4, 9.7, 15.9}}},
-			{{{0.25, 3.3, 2.6}, {1, 3.3, 4.8}, {1.25, 4.2, 5.6}, {2, 4.6, 7.4}, {2.5, 6.2, 11.4}, {4, 6.2, 14.7}}},
+			{{{0.125, 4.9, 7.5}, {0.5, 6.6, 8.3}, {1, 8.7, 12.5}, {1.02, 10.5, 18.2}, {2, 13.9, 23.5}, {2.02, 15.4, 30.0}, {3, 16.6, 35.7}}, 0.3},
+			{{{0.25, 3.5, 1.1}, {1, 3.5, 1.6}, {1.02, 5.3, 2.7}, {2, 5.7, 4.6}, {4, 7.9, 8.6}}},
+			{{{0.25, 3.6, 2.7}, {1, 3.7, 4.2}, {1.02, 6.0, 6.3}, {2, 6.0, 9.1}, {2.02, 8.2, 10.1}, {4, 10.3, 17.0}, {4.02, 12.8, 17.4}, {6, 14.2, 25.1}}},
+			{{{0.25, 3.0, 4.3}, {1, 3.3, 5.7}, {1.02, 4.3, 5.1}, {2, 4.2, 8.3}, {2.02, 5.7, 10.9}, {4, 7.1, 15.3}, {4.02, 8.2, 18.1}, {6, 8.6, 23.5}}},
 		},
 		{   // int8, head-normalising writers (wavefronts of 32 x 128)
-			{{{0.125, 5.4, 7.0}, {0.5, 6.4, 7.8}, {1, 7.9, 11.9}, {1.25, 10.8, 18.4}, {2, 13.7, 23.0}, {4, 17.4, 47.0}}},
-			{{{0.25, 4.5, 1.4}, {1, 4.9, 1.4}, {1.25, 7.5, 3.0}, {2, 6.4, 3.4}}},
-			{{{0.25, 4.8, 2.6}, {1, 5.1, 3.5}, {1.25, 7.7, 6.4}, {2, 8.4, 9.1}, {4, 12.7, 17.2}}},
-			{{{0.25, 4.5, 2.5}, {1, 4.7, 3.8}, {1.25, 5.3, 5.8}, {2, 6.2, 7.3}, {2.5, 8.1, 11.4}, {4, 8.4, 15.0}}},
+			{{{0.125, 5.4, 7.4}, {0.5, 6.3, 7.8}, {1, 7.2, 12.1}, {1.02, 9.5, 18.1}, {2, 11.9, 22.0}, {2.02, 12.4, 30.2}, {3, 12.6, 36.4}}, 0.3},
+			{{{0.25, 4.7, 1.4}, {1, 5.0, 1.6}, {1.02, 7.0, 3.4}, {2, 7.3, 5.9}, {4, 12.3, 7.9}}},
+			{{{0.25, 4.9, 2.7}, {1, 4.8, 4.5}, {1.02, 7.5, 6.4}, {2, 7.3, 9.4}, {2.02, 10.8, 10.0}, {4, 12.2, 18.7}, {4.02, 16.8, 17.5}, {6, 18.8, 26.3}}},
+			{{{0.25, 4.2, 4.2}, {1, 3.9, 6.6}, {1.02, 5.2, 5.4}, {2, 5.1, 8.5}, {2.02, 7.4, 11.1}, {4, 7.5, 17.2}, {4.02, 10.4, 18.1}, {6, 11.3, 24.2}}},
 		},
 		{   // e4m3 x e4m3
-			{{{0.125, 9.9, 7.1}, {0.5, 12.6, 7.8}, {1, 18.3, 10.5}, {1.25, 25.3, 17.6}, {2, 33.1, 21.1}, {4, 47.1, 43.6}}},
-			{{{0.25, 3.2, 1.2}, {1, 3.0, 1.7}, {1.25, 4.6, 2.9}, {2, 3.3, 4.0}}},
-			{{{0.25, 3.7, 2.9}, {1, 4.4, 4.0}, {1.25, 7.0, 6.8}, {2, 8.1, 8.2}, {4, 11.8, 16.2}}},
-			{{{0.25, 3.3, 3.1}, {1, 3.6, 5.0}, {1.25, 5.4, 5.7}, {2, 6.5, 7.3}, {2.5, 7.9, 11.2}, {4, 8.6, 15.2}}},
+			{{{0.125, 9.7, 7.7}, {0.5, 12.5, 8.2}, {1, 18.7, 10.5}, {1.02, 23.6, 17.1}, {2, 28.6, 21.0}, {2.02, 36.9, 27.4}, {3, 36.0, 33.9}}, 0.3},
+			{{{0.25, 3.7, 1.1}, {1, 3.6, 1.6}, {1.02, 4.5, 3.0}, {2, 5.0, 4.7}, {4, 6.3, 9.0}}},
+			{{{0.25, 3.9, 3.0}, {1, 4.3, 4.6}, {1.02, 6.9, 6.6}, {2, 6.5, 8.9}, {2.02, 9.4, 10.5}, {4, 11.5, 17.2}, {4.02, 14.1, 18.5}, {6, 17.2, 26.4}}},
+			{{{0.25, 3.3, 4.5}, {1, 3.5, 6.6}, {1.02, 5.0, 5.7}, {2, 5.8, 8.1}, {2.02, 6.8, 11.1}, {4, 8.7, 16.2}, {4.02, 10.4, 18.3}, {6, 12.0, 24.6}}},
 		},
 		{   // e4m3 x int8
-			{{{0.125, 6.0, 15.3}, {0.5, 8.0, 15.4}, {1, 11.3, 21.6}, {1.25, 13.7, 35.9}, {2, 19.5, 44.4}, {4, 24.2, 89.5}}},
-			{{{0.25, 2.5, 3.2}, {1, 2.6, 3.7}, {1.25, 3.8, 6.8}, {2, 2.7, 7.0}}},
-			{{{0.25, 3.0, 7.1}, {1, 3.2, 7.9}, {1.25, 5.0, 14.6}, {2, 5.3, 16.3}, {4, 7.5, 32.6}}},
-			{{{0.25, 2.8, 7.1}, {1, 3.2, 7.7}, {1.25, 3.7, 12.0}, {2, 3.7, 14.4}, {2.5, 5.3, 19.8}, {4, 4.3, 28.7}}},
+			{{{0.125, 6.2, 15.4}, {0.5, 8.3, 15.3}, {1, 11.2, 21.7}, {1.02, 12.8, 36.5}, {2, 17.1, 41.5}, {2.02, 18.9, 59.0}, {3, 19.6, 67.4}}, 0.3},
+			{{{0.25, 2.9, 3.1}, {1, 3.0, 3.7}, {1.02, 3.9, 6.5}, {2, 4.3, 8.2}, {4, 5.5, 14.2}}},
+			{{{0.25, 3.2, 7.1}, {1, 3.5, 7.9}, {1.02, 5.1, 14.7}, {2, 5.1, 16.0}, {2.02, 6.9, 21.8}, {4, 8.1, 32.0}, {4.02, 9.9, 37.3}, {6, 11.1, 49.8}}},
+			{{{0.25, 3.1, 7.1}, {1, 3.4, 7.7}, {1.02, 3.9, 11.4}, {2, 3.7, 14.1}, {2.02, 4.3, 19.0}, {4, 5.3, 28.2}, {4.02, 5.7, 32.4}, {6, 5.7, 43.8}}},
 		},
 	};
-	// What a small form has to gain by the estimate: the curves' spread.  Without it 10 of the 689 launches took a form
-	// slower than the 256 x 256 kernel, one by half; with it three do, by 6 % at most.
-	static constexpr double MARGIN = 1.06;
+	// What a small form has to gain by the estimate: the curves' spread.  Without it 23 of the 1721 launches take a form
+	// slower than the 256 x 256 kernel by more than 2 %, one by a fifth; with it 12 do, by 9 % at most.
+	static constexpr double MARGIN = 1.05;
 }
 
 GemmKernel::Small const *GemmKernel::form_for(size_t a_rows) const {
