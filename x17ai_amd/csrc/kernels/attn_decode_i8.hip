@@ -169,7 +169,8 @@ void kernel(
 	// then walk a sequence's rows nearly in step, which the DRAM pages like (64 sequences x 1024 keys: 57 us with 2, 60
 	// with 4; x 4096: 193 and 205) -- four where it is short (64 x 128: 11.9 and 10.9).  256 threads: eight, unless that
 	// reaches past a short window (128 x 1024: 98 us with 8, 106 with 4; 64 x 128: 17.5 and 16.5).  512 threads: eight
-	// (16 x 512: 10.9 us with 8, 11.2 with 4, 12.5 with 16).  1024: four.
+	// (16 x 512: 10.9 us with 8, 11.2 with 4, 12.5 with 16; against 16, ragged caches and windows of 2048 keys are 2-5 %
+	// faster, 30 .. 64 full caches of 4096 keys 1-2 % slower).  1024: four.
 	constexpr u32 MANY = dt::THREADS_PER_BLOCK == 128 ? 2 : dt::THREADS_PER_BLOCK <= 512 ? 8 : 4;
 	constexpr u32 SHORT_BYTES = dt::THREADS_PER_BLOCK == 128 ? 32 * 1024 : dt::THREADS_PER_BLOCK == 256 ? 16 * 1024 : 0;
 	if (SHORT_BYTES != 0 && n_keys * HD <= SHORT_BYTES) {     // (widths without a short case carry one copy of the loop)
