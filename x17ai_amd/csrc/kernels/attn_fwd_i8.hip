@@ -407,14 +407,20 @@ void kernel(
 		sc_src = (half == 0 ? k_scale : v_weight) + (size_t)head * ((size_t)gridDim.z * seq_len) + row_base
 		         + (size_t)kb_begin * at::KV_PER_STEP + qlane;
 #endif
-#define X17_REQUEST_SCALES(ring_slot) \
-		if (wave == 0) { \
-			__builtin_amdgcn_global_load_lds(X17_GLOBAL_PTR(sc_src), X17_LDS_PTR(smem + at::SCALE_RING_OFFSET + (ring_slot) * at::SCALE_TILE_BYTES), 4, 0, 0); \
-		}
+		// (by hand like the tile requests: in front of an LDS read the compiler waits for every direct-to-LDS load of its own,
+		// and with it for all that were requested behind that one.  With the builtin the first wavefront drained its three
+		// steps of prefetch every step: 65536 tokens, 32 heads of 128, window 4096: 3869 -> 3815 us; 1024 tokens, 8 heads
+		// of 64: 15.5 -> 15.1 us)
+		auto request_scales = [&](u32 ring_slot) __attribute__((always_inline)) {
+			if (wave == 0) {
+				asm volatile("s_add_i32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, off"
+				             :: "s"(lds_wave), "s"(at::SCALE_RING_OFFSET + ring_slot * at::SCALE_TILE_BYTES), "v"(sc_src) : "memory", "m0", "scc");
+			}
+		};
 		auto request_tiles = [&]<int SLOT>(u32 s) __attribute__((always_inline)) {
 			if constexpr (SLOT >= 0) {
 				if constexpr (ROW_SCALES) {
-					X17_REQUEST_SCALES((SLOT + 3) % 4)
+					request_scales((SLOT + 3) % 4);
 					sc_src += at::KV_PER_STEP;
 				}
 				if (CPR == 8 || stager) {
@@ -427,7 +433,7 @@ void kernel(
 			} else {
 				bool const more = at::further_tile_exists(s, n_steps);
 				if constexpr (ROW_SCALES) {
-					X17_REQUEST_SCALES((s + 3) % at::RING)
+					request_scales((s + 3) % at::RING);
 					sc_src += __builtin_amdgcn_readfirstlane(more ? at::KV_PER_STEP : 0u);
 				}
 				if (CPR == 8 || stager) {
@@ -671,7 +677,7 @@ void kernel(
 			load_to_lds_16(smem + at::RAW_V_RING_OFFSET + stage_lds, src, stage_v_src);
 			X17_UNROLL for (u32 j = 0; j < 3; ++j) {
 				if constexpr (ROW_SCALES) {
-					X17_REQUEST_SCALES(j)
+					request_scales(j);
 					sc_src += at::KV_PER_STEP;
 				}
 				load_to_lds_16(smem + at::K_RING_OFFSET + j * at::K_TILE_BYTES + stage_lds, src + j * TILE_STEP_BYTES, stage_k_src);
