@@ -14,7 +14,7 @@ constexpr unsigned THREADS_PER_BLOCK = at::THREADS_PER_BLOCK;
 constexpr unsigned Q_PER_BLOCK = at::Q_PER_BLOCK;
 // raw int8 K / V tiles are fetched PREFETCH steps ahead into rings of PREFETCH + 1 slots; one step before its use a
 // tile is widened to f16 by the threads that fetched it, into one of two f16 tiles
-constexpr unsigned PREFETCH = 2;
+constexpr unsigned PREFETCH = 3;
 constexpr unsigned RING = PREFETCH + 1;
 // 64 accumulators of dQ^T, the f16 dO fragments of all of head_dim and the forward's Q fragments stay in registers:
 // two wavefronts per SIMD

@@ -17,7 +17,7 @@
 //   * S^T = K . Q^T on v_mfma_i32_32x32x32_i8 exactly as in the forward (keys are the "A" operand: a lane owns one
 //     query and 8 keys of each 16-key tile).
 //   * dP^T = V . dO^T and dQ^T += K^T . dS^T run on v_mfma_f32_32x32x16_f16.  K and V arrive as int8 (global -> LDS
-//     directly, two steps ahead) and are widened to f16 once per workgroup, LDS -> LDS, one step ahead, by the
+//     directly, three steps ahead) and are widened to f16 once per workgroup, LDS -> LDS, one step ahead, by the
 //     threads that fetched them: K into the granule layout that ds_read_b64_tr_b16 reads transposed (the "A" operand
 //     K^T needs eight keys of one dim per lane), V into swizzled rows (the "A" operand V needs eight dims of one key).
 //   * dO is bf16 in memory.  Everything is linear in dO_i, so each query row is scaled by a power of two that brings
@@ -178,17 +178,8 @@ void kernel(
 			v_f16_dst0 = vrow_offset(tid / CPR, 2 * (tid % CPR));
 			v_f16_dst1 = vrow_offset(tid / CPR, 2 * (tid % CPR) + 1);
 		}
-		auto issue_kv_load = [&](u32 kb, u32 slot) {
-			if (stager) {
-				i8 const *src = kv_head + (size_t)(kb * at::KV_PER_STEP) * KV_STRIDE;
-				u8 *k_dst = smem + bt::RAW_K_RING_OFFSET + slot * bt::RAW_TILE_BYTES + wave * 1024;
-				u8 *v_dst = smem + bt::RAW_V_RING_OFFSET + slot * bt::RAW_TILE_BYTES + wave * 1024;
-				__builtin_amdgcn_global_load_lds(X17_GLOBAL_PTR(src + stage_k_src), X17_LDS_PTR(k_dst), 16, 0, 0);
-				__builtin_amdgcn_global_load_lds(X17_GLOBAL_PTR(src + stage_v_src), X17_LDS_PTR(v_dst), 16, 0, 0);
-			}
-		};
-		auto widen = [&](u32 slot, u32 buf) {
-			if (stager) {
+		auto widen = [&](u32 slot, u32 buf) __attribute__((always_inline)) {
+			if (CPR == 8 || stager) {          // (head_dim 128: every thread stages)
 				u32 w[8];
 				widen16(*reinterpret_cast<v4u const *>(smem + bt::RAW_K_RING_OFFSET + slot * bt::RAW_TILE_BYTES + tid * 16), w);
 				u8 *kd = smem + bt::K_F16_OFFSET + buf * bt::F16_TILE_BYTES + k_f16_dst;
@@ -200,15 +191,27 @@ void kernel(
 				*reinterpret_cast<v4u *>(vd + v_f16_dst1) = v4u{w[4], w[5], w[6], w[7]};
 			}
 		};
-		// two loads in flight per staging thread and prefetched step; they complete in issue order
-		auto wait_steps_in_flight = [&](u32 steps) {
-			if (steps >= 1) {
-				__builtin_amdgcn_s_waitcnt(0x0F72);          // vmcnt(2)
-			} else {
-				__builtin_amdgcn_s_waitcnt(0x0F70);          // vmcnt(0)
+		constexpr u32 TILE_STEP_BYTES = at::KV_PER_STEP * KV_STRIDE;
+		u32 const lds_wave = (u32)(size_t)X17_LDS_PTR(smem) + wave * 1024;
+		i8 const *src = kv_head + (size_t)(kb_begin * at::KV_PER_STEP) * KV_STRIDE;      // the tile the next request takes
+		auto request = [&](u32 slot) __attribute__((always_inline)) {
+			if (CPR == 8 || stager) {
+				// (a scalar write of M0 needs one wait state before a direct-to-LDS load reads it)
+				// (the slot is the same in every lane; reading its offset from the first one tells the compiler so)
+				u32 const slot_bytes = __builtin_amdgcn_readfirstlane(slot * bt::RAW_TILE_BYTES);
+				asm volatile("s_add_i32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3"
+				             :: "s"(lds_wave), "s"(bt::RAW_K_RING_OFFSET + slot_bytes), "v"(stage_k_src), "s"(src) : "memory", "m0", "scc");
+				asm volatile("s_add_i32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3"
+				             :: "s"(lds_wave), "s"(bt::RAW_V_RING_OFFSET + slot_bytes), "v"(stage_v_src), "s"(src) : "memory", "m0", "scc");
 			}
 		};
-		static_assert(bt::PREFETCH == 2, "the waits below are written for a prefetch distance of 2");
+		// the first tiles are requested ahead of the per-query set-up and land behind it
+		__syncthreads();                      // previous head's tiles are no longer read
+		// (every workgroup walks at least four tiles: 0 .. 3 exist)
+		X17_UNROLL for (u32 j = 0; j < bt::PREFETCH; ++j) {
+			request(j);
+			src += TILE_STEP_BYTES;
+		}
 
 		// ---- per-query set-up
 		v4i qf[K_SLICES];
@@ -265,15 +268,6 @@ void kernel(
 		}
 		sink_dot += partner_i32(sink_dot, half);
 		f32 const p_sink = sfu::ex2(f32(sink_dot) * temperature - l_hat);
-		f32 const w_sink = p_sink * ((dps8 - d8) * 0.125f);
-		v16f dq_acc[D_BLOCKS];               // dQ^T: lane = query, register r = dim 32 db + 8 (r / 4) + 4 half + r % 4
-		X17_UNROLL for (u32 db = 0; db < D_BLOCKS; ++db) {
-			X17_UNROLL for (int r4 = 0; r4 < 4; ++r4) {
-				u32 const word = *reinterpret_cast<u32 const *>(sink_k + (size_t)head * HD + 32 * db + 8 * r4 + 4 * half);
-				X17_UNROLL for (int b = 0; b < 4; ++b) dq_acc[db][4 * r4 + b] = w_sink * i8_of(word, b);
-			}
-		}
-
 		// lane offsets of the operand fragments (the forward's transposed-read addressing for K^T)
 		u32 kt_lane_off[D_BLOCKS];
 		[[maybe_unused]] u32 kt_lane_off8[D_BLOCKS];
@@ -285,62 +279,106 @@ void kernel(
 			}
 		}
 
-		// ---- pipeline prologue
-		__syncthreads();                      // previous head's tiles are no longer read
-		X17_UNROLL for (u32 j = 0; j < bt::PREFETCH; ++j) {
-			if (j < n_steps) issue_kv_load(kb_begin + j, j);
+		// ---- the key loop, built like the forward's (attn_fwd_i8.hip): a wave's steps fall into runs -- nothing to do, the
+		// window's edge, fully visible, the diagonal, nothing to do -- each its own loop; every step requests a tile by
+		// hand (past the end the last one again, into a slot nobody reads any more), so the waits are constants; the long
+		// run is unrolled over the four slots of the rings, so that every LDS address is a register plus an immediate.
+		// Per score what is left is a fused multiply-add, an exponential, a multiplication and half a conversion:
+		//  * The score accumulators start at the bits of 1.5 * 2^23: the int32 sum, read as a float, is 12582912 + dot
+		//    exactly, and one fused multiply-add makes the exponent's argument of it.  Its subtrahend mb, t * 12582912 + L
+		//    rounded, is constant per query here; so is the rest that the rounding leaves, and 2^rest is taken out of dq at the end.
+		//  * The dP accumulators start at -D, so that they end as dP - D.
+		//  * The 1 / 8 of dO . v (v codes) goes into the exponent.
+		// A temperature so large that the rest would matter (or one that is no number) takes the general step throughout,
+		// with accumulators from zero and a conversion per score.
+		// Bound by the rate at which a wavefront issues (one instruction in about ten clocks, two wavefronts per SIMD): a fully
+		// visible step is 183 instructions; it was 357, around requests that were drained in the step that made them.  16 heads
+		// of 128, 4 x 8192 tokens: 11.5 -> 7 us per 32 keys of window; window 512: 333 -> 272 us, of which 150 are set-up and output.
+		constexpr f32 DOT_BIAS = 12582912.0f;
+		f32 const head_temperature = u2f(__builtin_amdgcn_readfirstlane(f2u(attn_temperature[head])));
+		bool const biased = __builtin_fabsf(head_temperature) * (BASE_TEMPERATURE * 32.0f) <= 1.0f;      // |t| <= 1: lg2 of a u32 is at most 32
+		f32 const l_eighth = l_hat + 3.0f;
+		f32 const prod = biased ? temperature * DOT_BIAS : 0.0f;
+		f32 const low = biased ? fmaf32(temperature, DOT_BIAS, -prod) : 0.0f;
+		f32 const mb = prod + l_eighth;
+		f32 const rest = biased ? ((prod - mb) + l_eighth) + low : 0.0f;      // |rest| <= 1
+		f32 const fine = sfu::ex2(rest), inv_fine = sfu::ex2(-rest);
+		// dQ starts from the sink's share: the outer product of the sink key and w_sink by one matrix instruction per 32 dims.
+		// The weight is cut into three bf16 numbers of eight significand bits each (exact), in key slots 0 to 2 of the "B"
+		// operand next to three copies of the key's code.
+		f32 const w_sink = (p_sink * ((dps8 - d8) * 0.125f)) * fine;
+		f32 const w_high = u2f(f2u(w_sink) & 0xFFFF0000u);
+		f32 const w_left = w_high == w_sink ? 0.0f : w_sink - w_high;
+		f32 const w_mid = u2f(f2u(w_left) & 0xFFFF0000u);
+		f32 const w_low = w_left - w_mid;
+		v4u const w_slots = {half == 0 ? (f2u(w_high) >> 16) | f2u(w_mid) : 0u, half == 0 ? f2u(w_low) >> 16 : 0u, 0u, 0u};
+		v16f dq_acc[D_BLOCKS];               // dQ^T: lane = query, register r = dim 32 db + 8 (r / 4) + 4 half + r % 4
+		X17_UNROLL for (u32 db = 0; db < D_BLOCKS; ++db) {
+			u32 const code = f2u((f32)(i32)sink_k[(size_t)head * HD + 32 * db + qlane]) & 0xFFFF0000u;      // (int8 is exact in bf16)
+			v4u const k_slots = {half == 0 ? (code >> 16) | code : 0u, half == 0 ? code >> 16 : 0u, 0u, 0u};
+			v16f const zero = {0};
+			dq_acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, k_slots), __builtin_bit_cast(v8bf, w_slots), zero, 0, 0, 0);
 		}
-		wait_steps_in_flight((n_steps < bt::PREFETCH ? n_steps : bt::PREFETCH) - 1);
-		widen(0, 0);
+		v16i s_bias;
+		v16f neg_d8;
+		X17_UNROLL for (int r = 0; r < 16; ++r) {
+			s_bias[r] = biased ? 0x4B400000 : 0;
+			neg_d8[r] = -d8;
+		}
+		asm volatile("" : "+v"(s_bias), "+v"(neg_d8));      // (kept in registers: rebuilding them per step would cost what they save)
 
-		for (u32 i = 0; i < n_steps; ++i) {
-			u32 const kb = kb_begin + i;
-			u32 const slot = i % bt::RING;
-			// raw tile i + 1 has landed (this thread's chunks); at most step i + 2's loads stay in flight after the issue below
-			wait_steps_in_flight(0);
-			__builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0): own LDS traffic of step i - 1 is complete
-			__builtin_amdgcn_s_barrier();                // ... and so is everybody else's: tiles i are visible
-			if (i + bt::PREFETCH < n_steps) {
-				issue_kv_load(kb + bt::PREFETCH, (i + bt::PREFETCH) % bt::RING);
+		u32 k_lane_off[K_SLICES], v_lane_off[D_SLICES];
+		X17_UNROLL for (u32 sl = 0; sl < K_SLICES; ++sl) k_lane_off[sl] = k_chunk_offset(qlane, 2 * sl + half);
+		X17_UNROLL for (u32 sl = 0; sl < D_SLICES; ++sl) v_lane_off[sl] = vrow_offset(qlane, 2 * sl + half);
+
+		// SLOT: the step's position in the rings (s % RING) as a compile-time number, or -1 for "compute it"; SLOT >= 0 also
+		// says that tile s + 4 exists (the caller's loop bound)
+		auto stage = [&]<int SLOT>(u32 s) __attribute__((always_inline)) {
+			__builtin_amdgcn_s_waitcnt(0x0F72);          // vmcnt(2): tile s + 1 has landed (this thread's chunks), s + 2 may be in flight
+			__builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0): own LDS traffic of step s - 1 is complete
+			__builtin_amdgcn_s_barrier();                // ... and so is everybody else's: tiles s are visible
+			// step s requests tile min(s + 3, last) into the slot of tile s - 1, which nobody reads any more
+			request(SLOT >= 0 ? (SLOT + 3) % bt::RING : (s + 3) % bt::RING);
+			if (SLOT >= 0 || at::further_tile_exists(s, n_steps)) {
+				src += TILE_STEP_BYTES;
 			}
-			if (i + 1 < n_steps) {
-				widen((i + 1) % bt::RING, (i + 1) & 1);
-			}
-			if (kb < wave_kb_first || kb > wave_kb_last) {
-				continue;
-			}
+		};
+		static_assert(bt::PREFETCH == 3 && bt::RING == 4 && at::PREFETCH == 3, "the waits, the requests and the unrolled run are written for rings of four");
+		auto compute = [&]<bool MASKED, int SLOT>(u32 i) __attribute__((always_inline)) {
+			u32 const slot = SLOT >= 0 ? (u32)SLOT : i % bt::RING;
+			u32 const buf = SLOT >= 0 ? (u32)SLOT & 1u : i & 1u;
 			u8 const *k_raw = smem + bt::RAW_K_RING_OFFSET + slot * bt::RAW_TILE_BYTES;
-			u8 const *k_f16 = smem + bt::K_F16_OFFSET + (i & 1) * bt::F16_TILE_BYTES;
-			u8 const *v_f16 = smem + bt::V_F16_OFFSET + (i & 1) * bt::F16_TILE_BYTES;
-
-			// S^T block: rows = 32 keys, columns = this wave's 32 queries
-			v16i s_acc = {0};
+			u8 const *k_f16 = smem + bt::K_F16_OFFSET + buf * bt::F16_TILE_BYTES;
+			u8 const *v_f16 = smem + bt::V_F16_OFFSET + buf * bt::F16_TILE_BYTES;
+			// S^T block: rows = 32 keys, columns = this wave's 32 queries; dP'^T - D' (times 8: v codes) for the same keys
+			v16i s_acc = s_bias;
 			X17_UNROLL for (u32 s = 0; s < K_SLICES; ++s) {
-				v4i kf = *reinterpret_cast<v4i const *>(k_raw + k_chunk_offset(qlane, 2 * s + half));
+				v4i const kf = *reinterpret_cast<v4i const *>(k_raw + k_lane_off[s]);
 				s_acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf, qf[s], s_acc, 0, 0, 0);
 			}
-			// dP'^T block (times 8: v codes): rows = the same 32 keys
-			v16f dp_acc = {0};
+			if constexpr (MASKED) {
+				if (!biased) {
+					X17_UNROLL for (int r = 0; r < 16; ++r) s_acc[r] = (i32)f2u(f32(s_acc[r]));
+				}
+			}
+			v16f dp_acc = neg_d8;
 			X17_UNROLL for (u32 sl = 0; sl < D_SLICES; ++sl) {
-				v8h const vf = *reinterpret_cast<v8h const *>(v_f16 + vrow_offset(qlane, 2 * sl + half));
+				v8h const vf = *reinterpret_cast<v8h const *>(v_f16 + v_lane_off[sl]);
 				dp_acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, dofrag[sl], dp_acc, 0, 0, 0);
 			}
-
-			u32 const key0 = kb * at::KV_PER_STEP;
-			bool const need_mask = !(key0 + 31 < q_wave0 && (q_wave0 + 31 - key0) <= wr);
+			widen((slot + 1) % bt::RING, buf ^ 1u);       // (behind the matrix instructions, whose results are not ready yet)
 			X17_UNROLL for (u32 tile = 0; tile < 2; ++tile) {
 				// this lane's keys of the tile: 4 half + {0..3} and 8 + 4 half + {0..3}
 				f32 w[8];
-				u32 const first = qi - 1 - (key0 + 16 * tile + 4 * half);
+				[[maybe_unused]] u32 const first = qi - 1 - ((kb_begin + i) * at::KV_PER_STEP + 16 * tile + 4 * half);
 				X17_UNROLL for (u32 r = 0; r < 8; ++r) {
-					f32 const s = f32(s_acc[8 * tile + r]) * temperature;
-					f32 p = sfu::ex2(s - l_hat);
-					if (need_mask) {
+					f32 p = sfu::ex2(fmaf32(u2f((u32)s_acc[8 * tile + r]), temperature, -mb));
+					if constexpr (MASKED) {
 						// key j is visible iff the distance qi - 1 - j, as an unsigned number, is at most W' - 1
 						u32 const distance = first - (8 * (r / 4) + (r % 4));
 						p = distance <= vis_bound ? p : 0.0f;
 					}
-					w[r] = p * ((dp_acc[8 * tile + r] - d8) * 0.125f);
+					w[r] = p * dp_acc[8 * tile + r];
 				}
 				v8h wfrag;
 				X17_UNROLL for (u32 r = 0; r < 8; ++r) wfrag[r] = (_Float16)w[r];
@@ -353,10 +391,41 @@ void kernel(
 					dq_acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, both), wfrag, dq_acc[db], 0, 0, 0);
 				}
 			}
-		}
+		};
+		auto step = [&]<bool MASKED, int SLOT>(u32 i) __attribute__((always_inline)) {
+			stage.template operator()<SLOT>(i);
+			compute.template operator()<MASKED, SLOT>(i);
+		};
+		auto idle_step = [&](u32 i) __attribute__((always_inline)) {
+			stage.template operator()<-1>(i);
+			widen((i + 1) % bt::RING, (i + 1) & 1);
+		};
+		u32 const first_active = wave_kb_first - kb_begin;
+		u32 const diagonal = wave_kb_last - kb_begin;
+		// first block that lies inside the window of all 32 queries: q_wave0 + 31 - 32 kb <= wr
+		u32 const inside_kb = q_wave0 + 31 > wr ? (q_wave0 + 62 - wr) / 32 : 0;
+		u32 const inside_clamped = inside_kb < wave_kb_first ? wave_kb_first : (inside_kb > wave_kb_last ? wave_kb_last : inside_kb);
+		u32 const first_full = (biased ? inside_clamped : wave_kb_last) - kb_begin;
 
-		// ---- output: dq = 8 ln 2 * temperature * dq_acc / scale, D = d8 / (8 scale)
-		f32 const out_scale = (temperature * EIGHT_LN2) * inv_scale;
+		__builtin_amdgcn_s_waitcnt(0x0F74);   // vmcnt(4): tile 0 has landed
+		widen(0, 0);
+		u32 i = 0;
+		for (; i < first_active; ++i) idle_step(i);
+		for (; i < first_full; ++i) step.template operator()<true, -1>(i);
+		for (; i < diagonal && i % bt::RING != 0; ++i) step.template operator()<false, -1>(i);
+		for (; i + bt::RING <= diagonal && i + 2 * bt::RING <= n_steps; i += bt::RING) {
+			step.template operator()<false, 0>(i);
+			step.template operator()<false, 1>(i + 1);
+			step.template operator()<false, 2>(i + 2);
+			step.template operator()<false, 3>(i + 3);
+		}
+		for (; i < diagonal; ++i) step.template operator()<false, -1>(i);
+		step.template operator()<true, -1>(i);
+		for (++i; i < n_steps; ++i) idle_step(i);
+		__builtin_amdgcn_s_waitcnt(0x0F70);   // the last requests write LDS: they land before the tiles are reused
+
+		// ---- output: dq = 8 ln 2 * temperature * dq_acc / (scale * fine), D = d8 / (8 scale)
+		f32 const out_scale = ((temperature * EIGHT_LN2) * inv_scale) * inv_fine;
 		u16 *dq_row = d_q + (row_base + qi) * Q_STRIDE + (size_t)head * HD;
 		X17_UNROLL for (u32 db = 0; db < D_BLOCKS; ++db) {
 			X17_UNROLL for (int g = 0; g < 4; ++g) {
