@@ -1281,7 +1281,7 @@ std::unique_ptr<AttnKernel> AttnKernel::create(std::shared_ptr<HipDevice> device
 	if (!meta) return nullptr;
 	auto out = std::make_unique<AttnKernel>();
 	auto get = [&](char const *k) { auto v = kernel_build::meta_get(*meta, k); return v ? *v : size_t(0); };
-	out->metadata = AttnLauncherMetadata{get("THREADS_PER_BLOCK"), get("SMEM_BYTES"), get("Q_PER_BLOCK")};
+	out->metadata = AttnLauncherMetadata{get("THREADS_PER_BLOCK"), get("SMEM_BYTES"), get("Q_PER_BLOCK"), get("KEYS_PER_WORKGROUP")};
 	// attn.rs:333-342
 	if (out->metadata.THREADS_PER_BLOCK == 0 || out->metadata.SMEM_BYTES == 0 || !is_pow2(out->metadata.Q_PER_BLOCK)) {
 		diag.add_error("Invalid JSON metadata in " + built->meta_json_path);
@@ -1313,11 +1313,12 @@ size_t AttnKernel::heads_per_workgroup(size_t seq_len, size_t batch, size_t wind
 		{{3, 2.5, 0, 0.5}, {3, 1.5, 0.5, 0.25}}, {{3, 8, 0, 0.75}, {3, 4, 0, 0.75}}, {{1, 2.5, 0, 0.1}, {1, 1, 0, 0.1}},
 	};
 	Fit const &f = FITS[config.backward_q ? 1 : config.backward_kv ? 2 : 0][config.head_dim == 32 ? 0 : 1];
-	size_t const blocks = (seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK;
+	size_t const own_rows = metadata.rows_per_workgroup();
+	size_t const blocks = (seq_len + own_rows - 1) / own_rows;
 	size_t const w = window == 0 || window > seq_len ? seq_len : window;
 	// key steps of a block: its own, and those of the min(w, rows before it) keys it sees further back
-	size_t const growing = std::min(blocks, (w + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK);
-	double const own = double(metadata.Q_PER_BLOCK);
+	size_t const growing = std::min(blocks, (w + own_rows - 1) / own_rows);
+	double const own = double(own_rows);
 	double const mean = (own + (own * double(growing) * double(growing - 1) / 2.0 + double(blocks - growing) * double(w)) / double(blocks)) / 32.0;
 	double const longest = (own + std::min(own * double(blocks - 1), double(w))) / 32.0;
 	size_t best = 1;
@@ -1517,7 +1518,7 @@ Status AttnKernel::launch_d_kv(AttnKernelArgs const &a) {
 	void *q_ptr = a.q->ptr, *kv_ptr = a.kv->ptr, *tp = a.attn_temperature->ptr, *do_ptr = a.d_out->ptr, *l_ptr = a.l->ptr, *d_ptr = a.d->ptr;
 	void *dkv_ptr = a.d_kv->ptr;
 	void *raw_args[9] = {&seq_len_arg, &q_ptr, &kv_ptr, &tp, &do_ptr, &l_ptr, &d_ptr, &dkv_ptr, &window_arg};
-	size_t grid[3] = {(seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK, config.n_heads / heads_per_workgroup(seq_len, a.batch, a.window_size), a.batch};
+	size_t grid[3] = {(seq_len + metadata.rows_per_workgroup() - 1) / metadata.rows_per_workgroup(), config.n_heads / heads_per_workgroup(seq_len, a.batch, a.window_size), a.batch};
 	size_t block[3] = {metadata.THREADS_PER_BLOCK, 1, 1};
 	return kernel->launch(*device->stream, grid, block, metadata.SMEM_BYTES, raw_args);
 }

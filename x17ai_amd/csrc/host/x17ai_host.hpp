@@ -294,7 +294,11 @@ struct AttnKernelArgs {
 	Tensor const *d_kv = nullptr;
 };
 
-struct AttnLauncherMetadata { size_t THREADS_PER_BLOCK, SMEM_BYTES, Q_PER_BLOCK; };
+// Q_PER_BLOCK: queries of a workgroup, and the shortest sequence; KEYS_PER_WORKGROUP: what the dK / dV kernel's grid counts (0: Q_PER_BLOCK)
+struct AttnLauncherMetadata {
+	size_t THREADS_PER_BLOCK, SMEM_BYTES, Q_PER_BLOCK, KEYS_PER_WORKGROUP;
+	size_t rows_per_workgroup() const { return KEYS_PER_WORKGROUP != 0 ? KEYS_PER_WORKGROUP : Q_PER_BLOCK; }
+};
 
 struct AttnKernel {
 	std::string name;

@@ -1,5 +1,6 @@
 // Prints the launch geometry of the attention backward (dK, dV) kernel configured by common.h as JSON, with the keys
-// the attention launcher reads (reference: templates/attn/meta.cu); Q_PER_BLOCK is the key block here.
+// the attention launcher reads (reference: templates/attn/meta.cu); Q_PER_BLOCK is the smallest sequence, KEYS_PER_WORKGROUP
+// the keys a workgroup takes at a time.
 #include "common.h"
 #include "attn_bwd_kv_tile.h"
 #include <cstdio>
@@ -9,6 +10,7 @@ int main() {
 	std::printf("{\n");
 	std::printf("\t\"THREADS_PER_BLOCK\": %u,\n", kt::THREADS_PER_BLOCK);
 	std::printf("\t\"SMEM_BYTES\": %u,\n", kt::SMEM_BYTES);
-	std::printf("\t\"Q_PER_BLOCK\": %u\n", kt::KEYS_PER_BLOCK);
+	std::printf("\t\"Q_PER_BLOCK\": %u,\n", kt::LAUNCH_BLOCK);
+	std::printf("\t\"KEYS_PER_WORKGROUP\": %u\n", kt::KEYS_PER_BLOCK);
 	std::printf("}\n");
 }

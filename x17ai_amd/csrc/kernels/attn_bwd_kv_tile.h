@@ -11,44 +11,54 @@ namespace x17 { namespace attn_bwd_kv_tile {
 namespace at = x17::attn_tile;
 
 constexpr unsigned HEAD_DIM = at::HEAD_DIM;
-constexpr unsigned KEY_WAVES = 8;
+constexpr unsigned KEY_WAVES = 4;
 constexpr unsigned KEYS_PER_WAVE = 16;
-constexpr unsigned KEYS_PER_BLOCK = KEY_WAVES * KEYS_PER_WAVE;        // 128 keys of one head per workgroup
+constexpr unsigned KEYS_PER_BLOCK = KEY_WAVES * KEYS_PER_WAVE;        // 64 keys of one head per workgroup at a time
 constexpr unsigned Q_PER_STEP = 32;                                    // queries staged per pipeline step
 constexpr unsigned THREADS_PER_BLOCK = at::WAVE * KEY_WAVES;
-static_assert(KEYS_PER_BLOCK == at::Q_PER_BLOCK, "the launcher's grid and its smallest sequence are the forward's");
-// tiles are requested PREFETCH steps ahead into rings of PREFETCH + 1 slots; one step before its use the int8 Q tile
-// is widened to bf16
-constexpr unsigned PREFETCH = 2;
-constexpr unsigned RING = PREFETCH + 1;
+// The launcher's smallest sequence is the forward's query block.  gridDim.x says into how many runs the sequence's key blocks
+// are cut (a block each by this library's launchers, two where a grid is made of the forward's blocks).
+constexpr unsigned LAUNCH_BLOCK = at::Q_PER_BLOCK;
+constexpr unsigned blocks_per_run(unsigned seq_len, unsigned runs) { return (seq_len / KEYS_PER_BLOCK + runs - 1) / runs; }
 // 16 keys per wavefront on the 16 x 16 matrix instructions: 64 accumulators (dK^T and dV^T of 16 keys x head_dim 128)
-// and the keys' own K and V fragments leave room for two wavefronts per SIMD, which a lone wavefront's issue rate needs
-constexpr unsigned WAVES_PER_SIMD = 2;
+// and the keys' own K and V fragments leave room for three wavefronts per SIMD, i.e. three workgroups per compute unit.
+// A wavefront issues one instruction in about ten clocks whatever its neighbours do, so a step takes its number of
+// instructions times that, and what counts is how many wavefronts a SIMD has (four, at 128 registers, spill inside the
+// loop; with smaller heads they do not).
+constexpr unsigned WAVES_PER_SIMD = HEAD_DIM == 128 ? 3 : 4;
 
 constexpr unsigned CPR = at::CHUNKS_PER_ROW;                // 16-byte chunks of an int8 row of the head
 constexpr unsigned WIDE_CPR = 2 * CPR;                      // ... of a bf16 row
-constexpr unsigned Q_STAGERS = Q_PER_STEP * CPR;            // threads that request the raw Q tile: 16-byte chunk t each
-constexpr unsigned WIDE_STAGERS = Q_PER_STEP * WIDE_CPR;    // threads that request the dO tile: chunk t of each of its two layouts
-static_assert(WIDE_STAGERS <= THREADS_PER_BLOCK && Q_STAGERS % at::WAVE == 0, "whole wavefronts request, one chunk per lane");
+constexpr unsigned Q_STAGERS = Q_PER_STEP * CPR;            // threads that request the raw Q tile: 16-byte chunk t each; they widen it
+constexpr unsigned WIDE_CHUNKS = Q_PER_STEP * WIDE_CPR;
+// dO requests: thread t < WIDE_STAGERS asks for chunk t and, where the tile has more chunks than the workgroup threads, for
+// chunk t + WIDE_STAGERS, sixteen rows further
+constexpr unsigned WIDE_STAGERS = WIDE_CHUNKS < THREADS_PER_BLOCK ? WIDE_CHUNKS : THREADS_PER_BLOCK;
+constexpr unsigned WIDE_PASSES = WIDE_CHUNKS / WIDE_STAGERS;
+static_assert(WIDE_STAGERS % at::WAVE == 0 && Q_STAGERS % at::WAVE == 0 && Q_STAGERS <= THREADS_PER_BLOCK, "whole wavefronts request, one chunk per lane");
+static_assert(WIDE_PASSES == 1 || (WIDE_PASSES == 2 && WIDE_STAGERS == 16 * WIDE_CPR), "the second pass starts sixteen rows further");
+constexpr unsigned LD_WAVE = KEY_WAVES - 1;                 // the wavefront that requests the tile's L and D and makes its constants
 constexpr unsigned Q_RAW_BYTES = Q_PER_STEP * HEAD_DIM;     // int8 queries as they arrive
 constexpr unsigned WIDE_BYTES = Q_PER_STEP * HEAD_DIM * 2;  // a bf16 tile (dO as it arrives, Q widened)
-constexpr unsigned LD_BYTES_PER_WAVE = 2 * Q_PER_STEP * 4;  // the tile's L and D values (f32), one copy per wavefront
-// one ring slot: raw Q | dO laid out for row reads | dO laid out for transposed reads | L and D (per wavefront)
+constexpr unsigned LD_BYTES = 2 * Q_PER_STEP * 4;           // the tile's L and D values (f32)
+constexpr unsigned CONST_BYTES = 3 * Q_PER_STEP * 4;        // the per-query constants temperature | L - lg2(255) | -8 D
+// LDS: raw Q ring (tiles requested three steps ahead, widened to bf16 one step before their use) | L and D ring | two dO tiles
+// (requested one step ahead: a third one is the LDS of the third workgroup) | two widened Q tiles | two blocks of constants
+constexpr unsigned RING = 4;
 constexpr unsigned Q_RAW_OFFSET = 0;
-constexpr unsigned DO_ROWS_OFFSET = Q_RAW_OFFSET + Q_RAW_BYTES;
-constexpr unsigned DO_TR_OFFSET = DO_ROWS_OFFSET + WIDE_BYTES;
-constexpr unsigned LD_OFFSET = DO_TR_OFFSET + WIDE_BYTES;
-constexpr unsigned SLOT_BYTES = LD_OFFSET + KEY_WAVES * LD_BYTES_PER_WAVE;
-// behind the ring, with the slot numbering of the ring (so that one compile-time slot number addresses a step's
-// operands everywhere): the bf16 Q tiles and, per wavefront, the per-query constants temperature | L - lg2(255) | D
-constexpr unsigned Q_WIDE_OFFSET = RING * SLOT_BYTES;
-constexpr unsigned CONST_BYTES_PER_WAVE = 3 * Q_PER_STEP * 4;
-constexpr unsigned CONST_OFFSET = Q_WIDE_OFFSET + RING * WIDE_BYTES;
-constexpr unsigned SMEM_BYTES = CONST_OFFSET + RING * KEY_WAVES * CONST_BYTES_PER_WAVE;
+constexpr unsigned LD_OFFSET = Q_RAW_OFFSET + RING * Q_RAW_BYTES;
+constexpr unsigned DO_OFFSET = LD_OFFSET + RING * LD_BYTES;
+constexpr unsigned Q_WIDE_OFFSET = DO_OFFSET + 2 * WIDE_BYTES;
+constexpr unsigned CONST_OFFSET = Q_WIDE_OFFSET + 2 * WIDE_BYTES;
+constexpr unsigned SMEM_BYTES = CONST_OFFSET + 2 * CONST_BYTES;
+// at the end every wavefront turns its keys' rows (dK then dV, bf16) around in a region of its own over all of this
+constexpr unsigned OUT_CPR = HEAD_DIM / 4;                  // 16-byte chunks of such a row
+constexpr unsigned OUT_BYTES_PER_WAVE = KEYS_PER_WAVE * OUT_CPR * 16;
+static_assert(KEY_WAVES * OUT_BYTES_PER_WAVE <= SMEM_BYTES, "the rows fit the workgroup's LDS");
+constexpr unsigned out_offset(unsigned row, unsigned c) { return (row * OUT_CPR + (c ^ (row & (OUT_CPR - 1)))) * 16; }
 
-// ---- the walk.  Key blocks are placed like the forward's query blocks (a last block that would overhang starts
-// earlier and recomputes some of its neighbour's keys, storing the same values).
-constexpr unsigned block_first_key(unsigned key_block_index, unsigned seq_len) { return at::block_first_query(key_block_index, seq_len); }
+// ---- the walk (sequence lengths are multiples of 64: key blocks divide them)
+constexpr unsigned block_first_key(unsigned key_block_index) { return key_block_index * KEYS_PER_BLOCK; }
 // last query that sees a key of [.., last_key]: query i sees key j iff j < i <= j + W' (wr: the rounded window, 2^32 - 1 = none)
 constexpr unsigned last_seeing_query(unsigned last_key, unsigned wr, unsigned seq_len) {
 	return wr >= seq_len || wr >= seq_len - 1 - last_key ? seq_len - 1 : last_key + wr;
@@ -76,31 +86,31 @@ constexpr unsigned q_raw_source(unsigned p, unsigned row_stride_bytes) {
 	unsigned const n = q_raw_logical_chunk(p);
 	return (n / CPR) * row_stride_bytes + (n % CPR) * 16;
 }
-// bf16 tile read by rows (eight dims of one query per lane): a row is WIDE_CPR chunks of 16 bytes; 16 / WIDE_CPR rows
-// share a 256-byte line and chunk c of a row sits at position c ^ line inside its row's part of the line
+// bf16 tile: a row is WIDE_CPR chunks of 16 bytes; 16 / WIDE_CPR rows share a 256-byte line and chunk c of a row sits at
+// position c ^ key(line) inside its row's part of the line.  It is read in two ways, both without bank conflicts: by rows
+// (eight dims of one query per lane; the same chunk of sixteen rows lands in sixteen different positions, key being a
+// bijection), and transposed (eight queries of one dim per lane: the 32 lanes a ds_read_b64_tr_b16 serves at a time ask for the
+// same two chunks of eight consecutive rows, which lie in eight different 32-byte columns, key / 2 being different for
+// the lines of eight consecutive rows)
+constexpr unsigned line_key(unsigned line) { return ((line << 1) | ((line & (WIDE_CPR - 1)) / (WIDE_CPR / 2))) & (WIDE_CPR - 1); }
 constexpr unsigned rows_offset(unsigned row, unsigned c) {
 	constexpr unsigned RPL = 16 / WIDE_CPR;
 	unsigned const line = row / RPL;
-	return line * 256 + ((row % RPL) * WIDE_CPR + (c ^ (line & (WIDE_CPR - 1)))) * 16;
+	return line * 256 + ((row % RPL) * WIDE_CPR + (c ^ line_key(line))) * 16;
 }
 constexpr unsigned rows_source(unsigned p, unsigned row_stride_bytes) {
 	constexpr unsigned RPL = 16 / WIDE_CPR;
 	unsigned const line = p / 16, slot = p % 16;
-	return (line * RPL + slot / WIDE_CPR) * row_stride_bytes + ((slot % WIDE_CPR) ^ (line & (WIDE_CPR - 1))) * 16;
+	return (line * RPL + slot / WIDE_CPR) * row_stride_bytes + ((slot % WIDE_CPR) ^ line_key(line)) * 16;
 }
-// bf16 tile read transposed (eight queries of one dim per lane): 32-byte granule n = row * CPR + g (16 dims) in
-// 256-byte line n / 8 at position (n % 8) ^ (line % CPR): the 32 lanes a ds_read_b64_tr_b16 serves at a time ask for
-// granule g of eight consecutive rows, which then lie in eight different 32-byte columns
-constexpr unsigned granule_offset(unsigned row, unsigned g) {
-	unsigned const n = row * CPR + g, line = n >> 3;
-	return (line << 8) | (((n & 7) ^ (line & (CPR - 1))) << 5);
+// the eight bytes at dims 4 piece .. 4 piece + 3 of a row, as a transposed read asks for them
+constexpr unsigned piece_offset(unsigned row, unsigned piece) { return rows_offset(row, piece / 2) + 8 * (piece % 2); }
+// the same row's chunk (piece) `dims` dims further, dims a multiple of 16 above the lane's own: those address bits are flipped
+constexpr unsigned dims_flip(unsigned dims) { return dims * 2; }
+// Q tile int8 -> bf16: a staging thread widens the chunk it requested (16 codes), into two chunks that differ in address bit 4
+constexpr unsigned widened_offset(unsigned tid) {
+	unsigned const n = q_raw_logical_chunk(tid);
+	return rows_offset(n / CPR, 2 * (n % CPR));
 }
-constexpr unsigned granule_source(unsigned p, unsigned row_stride_bytes) {
-	unsigned const gp = p / 2, line = gp / 8;
-	unsigned const n = line * 8 + ((gp % 8) ^ (line & (CPR - 1)));
-	return (n / CPR) * row_stride_bytes + (2 * (n % CPR) + p % 2) * 16;
-}
-// Q tile int8 -> bf16: thread t < 2 * Q_STAGERS widens half a chunk (eight codes) of raw position t / 2
-constexpr bool is_widener(unsigned tid) { return tid < 2 * Q_STAGERS; }
 
 }} // namespace x17::attn_bwd_kv_tile
