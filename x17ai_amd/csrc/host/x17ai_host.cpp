@@ -1306,11 +1306,11 @@ std::unique_ptr<AttnKernel> AttnKernel::create(std::shared_ptr<HipDevice> device
 // rows, windows of 64 .. 4096 and none: 0.1-0.8 % behind the best choice in the mean.  us, one head / the whole group:
 //   forward, 8 heads of 64:    1024 rows, no window 23 / 42    16384 rows in sequences of 128 16.2 / 14.7
 //   dQ, 64 heads of 32:        8192 rows, window 64, 8 sequences 73 / 66
-//   dK / dV, 64 heads of 32:   1024 rows, no window 36 / 104   16384 rows in sequences of 128 193 / 178
+//   dK / dV, 64 heads of 32:   1024 rows, no window 24 / 70    16384 rows in sequences of 128 103 / 94
 size_t AttnKernel::heads_per_workgroup(size_t seq_len, size_t batch, size_t window) const {
 	struct Fit { double resident, start, last_round, tail; };
 	static constexpr Fit FITS[3][2] = {       // forward, dQ, dK / dV; head_dim 32 and 64
-		{{3, 2.5, 0, 0.5}, {3, 1.5, 0.5, 0.25}}, {{3, 8, 0, 0.75}, {3, 4, 0, 0.75}}, {{1, 2.5, 0, 0.1}, {1, 1, 0, 0.1}},
+		{{3, 2.5, 0, 0.5}, {3, 1.5, 0.5, 0.25}}, {{3, 8, 0, 0.75}, {3, 4, 0, 0.75}}, {{3, 2, 0, 0.25}, {5, 1, 0.5, 0.1}},
 	};
 	Fit const &f = FITS[config.backward_q ? 1 : config.backward_kv ? 2 : 0][config.head_dim == 32 ? 0 : 1];
 	size_t const own_rows = metadata.rows_per_workgroup();
