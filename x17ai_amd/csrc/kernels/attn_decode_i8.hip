@@ -19,6 +19,10 @@
 //   32 x 1024                  43 / 31 / 32 / 46    32 x 4096  141 / 103 / 97 / 109  32 x 128  9.1 / 8.7 / 16 / 28
 //   48 x 1024                  50 / 46 / 46 / 67    48 x 4096  158 / 148 / 137 / 157 (266, 271)
 //   64 x 128                 10.9 / 17 / 31 / 57    64 x 4096  193 / 192 / 184 / 206 (349, 343)
+// (the table was measured before phases 3 and 4 took their present form, which took 0.5 to 4 us off a launch at every width.)
+// What the tail behind the scores costs counts where few workgroups run: the slowest heads, with 100 to 180 listed tiles of 240,
+// spent 9 to 13 of their 22 us in phases 3 and 4.  Four keys per dot product, the partial sums beside the O chain and the
+// listed tiles' factors in a list of their own: 3 ragged caches 22.0 -> 19.3 us, 8 31.9 -> 27.5, 64 full ones 185.8 -> 183.5.
 // The recurrence is cut into phases so that only two cheap scans remain sequential:
 //   1  scores: HD/16 lanes per key row (16-byte coalesced loads), v_dot4 + lane reduction
 //   2  per-tile max, prefix max over tiles (exact), rescale factors, probabilities, quad sums
@@ -93,6 +97,7 @@ void kernel(
 	f32 *s_score = reinterpret_cast<f32 *>(smem);                               // [CAP], quad slots (see quad_slot)
 	f32 *s_mrun = reinterpret_cast<f32 *>(smem + dt::TILE_STATE_OFFSET);         // [MAX_TILES] tile max, then running max
 	f32 *s_tmax = s_mrun;
+	f32 *s_ract = s_mrun;                                                        // from phase 3 on: the listed tiles' rescale factors
 	f32 *s_resc = s_mrun + dt::MAX_TILES;                                        // [MAX_TILES]
 	f32 *s_bmax = s_resc + dt::MAX_TILES;                                        // [MAX_SLOTS] one per wavefront
 	f32 *s_sum = s_bmax + dt::MAX_SLOTS;                                                     // [4]
@@ -240,6 +245,7 @@ void kernel(
 	}
 	__syncthreads();
 
+	f32 const m_final = n_tiles == 0 ? m0 : s_mrun[n_tiles - 1];      // (the array is another list from phase 3 on)
 	// ---- phase 2c: probabilities and quad sums (:265-290); one key quad per thread per pass
 	for (u32 quad = tid; quad < n_tiles * 4; quad += dt::THREADS_PER_BLOCK) {
 		f32 m = s_mrun[quad / 4];
@@ -268,22 +274,29 @@ void kernel(
 	}
 	__syncthreads();
 
-	// ---- phase 3: the four partial-sum chains, one per lane of the first four, while the last wavefront lists the
-	// tiles for phase 4.  The chain is serial; what costs time is fetching its operands from LDS, so they are
-	// fetched 32 tiles at a time (the registers are free at this point) and the chain waits once per 32 steps.
-	if (tid < 4) {
-		constexpr u32 STEPS = 32;
+	// ---- phase 3: the four partial-sum chains, one per lane of the first four of a wavefront.  A chain is serial, and nothing
+	// needs it before the end: where the workgroup has a wavefront that owns no output dimension, that one runs it beside the
+	// first O chain; else the first one does while the last one lists the tiles for phase 4.  What costs time is fetching its
+	// operands from LDS: they are fetched SUM_STEPS tiles at a time (as many as the registers hold next to the value rows
+	// in flight) and the chain waits once per SUM_STEPS steps.
+	constexpr bool LATE_SUMS = dt::THREADS_PER_BLOCK >= HD + 64;
+	constexpr u32 SUM_STEPS = LATE_SUMS ? 16 : 32, SUM_THREAD0 = LATE_SUMS ? (HD + 63) / 64 * 64 : 0;
+	auto partial_sums = [&]() {
+		u32 const quad = tid - SUM_THREAD0;
 		f32 sum = 63.75f;
 		u32 t = 0;
-		for (; t + STEPS <= n_tiles; t += STEPS) {
-			v4f r[STEPS / 4];
-			f32 a[STEPS];
-			X17_UNROLL for (u32 i = 0; i < STEPS / 4; ++i) r[i] = *reinterpret_cast<v4f const *>(s_resc + t + 4 * i);
-			X17_UNROLL for (u32 i = 0; i < STEPS; ++i) a[i] = *reinterpret_cast<f32 const *>(quad_slot(smem, (t + i) * 4 + tid));
-			X17_UNROLL for (u32 i = 0; i < STEPS; ++i) sum = fmaf32(sum, r[i / 4][i % 4], a[i]);
+		for (; t + SUM_STEPS <= n_tiles; t += SUM_STEPS) {
+			v4f r[SUM_STEPS / 4];
+			f32 a[SUM_STEPS];
+			X17_UNROLL for (u32 i = 0; i < SUM_STEPS / 4; ++i) r[i] = *reinterpret_cast<v4f const *>(s_resc + t + 4 * i);
+			X17_UNROLL for (u32 i = 0; i < SUM_STEPS; ++i) a[i] = *reinterpret_cast<f32 const *>(quad_slot(smem, (t + i) * 4 + quad));
+			X17_UNROLL for (u32 i = 0; i < SUM_STEPS; ++i) sum = fmaf32(sum, r[i / 4][i % 4], a[i]);
 		}
-		for (; t < n_tiles; ++t) sum = fmaf32(sum, s_resc[t], *reinterpret_cast<f32 const *>(quad_slot(smem, t * 4 + tid)));
-		s_sum[tid] = sum;
+		for (; t < n_tiles; ++t) sum = fmaf32(sum, s_resc[t], *reinterpret_cast<f32 const *>(quad_slot(smem, t * 4 + quad)));
+		s_sum[quad] = sum;
+	};
+	if constexpr (!LATE_SUMS) {
+		if (tid < 4) partial_sums();
 	}
 
 	// ---- phase 4: O chains.  Lane d < HD owns output dim d.
@@ -303,7 +316,9 @@ void kernel(
 			}
 			unsigned long long const mask = __ballot(active);
 			if (active) {
-				s_act[count + __builtin_popcountll(mask & ((1ull << lane) - 1ull))] = (u16)t;
+				u32 const at = count + (u32)__builtin_popcountll(mask & ((1ull << lane) - 1ull));
+				s_act[at] = (u16)t;
+				s_ract[at] = s_resc[t];
 			}
 			count += (u32)__builtin_popcountll(mask);
 		}
@@ -344,22 +359,34 @@ void kernel(
 	};
 	if (n_act > 0) {
 		request_rows(0);
+	} else if (LATE_SUMS && tid >= SUM_THREAD0 && tid < SUM_THREAD0 + 4) {
+		partial_sums();
 	}
 	for (u32 chunk = 0; chunk < n_act; chunk += dt::CHUNK_TILES) {
 		u32 const tiles_here = n_act - chunk < dt::CHUNK_TILES ? n_act - chunk : dt::CHUNK_TILES;
 		if (tl < tiles_here) {
-			i32 acc[16];
-			X17_UNROLL for (int i = 0; i < 16; ++i) acc[i] = 0;
-			X17_UNROLL for (int k = 0; k < 16; ++k) {
-				i32 p = (i32)((probs[k / 4] >> (8 * (k % 4))) & 0xFFu);
-				if (p != 0) {     // after the 8-bit quantisation most keys far below the maximum carry no weight
-					X17_UNROLL for (int i = 0; i < 16; ++i) {
-						acc[i] += p * (i32)(i8)(((u32)vv[k][i / 4] >> (8 * (i % 4))) & 0xFFu);
+			// sum_k P_k v_k as sum_k P_k (v_k + 128) - 128 sum_k P_k: four keys of one dim per unsigned dot product, behind a
+			// transposition of 4 keys x 4 dims at a time (16 instructions for 16 products; byte by byte it was 33)
+			u32 p_sum = 0;
+			X17_UNROLL for (int q = 0; q < 4; ++q) p_sum = __builtin_amdgcn_udot4(probs[q], 0x01010101u, p_sum, false);
+			u32 acc[16];
+			X17_UNROLL for (int i = 0; i < 16; ++i) acc[i] = p_sum * (u32)-128;
+			X17_UNROLL for (int q = 0; q < 4; ++q) {
+				if (probs[q] != 0) {     // after the 8-bit quantisation most keys far below the maximum carry no weight
+					X17_UNROLL for (int w = 0; w < 4; ++w) {
+						u32 k[4];
+						X17_UNROLL for (int i = 0; i < 4; ++i) k[i] = (u32)vv[4 * q + i][w] ^ 0x80808080u;
+						u32 const lo01 = __builtin_amdgcn_perm(k[1], k[0], 0x05010400u), hi01 = __builtin_amdgcn_perm(k[1], k[0], 0x07030602u);
+						u32 const lo23 = __builtin_amdgcn_perm(k[3], k[2], 0x05010400u), hi23 = __builtin_amdgcn_perm(k[3], k[2], 0x07030602u);
+						acc[4 * w] = __builtin_amdgcn_udot4(__builtin_amdgcn_perm(lo23, lo01, 0x05040100u), probs[q], acc[4 * w], false);
+						acc[4 * w + 1] = __builtin_amdgcn_udot4(__builtin_amdgcn_perm(lo23, lo01, 0x07060302u), probs[q], acc[4 * w + 1], false);
+						acc[4 * w + 2] = __builtin_amdgcn_udot4(__builtin_amdgcn_perm(hi23, hi01, 0x05040100u), probs[q], acc[4 * w + 2], false);
+						acc[4 * w + 3] = __builtin_amdgcn_udot4(__builtin_amdgcn_perm(hi23, hi01, 0x07060302u), probs[q], acc[4 * w + 3], false);
 					}
 				}
 			}
 			X17_UNROLL for (int i = 0; i < 16; i += 2) {
-				*reinterpret_cast<v2i *>(pv_word(smem, tl, 16 * c + i)) = v2i{acc[i], acc[i + 1]};
+				*reinterpret_cast<v2i *>(pv_word(smem, tl, 16 * c + i)) = v2i{(i32)acc[i], (i32)acc[i + 1]};
 			}
 		}
 		__syncthreads();
@@ -368,20 +395,24 @@ void kernel(
 		}
 		// 4b: one f32 multiply (rescale) and one f32 add per tile (:247-252, :588-605)
 		if (tid < HD) {
+			constexpr u32 STEPS = 16;
 			u32 tl2 = 0;
-			for (; tl2 + 8 <= tiles_here; tl2 += 8) {
-				f32 r[8];
-				i32 a[8];
-				X17_UNROLL for (int i = 0; i < 8; ++i) { r[i] = s_resc[s_act[chunk + tl2 + i]]; a[i] = *pv_word(smem, tl2 + i, tid); }
-				X17_UNROLL for (int i = 0; i < 8; ++i) {
-					o = o * r[i];
+			for (; tl2 + STEPS <= tiles_here; tl2 += STEPS) {
+				v4f r[STEPS / 4];
+				i32 a[STEPS];
+				X17_UNROLL for (u32 i = 0; i < STEPS / 4; ++i) r[i] = *reinterpret_cast<v4f const *>(s_ract + chunk + tl2 + 4 * i);
+				X17_UNROLL for (u32 i = 0; i < STEPS; ++i) a[i] = *pv_word(smem, tl2 + i, tid);
+				X17_UNROLL for (u32 i = 0; i < STEPS; ++i) {
+					o = o * r[i / 4][i % 4];
 					o = o + f32(a[i]);
 				}
 			}
 			for (; tl2 < tiles_here; ++tl2) {
-				o = o * s_resc[s_act[chunk + tl2]];
+				o = o * s_ract[chunk + tl2];
 				o = o + f32(*pv_word(smem, tl2, tid));
 			}
+		} else if (LATE_SUMS && chunk == 0 && tid >= SUM_THREAD0 && tid < SUM_THREAD0 + 4) {
+			partial_sums();
 		}
 		__syncthreads();
 	}
@@ -389,7 +420,6 @@ void kernel(
 	// ---- finish (:293-351)
 	__syncthreads();
 	f32 const total = (s_sum[0] + s_sum[1]) + (s_sum[2] + s_sum[3]);
-	f32 const m_final = n_tiles == 0 ? m0 : s_mrun[n_tiles - 1];
 	if (tid == 0 && l_out != nullptr) {
 		l_out[(size_t)seq * N_HEADS + head] = strict::lg2(total) + m_final;
 	}
