@@ -315,6 +315,36 @@ def test_attn_row_scaled_fast_within_tolerance(dev, t, h, hd, w):
 	assert np.max(np.abs(got_l - want_l)) < 1e-4
 
 
+@pytest.mark.parametrize("t,h,hd,w,batch", [(128, 4, 32, 0, 2), (192, 2, 64, 16, 3), (320, 2, 128, 48, 1), (256, 8, 64, 256, 1), (128, 2, 128, 0, 1)])
+@pytest.mark.parametrize("rows", [False, True])
+def test_attn_fast_sixteen_queries_per_wavefront(dev, t, h, hd, w, batch, rows):
+	"""The form of small launches against the strict definition, with the speed builds' bounds: sequences of one and two query
+	blocks, walks shorter than the rings, a window that ends inside a block, a head with a negative temperature."""
+	rng = rng_for("attn-narrow", t, h, hd, w, batch)
+	if rows:
+		q, kv, qs, ks, vs, sk, sv, temp = _row_scaled_inputs(rng, t * batch, h, hd)
+	else:
+		q, kv, sk, sv, temp = _attn_inputs(rng, t * batch, h, hd)
+	temp[0] = -temp[0]
+	if rows:
+		vw, sw, osc = recipes.attn_row_scale_operands(vs, X.INT8)
+		kern = recipes.attn_row_scaled_kernel(dev, h, hd, X.INT8, False)
+		got, got_l = _run_row_scaled(dev, kern, q, kv, sk, sv, temp, w, qs, ks, vw, sw, osc, batch=batch)
+	else:
+		kern = recipes.attn_kernel(dev, h, hd, False)
+		got, got_l = _run_attn(dev, kern, q, kv, sk, sv, temp, w, batch=batch)
+	assert kern.queries_per_wavefront(t, batch, w) == 16
+	for i in range(batch):
+		r = slice(i * t, (i + 1) * t)
+		if rows:
+			want, want_l = S.attn_fwd_i8_row_scaled(q[r], kv[r], sk, sv, temp, h, hd, w, *(np.ascontiguousarray(a[:, r]) for a in (qs, ks, vw)), sw, osc)
+		else:
+			want, want_l = S.attn_fwd_i8(q[r], kv[r], sk, sv, temp, h, hd, w)
+		d = np.abs(got[r].astype(np.int32) - want.astype(np.int32))
+		assert d.max() <= 1 and np.mean(d > 0) < 0.02, (d.max(), np.mean(d > 0))
+		assert np.max(np.abs(got_l[:, r] - want_l)) < 1e-4
+
+
 def test_attn_row_scaled_launch_checks(dev):
 	t, h, hd = 128, 2, 64
 	rng = rng_for("attn-rows-checks")

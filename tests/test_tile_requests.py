@@ -99,6 +99,27 @@ def test_attention_tile_requests_stay_inside_their_sequence(tmp_path, label, mak
 	assert rc != 0 and not rep["ok"]
 
 
+NARROWS = [
+	("head_dim 128", lambda: recipes.attn_kernel(None, 16, 128, False), ((256, 1, 512), (1088, 3, 512), (192, 2, 16))),
+	("row scales, head_dim 64", lambda: recipes.attn_row_scaled_kernel(None, 8, 64, X.BF16, False), ((1024, 1, 256), (128, 1, 0), (320, 2, 48))),
+	("head_dim 32", lambda: recipes.attn_kernel(None, 4, 32, False), ((768, 1, 64), (192, 1, 0))),
+]
+
+
+@pytest.mark.parametrize("label,make,shapes", NARROWS, ids=[a[0] for a in NARROWS])
+def test_narrow_attention_requests_reads_and_walks(tmp_path, label, make, shapes):
+	"""attn_narrow_tile.h: reads name what requests and widening wrote, every workgroup's walk covers the keys its queries see."""
+	kern = make()
+	for seq_len, batch, window in shapes:
+		rep, rc = _audit(tmp_path, kern, "attn_narrow_requests_audit.cpp", seq_len, batch, window, form="q16")
+		assert rc == 0 and rep["ok"] and rep["kv_extent"] == rep["kv_bytes"], (label, seq_len, batch, window, rep)
+	seq_len, batch, window = shapes[0]
+	rep, rc = _audit(tmp_path, kern, "attn_narrow_requests_audit.cpp", seq_len, batch, window, seq_len * batch - 1, form="q16")
+	assert rc != 0 and not rep["ok"] and "past the end" in rep["error"], rep
+	rep, rc = _audit(tmp_path, kern, "attn_narrow_requests_audit.cpp", 64, 1, 0, form="q16")
+	assert rc != 0 and not rep["ok"]
+
+
 D_KVS = [
 	("config 4", lambda: recipes.attn_d_kv_kernel(None, 16, 128, False), ((2048, 16, 512), (128, 1, 0), (192, 3, 16), (320, 2, 4096))),
 	("head_dim 64 (two staging wavefronts)", lambda: recipes.attn_d_kv_kernel(None, 8, 64, True), ((1024, 1, 256), (192, 2, 0), (128, 1, 16))),

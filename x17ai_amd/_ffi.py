@@ -113,6 +113,8 @@ def host() -> ctypes.CDLL:
 	h.x17h_attn_kernel_free.restype = None
 	h.x17h_attn_kernel_heads_per_workgroup.argtypes = [P, SZ, SZ, SZ]
 	h.x17h_attn_kernel_heads_per_workgroup.restype = SZ
+	h.x17h_attn_kernel_queries_per_wavefront.argtypes = [P, SZ, SZ, SZ]
+	h.x17h_attn_kernel_queries_per_wavefront.restype = SZ
 	h.x17h_attn_kernel_launch.argtypes = [P, P, P, P, P, P, P, P, SZ, SZ]
 	h.x17h_attn_kernel_launch_row_scaled.argtypes = [P, P, P, P, P, P, P, P, SZ, SZ, P, P, P, P, P]
 	h.x17h_attn_kernel_launch_d_q.argtypes = [P, P, P, P, P, P, P, P, P, P, P, SZ, SZ]

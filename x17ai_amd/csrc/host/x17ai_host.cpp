@@ -1273,9 +1273,13 @@ std::unique_ptr<AttnKernel> AttnKernel::create(std::shared_ptr<HipDevice> device
 		diag.add_error("an attention kernel is the forward, the backward with respect to q, or the backward with respect to k and v: backward_q and backward_kv are both set");
 		return nullptr;
 	}
-	auto built = config.backward_q  ? kernel_build::build(kernel_name, common.str(), "attn_d_q_i8.hip", "attn_bwd_meta.cpp", diag)
-	           : config.backward_kv ? kernel_build::build(kernel_name, common.str(), "attn_d_kv_i8.hip", "attn_bwd_kv_meta.cpp", diag)
-	                                : kernel_build::build(kernel_name, common.str(), "attn_fwd_i8.hip", "attn_meta.cpp", diag);
+	std::vector<kernel_build::Form> forms{config.backward_q  ? kernel_build::Form{"", "", "attn_d_q_i8.hip", "attn_bwd_meta.cpp"}
+	                                    : config.backward_kv ? kernel_build::Form{"", "", "attn_d_kv_i8.hip", "attn_bwd_kv_meta.cpp"}
+	                                                         : kernel_build::Form{"", "", "attn_fwd_i8.hip", "attn_meta.cpp"}};
+	if (!config.backward_q && !config.backward_kv && !strict_math) forms.push_back({"q16", "", "attn_fwd_i8_narrow.hip", "attn_narrow_meta.cpp"});
+	std::vector<kernel_build::BuiltForm> built_forms = kernel_build::build_forms(kernel_name, common.str(), forms);
+	for (Diagnostic const &d : built_forms[0].diag.list) d.is_error ? diag.add_error(d.message) : diag.add_warning(d.message);
+	std::optional<kernel_build::BuiltKernel> const &built = built_forms[0].files;
 	if (!built) return nullptr;
 	auto meta = kernel_build::read_metadata_json(built->meta_json_path, diag);
 	if (!meta) return nullptr;
@@ -1293,9 +1297,52 @@ std::unique_ptr<AttnKernel> AttnKernel::create(std::shared_ptr<HipDevice> device
 	if (device) {
 		out->kernel = kernel_build::load_kernel(*device->stream, built->code_object_path, "kernel", out->metadata.SMEM_BYTES, diag);
 		if (!out->kernel) return nullptr;
-		out->device = std::move(device);
 	}
+	if (forms.size() > 1) {
+		kernel_build::BuiltForm &b = built_forms[1];
+		auto load = [&]() -> std::optional<Narrow> {
+			if (!b.files) return std::nullopt;
+			auto narrow_meta = kernel_build::read_metadata_json(b.files->meta_json_path, b.diag);
+			if (!narrow_meta) return std::nullopt;
+			auto get_narrow = [&](char const *k) { auto v = kernel_build::meta_get(*narrow_meta, k); return v ? *v : size_t(0); };
+			Narrow n{{get_narrow("THREADS_PER_BLOCK"), get_narrow("SMEM_BYTES"), get_narrow("Q_PER_BLOCK"), 0}, nullptr};
+			if (n.metadata.THREADS_PER_BLOCK == 0 || n.metadata.Q_PER_BLOCK != 64) {
+				b.diag.add_error("Invalid JSON metadata in " + b.files->meta_json_path);
+				return std::nullopt;
+			}
+			if (device) {
+				n.kernel = kernel_build::load_kernel(*device->stream, b.files->code_object_path, "kernel", n.metadata.SMEM_BYTES, b.diag);
+				if (!n.kernel) return std::nullopt;
+			}
+			return n;
+		};
+		out->narrow = load();
+		if (out->narrow) {
+			for (Diagnostic const &d : b.diag.list) diag.add_warning(d.message);
+		} else {
+			kernel_build::leave_out(kernel_name, forms[1].name, b.diag, diag);
+		}
+	}
+	out->device = std::move(device);
 	return out;
+}
+
+// Sixteen queries per wavefront and 64 per workgroup while the 32-query kernel's workgroups of 128 leave most of the chip idle;
+// beyond that the shorter the walk, the longer it stays ahead (it then is the set-up and the output that fill the chip).
+// Fitted to 168 launches of 4 .. 32 heads of 32, 64 and 128; us with 32 / 16 queries, windows of 64 | 256 | 1024:
+//    32 workgroups of 128   8 heads of 64, row scales   10.5 / 6.8 | 15.4 / 11.3 | 17.0 / 15.2
+//   128                     8 heads of 64, row scales   10.8 / 7.1 | 15.8 / 11.7 | 32.6 / 28.7
+//                           16 heads of 128             10.8 / 7.8 | 15.8 / 12.2 | 28.7 / 25.2
+//   256                     8 heads of 64, row scales   11.2 / 8.4 | 16.3 / 14.0 | 33.7 / 33.6
+//                           16 heads of 128             11.1 / 9.6 | 16.3 / 17.1 | 33.5 / 35.1
+//   448                     16 heads of 128             14.8 / 16.0 | 21.8 / 27.2 | 44.5 / 62.3
+bool AttnKernel::narrow_for(size_t seq_len, size_t batch, size_t window) const {
+	if (!narrow) return false;
+	size_t const workgroups = (seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK * config.n_heads * batch;
+	size_t const walk_bytes = (window == 0 ? seq_len : std::min(window, seq_len)) * config.head_dim;
+	return workgroups <= COMPUTE_UNITS / 2
+		|| (workgroups <= COMPUTE_UNITS * 3 / 4 && walk_bytes <= 32 * 1024)
+		|| (workgroups <= COMPUTE_UNITS * 5 / 4 && walk_bytes <= 16 * 1024);
 }
 
 // Heads a workgroup takes one behind the other (a power of two up to 128 / head_dim, the reference's group,
@@ -1412,6 +1459,11 @@ Status AttnKernel::launch(AttnKernelArgs const &a) {
 	// the plain kernel takes the first nine arguments only
 	void *raw_args[14] = {&seq_len_arg, &q_ptr, &kv_ptr, &sk, &sv, &tp, &out_ptr, &l_ptr, &window_arg,
 	                      &scale_ptrs[0], &scale_ptrs[1], &scale_ptrs[2], &scale_ptrs[3], &scale_ptrs[4]};
+	if (narrow_for(seq_len, a.batch, a.window_size)) {
+		size_t grid[3] = {seq_len / narrow->metadata.Q_PER_BLOCK, config.n_heads, a.batch};
+		size_t block[3] = {narrow->metadata.THREADS_PER_BLOCK, 1, 1};
+		return narrow->kernel->launch(*device->stream, grid, block, narrow->metadata.SMEM_BYTES, raw_args);
+	}
 	size_t grid[3] = {(seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK, config.n_heads / heads_per_workgroup(seq_len, a.batch, a.window_size), a.batch};
 	size_t block[3] = {metadata.THREADS_PER_BLOCK, 1, 1};
 	return kernel->launch(*device->stream, grid, block, metadata.SMEM_BYTES, raw_args);
@@ -2041,6 +2093,9 @@ int x17h_attn_kernel_launch_d_kv(X17hAttnKernel *k, X17hTensor *q, X17hTensor *k
 double x17h_attn_kernel_n_ops(X17hAttnKernel *k, size_t seq_len, size_t window_size) { return k->k->config.n_ops(seq_len, window_size); }
 size_t x17h_attn_kernel_heads_per_workgroup(X17hAttnKernel *k, size_t seq_len, size_t batch, size_t window_size) {
 	return k->k->heads_per_workgroup(seq_len, batch, window_size);
+}
+size_t x17h_attn_kernel_queries_per_wavefront(X17hAttnKernel *k, size_t seq_len, size_t batch, size_t window_size) {
+	return k->k->narrow_for(seq_len, batch, window_size) ? 16 : 32;
 }
 int x17h_attn_kernel_metadata(X17hAttnKernel *k, size_t out[3]) {
 	out[0] = k->k->metadata.THREADS_PER_BLOCK; out[1] = k->k->metadata.SMEM_BYTES; out[2] = k->k->metadata.Q_PER_BLOCK;

@@ -308,6 +308,10 @@ struct AttnKernel {
 	std::shared_ptr<HipDevice> device;
 	std::unique_ptr<HipKernel> kernel;
 	size_t heads_per_workgroup(size_t seq_len, size_t batch, size_t window) const;     // what a launch takes
+	// forward, speed build: the same kernel with sixteen queries per wavefront, for launches that leave most of the chip idle
+	struct Narrow { AttnLauncherMetadata metadata; std::unique_ptr<HipKernel> kernel; };
+	std::optional<Narrow> narrow;
+	bool narrow_for(size_t seq_len, size_t batch, size_t window) const;                // whether a launch takes it
 	static std::unique_ptr<AttnKernel> create(std::shared_ptr<HipDevice> device, std::string const &kernel_name,
 	                                           AttnKernelConfig const &config, bool strict_math, Diagnostics &diag);
 	Status launch(AttnKernelArgs const &args);

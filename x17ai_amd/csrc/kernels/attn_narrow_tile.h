@@ -1,0 +1,45 @@
+// attn_narrow_tile.h -- tile geometry and LDS layouts of the attention kernel with sixteen queries per wavefront
+// (attn_fwd_i8_narrow.hip) as plain constexprs, shared with the host program that prints its meta.json and with the
+// request audit (attn_requests_audit.cpp).  Key tiles, their requests and their rings are attn_tile.h's.
+#pragma once
+
+#include "attn_tile.h"
+
+namespace x17 { namespace attn_narrow_tile {
+
+namespace at = x17::attn_tile;
+
+constexpr unsigned Q_PER_WAVE = 16;
+constexpr unsigned Q_PER_BLOCK = at::Q_WAVES * Q_PER_WAVE;      // 64 queries of one head per workgroup
+constexpr unsigned THREADS_PER_BLOCK = at::THREADS_PER_BLOCK;
+constexpr unsigned RING = at::RING;
+
+// LDS map: that of attn_tile.h
+constexpr unsigned K_RING_OFFSET = at::K_RING_OFFSET;
+constexpr unsigned RAW_V_RING_OFFSET = at::RAW_V_RING_OFFSET;
+constexpr unsigned V_TILES_OFFSET = at::V_TILES_OFFSET;
+constexpr unsigned SCALE_RING_OFFSET = at::SCALE_RING_OFFSET;
+constexpr unsigned SMEM_BYTES = at::SMEM_BYTES;
+
+// (sequence lengths are multiples of 64: query blocks divide them.)  One past the last key block a workgroup walks
+constexpr unsigned end_key_block(unsigned q_block0) { return q_block0 / at::KV_PER_STEP + Q_PER_BLOCK / at::KV_PER_STEP; }
+// first key block inside the window of all sixteen queries of a wavefront: q_wave0 + 15 - 32 kb <= wr
+constexpr unsigned first_inside_block(unsigned q_wave0, unsigned wr) {
+	return q_wave0 + Q_PER_WAVE - 1 > wr ? (q_wave0 + Q_PER_WAVE - 1 - wr + at::KV_PER_STEP - 1) / at::KV_PER_STEP : 0;
+}
+
+// K tile: as requested (attn_tile.h: linear 16-byte chunk n = key * CPR + c in 128-byte line n / 8 at position (n % 8) ^ ((line / 2) % 8))
+constexpr unsigned k_chunk_offset(unsigned key, unsigned c) {
+	unsigned const n = key * at::CHUNKS_PER_ROW + c, line = n >> 3;
+	return (line << 7) | (((n & 7) ^ ((line >> 1) & 7)) << 4);
+}
+// f16 V tile, read transposed: 32-byte granule n = key * CPR + c (16 dims) in 256-byte line n / 8 at position (n % 8) ^ (line % CPR):
+// the 32 lanes a ds_read_b64_tr_b16 serves at a time ask for one granule of eight consecutive keys, which then lie in eight
+// different 32-byte columns
+constexpr unsigned v_granule_offset(unsigned key, unsigned c) {
+	unsigned const n = key * at::CHUNKS_PER_ROW + c, line = n >> 3;
+	return (line << 8) | (((n & 7) ^ (line & (at::CHUNKS_PER_ROW - 1))) << 5);
+}
+constexpr unsigned SIXTEEN_KEYS = 16 * at::HEAD_DIM * 2;       // bytes from a key's granule to that of the key sixteen further
+
+}} // namespace x17::attn_narrow_tile

@@ -68,6 +68,8 @@ def _specs():
 		add(("attn_rows", h, hd, out, True))
 	for h, hd in ((8, 64), (2, 128)):
 		add(("attn_rows", h, hd, BF16, False))
+	for h, hd in ((4, 32), (2, 64), (2, 128), (8, 64)):      # sixteen queries per wavefront
+		add(("attn_rows", h, hd, INT8, False))
 	# ---- tests/test_gpu_attn_bwd.py
 	for h, hd in ((8, 64), (2, 128), (4, 32), (2, 64)):
 		add(("attn_d_q", h, hd, True))
