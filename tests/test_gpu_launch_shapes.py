@@ -298,3 +298,39 @@ def test_a_row_of_an_e4m3_product_does_not_depend_on_the_rows_launched_with_it(n
 	whole = launch(m)
 	for rows in (256, 320, 448, 1024, 2368, 8192):
 		assert np.array_equal(launch(rows), whole[:rows]), (name, rows)
+
+
+@pytest.mark.parametrize("k", [256, 768, 1280])
+@pytest.mark.parametrize("rows", [256, 320])
+def test_weights_widened_once_per_workgroup(shim, k, rows):  # noqa: F811
+	"""The 64 x 64 form of e4m3 x int8 at K steps (of 128 bytes) short of, equal to and past its rings of six, and with an
+	overhanging token tile: the 256 x 256 kernel's bytes, and within a bf16 step (2^-8) plus float32 summation (K roundings
+	of 2^-24 of the terms' magnitudes, in any order) of the product in 64 bits."""
+	dev = X.Device(0)
+	rng = rng_for("widened once", k, rows)
+	n = 384
+	t = lambda a, dtype: X.Tensor.from_numpy(dev, np.ascontiguousarray(a), dtype)
+	a, b = e4m3_bytes(rng, (rows, k)), i8_codes(rng, (n, k))
+	rs, cs = (0.01 + 0.01 * rng.random(rows)).astype(np.float32), (0.01 + 0.01 * rng.random(n)).astype(np.float32)
+	kernel = recipes.dequant_gemm_kernel(None, k, n, X.E4M3, X.INT8, False, True)
+	ta, tb, trs, tcs = t(a, X.E4M3), t(b, X.INT8), t(rs, X.F32), t(cs, X.F32)
+	results = []
+	for form in ("", "s64x4"):
+		path = os.path.join(_ffi.kernel_cache_dir(), kernel.name, form)
+		with open(os.path.join(path, "meta.json")) as f:
+			meta = json.load(f)
+		c = t(np.full((rows, n), 0x5A5A, np.uint16), X.BF16)
+		dev.synchronize()
+		_launch(shim, path, meta, (-(-rows // meta["M_PER_BLOCK"]) * -(-n // meta["N_PER_BLOCK"]), 1, 1), [ta, rows, tb, n, c, trs, tcs])
+		results.append(np.ascontiguousarray(c.download()).view(np.uint16))
+	assert np.array_equal(results[0], results[1])
+	values = np.zeros(a.shape)
+	exponent, mantissa = (a >> 3 & 15).astype(np.int32), (a & 7).astype(np.float64)
+	normal = exponent > 0
+	values[normal] = ((1 + mantissa / 8) * np.exp2(exponent - 7))[normal]
+	values[a >= 128] *= -1
+	scale = rs[:, None].astype(np.float64) * cs
+	want = values @ b.T.astype(np.float64) * scale
+	magnitude = np.abs(values) @ np.abs(b.T.astype(np.float64)) * scale
+	got = (results[1].astype(np.uint32) << 16).view(np.float32).reshape(rows, n)
+	assert np.all(np.abs(got - want) <= np.abs(want) * 2.0 ** -8 + magnitude * k * 2.0 ** -24)

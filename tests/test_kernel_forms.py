@@ -51,6 +51,13 @@ def test_the_form_a_launch_takes(make, picks):
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
+@pytest.mark.parametrize("k", [2048, 8192])
+def test_widened_weights_pay_up_to_two_rounds_of_workgroups(k):
+	kernel = recipes.ffn_y_kernel(None, 2048, k, k == 2048)
+	assert {rows: kernel.form(rows) for rows in (256, 320, 512, 576)} == {256: "s64x4", 320: "s64x4", 512: "s64x4", 576: "s128x2"}
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
 @pytest.mark.parametrize("make,picks", [
 	(lambda: recipes.attn_decode_kernel(None, 32, 128, 4096), {
 		(1, 256): 256, (8, 256): 256, (8, 512): 512, (8, 4096): 1024,          # at most one workgroup per compute unit

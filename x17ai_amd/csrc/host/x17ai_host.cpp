@@ -1111,7 +1111,7 @@ namespace gemm_cost {
 		}
 	};
 	struct Curves { Curve large, tile64, tile128_deep, tile128; };   // 256 x 256 | 64 x 64 | 128 x 128, four stages | two
-	static Curves const CURVES[4] = {
+	static Curves const CURVES[5] = {
 		{   // int8
 			{{{0.125, 4.9, 7.5}, {0.5, 6.6, 8.3}, {1, 8.7, 12.5}, {1.02, 10.5, 18.2}, {2, 13.9, 23.5}, {2.02, 15.4, 30.0}, {3, 16.6, 35.7}}, 0.3},
 			{{{0.25, 3.5, 1.1}, {1, 3.5, 1.6}, {1.02, 5.3, 2.7}, {2, 5.7, 4.6}, {4, 7.9, 8.6}}},
@@ -1130,7 +1130,15 @@ namespace gemm_cost {
 			{{{0.25, 3.9, 3.0}, {1, 4.3, 4.6}, {1.02, 6.9, 6.6}, {2, 6.5, 8.9}, {2.02, 9.4, 10.5}, {4, 11.5, 17.2}, {4.02, 14.1, 18.5}, {6, 17.2, 26.4}}},
 			{{{0.25, 3.3, 4.5}, {1, 3.5, 6.6}, {1.02, 5.0, 5.7}, {2, 5.8, 8.1}, {2.02, 6.8, 11.1}, {4, 8.7, 16.2}, {4.02, 10.4, 18.3}, {6, 12.0, 24.6}}},
 		},
-		{   // e4m3 x int8
+		{   // e4m3 x int8: the 64 x 64 form widens its weights once per workgroup, and with two workgroups on a compute unit it
+		    // beats 128 x 128 up to two rounds (4096 columns, weights from memory, 320 .. 512 rows: K = 8192 44-52 us and 63, K = 2048
+		    // 15-17 and 21), behind them no longer (576 rows: 67 and 64, 23 and 22)
+			{{{0.125, 6.2, 15.4}, {0.5, 8.3, 15.3}, {1, 11.2, 21.7}, {1.02, 12.8, 36.5}, {2, 17.1, 41.5}, {2.02, 18.9, 59.0}, {3, 19.6, 67.4}}, 0.3},
+			{{{0.125, 3.4, 2.8}, {1, 3.2, 3.85}, {1.02, 5.8, 4.8}, {2, 6.0, 5.85}, {2.02, 8.3, 7.3}, {3, 7.9, 8.45}, {4, 14.6, 10.3}}},
+			{{{0.25, 3.2, 7.1}, {1, 3.5, 7.9}, {1.02, 5.1, 14.7}, {2, 5.1, 16.0}, {2.02, 6.9, 21.8}, {4, 8.1, 32.0}, {4.02, 9.9, 37.3}, {6, 11.1, 49.8}}},
+			{{{0.25, 3.1, 7.1}, {1, 3.4, 7.7}, {1.02, 3.9, 11.4}, {2, 3.7, 14.1}, {2.02, 4.3, 19.0}, {4, 5.3, 28.2}, {4.02, 5.7, 32.4}, {6, 5.7, 43.8}}},
+		},
+		{   // int8 x e4m3, and e4m3 x int8 through the head-normalising writers: every wavefront widens what it reads
 			{{{0.125, 6.2, 15.4}, {0.5, 8.3, 15.3}, {1, 11.2, 21.7}, {1.02, 12.8, 36.5}, {2, 17.1, 41.5}, {2.02, 18.9, 59.0}, {3, 19.6, 67.4}}, 0.3},
 			{{{0.25, 2.9, 3.1}, {1, 3.0, 3.7}, {1.02, 3.9, 6.5}, {2, 4.3, 8.2}, {4, 5.5, 14.2}}},
 			{{{0.25, 3.2, 7.1}, {1, 3.5, 7.9}, {1.02, 5.1, 14.7}, {2, 5.1, 16.0}, {2.02, 6.9, 21.8}, {4, 8.1, 32.0}, {4.02, 9.9, 37.3}, {6, 11.1, 49.8}}},
@@ -1148,7 +1156,7 @@ GemmKernel::Small const *GemmKernel::form_for(size_t a_rows) const {
 		return ((a_rows + m.M_PER_BLOCK - 1) >> ctz(m.M_PER_BLOCK)) * ((n_raw + m.N_PER_BLOCK - 1) >> ctz(m.N_PER_BLOCK));
 	};
 	bool const natural = epilogue_kind == 3 || epilogue_kind == 5 || epilogue_kind == 6;
-	gemm_cost::Curves const &c = gemm_cost::CURVES[a_dtype != b_dtype ? 3 : a_dtype == DType::E4m3 ? 2 : natural ? 1 : 0];
+	gemm_cost::Curves const &c = gemm_cost::CURVES[a_dtype != b_dtype ? (a_dtype == DType::E4m3 && !natural ? 3 : 4) : a_dtype == DType::E4m3 ? 2 : natural ? 1 : 0];
 	double best = c.large.us(tiles_of(metadata), double(a_cols));
 	Small const *chosen = nullptr;
 	for (Small const &s : small) {

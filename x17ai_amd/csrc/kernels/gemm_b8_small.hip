@@ -10,8 +10,14 @@
 // a block of its own (32 x 32 of the 64 x 64; of the 128 x 128 64 x 32, and 64 x 64 of e4m3 x int8), in the 256 x 256
 // kernel's order, and every form gives that kernel's bytes.
 // What bounds int8 and e4m3 is the stream of tiles from L2 / HBM into LDS: X17_SMALL_STAGES - 1 K steps of requests are
-// kept in flight per workgroup, one barrier per step.  e4m3 x int8 in 64 x 64 tiles is bound by widening to f16 (256 rows,
-// 4096 columns, K = 8192: 33 us, vector ALU 50 % busy, matrix cores 24 %, one wavefront per SIMD).
+// kept in flight per workgroup, one barrier per step.
+// e4m3 x int8 in 64 x 64 tiles is bound by the instructions around the f16 matrix instructions, which one wavefront per SIMD
+// issues at one in about ten clocks.  Of 34 per 32 bytes of K twenty widened a weight fragment, the same one in two
+// wavefronts; four further wavefronts now do that once, from memory through registers, and leave f16 in LDS (gemm_small_tile.h:
+// WIDEN_ONCE).  256 rows, 4096 columns, K = 8192: 34.8 -> 30.7 us (39.1 -> 34 with weights from memory; vector ALU 29 %, matrix
+// cores 21 %, LDS 38 % busy: the step's chain barrier - reads - widening - multiplications bounds it); 320 rows, two
+// workgroups per compute unit: 61 -> 44 us.  Tried: token tiles through the same registers 34.6 / 49.7 us, half a step's
+// fragments read across the barrier from a third widened tile 32.2 / 45.5 us.
 
 #include "common.h"
 #include "x17_device.h"
@@ -55,6 +61,63 @@ constexpr u32 owner(int j) { return gt::NATURAL ? 0 : (u32)j * gt::WAVES_K / BLO
 constexpr u32 GROUP_BYTES = BLOCKS * (gt::WAVES_K - 1) * BLOCK_BYTES;
 X17_DEV u32 exchange_offset(int j, u32 from) { return (j * (gt::WAVES_K - 1) + (from < owner(j) ? from : from - 1)) * BLOCK_BYTES; }
 static_assert(gt::WAVES / gt::WAVES_K * GROUP_BYTES <= gt::SMEM_BYTES, "the exchange fits the ring");
+
+// The barrier of a K step of the widening form, behind this wavefront's LDS reads and writes
+X17_DEV void step_barrier() {
+	asm volatile("" ::: "memory");
+	__builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0)
+	__builtin_amdgcn_s_barrier();
+	__builtin_amdgcn_sched_barrier(0);
+	asm volatile("" ::: "memory");
+}
+
+// The widening form's second half of a workgroup: weights from memory into registers, WIDENER_DEPTH K steps ahead, and from
+// there as f16 into the tile behind the one the matrix wavefronts are at, widened one step before that.  Past the
+// end the last step is loaded again, into tiles nobody reads any more.
+[[maybe_unused]] X17_DEV void widen_and_store(u8 *smem, u8 const *b_tile, u32 widener, u32 lane) {
+	constexpr u32 UNITS = gt::WIDENER_UNITS;
+	u32 src[UNITS];
+	u8 *dst[UNITS][2];
+	X17_UNROLL for (u32 u = 0; u < UNITS; ++u) {
+		u32 const row = gt::widener_row(widener, u, lane), chunk = gt::widener_chunk(lane);
+		src[u] = gt::w_source_row(row) * K_TOTAL + 16 * chunk;
+		X17_UNROLL for (u32 h = 0; h < 2; ++h) dst[u][h] = smem + gt::WIDE_OFFSET + gt::wide_offset(row, 2 * chunk + h);
+	}
+	// (buffer loads: lane offset and step's offset need no vector arithmetic; bounded by the tile's rows)
+	auto const rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<u8 *>(b_tile), 0, gt::N_PER_BLOCK * K_TOTAL, 0x00020000);
+	v4i raw[gt::WIDENER_DEPTH][UNITS];
+	v8h wide[UNITS][2];
+	auto load = [&](u32 step, u32 slot) __attribute__((always_inline)) {
+		u32 const k0 = (step < K_STEPS ? step : K_STEPS - 1) * gt::K_STEP;
+		X17_UNROLL for (u32 u = 0; u < UNITS; ++u) raw[slot][u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rows, src[u], k0, 0));
+	};
+	auto widen = [&](u32 slot) __attribute__((always_inline)) {
+		X17_UNROLL for (u32 u = 0; u < UNITS; ++u) {
+			X17_UNROLL for (u32 h = 0; h < 2; ++h) wide[u][h] = widen8(raw[slot][u][2 * h], raw[slot][u][2 * h + 1], B_KIND);
+		}
+	};
+	auto store = [&](u32 tile) __attribute__((always_inline)) {
+		X17_UNROLL for (u32 u = 0; u < UNITS; ++u) {
+			X17_UNROLL for (u32 h = 0; h < 2; ++h) *reinterpret_cast<v8h *>(dst[u][h] + tile * gt::WIDE_BYTES) = wide[u][h];
+		}
+	};
+	X17_UNROLL for (u32 d = 0; d < gt::WIDENER_DEPTH; ++d) load(d, d);
+	X17_UNROLL for (u32 d = 0; d < gt::WIDE_TILES; ++d) {
+		widen(d);
+		load(d + gt::WIDENER_DEPTH, d);
+		if (d + 1 < gt::WIDE_TILES) store(d);
+	}
+	for (u32 base = 0; base < K_STEPS; base += gt::WIDENER_DEPTH) {
+		X17_UNROLL for (u32 j = 0; j < gt::WIDENER_DEPTH; ++j) {
+			if (base + j < K_STEPS) {
+				step_barrier();
+				store((j + 1) % gt::WIDE_TILES);
+				widen((j + 2) % gt::WIDENER_DEPTH);
+				load(base + j + 2 + gt::WIDENER_DEPTH, (j + 2) % gt::WIDENER_DEPTH);
+			}
+		}
+	}
+}
 
 } // namespace
 
@@ -100,6 +163,13 @@ void kernel(
 	u8 const *b_tile = b + (size_t)tile.n * K_TOTAL;
 #endif
 
+	if constexpr (gt::WIDEN_ONCE) {
+		if (wave >= gt::WAVES) {
+			widen_and_store(smem, b_tile, wave - gt::WAVES, lane);
+			return;
+		}
+	}
+
 	// ---- requests: this wavefront's units of the token tile and of the weight tile
 	u32 x_src[gt::X_UNITS], w_src[gt::W_UNITS];
 	X17_UNROLL for (u32 u = 0; u < gt::X_UNITS; ++u) {
@@ -118,7 +188,9 @@ void kernel(
 		X17_UNROLL for (u32 u = 0; u < gt::X_UNITS; ++u) load_to_lds_16(x_dst + slot * gt::STAGE_BYTES + u * 1024, a_tile + k0, x_src[u]);
 		X17_UNROLL for (u32 u = 0; u < gt::W_UNITS; ++u) load_to_lds_16(w_dst + slot * gt::STAGE_BYTES + u * 1024, b_tile + k0, w_src[u]);
 	};
-	X17_UNROLL for (u32 s = 0; s + 1 < gt::STAGES; ++s) request(s, s);
+	if constexpr (!gt::WIDEN_ONCE) {
+		X17_UNROLL for (u32 s = 0; s + 1 < gt::STAGES; ++s) request(s, s);
+	}
 
 	Acc acc[BN][BM];
 	X17_UNROLL for (int bn = 0; bn < BN; ++bn) {
@@ -130,9 +202,50 @@ void kernel(
 	u32 const x_off = (wm * gt::WAVE_M + lane % 32) * ROW_BYTES;
 	u32 const w_off = X_TILE_BYTES + (wn * gt::WAVE_N + lane % 32) * ROW_BYTES;
 
+	if constexpr (gt::WIDEN_ONCE) {
+		// a lane's fragments in a token and in a widened tile; the rings' positions are immediates beside them
+		u8 const *x_at[SLICES], *w_at[SLICES][2];
+		X17_UNROLL for (u32 s = 0; s < SLICES; ++s) {
+			x_at[s] = smem + x_off + (((2 * s + half) ^ swz) << 4);
+			X17_UNROLL for (u32 h = 0; h < 2; ++h) {
+				w_at[s][h] = smem + gt::WIDE_OFFSET + gt::wide_offset(wn * gt::WAVE_N + lane % 32, 4 * s + 2 * half + h);
+			}
+		}
+		auto request_x = [&](u32 step, u32 to) __attribute__((always_inline)) {
+			u8 const *const from = a_tile + (step < K_STEPS ? step : K_STEPS - 1) * gt::K_STEP;
+			X17_UNROLL for (u32 u = 0; u < gt::X_UNITS; ++u) load_to_lds_16(x_dst + to * gt::STAGE_BYTES + u * 1024, from, x_src[u]);
+		};
+		X17_UNROLL for (u32 s = 0; s + 1 < gt::STAGES; ++s) request_x(s, s);
+		static_assert(!gt::WIDEN_ONCE || gt::STAGES % gt::WIDE_TILES == 0, "one loop over both rings");
+		for (u32 base = 0; base < K_STEPS; base += gt::STAGES) {
+			X17_UNROLL for (u32 j = 0; j < gt::STAGES; ++j) {
+				if (base + j < K_STEPS) {
+					// this wavefront's requests of the step have landed and its reads of the step before are done; behind the barrier
+					// so are everybody's, the step's weights are widened, and the slot of the token tile before is free
+					wait_vmcnt<(gt::STAGES - 2) * gt::X_UNITS>();
+					step_barrier();
+					v4i raw[SLICES];
+					v8h wide[SLICES][2];
+					X17_UNROLL for (u32 s = 0; s < SLICES; ++s) {
+						raw[s] = *reinterpret_cast<v4i const *>(x_at[s] + j * gt::STAGE_BYTES);
+						X17_UNROLL for (u32 h = 0; h < 2; ++h) wide[s][h] = *reinterpret_cast<v8h const *>(w_at[s][h] + j % gt::WIDE_TILES * gt::WIDE_BYTES);
+					}
+					__builtin_amdgcn_sched_barrier(0);      // (all reads are on their way before anything waits for one)
+					request_x(base + j + gt::STAGES - 1, (j + gt::STAGES - 1) % gt::STAGES);
+					X17_UNROLL for (u32 s = 0; s < SLICES; ++s) {
+						X17_UNROLL for (u32 h = 0; h < 2; ++h) {        // mma_slice's order
+							v8h const xf = widen8(raw[s][2 * h], raw[s][2 * h + 1], A_KIND);
+							v16f const r = __builtin_amdgcn_mfma_f32_32x32x16_f16(wide[s][h], xf, __builtin_bit_cast(v16f, acc[0][0]), 0, 0, 0);
+							acc[0][0] = __builtin_bit_cast(Acc, r);
+						}
+					}
+				}
+			}
+		}
+	}
 	u32 slot = 0;
 	X17_SMALL_LOOP_PRAGMA
-	for (u32 ks = 0; ks < K_STEPS; ++ks) {
+	for (u32 ks = 0; ks < (gt::WIDEN_ONCE ? 0 : K_STEPS); ++ks) {
 		// this wavefront's requests of step ks have landed and its reads of step ks - 1 are done; behind the barrier so
 		// are everybody's, and the slot of step ks - 1 takes the requests of step ks + STAGES - 1
 		wait_vmcnt<(gt::STAGES - 2) * LOADS_PER_STAGE>();

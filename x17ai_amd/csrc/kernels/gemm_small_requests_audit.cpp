@@ -69,7 +69,30 @@ int main(int argc, char **argv) {
 		return nullptr;
 	};
 	if (char const *what = pattern(gt::M_PER_BLOCK, gt::X_UNITS, false)) return fail(what, gt::M_PER_BLOCK, 0);
-	if (char const *what = pattern(gt::N_PER_BLOCK, gt::W_UNITS, true)) return fail(what, gt::N_PER_BLOCK, 0);
+	// the widening form: every chunk of the weights is loaded by one widener lane, and every 16 bytes of a widened tile are
+	// written once and read as one fragment
+	auto widened = [&]() -> char const * {
+		std::vector<unsigned> source(gt::N_PER_BLOCK * gt::CHUNKS, 0), stored(gt::WIDE_BYTES / 16, 0), read(gt::WIDE_BYTES / 16, 0);
+		auto touch = [&](std::vector<unsigned> &v, unsigned at) { return at % 16 == 0 && at / 16 < v.size() ? (++v[at / 16], true) : false; };
+		for (unsigned wave = 0; wave < gt::WIDENERS; ++wave) for (unsigned u = 0; u < gt::WIDENER_UNITS; ++u) for (unsigned lane = 0; lane < 64; ++lane) {
+			unsigned const row = gt::widener_row(wave, u, lane), chunk = gt::widener_chunk(lane);
+			if (row >= gt::N_PER_BLOCK || gt::w_source_row(row) >= gt::N_PER_BLOCK) return "row of a widener's load outside its tile";
+			if (chunk >= gt::CHUNKS) return "chunk of a widener's load outside the K step";
+			++source[gt::w_source_row(row) * gt::CHUNKS + chunk];
+			max_chunk = chunk > max_chunk ? chunk : max_chunk;
+			for (unsigned h = 0; h < 2; ++h) if (!touch(stored, gt::wide_offset(row, 2 * chunk + h))) return "a widened chunk is stored outside its tile";
+			++per_step;
+		}
+		// fragment reads: 32-byte slice s, K half of the lane, matrix instruction h
+		for (unsigned row = 0; row < gt::N_PER_BLOCK; ++row) for (unsigned s = 0; s < gt::K_STEP / 32; ++s) for (unsigned half = 0; half < 2; ++half) {
+			for (unsigned h = 0; h < 2; ++h) if (!touch(read, gt::wide_offset(row, 4 * s + 2 * half + h))) return "a widened chunk is read outside its tile";
+		}
+		for (unsigned v : source) if (v != 1) return "a weight-tile chunk is not loaded exactly once";
+		for (unsigned v : stored) if (v != 1) return "a position of the widened tile is not filled exactly once";
+		for (unsigned v : read) if (v != 1) return "a position of the widened tile is not one fragment's";
+		return nullptr;
+	};
+	if (char const *what = gt::WIDEN_ONCE ? widened() : pattern(gt::N_PER_BLOCK, gt::W_UNITS, true)) return fail(what, gt::N_PER_BLOCK, 0);
 	// matrix block bn of a wavefront, register r of a lane half: the writer takes it as column (WAVE_N / 2) * half + 16 * bn + r
 	if (!gt::NATURAL) {
 		for (unsigned wn = 0; wn < gt::WAVES_N; ++wn) for (unsigned bn = 0; bn < gt::WAVE_N / 32; ++bn) for (unsigned half = 0; half < 2; ++half) for (unsigned r = 0; r < 16; ++r) {
@@ -92,7 +115,8 @@ int main(int argc, char **argv) {
 		bool const kv_side = o.n >= Q_COLS;
 		if (!kv_side && o.n + gt::N_PER_BLOCK > Q_COLS) return fail("a tile straddles the q and kv weights", o.n + gt::N_PER_BLOCK, Q_COLS);
 		unsigned long long const w_first = kv_side ? o.n - Q_COLS : o.n, w_rows = kv_side ? N_RAW - Q_COLS : Q_COLS;
-		for (unsigned step = 0; step < K_STEPS + gt::STAGES - 1; ++step) {
+		// (requests run STAGES - 1 steps ahead, a widener's loads WIDENER_DEPTH + 2)
+		for (unsigned step = 0; step < K_STEPS + (gt::WIDEN_ONCE ? gt::WIDENER_DEPTH + 2 : gt::STAGES - 1); ++step) {
 			unsigned long long const k0 = (step < K_STEPS ? step : K_STEPS - 1) * (unsigned long long)gt::K_STEP;
 			unsigned long long const col_end = k0 + 16ull * max_chunk + 16;
 			if (col_end > K) return fail("request leaves its operand row", col_end, K);

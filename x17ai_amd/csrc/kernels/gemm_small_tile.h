@@ -28,16 +28,25 @@ constexpr unsigned WAVES_M = MID ? 128 / WAVE_M : SPLIT_K ? 1 : 64 / WAVE_M;
 constexpr unsigned WAVES_N = MID ? 128 / WAVE_N : SPLIT_K ? 1 : 64 / WAVE_N;
 constexpr unsigned WAVES_K = !SPLIT_K ? 1 : MID ? 2 : 4;                              // wavefronts that share an output block
 constexpr unsigned WAVES = WAVES_M * WAVES_N * WAVES_K;
-constexpr unsigned THREADS_PER_BLOCK = 64 * WAVES;
+// The 64 x 64 form of e4m3 x int8: four more wavefronts bring the weights into LDS and widen them to f16 on the way, once for
+// the workgroup.  (An int8 fragment is twenty instructions, an e4m3 one eight: widening the tokens there as well adds more
+// LDS traffic than it takes instructions out.)
+constexpr bool WIDEN_ONCE = X17_A_KIND == 1 && X17_B_KIND == 0 && !MID && !NATURAL;
+constexpr unsigned WIDENERS = WIDEN_ONCE ? 4 : 0;
+constexpr unsigned THREADS_PER_BLOCK = 64 * (WAVES + WIDENERS);
 constexpr unsigned M_PER_BLOCK = WAVE_M * WAVES_M;
 constexpr unsigned N_PER_BLOCK = WAVE_N * WAVES_N;
 
 // bytes of K per pipeline step: four e4m3 slices of 64 need 256
-constexpr unsigned K_STEP = MID ? 128 : 256;
-constexpr unsigned STAGES = X17_SMALL_STAGES;               // LDS ring depth
-constexpr unsigned STAGE_BYTES = (M_PER_BLOCK + N_PER_BLOCK) * K_STEP;
-constexpr unsigned SMEM_BYTES = STAGES * STAGE_BYTES;
-constexpr unsigned WAVES_PER_SIMD = 160 * 1024 / SMEM_BYTES * WAVES / 4;      // as many workgroups as the LDS holds
+constexpr unsigned K_STEP = MID || WIDEN_ONCE ? 128 : 256;
+constexpr unsigned STAGES = WIDEN_ONCE ? 6 : X17_SMALL_STAGES;      // LDS ring depth
+constexpr unsigned STAGE_BYTES = (M_PER_BLOCK + (WIDEN_ONCE ? 0 : N_PER_BLOCK)) * K_STEP;
+// two widened weight tiles behind the token tiles: one is read while the next one is written
+constexpr unsigned WIDE_TILES = 2;
+constexpr unsigned WIDE_OFFSET = STAGES * STAGE_BYTES;
+constexpr unsigned WIDE_BYTES = N_PER_BLOCK * 2 * K_STEP;
+constexpr unsigned SMEM_BYTES = WIDE_OFFSET + (WIDEN_ONCE ? WIDE_TILES * WIDE_BYTES : 0);
+constexpr unsigned WAVES_PER_SIMD = 160 * 1024 / SMEM_BYTES * (WAVES + WIDENERS) / 4;      // as many workgroups as the LDS holds
 static_assert(X17_A_COLS % K_STEP == 0, "K must be whole steps");
 static_assert(SMEM_BYTES <= 160 * 1024, "LDS ring does not fit");
 
@@ -57,6 +66,15 @@ constexpr unsigned w_source_row(unsigned r) {
 	unsigned const i = r % 32, bn = (r % WAVE_N) / 32;
 	return NATURAL ? r : WAVE_N * (r / WAVE_N) + (WAVE_N / 2) * ((i / 4) % 2) + 16 * bn + 4 * (i / 8) + i % 4;
 }
+// ---- the widening form: a widener's 16-byte loads of a step's weights (consecutive lanes read consecutive bytes of a row), and
+// where the eight f16 of raw bytes 8 c .. 8 c + 7 of row r are stored in a widened tile.  What eight lanes write, and the
+// sixteen rows a read serves at a time, lie in different 16-byte columns of the 256-byte bank line.
+constexpr unsigned WIDENER_UNITS = WIDEN_ONCE ? N_PER_BLOCK / UNIT_ROWS / WIDENERS : 1;
+constexpr unsigned widener_row(unsigned wave, unsigned u, unsigned lane) { return unit_row(wave * WIDENER_UNITS + u, lane); }
+constexpr unsigned widener_chunk(unsigned lane) { return lane % CHUNKS; }
+constexpr unsigned wide_offset(unsigned row, unsigned c) { return row * 2 * K_STEP + ((c ^ (row & 15)) << 4); }
+constexpr unsigned WIDENER_DEPTH = 6;                        // K steps of weights on their way, in registers
+static_assert(WIDENER_DEPTH % WIDE_TILES == 0, "one loop over both rings");
 // First token row and raw column of workgroup `lin`: each XCD (workgroups are dealt round-robin to 8 of them) gets a
 // contiguous run of tiles, column tiles slowest inside bands of BAND token tiles, so that an XCD reads its weight
 // columns once.  A last token tile that would overhang is moved back to end at the matrix edge.

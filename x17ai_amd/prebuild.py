@@ -135,6 +135,8 @@ def _specs():
 	add(("dequant", 4096, 384, E4M3, E4M3, False, True))
 	add(("dequant", 4096, 384, E4M3, INT8, False, True))
 	add(("ffn_y", 256, 4096, True, E4M3, INT8))
+	for k in (256, 768, 1280):           # weights widened once per workgroup, around the rings' six steps
+		add(("dequant", k, 384, E4M3, INT8, False, True))
 	# ---- x17ai_amd.block: benchmark config 4 (bench.py, tests/config4_chain.py) and the reference's own configuration
 	for strict in (True, False):
 		add(("block", 2048, 16, 128, 8192, BF16, strict))
