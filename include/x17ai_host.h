@@ -148,7 +148,8 @@ int x17h_attn_kernel_new(X17hDevice *dev, char const *kernel_name, X17hAttnConfi
 void x17h_attn_kernel_free(X17hAttnKernel *k);
 /* heads a workgroup of a launch takes one behind the other (1 .. 128 / head_dim; every choice gives the same bytes) */
 size_t x17h_attn_kernel_heads_per_workgroup(X17hAttnKernel *k, size_t seq_len, size_t batch, size_t window_size);
-/* queries a wavefront of a forward launch takes: 32, or 16 where a speed build's launch would leave most of the chip idle */
+/* queries a wavefront of a forward launch takes: 32, or 16 where a speed build's launch would leave most of the chip idle
+ * (either gives the same bytes) */
 size_t x17h_attn_kernel_queries_per_wavefront(X17hAttnKernel *k, size_t seq_len, size_t batch, size_t window_size);
 /* AttnKernel::launch, attn.rs:234-236 / 353-447.  l may be NULL.  batch > 1 is an extension:
  * the rows of q/kv/out are `batch` independent sequences of equal length. */

@@ -334,3 +334,78 @@ def test_weights_widened_once_per_workgroup(shim, k, rows):  # noqa: F811
 	magnitude = np.abs(values) @ np.abs(b.T.astype(np.float64)) * scale
 	got = (results[1].astype(np.uint32) << 16).view(np.float32).reshape(rows, n)
 	assert np.all(np.abs(got - want) <= np.abs(want) * 2.0 ** -8 + magnitude * k * 2.0 ** -24)
+
+
+# (head_dim, heads, row scales, bf16 out, tokens, batch, window)
+QUERY_WIDTHS = [
+	(64, 8, True, True, 1024, 1, 256), (64, 8, False, False, 576, 2, 0), (64, 2, False, False, 192, 3, 16), (64, 2, True, False, 448, 1, 48),
+	(32, 4, False, False, 768, 2, 64), (32, 4, True, False, 320, 1, 0),
+	(128, 16, False, False, 256, 3, 512), (128, 2, False, False, 1088, 1, 112), (128, 2, True, True, 640, 2, 0), (128, 2, True, False, 128, 1, 0),
+]
+
+
+@pytest.mark.parametrize("hd,h,row_scales,out_bf16,seq,batch,window", QUERY_WIDTHS)
+@pytest.mark.parametrize("spread", [0.25, 1.0, 3.0], ids=["flat", "gaussian", "peaked"])
+def test_a_querys_attention_does_not_depend_on_the_queries_a_wavefront_takes(shim, hd, h, row_scales, out_bf16, seq, batch, window, spread):  # noqa: F811
+	"""The speed build's two code objects give the same bytes, outputs and log-sum-exp: scores flat enough never to bring the
+	accumulators down and peaked enough to do it many times, some heads at a negative temperature and one at zero."""
+	dev = X.Device(0)
+	rng = rng_for("query widths", hd, h, row_scales, seq, batch, window, spread)
+	rows, width = seq * batch, h * hd
+	t = lambda a, dtype: X.Tensor.from_numpy(dev, np.ascontiguousarray(a), dtype)
+	temp = ((0.5 + rng.random(h)) * spread).astype(np.float32)
+	temp[0] = -temp[0]
+	if h > 2:
+		temp[2] = 0.0
+	args = [t(i8_codes(rng, (rows, width)), X.INT8), t(i8_codes(rng, (rows, 2 * width)), X.INT8), t(i8_codes(rng, (h, hd)), X.INT8),
+	        t(i8_codes(rng, (h, hd)), X.INT8), t(temp, X.F32)]
+	tail = []
+	if row_scales:
+		kernel = recipes.attn_row_scaled_kernel(None, h, hd, X.BF16 if out_bf16 else X.INT8, False)
+		qs, ks, vs = (0.125 * np.exp(0.5 * rng.standard_normal((h, rows))).astype(np.float32) for _ in range(3))
+		tail = [t(a, X.F32) for a in (qs, ks, *recipes.attn_row_scale_operands(vs, X.BF16 if out_bf16 else X.INT8))]
+	else:
+		kernel = recipes.attn_kernel(None, h, hd, False)
+	results = []
+	for form in ("", "q16"):
+		path = os.path.join(_ffi.kernel_cache_dir(), kernel.name, form)
+		with open(os.path.join(path, "meta.json")) as f:
+			meta = json.load(f)
+		out, l = t(np.full((rows, width), 0x55, np.uint16 if out_bf16 else np.int8), X.BF16 if out_bf16 else X.INT8), t(np.full((h, rows), 7.0, np.float32), X.F32)
+		dev.synchronize()
+		_launch(shim, path, meta, (-(-seq // meta["Q_PER_BLOCK"]), h, batch), [seq, *args, out, l, window, *tail])
+		results.append((np.ascontiguousarray(out.download()), l.download()))
+	assert np.array_equal(results[0][1].view(np.uint32), results[1][1].view(np.uint32))
+	assert np.array_equal(results[0][0].view(np.uint8), results[1][0].view(np.uint8))
+
+
+@pytest.mark.parametrize("h,hd,row_scales", [(8, 64, True), (16, 128, False), (4, 32, False)])
+def test_a_sequences_attention_does_not_depend_on_what_is_launched_with_it(h, hd, row_scales):
+	"""One prompt alone, in a batch, and as the beginning of a longer sequence (causal: its tokens see the same keys): the same bytes,
+	whichever code object the launches take."""
+	dev = X.Device(0)
+	rng = rng_for("launched with it", h, hd, row_scales)
+	seq, window, many = 448, 128, 32
+	width = h * hd
+	q, kv = i8_codes(rng, (seq * many, width)), i8_codes(rng, (seq * many, 2 * width))
+	sk, sv, temp = i8_codes(rng, (h, hd)), i8_codes(rng, (h, hd)), (0.5 + rng.random(h)).astype(np.float32)
+	qs, ks, vw = (0.125 * (0.75 + 0.5 * rng.random((h, seq * many))).astype(np.float32) for _ in range(3))
+	sw, osc = np.ones(h, np.float32), np.full(h, 0.125, np.float32)
+	t = lambda a, dtype: X.Tensor.from_numpy(dev, np.ascontiguousarray(a), dtype)
+	kernel = recipes.attn_row_scaled_kernel(dev, h, hd, X.BF16, False) if row_scales else recipes.attn_kernel(dev, h, hd, False)
+
+	def launch(rows, batch):
+		out, l = X.Tensor(dev, (rows, width), X.BF16 if row_scales else X.INT8), X.Tensor(dev, (h, rows), X.F32)
+		args = (t(q[:rows], X.INT8), t(kv[:rows], X.INT8), t(sk, X.INT8), t(sv, X.INT8), t(temp, X.F32), out, l, window)
+		if row_scales:
+			kernel.launch_row_scaled(*args, *(t(a[:, :rows], X.F32) for a in (qs, ks, vw)), t(sw, X.F32), t(osc, X.F32), batch)
+		else:
+			kernel.launch(*args, batch)
+		return np.ascontiguousarray(out.download()), l.download()
+	alone = launch(seq, 1)
+	widths = {kernel.queries_per_wavefront(seq, 1, window), kernel.queries_per_wavefront(seq, many, window), kernel.queries_per_wavefront(seq * many, 1, window)}
+	assert widths == {16, 32}
+	for rows, batch in ((seq * 3, 3), (seq * many, many), (seq * 2, 1), (seq * many, 1)):
+		out, l = launch(rows, batch)
+		assert np.array_equal(out[:seq].view(np.uint8), alone[0].view(np.uint8)), (rows, batch)
+		assert np.array_equal(l[:, :seq].view(np.uint32), alone[1].view(np.uint32)), (rows, batch)

@@ -89,8 +89,8 @@ def test_the_heads_a_workgroup_takes(make, picks):
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="needs hipcc")
 @pytest.mark.parametrize("make,picks", [
-	(lambda: recipes.attn_row_scaled_kernel(None, 8, 64, X.BF16, False), {(1024, 1, 256): 16, (2048, 1, 0): 16, (3072, 1, 512): 16, (3072, 1, 1024): 32, (5120, 1, 256): 16, (5120, 1, 512): 32, (8192, 1, 64): 32}),
-	(lambda: recipes.attn_kernel(None, 16, 128, False), {(256, 1, 512): 16, (1024, 1, 0): 16, (1536, 1, 256): 16, (1536, 1, 512): 32, (2048, 1, 64): 16, (8192, 4, 512): 32}),
+	(lambda: recipes.attn_row_scaled_kernel(None, 8, 64, X.BF16, False), {(1024, 1, 256): 16, (2048, 1, 0): 16, (3072, 1, 256): 16, (3072, 1, 512): 32, (6144, 1, 128): 16, (6144, 1, 256): 32, (8192, 1, 64): 32}),
+	(lambda: recipes.attn_kernel(None, 16, 128, False), {(256, 1, 512): 16, (1024, 1, 0): 16, (1536, 1, 64): 16, (1536, 1, 128): 32, (2048, 1, 64): 16, (8192, 4, 512): 32}),
 	# the strict build has one order of operations; the backward kernels have no such form
 	(lambda: recipes.attn_kernel(None, 2, 64, True), {(128, 1, 0): 32}),
 	(lambda: recipes.attn_d_q_kernel(None, 4, 32), {(128, 1, 0): 32}),

@@ -419,8 +419,8 @@ class AttnKernel:
 		return int(_ffi.host().x17h_attn_kernel_heads_per_workgroup(self._h, seq_len, batch, window_size))
 
 	def queries_per_wavefront(self, seq_len: int, batch: int, window_size: int) -> int:
-		"""Queries a wavefront of such a forward launch takes: 32, or 16 in the speed build's small launches (same recurrence;
-		float32 sums in another order)."""
+		"""Queries a wavefront of such a forward launch takes: 32, or 16 in the speed build's small launches; both give
+		the same bytes."""
 		return int(_ffi.host().x17h_attn_kernel_queries_per_wavefront(self._h, seq_len, batch, window_size))
 
 	def n_ops(self, seq_len: int, window_size: int) -> float:

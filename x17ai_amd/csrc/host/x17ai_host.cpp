@@ -1336,21 +1336,23 @@ std::unique_ptr<AttnKernel> AttnKernel::create(std::shared_ptr<HipDevice> device
 }
 
 // Sixteen queries per wavefront and 64 per workgroup while the 32-query kernel's workgroups of 128 leave most of the chip idle;
-// beyond that the shorter the walk, the longer it stays ahead (it then is the set-up and the output that fill the chip).
-// Fitted to 168 launches of 4 .. 32 heads of 32, 64 and 128; us with 32 / 16 queries, windows of 64 | 256 | 1024:
-//    32 workgroups of 128   8 heads of 64, row scales   10.5 / 6.8 | 15.4 / 11.3 | 17.0 / 15.2
-//   128                     8 heads of 64, row scales   10.8 / 7.1 | 15.8 / 11.7 | 32.6 / 28.7
-//                           16 heads of 128             10.8 / 7.8 | 15.8 / 12.2 | 28.7 / 25.2
-//   256                     8 heads of 64, row scales   11.2 / 8.4 | 16.3 / 14.0 | 33.7 / 33.6
-//                           16 heads of 128             11.1 / 9.6 | 16.3 / 17.1 | 33.5 / 35.1
-//   448                     16 heads of 128             14.8 / 16.0 | 21.8 / 27.2 | 44.5 / 62.3
+// beyond that the shorter the walk, the longer it stays ahead (it then is the set-up and the output that fill the chip).  Both give
+// the same bytes.  Fitted to 576 launches of 4 .. 32 heads of 32, 64 and 128, 32 .. 448 workgroups: 0.07 % behind the faster one
+// in the mean, 3 % at most.  us with 32 / 16 queries, windows of 64 | 256 | 1024:
+//    32 workgroups of 128   8 heads of 64, row scales   10.1 / 7.2 | 15.0 / 11.3 | 16.6 / 14.6
+//   128                     8 heads of 64, row scales   10.2 / 7.5 | 15.2 / 11.8 | 32.2 / 28.0
+//                           16 heads of 128             10.2 / 8.3 | 15.2 / 13.5 | 28.2 / 27.4
+//   256                     8 heads of 64, row scales   10.5 / 9.1 | 15.6 / 14.8 | 32.4 / 33.9
+//                           16 heads of 128             10.6 / 10.9 | 15.6 / 19.0 | 32.9 / 40.0
+//   384                     8 heads of 64, row scales   12.2 / 10.9 | 18.3 / 18.1 | 39.7 / 41.0
+//   448                     16 heads of 128             14.2 / 18.3 | 20.9 / 30.5 | 43.7 / 70.1
 bool AttnKernel::narrow_for(size_t seq_len, size_t batch, size_t window) const {
 	if (!narrow) return false;
 	size_t const workgroups = (seq_len + metadata.Q_PER_BLOCK - 1) / metadata.Q_PER_BLOCK * config.n_heads * batch;
 	size_t const walk_bytes = (window == 0 ? seq_len : std::min(window, seq_len)) * config.head_dim;
 	return workgroups <= COMPUTE_UNITS / 2
-		|| (workgroups <= COMPUTE_UNITS * 3 / 4 && walk_bytes <= 32 * 1024)
-		|| (workgroups <= COMPUTE_UNITS * 5 / 4 && walk_bytes <= 16 * 1024);
+		|| (workgroups <= COMPUTE_UNITS && config.row_scales && walk_bytes <= 16 * 1024)
+		|| (workgroups <= COMPUTE_UNITS * 3 / 2 && walk_bytes <= 8 * 1024);
 }
 
 // Heads a workgroup takes one behind the other (a power of two up to 128 / head_dim, the reference's group,

@@ -3,18 +3,25 @@
 //
 // A launch of few workgroups takes as long as one wavefront's walk over its window, and a wavefront alone on its SIMD issues
 // one instruction in about ten clocks: the walk is bound by its number of instructions.  Sixteen queries on the 16 x 16
-// matrix instructions instead of thirty-two halve what a 32-key step spends on scores, and blocks of 64 queries instead of
-// 128 make twice the workgroups and walk two steps less.  1024 tokens, 8 heads of 64, window 256, row scales: 64 workgroups,
-// 12 steps of 0.9 us -> 128 workgroups, 10 steps of 0.6 us; the launch 15.1 -> 11.0 us.  Once the chip is full the 32-query kernel
-// is ahead: it widens and reads a tile for twice the queries.
+// matrix instructions instead of thirty-two halve what a 32-key step spends on probabilities and output, and blocks of 64
+// queries instead of 128 make twice the workgroups and walk two steps less.  1024 tokens, 8 heads of 64, window 256, row scales: 64
+// workgroups and 12 steps, 128 and 10; the launch 15.5 -> 11.4 us.  Once the chip is full the 32-query kernel is ahead: it
+// widens and reads a tile for twice the queries.
 //
 // What differs from attn_fwd_i8.hip, whose comments explain the recurrence and the arithmetic of the speed build:
 //   * One workgroup = 4 wavefronts = 64 queries of one head (grid: query blocks of 64, heads, sequences).
-//   * S^T = K . Q^T on v_mfma_i32_16x16x64_i8 (a lane owns query lane % 16 and the four keys 4 g .. 4 g + 3, g = lane / 16, of each
-//     16-key tile); O^T += V^T . P^T on v_mfma_f32_16x16x16_f16, whose "B" operand those four probabilities are.  Lane group g
-//     holds exactly the reference's partial sum g.
+//   * S^T = K . Q^T on v_mfma_i32_16x16x64_i8 (a lane owns query lane % 16 and four keys of each 16-key tile); O^T += V^T . P^T on
+//     v_mfma_f32_16x16x16_f16, whose "B" operand those four probabilities are.
 //   * The row maximum crosses four lanes instead of two when it moves.
 //   * The f16 V tile's layout: eight keys of one 32-byte granule (what 32 lanes of a transposed read ask for) in eight columns.
+// The bytes are the 32-query kernel's, so that a token's result does not depend on what is launched with it:
+//   * Lane group g owns keys 4 j .. 4 j + 3 with j = 0, 2, 1, 3 (nt::key_of_row): the order in which the 32 x 32 x 16 instruction of
+//     the other kernel takes its sixteen products.  With it the 16 x 16 x 16 instruction rounds as that one does (4 million results
+//     over four distributions of operands: all the same; with keys in their own order 13 to 37 % differ).
+//   * There a whole wavefront brings O and its sums down when one of its 32 queries asks for it.  So a wavefront follows its
+//     twin, the sixteen queries that share such a 32 with it: their scores (the key fragments are there), their running maximum in
+//     lanes, and whether that asks.  It walks the blocks of the 32.  (0.4 of the 11.4 us.)
+//   * Everything else is the same operations per query; the partial sums are added in the reference's order.
 //
 // common.h: as for attn_fwd_i8.hip, X17_STRICT_MATH 0.
 
@@ -52,8 +59,7 @@ constexpr f32 BASE_TEMPERATURE = ROW_SCALES ? f32(constexpr_inv_sqrt(f64(HD)))
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 
-// every lane's value and those of the three lanes that own the same query, combined (op commutative and associative, or the
-// order (g0 op g1) op (g2 op g3) wanted)
+// every lane's value and those of the three lanes that own the same query, combined (op commutative and associative)
 template <class Op>
 X17_DEV u32 over_groups(u32 x, Op op) {
 	auto const a = __builtin_amdgcn_permlane16_swap(x, x, false, false);
@@ -99,14 +105,16 @@ void kernel(
 	size_t const all_rows = (size_t)gridDim.z * seq_len;
 	u32 const q_block0 = (gridDim.x - 1 - blockIdx.x) * nt::Q_PER_BLOCK;
 	u32 const q_wave0 = q_block0 + wave * nt::Q_PER_WAVE;
-	u32 const qi = q_wave0 + qlane;
+	u32 const qi = q_wave0 + qlane, twin_qi = qi ^ nt::Q_PER_WAVE;
+	u32 const q_pair0 = q_wave0 & ~(2 * nt::Q_PER_WAVE - 1);
+	u32 const own_keys = nt::key_of_row(4 * group);          // this lane's keys of a 16-key tile: own_keys .. + 3
 
 	u32 const wr = at::rounded_window(window_size);
 	u32 const vis_bound = wr - 1 < 0x7FFFFFFFu ? wr - 1 : 0x7FFFFFFFu;
 	u32 const kb_begin = at::first_key_block(q_block0, wr);
 	u32 const n_steps = nt::end_key_block(q_block0) - kb_begin;
-	u32 const wave_kb_first = at::first_key_block(q_wave0, wr);
-	u32 const wave_kb_last = q_wave0 / at::KV_PER_STEP;
+	u32 const wave_kb_first = at::first_key_block(q_pair0, wr);
+	u32 const wave_kb_last = q_pair0 / at::KV_PER_STEP;
 
 	i8 const *q_head = q + row_base * Q_STRIDE + (size_t)head * HD;
 	i8 const *kv_head = kv + row_base * KV_STRIDE + (size_t)head * 2 * HD;
@@ -150,30 +158,42 @@ void kernel(
 
 	// ---- per-query setup (cuda/attn_fwd_i8.cuh:444-517), behind the requests
 	bool const group_in_row = 16 * group < HD;            // (head_dim 32: the row has half the bytes of a slice)
-	v4i qf[K_SLICES];
-	i32 sink_dot = 0;
+	v4i qf[K_SLICES], twin_qf[K_SLICES];
+	i32 sink_dot = 0, twin_sink_dot = 0;
 	X17_UNROLL for (u32 s = 0; s < K_SLICES; ++s) {
-		qf[s] = v4i{0, 0, 0, 0};
+		qf[s] = twin_qf[s] = v4i{0, 0, 0, 0};
 		if (group_in_row) {
 			qf[s] = *reinterpret_cast<v4i const *>(q_head + (size_t)qi * Q_STRIDE + 64 * s + 16 * group);
+			twin_qf[s] = *reinterpret_cast<v4i const *>(q_head + (size_t)twin_qi * Q_STRIDE + 64 * s + 16 * group);
 			v4i const sk = *reinterpret_cast<v4i const *>(sink_k + (size_t)head * HD + 64 * s + 16 * group);
-			X17_UNROLL for (int w = 0; w < 4; ++w) sink_dot = __builtin_amdgcn_sdot4(qf[s][w], sk[w], sink_dot, false);
+			X17_UNROLL for (int w = 0; w < 4; ++w) {
+				sink_dot = __builtin_amdgcn_sdot4(qf[s][w], sk[w], sink_dot, false);
+				twin_sink_dot = __builtin_amdgcn_sdot4(twin_qf[s][w], sk[w], twin_sink_dot, false);
+			}
 		}
 	}
-	sink_dot = (i32)over_groups((u32)sink_dot, [](u32 a, u32 b) { return a + b; });
-	u32 const visible = qi < wr ? qi : wr;
-	f32 temperature = BASE_TEMPERATURE * strict::lg2(f32(visible + 4u));
-	temperature = temperature * attn_temperature[head];
+	auto const add = [](u32 a, u32 b) { return a + b; };
+	sink_dot = (i32)over_groups((u32)sink_dot, add);
+	twin_sink_dot = (i32)over_groups((u32)twin_sink_dot, add);
+	// (the lower 32 lanes compute the wavefront's temperatures, the upper ones the twin's)
+	u32 const some_qi = group < 2 ? qi : twin_qi;
+	u32 const visible = some_qi < wr ? some_qi : wr;
+	f32 some_temperature = BASE_TEMPERATURE * strict::lg2(f32(visible + 4u));
+	some_temperature = some_temperature * attn_temperature[head];
 #if X17_ATTN_ROW_SCALES
-	temperature = temperature * q_scale[(size_t)head * all_rows + row_base + qi];
+	some_temperature = some_temperature * q_scale[(size_t)head * all_rows + row_base + some_qi];
 #endif
+	auto const both_temperatures = __builtin_amdgcn_permlane32_swap(f2u(some_temperature), f2u(some_temperature), false, false);
+	f32 const temperature = u2f((u32)both_temperatures[0]);
 	bool const positive_temperature = __builtin_amdgcn_readfirstlane(f2u(attn_temperature[head])) - 1u < 0x7F7FFFFFu;
 
 	v4i s_bias;
 	X17_UNROLL for (int r = 0; r < 4; ++r) s_bias[r] = ROW_SCALES ? 0 : 0x4B400000;
-	f32 const abs_t = __builtin_fabsf(temperature);
+	f32 const abs_t = __builtin_fabsf(temperature), twin_abs_t = __builtin_fabsf(u2f((u32)both_temperatures[1]));
 	f32 const sgn = positive_temperature ? 1.0f : -1.0f;
-	f32 ext = ROW_SCALES ? (f32(sink_dot) * 0.125f) * sgn : (f32(sink_dot) + DOT_BIAS) * sgn;
+	auto const sink_extreme = [&](i32 dot) { return ROW_SCALES ? (f32(dot) * 0.125f) * sgn : (f32(dot) + DOT_BIAS) * sgn; };
+	f32 ext = sink_extreme(sink_dot);
+	f32 twin_ext = sink_extreme(twin_sink_dot), twin_ext_ref = twin_ext;      // (twin_ext: of this lane's keys and the sink)
 	f32 mb, fine;
 	auto set_subtrahend = [&]() {
 		if constexpr (ROW_SCALES) {
@@ -191,7 +211,7 @@ void kernel(
 	f32 ext_ref = ext;                       // O and the sum refer to the maximum HEADROOM above this extreme's score
 	f32 lift = LIFT0, sum_lift = LIFT0 * fine;
 	v2h lift2 = {(_Float16)LIFT0, (_Float16)LIFT0}, neg_bias2 = {(_Float16)(-1024.0f * LIFT0), (_Float16)(-1024.0f * LIFT0)};
-	f32 sum = 0.25f * PROB_SCALE * LIFT0;    // the reference's partial sum `group`
+	f32 sum = 0.25f * PROB_SCALE * LIFT0;    // the reference's partial sum own_keys / 4
 	v4f o_acc[D_TILES];                      // O^T: lane = query, register r = dim 16 dt + 4 group + r
 	{
 #if X17_ATTN_ROW_SCALES
@@ -212,10 +232,10 @@ void kernel(
 	// ---- lane offsets of the operand reads and of the widening
 	u32 k_lane_off[2][K_SLICES], v_lane_off[D_TILES];
 	X17_UNROLL for (u32 tile = 0; tile < 2; ++tile) {
-		X17_UNROLL for (u32 s = 0; s < K_SLICES; ++s) k_lane_off[tile][s] = nt::k_chunk_offset(16 * tile + qlane, group_in_row ? 4 * s + group : 0);
+		X17_UNROLL for (u32 s = 0; s < K_SLICES; ++s) k_lane_off[tile][s] = nt::k_chunk_offset(16 * tile + nt::key_of_row(qlane), group_in_row ? 4 * s + group : 0);
 	}
 	X17_UNROLL for (u32 dt = 0; dt < D_TILES; ++dt) v_lane_off[dt] = nt::v_granule_offset(4 * group + (qlane >> 2), dt) + 8 * (qlane & 3);
-	u32 const widen_dst = stager ? nt::v_granule_offset(tid / CPR, tid % CPR) : 0;
+	u32 const widen_dst = stager ? nt::widened_offset(tid) : 0;
 	auto widen_v = [&](u32 slot, u32 buf) __attribute__((always_inline)) {
 		if (CPR == 8 || stager) {
 			v4u const raw = *reinterpret_cast<v4u const *>(smem + nt::RAW_V_RING_OFFSET + slot * at::RAW_V_TILE_BYTES + tid * 16);
@@ -251,51 +271,66 @@ void kernel(
 		u32 const slot = SLOT >= 0 ? (u32)SLOT : i % nt::RING;
 		widen_v((slot + 1) % nt::RING, (slot + 1) & 1);
 	};
+	static_assert(MAX_LIFT == 32.0f);
+	auto const larger = [](u32 a, u32 b) { return f2u(__builtin_fmaxf(u2f(a), u2f(b))); };
 	auto compute = [&]<bool MASKED, int SLOT>(u32 i) __attribute__((always_inline)) {
 		u32 const slot = SLOT >= 0 ? (u32)SLOT : i % nt::RING;
 		u8 const *k_tile = smem + nt::K_RING_OFFSET + slot * at::K_TILE_BYTES;
 		u8 const *v_tile = smem + nt::V_TILES_OFFSET + (slot & 1) * at::V_TILE_BYTES;
-		v4i s_acc[2];
+		v4i s_acc[2], twin_s_acc[2];
 		X17_UNROLL for (u32 tile = 0; tile < 2; ++tile) {
-			s_acc[tile] = s_bias;
+			s_acc[tile] = twin_s_acc[tile] = s_bias;
 			X17_UNROLL for (u32 s = 0; s < K_SLICES; ++s) {
 				v4i const kf = *reinterpret_cast<v4i const *>(k_tile + k_lane_off[tile][s]);
 				s_acc[tile] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf, qf[s], s_acc[tile], 0, 0, 0);
+				twin_s_acc[tile] = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf, twin_qf[s], twin_s_acc[tile], 0, 0, 0);
 			}
 		}
 		widen_next.template operator()<SLOT>(i);
 		X17_UNROLL for (u32 tile = 0; tile < 2; ++tile) {
-			// this lane's keys of the tile: 4 group .. 4 group + 3
-			f32 y[4];
+			f32 y[4], twin_y[4];
 			[[maybe_unused]] bool vis[4];
 			[[maybe_unused]] f32 const *sc = nullptr;
-			f32 tmax;
 			if constexpr (ROW_SCALES) {
-				sc = reinterpret_cast<f32 const *>(smem + nt::SCALE_RING_OFFSET + slot * at::SCALE_TILE_BYTES) + 16 * tile + 4 * group;
+				sc = reinterpret_cast<f32 const *>(smem + nt::SCALE_RING_OFFSET + slot * at::SCALE_TILE_BYTES) + 16 * tile + own_keys;
 				v4f const ks = *reinterpret_cast<v4f const *>(sc);
-				X17_UNROLL for (u32 r = 0; r < 4; ++r) y[r] = f32(s_acc[tile][r]) * ks[r];
+				X17_UNROLL for (u32 r = 0; r < 4; ++r) {
+					y[r] = f32(s_acc[tile][r]) * ks[r];
+					twin_y[r] = f32(twin_s_acc[tile][r]) * ks[r];
+				}
 			} else {
-				X17_UNROLL for (u32 r = 0; r < 4; ++r) y[r] = u2f((u32)s_acc[tile][r]);
+				X17_UNROLL for (u32 r = 0; r < 4; ++r) {
+					y[r] = u2f((u32)s_acc[tile][r]);
+					twin_y[r] = u2f((u32)twin_s_acc[tile][r]);
+				}
 			}
+			auto const largest = [](f32 const (&x)[4]) { return __builtin_fmaxf(__builtin_fmaxf(x[0], x[1]), __builtin_fmaxf(x[2], x[3])); };
+			f32 tmax, twin_tmax;
 			if constexpr (!MASKED) {
 				// (positive temperature: sgn = 1)
-				tmax = __builtin_fmaxf(__builtin_fmaxf(y[0], y[1]), __builtin_fmaxf(y[2], y[3]));
+				tmax = largest(y);
+				twin_tmax = largest(twin_y);
 			} else {
-				u32 const first = qi - 1 - ((kb_begin + i) * at::KV_PER_STEP + 16 * tile + 4 * group);
-				f32 ym[4];
+				u32 const first_key = (kb_begin + i) * at::KV_PER_STEP + 16 * tile + own_keys;
+				f32 ym[4], twin_ym[4];
 				X17_UNROLL for (u32 r = 0; r < 4; ++r) {
-					vis[r] = first - r <= vis_bound;
+					vis[r] = qi - 1 - first_key - r <= vis_bound;
 					y[r] = y[r] * sgn;
 					ym[r] = vis[r] ? y[r] : -__builtin_inff();
+					twin_ym[r] = twin_qi - 1 - first_key - r <= vis_bound ? twin_y[r] * sgn : -__builtin_inff();
 				}
-				tmax = __builtin_fmaxf(__builtin_fmaxf(ym[0], ym[1]), __builtin_fmaxf(ym[2], ym[3]));
+				tmax = largest(ym);
+				twin_tmax = largest(twin_ym);
 			}
-			if (__any(tmax > ext)) {
-				tmax = u2f(over_groups(f2u(tmax), [](u32 a, u32 b) { return f2u(__builtin_fmaxf(u2f(a), u2f(b))); }));
+			// The twin asks for a smaller scale when its lift, 2^(this), is above MAX_LIFT = 2^5
+			twin_ext = __builtin_fmaxf(twin_ext, twin_tmax);
+			bool const twin_asks = __any(fmaf32(twin_ext - twin_ext_ref, twin_abs_t, -HEADROOM) > 5.0f);
+			if (__any(tmax > ext) || twin_asks) {
+				tmax = u2f(over_groups(f2u(tmax), larger));
 				ext = tmax > ext ? tmax : ext;
 				set_subtrahend();
 				lift = hw::ex2(fmaf32(ext - ext_ref, abs_t, -HEADROOM));      // (the difference is exact)
-				if (__any(lift > MAX_LIFT)) {
+				if (__any(lift > MAX_LIFT) || twin_asks) {
 					// O and the partial sum come down to the scale of the new maximum
 					f32 const down = hw::rcp(lift) * LIFT0;
 					X17_UNROLL for (u32 dt = 0; dt < D_TILES; ++dt) {
@@ -304,6 +339,7 @@ void kernel(
 					sum = sum * down;
 					ext_ref = ext;
 					lift = LIFT0;
+					twin_ext = twin_ext_ref = u2f(over_groups(f2u(twin_ext), larger));
 				}
 				lift2 = v2h{(_Float16)lift, (_Float16)lift};
 				neg_bias2 = lift2 * v2h{(_Float16)-1024.0f, (_Float16)-1024.0f};     // exact
@@ -352,7 +388,7 @@ void kernel(
 	widen_v(0, 0);
 	u32 const first_active = wave_kb_first - kb_begin;
 	u32 const diagonal = wave_kb_last - kb_begin;
-	u32 const inside_kb = nt::first_inside_block(q_wave0, wr);
+	u32 const inside_kb = nt::first_inside_block(q_pair0, wr);
 	u32 const inside_clamped = inside_kb < wave_kb_first ? wave_kb_first : (inside_kb > wave_kb_last ? wave_kb_last : inside_kb);
 	u32 const first_full = (positive_temperature ? inside_clamped : wave_kb_last) - kb_begin;
 	u32 i = 0;
@@ -372,7 +408,11 @@ void kernel(
 
 	// ---- finish (cuda/attn_fwd_i8.cuh:293-351): the sums are at the scale of the maximum HEADROOM above ext_ref's score
 	f32 const m = ROW_SCALES ? fmaf32(ext_ref * sgn, temperature, HEADROOM) : fmaf32(fmaf32(ext_ref, sgn, -DOT_BIAS), temperature, HEADROOM);
-	f32 const total = u2f(over_groups(f2u(sum), [](u32 a, u32 b) { return f2u(u2f(a) + u2f(b)); }));      // (s0 + s1) + (s2 + s3)
+	// (s0 + s1) + (s2 + s3): lane groups 0 and 2 hold s0 and s1
+	auto const across = __builtin_amdgcn_permlane32_swap(f2u(sum), f2u(sum), false, false);
+	f32 const half_total = u2f((u32)across[0]) + u2f((u32)across[1]);
+	auto const beside = __builtin_amdgcn_permlane16_swap(f2u(half_total), f2u(half_total), false, false);
+	f32 const total = u2f((u32)beside[0]) + u2f((u32)beside[1]);
 	if (l_out != nullptr && group == 0) {
 		l_out[(size_t)head * all_rows + row_base + qi] = sfu::lg2(total) + m;
 	}

@@ -48,11 +48,20 @@ int main(int argc, char **argv) {
 	for (unsigned tid = 0; tid < at::THREADS_PER_BLOCK; ++tid) {
 		if (!at::is_stager(tid)) continue;
 		if (at::stage_v_offset(tid, KV_STRIDE) != (tid / CPR) * KV_STRIDE + HD + 16 * (tid % CPR)) return fail("a V chunk is not in order", tid, 0);
-		unsigned const dst = nt::v_granule_offset(tid / CPR, tid % CPR);
+		unsigned const dst = nt::widened_offset(tid);
 		if (dst % 32 != 0 || dst + 32 > at::V_TILE_BYTES) return fail("a widened granule leaves the tile", dst + 32, at::V_TILE_BYTES);
 		++written[dst / 32];
 	}
 	for (unsigned v : written) if (v != 1) return fail("a granule of the f16 tile is not written exactly once", v, 1);
+	// scores, probabilities and values meet in matrix row r of a 16-key tile: K read there, V stored there, keys 0-3, 8-11, 4-7, 12-15
+	unsigned const quad_of_group[4] = {0, 2, 1, 3};
+	for (unsigned r = 0; r < 16; ++r) {
+		unsigned const key = nt::key_of_row(r);
+		if (key != 4 * quad_of_group[r / 4] + r % 4) return fail("a matrix row holds another key", r, key);
+		for (unsigned t = 0; t < 2; ++t) for (unsigned c = 0; c < CPR; ++c) {
+			if (nt::widened_offset((16 * t + key) * CPR + c) != nt::v_granule_offset(16 * t + r, c)) return fail("a key's values are not in its scores' row", r, key);
+		}
+	}
 	for (unsigned dt = 0; dt < HD / 16; ++dt) for (unsigned row0 = 0; row0 < 16; row0 += 8) {
 		unsigned mask = 0;
 		for (unsigned r = 0; r < 8; ++r) {
@@ -71,14 +80,16 @@ int main(int argc, char **argv) {
 		unsigned const begin = at::first_key_block(q0, wr), end = nt::end_key_block(q0);
 		if (end <= begin || end * KEYS > seq_len) return fail("the walk is empty or reaches behind its sequence", end * KEYS, seq_len);
 		for (unsigned w = 0; w < at::Q_WAVES; ++w) {
-			unsigned const qw = q0 + w * nt::Q_PER_WAVE, first = at::first_key_block(qw, wr), last = qw / KEYS;
+			// the walk is that of the 32 queries the wavefront shares with its twin
+			unsigned const qw = (q0 + w * nt::Q_PER_WAVE) & ~(nt::PAIR - 1), first = at::first_key_block(qw, wr), last = qw / KEYS;
 			if (first < begin || last >= end) return fail("a wavefront's keys are outside its workgroup's walk", last, end);
-			// every key a query of the wavefront sees: max(0, i - W') .. i - 1
-			unsigned const lowest = qw > wr ? qw - wr : 0, highest = qw + nt::Q_PER_WAVE - 2;
+			if (((q0 + w * nt::Q_PER_WAVE) ^ nt::Q_PER_WAVE) / nt::Q_PER_BLOCK != q0 / nt::Q_PER_BLOCK) return fail("a twin is in another workgroup", q0, w);
+			// every key a query of the 32 sees: max(0, i - W') .. i - 1
+			unsigned const lowest = qw > wr ? qw - wr : 0, highest = qw + nt::PAIR - 2;
 			if (lowest / KEYS < first || highest / KEYS > last) return fail("a visible key is outside the wavefront's blocks", highest / KEYS, last);
 			unsigned const inside = nt::first_inside_block(qw, wr);
 			for (unsigned kb = first; kb < last; ++kb) {
-				bool const whole = kb * KEYS + KEYS - 1 < qw && (unsigned long long)qw + nt::Q_PER_WAVE - 1 - kb * KEYS <= wr;
+				bool const whole = kb * KEYS + KEYS - 1 < qw && (unsigned long long)qw + nt::PAIR - 1 - kb * KEYS <= wr;
 				if (whole != (kb >= inside)) return fail("a block is taken as fully visible and is not, or the other way round", kb, inside);
 			}
 		}
