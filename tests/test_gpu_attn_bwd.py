@@ -7,6 +7,8 @@ whose gradient cancels to zero).
 dK / dV multiply on the bf16 matrix cores (P and dS rounded to bf16 as attn_d_kv.cuh:330-365 does) and write bf16:
 relative L2 error below 4e-3 for each of dK and dV, and every element within 2^-8 of the sum of the magnitudes of its
 terms (each term carries one bf16 rounding of P or dS, 2^-9 relative) plus one bf16 step of its own value."""
+import zlib
+
 import numpy as np
 import pytest
 
@@ -320,3 +322,61 @@ def test_backward_launches_are_repeatable_and_long_walks_are_homogeneous(dev):
 	assert np.array_equal(dq4, 4.0 * dq1) and np.array_equal(d4, 4.0 * d1) and np.array_equal(dkv4, 4.0 * dkv1)
 	assert np.isfinite(dkv1).all() and np.abs(dkv1).max() > 1e-4 and np.abs(dq1).max() > 1e-4
 	assert not dq1[0].any() and not dkv1[t - 1].any()
+
+
+# (heads, head_dim, tokens, sequences, window, head temperatures): zlib.crc32 of dq, d and d_kv
+GRADIENT_BYTES = [
+	(2, 128, 384, 1, 0, (0.8, -0.7), (3901675327, 3502591762, 56544525)),
+	(2, 64, 320, 2, 48, (6.0, -1.3), (123789717, 2027738705, 1177496629)),
+	(4, 32, 256, 3, 16, (1.1, -24.0, 0.0, 12.0), (343545148, 3163788278, 3631568396)),
+]
+
+
+def _gradient_crcs(dev, h, hd, t, batch, w, temperatures):
+	rng = rng_for("gradient bytes", h, hd, t, batch, w)
+	rows = t * batch
+	q, kv, sk, sv, _ = _inputs(rng, rows, h, hd)
+	up = lambda a, dt: X.Tensor.from_numpy(dev, a, dt)
+	tq, tkv, tsk, tsv, tt = up(q, X.INT8), up(kv, X.INT8), up(sk, X.INT8), up(sv, X.INT8), up(np.array(temperatures, np.float32), X.F32)
+	out, l, d = X.Tensor(dev, (rows, h * hd), X.INT8), X.Tensor(dev, (h, rows), X.F32), X.Tensor(dev, (h, rows), X.F32)
+	t_do, dq, d_kv = up(_bf16_bits(rng.standard_normal((rows, h * hd))), X.BF16), X.Tensor(dev, (rows, h * hd), X.BF16), X.Tensor(dev, (rows, 2 * h * hd), X.BF16)
+	recipes.attn_kernel(dev, h, hd, True).launch(tq, tkv, tsk, tsv, tt, out, l, w, batch)
+	recipes.attn_d_q_kernel(dev, h, hd, False).launch_d_q(tq, tkv, tsk, tsv, tt, out, t_do, dq, l, d, w, batch)
+	recipes.attn_d_kv_kernel(dev, h, hd, False).launch_d_kv(tq, tkv, tt, t_do, l, d, d_kv, w, batch)
+	return tuple(zlib.crc32(np.ascontiguousarray(x.download()).tobytes()) for x in (dq, d, d_kv))
+
+
+@pytest.mark.parametrize("h,hd,t,batch,w,temperatures,crcs", GRADIENT_BYTES)
+def test_the_bytes_of_the_gradients(dev, h, hd, t, batch, w, temperatures, crcs):
+	"""A training run repeats itself under another version of these kernels: the order and the rounding of the speed build's
+	operations are pinned by checksums of its outputs (gradients as they were before the key loops were requested by hand), at small,
+	negative, zero and large head temperatures."""
+	assert _gradient_crcs(dev, h, hd, t, batch, w, temperatures) == crcs
+
+
+@pytest.mark.parametrize("strict", [True, False])
+@pytest.mark.parametrize("h,hd", [(2, 128), (2, 64), (4, 32)])
+def test_a_row_of_infinite_log_sum_exp_weighs_nothing(dev, h, hd, strict):
+	"""exp2(s - inf) = 0: a query whose L a caller has set to +inf has no gradient and gives none to keys and values; the other rows keep
+	theirs, byte for byte."""
+	t, w = 192, 64
+	rng = rng_for("infinite L", h, hd)
+	q, kv, sk, sv, temp = _inputs(rng, t, h, hd)
+	up = lambda a, dt: X.Tensor.from_numpy(dev, a, dt)
+	tq, tkv, tsk, tsv, tt, t_do = up(q, X.INT8), up(kv, X.INT8), up(sk, X.INT8), up(sv, X.INT8), up(temp, X.F32), up(_bf16_bits(rng.standard_normal((t, h * hd))), X.BF16)
+	out, l = X.Tensor(dev, (t, h * hd), X.INT8), X.Tensor(dev, (h, t), X.F32)
+	recipes.attn_kernel(dev, h, hd, True).launch(tq, tkv, tsk, tsv, tt, out, l, w)
+	l_h = l.download()
+	gone = np.array([3, 40, 41, 127, 128, t - 1])
+	results = []
+	for drop in (gone[:0], gone, np.arange(t)):
+		l_h2 = l_h.copy()
+		l_h2[:, drop] = np.inf
+		tl, dq, d, d_kv = up(l_h2, X.F32), X.Tensor(dev, (t, h * hd), X.BF16), X.Tensor(dev, (h, t), X.F32), X.Tensor(dev, (t, 2 * h * hd), X.BF16)
+		recipes.attn_d_q_kernel(dev, h, hd, strict).launch_d_q(tq, tkv, tsk, tsv, tt, out, t_do, dq, tl, d, w)
+		recipes.attn_d_kv_kernel(dev, h, hd, strict).launch_d_kv(tq, tkv, tt, t_do, tl, d, d_kv, w)
+		results.append((dq.download(), _bf16_value(d_kv.download())))
+	kept = np.setdiff1d(np.arange(t), gone)
+	assert np.array_equal(results[1][0][kept], results[0][0][kept])
+	assert not _bf16_value(results[1][0][gone]).any() and not _bf16_value(results[2][0]).any()
+	assert np.isfinite(results[1][1]).all() and not results[2][1].any()

@@ -41,7 +41,7 @@ constexpr unsigned LD_WAVE = KEY_WAVES - 1;                 // the wavefront tha
 constexpr unsigned Q_RAW_BYTES = Q_PER_STEP * HEAD_DIM;     // int8 queries as they arrive
 constexpr unsigned WIDE_BYTES = Q_PER_STEP * HEAD_DIM * 2;  // a bf16 tile (dO as it arrives, Q widened)
 constexpr unsigned LD_BYTES = 2 * Q_PER_STEP * 4;           // the tile's L and D values (f32)
-constexpr unsigned CONST_BYTES = 3 * Q_PER_STEP * 4;        // the per-query constants temperature | L - lg2(255) | -8 D
+constexpr unsigned CONST_BYTES = 3 * Q_PER_STEP * 4;        // the per-query constants temperature | L - lg2(255) | D
 // LDS: raw Q ring (tiles requested three steps ahead, widened to bf16 one step before their use) | L and D ring | two dO tiles
 // (requested one step ahead: a third one is the LDS of the third workgroup) | two widened Q tiles | two blocks of constants
 constexpr unsigned RING = 4;

@@ -22,12 +22,11 @@
 //     dV^T += dO^T . P and dK^T += Q^T . dS; no lane exchange, no LDS round trip.
 //   * S runs on v_mfma_i32_16x16x64_i8 from the raw int8 Q tile; dP, dV^T, dK^T on v_mfma_f32_16x16x32_bf16 (dO is bf16
 //     in memory and is used as it is; int8 codes are exact in bf16): 28 matrix instructions per step for head_dim 128.
-//     The dP accumulators start at -8 D, so that they end as 8 (dP - D).
 //   * Tiles of 32 queries arrive global -> LDS directly, by hand-written requests with constant waits: the raw Q rows and the
 //     tile's L and D values three steps ahead, the dO rows one step ahead -- one copy that is read by rows ("A" of dP: eight
 //     dims of one query) as well as by ds_read_b64_tr_b16 ("A" of dV^T: eight queries of one dim); the layout is chosen by which source
 //     chunk a lane requests.  One step ahead the workgroup widens the Q tile to bf16 into the same layout ("A" of dK^T)
-//     and one wavefront writes the tile's per-query constants (temperature, L - lg2 255, -8 D).
+//     and one wavefront writes the tile's per-query constants (temperature, L - lg2 255, D).
 //
 // common.h (generated per kernel) provides X17_N_HEADS, X17_HEAD_DIM, X17_Q_STRIDE, X17_KV_STRIDE, X17_O_STRIDE,
 // X17_STRICT_MATH.  gridDim = (runs of key blocks, head groups, sequences).
@@ -56,21 +55,25 @@ constexpr u32 CPR = kt::CPR;
 
 static_assert(HD == 32 || HD == 64 || HD == 128, "head_dim must be 32, 64 or 128");
 static_assert(N_HEADS % HPK == 0, "n_heads must be divisible by heads_per_kernel");
+// Registers next to the 64 accumulators: D is read when P is there, and the strict build, whose exponential needs more of them,
+// multiplies dP then as well (in the speed build that costs 0.5 %)
+constexpr bool DP_LATE = X17_STRICT_MATH && HD == 128;
+
 static_assert(kt::RING == 4, "the pipeline below is written for a ring of four and pairs of tiles");
 
 constexpr f32 LOG2_PROB_SCALE = 7.9943534368588578f;                       // lg2(255): the forward's L carries it
 constexpr f32 BASE_TEMPERATURE = f32(constexpr_inv_sqrt(f64(HD)) / 64.0);  // for dots of codes (8 q . 8 k)
 // dk = t_real * ln 2 * sum_i w_i q_i with t_real = 64 * temperature (the temperature below is for dots of codes)
-// and q = code / 8: 64 * ln 2 / 8, and w_i carries 8 (dP - D)
-constexpr f32 LN2_F32 = 0.6931471805599453f;
+// and q = code / 8: 64 * ln 2 / 8
+constexpr f32 EIGHT_LN2 = 5.5451774444795625f;
 
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef short v8s __attribute__((ext_vector_type(8)));
 
-// four int8 codes as four bf16, exact
-X17_DEV v2u widen4(u32 word) {
+// four int8 codes, times a power of two, as four bf16, exact
+X17_DEV v2u widen4(u32 word, f32 factor = 1.0f) {
 	f32 f[4];
-	X17_UNROLL for (int b = 0; b < 4; ++b) f[b] = f32((i32)(i8)((word >> (8 * b)) & 0xFFu));
+	X17_UNROLL for (int b = 0; b < 4; ++b) f[b] = f32((i32)(i8)((word >> (8 * b)) & 0xFFu)) * factor;
 	return v2u{pack2_bf16_rne(f[0], f[1]), pack2_bf16_rne(f[2], f[3])};
 }
 
@@ -206,7 +209,7 @@ void kernel(
 			if (wave == kt::LD_WAVE) {
 				f32 const landed = *reinterpret_cast<f32 const *>(smem + kt::LD_OFFSET + slot * kt::LD_BYTES + lane * 4);
 				f32 *cst = reinterpret_cast<f32 *>(smem + kt::CONST_OFFSET + buf * kt::CONST_BYTES);
-				cst[kt::Q_PER_STEP + lane] = lane < 32 ? landed - LOG2_PROB_SCALE : landed * -8.0f;       // L - lg2 255 | -8 D
+				cst[kt::Q_PER_STEP + lane] = lane < 32 ? landed - LOG2_PROB_SCALE : landed;       // L - lg2 255 | D
 				if (lane < 32) {
 					u32 const qi = tile * kt::Q_PER_STEP + lane;
 					u32 const visible = qi < wr ? qi : wr;
@@ -229,10 +232,10 @@ void kernel(
 			kf[s] = v4i{0, 0, 0, 0};
 			if (k_group_in_row) kf[s] = *reinterpret_cast<v4i const *>(kv_head + (size_t)key * KV_STRIDE + 64 * s + 16 * group);
 		}
-		v8bf vfrag[D_SLICES];                // "B" of dP: lane = key, dims 32 sl + 8 group + 0..7 as bf16
+		v8bf vfrag[D_SLICES];                // "B" of dP: lane = key, dims 32 sl + 8 group + 0..7 as bf16, real values (code / 8)
 		X17_UNROLL for (u32 sl = 0; sl < D_SLICES; ++sl) {
 			v2u const raw = *reinterpret_cast<v2u const *>(kv_head + (size_t)key * KV_STRIDE + HD + 32 * sl + 8 * group);
-			v2u const a = widen4(raw[0]), b = widen4(raw[1]);
+			v2u const a = widen4(raw[0], 0.125f), b = widen4(raw[1], 0.125f);
 			vfrag[sl] = __builtin_bit_cast(v8bf, (v4u{a[0], a[1], b[0], b[1]}));
 		}
 		v4f dk_acc[D_TILES], dv_acc[D_TILES];    // (dims x keys): lane = key, register r = dim 16 dt + 4 group + r
@@ -271,28 +274,31 @@ void kernel(
 			u8 const *q_raw = smem + kt::Q_RAW_OFFSET + slot * kt::Q_RAW_BYTES;
 			u8 const *d_o = smem + kt::DO_OFFSET + (slot & 1) * kt::WIDE_BYTES;
 			u8 const *q_wide = smem + kt::Q_WIDE_OFFSET + (slot & 1) * kt::WIDE_BYTES;
-			f32 const *cst = reinterpret_cast<f32 const *>(smem + kt::CONST_OFFSET + (slot & 1) * kt::CONST_BYTES) + 4 * group;
-			u32 do_off = do_read_base, tr_off = tr_base;
+			u8 const *cst = smem + kt::CONST_OFFSET + (slot & 1) * kt::CONST_BYTES;
+			u32 do_off = do_read_base, tr_off = tr_base, cst_off = 16 * group;
 			asm volatile("" : "+v"(do_off), "+v"(tr_off));      // (keeps the flipped addresses out of registers that live across steps)
 			u32 pw[2 * Q_TILES], ww[2 * Q_TILES];     // P and the dK weights as bf16 pairs: "B" operands, slots = this lane's 8 queries
 			X17_UNROLL for (u32 qt = 0; qt < Q_TILES; ++qt) {
-				// S and 8 (dP - D) blocks (v codes): rows = 16 queries of the tile, columns = this wave's 16 keys
+				// S and dP blocks: rows = 16 queries of the tile, columns = this wave's 16 keys
 				v4i s_acc = {0, 0, 0, 0};
 				X17_UNROLL for (u32 s = 0; s < K_SLICES; ++s) {
 					v4i qa = *reinterpret_cast<v4i const *>(q_raw + q_read_off[qt][s]);
 					if (!k_group_in_row) qa = v4i{0, 0, 0, 0};
 					s_acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(qa, kf[s], s_acc, 0, 0, 0);
 				}
-				v4f dp_acc = *reinterpret_cast<v4f const *>(cst + 2 * kt::Q_PER_STEP + 16 * qt);
-				X17_UNROLL for (u32 sl = 0; sl < D_SLICES; ++sl) {
-					v8bf const da = *reinterpret_cast<v8bf const *>(d_o + (do_off ^ kt::dims_flip(32 * sl)) + qt * SIXTEEN_ROWS);
-					dp_acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(da, vfrag[sl], dp_acc, 0, 0, 0);
-				}
+				v4f dp_acc = {0.0f, 0.0f, 0.0f, 0.0f};
+				auto multiply_dp = [&]() __attribute__((always_inline)) {
+					X17_UNROLL for (u32 sl = 0; sl < D_SLICES; ++sl) {
+						v8bf const da = *reinterpret_cast<v8bf const *>(d_o + (do_off ^ kt::dims_flip(32 * sl)) + qt * SIXTEEN_ROWS);
+						dp_acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(da, vfrag[sl], dp_acc, 0, 0, 0);
+					}
+				};
+				if constexpr (!DP_LATE) multiply_dp();
 				// register r belongs to query 32 tile + 16 qt + 4 group + r; key j is visible to query i iff the distance
 				// i - 1 - j, as an unsigned number, is at most W' - 1
 				[[maybe_unused]] u32 const first = (tile_begin + i) * kt::Q_PER_STEP + 16 * qt + 4 * group - 1 - key;
-				v4f const ct = *reinterpret_cast<v4f const *>(cst + 16 * qt);
-				v4f const cl = *reinterpret_cast<v4f const *>(cst + kt::Q_PER_STEP + 16 * qt);
+				v4f const ct = *reinterpret_cast<v4f const *>(cst + cst_off + 64 * qt);
+				v4f const cl = *reinterpret_cast<v4f const *>(cst + cst_off + 4 * kt::Q_PER_STEP + 64 * qt);
 				f32 p[4], w[4];
 				X17_UNROLL for (u32 r = 0; r < 4; ++r) {
 					f32 pe = sfu::ex2(fmaf32(f32(s_acc[r]), ct[r], -cl[r]));
@@ -300,8 +306,14 @@ void kernel(
 						pe = first + r <= vis_bound ? pe : 0.0f;
 					}
 					p[r] = pe;
-					w[r] = (pe * dp_acc[r]) * ct[r];
 				}
+				asm volatile("" : "+v"(cst_off) : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]));
+				if constexpr (DP_LATE) {
+					asm volatile("" : "+v"(do_off) : "v"(cst_off));
+					multiply_dp();
+				}
+				v4f const cd = *reinterpret_cast<v4f const *>(cst + cst_off + 8 * kt::Q_PER_STEP + 64 * qt);
+				X17_UNROLL for (u32 r = 0; r < 4; ++r) w[r] = (p[r] * (dp_acc[r] - cd[r])) * ct[r];
 				pw[2 * qt] = pack2_bf16_rne(p[0], p[1]);
 				pw[2 * qt + 1] = pack2_bf16_rne(p[2], p[3]);
 				ww[2 * qt] = pack2_bf16_rne(w[0], w[1]);
@@ -352,7 +364,7 @@ void kernel(
 		for (; i < active_end; ++i) step.template operator()<true, -1>(i);
 		for (; i < n_steps; ++i) idle_step(i);
 
-		// ---- output: dk = ln 2 * dk_acc, dv = dv_acc.  A key's dK and dV are one run of memory, a lane holds eight bytes of it at
+		// ---- output: dk = 8 ln 2 * dk_acc, dv = dv_acc.  A key's dK and dV are one run of memory, a lane holds eight bytes of it at
 		// a time: turned around in LDS they leave as whole rows, 16 bytes per lane (8-byte stores straight from the
 		// registers, 32 bytes per row and instruction: a fifth of the launch at 4 x 8192 tokens).
 		__builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0): the last requests write LDS
@@ -362,7 +374,7 @@ void kernel(
 		u32 const out_key = out_lane % 16, out_group = out_lane / 16;
 		u8 *rows_lds = smem + wave * kt::OUT_BYTES_PER_WAVE;
 		X17_UNROLL for (u32 dt = 0; dt < D_TILES; ++dt) {
-			v2u const k_pair = {pack2_bf16_rne(dk_acc[dt][0] * LN2_F32, dk_acc[dt][1] * LN2_F32), pack2_bf16_rne(dk_acc[dt][2] * LN2_F32, dk_acc[dt][3] * LN2_F32)};
+			v2u const k_pair = {pack2_bf16_rne(dk_acc[dt][0] * EIGHT_LN2, dk_acc[dt][1] * EIGHT_LN2), pack2_bf16_rne(dk_acc[dt][2] * EIGHT_LN2, dk_acc[dt][3] * EIGHT_LN2)};
 			v2u const v_pair = {pack2_bf16_rne(dv_acc[dt][0], dv_acc[dt][1]), pack2_bf16_rne(dv_acc[dt][2], dv_acc[dt][3])};
 			*reinterpret_cast<v2u *>(rows_lds + kt::out_offset(out_key, 2 * dt + out_group / 2) + 8 * (out_group % 2)) = k_pair;
 			*reinterpret_cast<v2u *>(rows_lds + kt::out_offset(out_key, HD / 8 + 2 * dt + out_group / 2) + 8 * (out_group % 2)) = v_pair;

@@ -97,13 +97,17 @@ X17_DEV u32 vrow_offset(u32 key, u32 c16) {
 }
 
 // sixteen int8 (four words) -> sixteen f16 (eight words), exact: flip the sign bit (b + 128 as an unsigned byte u),
-// splice u under the f16 exponent of 1024 (0x6400 | u == 1024 + u), subtract 1152
+// splice u under the f16 exponent of 1024 (0x6400 | u == 1024 + u), subtract 1152; or (EIGHTHS) an eighth of each code, its real
+// value: under the exponent of 128, whose last place is an eighth, less 144
+template <bool EIGHTHS>
 X17_DEV void widen16(v4u raw, u32 (&w)[8]) {
-	v2h const bias = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+	_Float16 const less = (_Float16)(EIGHTHS ? -144.0f : -1152.0f);
+	u32 const exponent = EIGHTHS ? 0x58585858u : 0x64646464u;
+	v2h const bias = {less, less};
 	X17_UNROLL for (int i = 0; i < 4; ++i) {
 		u32 word = raw[i] ^ 0x80808080u;
-		u32 lo = __builtin_amdgcn_perm(0x64646464u, word, 0x04010400u);
-		u32 hi = __builtin_amdgcn_perm(0x64646464u, word, 0x04030402u);
+		u32 lo = __builtin_amdgcn_perm(exponent, word, 0x04010400u);
+		u32 hi = __builtin_amdgcn_perm(exponent, word, 0x04030402u);
 		w[2 * i] = __builtin_bit_cast(u32, __builtin_bit_cast(v2h, lo) + bias);
 		w[2 * i + 1] = __builtin_bit_cast(u32, __builtin_bit_cast(v2h, hi) + bias);
 	}
@@ -181,11 +185,11 @@ void kernel(
 		auto widen = [&](u32 slot, u32 buf) __attribute__((always_inline)) {
 			if (CPR == 8 || stager) {          // (head_dim 128: every thread stages)
 				u32 w[8];
-				widen16(*reinterpret_cast<v4u const *>(smem + bt::RAW_K_RING_OFFSET + slot * bt::RAW_TILE_BYTES + tid * 16), w);
+				widen16<false>(*reinterpret_cast<v4u const *>(smem + bt::RAW_K_RING_OFFSET + slot * bt::RAW_TILE_BYTES + tid * 16), w);
 				u8 *kd = smem + bt::K_F16_OFFSET + buf * bt::F16_TILE_BYTES + k_f16_dst;
 				*reinterpret_cast<v4u *>(kd) = v4u{w[0], w[1], w[2], w[3]};
 				*reinterpret_cast<v4u *>(kd + 16) = v4u{w[4], w[5], w[6], w[7]};
-				widen16(*reinterpret_cast<v4u const *>(smem + bt::RAW_V_RING_OFFSET + slot * bt::RAW_TILE_BYTES + tid * 16), w);
+				widen16<true>(*reinterpret_cast<v4u const *>(smem + bt::RAW_V_RING_OFFSET + slot * bt::RAW_TILE_BYTES + tid * 16), w);
 				u8 *vd = smem + bt::V_F16_OFFSET + buf * bt::F16_TILE_BYTES;
 				*reinterpret_cast<v4u *>(vd + v_f16_dst0) = v4u{w[0], w[1], w[2], w[3]};
 				*reinterpret_cast<v4u *>(vd + v_f16_dst1) = v4u{w[4], w[5], w[6], w[7]};
@@ -283,50 +287,23 @@ void kernel(
 		// window's edge, fully visible, the diagonal, nothing to do -- each its own loop; every step requests a tile by
 		// hand (past the end the last one again, into a slot nobody reads any more), so the waits are constants; the long
 		// run is unrolled over the four slots of the rings, so that every LDS address is a register plus an immediate.
-		// Per score what is left is a fused multiply-add, an exponential, a multiplication and half a conversion:
-		//  * The score accumulators start at the bits of 1.5 * 2^23: the int32 sum, read as a float, is 12582912 + dot
-		//    exactly, and one fused multiply-add makes the exponent's argument of it.  Its subtrahend mb, t * 12582912 + L
-		//    rounded, is constant per query here; so is the rest that the rounding leaves, and 2^rest is taken out of dq at the end.
-		//  * The dP accumulators start at -D, so that they end as dP - D.
-		//  * The 1 / 8 of dO . v (v codes) goes into the exponent.
-		// A temperature so large that the rest would matter (or one that is no number) takes the general step throughout,
-		// with accumulators from zero and a conversion per score.
+		// A score costs a conversion, a multiplication, a subtraction, an exponential, dP - D, the product and half a conversion to
+		// f16, each rounded by itself.  (One fused multiply-add on accumulators that start at a bias, and dP accumulators that
+		// start at -D, are 57 instructions fewer per step and 5 % of the launch, but round otherwise: a gradient's bytes
+		// then depend on the version.  They also make NaN of a row whose L is +inf, which weighs nothing.)  V is widened
+		// to its real value, code / 8, so that D needs no factor.
 		// Bound by the rate at which a wavefront issues (one instruction in about ten clocks, two wavefronts per SIMD): a fully
-		// visible step is 183 instructions; it was 357, around requests that were drained in the step that made them.  16 heads
-		// of 128, 4 x 8192 tokens: 11.5 -> 7 us per 32 keys of window; window 512: 333 -> 272 us, of which 150 are set-up and output.
-		constexpr f32 DOT_BIAS = 12582912.0f;
-		f32 const head_temperature = u2f(__builtin_amdgcn_readfirstlane(f2u(attn_temperature[head])));
-		bool const biased = __builtin_fabsf(head_temperature) * (BASE_TEMPERATURE * 32.0f) <= 1.0f;      // |t| <= 1: lg2 of a u32 is at most 32
-		f32 const l_eighth = l_hat + 3.0f;
-		f32 const prod = biased ? temperature * DOT_BIAS : 0.0f;
-		f32 const low = biased ? fmaf32(temperature, DOT_BIAS, -prod) : 0.0f;
-		f32 const mb = prod + l_eighth;
-		f32 const rest = biased ? ((prod - mb) + l_eighth) + low : 0.0f;      // |rest| <= 1
-		f32 const fine = sfu::ex2(rest), inv_fine = sfu::ex2(-rest);
-		// dQ starts from the sink's share: the outer product of the sink key and w_sink by one matrix instruction per 32 dims.
-		// The weight is cut into three bf16 numbers of eight significand bits each (exact), in key slots 0 to 2 of the "B"
-		// operand next to three copies of the key's code.
-		f32 const w_sink = (p_sink * ((dps8 - d8) * 0.125f)) * fine;
-		f32 const w_high = u2f(f2u(w_sink) & 0xFFFF0000u);
-		f32 const w_left = w_high == w_sink ? 0.0f : w_sink - w_high;
-		f32 const w_mid = u2f(f2u(w_left) & 0xFFFF0000u);
-		f32 const w_low = w_left - w_mid;
-		v4u const w_slots = {half == 0 ? (f2u(w_high) >> 16) | f2u(w_mid) : 0u, half == 0 ? f2u(w_low) >> 16 : 0u, 0u, 0u};
+		// visible step is 237 instructions; it was 357, around requests that were drained in the step that made them.  16 heads
+		// of 128, 4 x 8192 tokens, window 512: 333 -> 284 us, of which 160 are set-up, output and the first steps (window 32).
+		f32 const w_sink = p_sink * ((dps8 - d8) * 0.125f);
 		v16f dq_acc[D_BLOCKS];               // dQ^T: lane = query, register r = dim 32 db + 8 (r / 4) + 4 half + r % 4
 		X17_UNROLL for (u32 db = 0; db < D_BLOCKS; ++db) {
-			u32 const code = f2u((f32)(i32)sink_k[(size_t)head * HD + 32 * db + qlane]) & 0xFFFF0000u;      // (int8 is exact in bf16)
-			v4u const k_slots = {half == 0 ? (code >> 16) | code : 0u, half == 0 ? code >> 16 : 0u, 0u, 0u};
-			v16f const zero = {0};
-			dq_acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, k_slots), __builtin_bit_cast(v8bf, w_slots), zero, 0, 0, 0);
+			X17_UNROLL for (int r4 = 0; r4 < 4; ++r4) {
+				u32 const word = *reinterpret_cast<u32 const *>(sink_k + (size_t)head * HD + 32 * db + 8 * r4 + 4 * half);
+				X17_UNROLL for (int b = 0; b < 4; ++b) dq_acc[db][4 * r4 + b] = w_sink * i8_of(word, b);
+			}
 		}
-		v16i s_bias;
-		v16f neg_d8;
-		X17_UNROLL for (int r = 0; r < 16; ++r) {
-			s_bias[r] = biased ? 0x4B400000 : 0;
-			neg_d8[r] = -d8;
-		}
-		asm volatile("" : "+v"(s_bias), "+v"(neg_d8));      // (kept in registers: rebuilding them per step would cost what they save)
-
+		f32 const d1 = d8 * 0.125f;           // D in the units of dO . v (real v)
 		u32 k_lane_off[K_SLICES], v_lane_off[D_SLICES];
 		X17_UNROLL for (u32 sl = 0; sl < K_SLICES; ++sl) k_lane_off[sl] = k_chunk_offset(qlane, 2 * sl + half);
 		X17_UNROLL for (u32 sl = 0; sl < D_SLICES; ++sl) v_lane_off[sl] = vrow_offset(qlane, 2 * sl + half);
@@ -350,18 +327,13 @@ void kernel(
 			u8 const *k_raw = smem + bt::RAW_K_RING_OFFSET + slot * bt::RAW_TILE_BYTES;
 			u8 const *k_f16 = smem + bt::K_F16_OFFSET + buf * bt::F16_TILE_BYTES;
 			u8 const *v_f16 = smem + bt::V_F16_OFFSET + buf * bt::F16_TILE_BYTES;
-			// S^T block: rows = 32 keys, columns = this wave's 32 queries; dP'^T - D' (times 8: v codes) for the same keys
-			v16i s_acc = s_bias;
+			// S^T block: rows = 32 keys, columns = this wave's 32 queries; dP'^T for the same keys
+			v16i s_acc = {0};
 			X17_UNROLL for (u32 s = 0; s < K_SLICES; ++s) {
 				v4i const kf = *reinterpret_cast<v4i const *>(k_raw + k_lane_off[s]);
 				s_acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf, qf[s], s_acc, 0, 0, 0);
 			}
-			if constexpr (MASKED) {
-				if (!biased) {
-					X17_UNROLL for (int r = 0; r < 16; ++r) s_acc[r] = (i32)f2u(f32(s_acc[r]));
-				}
-			}
-			v16f dp_acc = neg_d8;
+			v16f dp_acc = {0};
 			X17_UNROLL for (u32 sl = 0; sl < D_SLICES; ++sl) {
 				v8h const vf = *reinterpret_cast<v8h const *>(v_f16 + v_lane_off[sl]);
 				dp_acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, dofrag[sl], dp_acc, 0, 0, 0);
@@ -372,13 +344,14 @@ void kernel(
 				f32 w[8];
 				[[maybe_unused]] u32 const first = qi - 1 - ((kb_begin + i) * at::KV_PER_STEP + 16 * tile + 4 * half);
 				X17_UNROLL for (u32 r = 0; r < 8; ++r) {
-					f32 p = sfu::ex2(fmaf32(u2f((u32)s_acc[8 * tile + r]), temperature, -mb));
+					f32 const score = f32(s_acc[8 * tile + r]) * temperature;
+					f32 p = sfu::ex2(score - l_hat);
 					if constexpr (MASKED) {
 						// key j is visible iff the distance qi - 1 - j, as an unsigned number, is at most W' - 1
 						u32 const distance = first - (8 * (r / 4) + (r % 4));
 						p = distance <= vis_bound ? p : 0.0f;
 					}
-					w[r] = p * dp_acc[8 * tile + r];
+					w[r] = p * (dp_acc[8 * tile + r] - d1);
 				}
 				v8h wfrag;
 				X17_UNROLL for (u32 r = 0; r < 8; ++r) wfrag[r] = (_Float16)w[r];
@@ -405,7 +378,7 @@ void kernel(
 		// first block that lies inside the window of all 32 queries: q_wave0 + 31 - 32 kb <= wr
 		u32 const inside_kb = q_wave0 + 31 > wr ? (q_wave0 + 62 - wr) / 32 : 0;
 		u32 const inside_clamped = inside_kb < wave_kb_first ? wave_kb_first : (inside_kb > wave_kb_last ? wave_kb_last : inside_kb);
-		u32 const first_full = (biased ? inside_clamped : wave_kb_last) - kb_begin;
+		u32 const first_full = inside_clamped - kb_begin;
 
 		__builtin_amdgcn_s_waitcnt(0x0F74);   // vmcnt(4): tile 0 has landed
 		widen(0, 0);
@@ -424,8 +397,8 @@ void kernel(
 		for (++i; i < n_steps; ++i) idle_step(i);
 		__builtin_amdgcn_s_waitcnt(0x0F70);   // the last requests write LDS: they land before the tiles are reused
 
-		// ---- output: dq = 8 ln 2 * temperature * dq_acc / (scale * fine), D = d8 / (8 scale)
-		f32 const out_scale = ((temperature * EIGHT_LN2) * inv_scale) * inv_fine;
+		// ---- output: dq = 8 ln 2 * temperature * dq_acc / scale, D = d8 / (8 scale)
+		f32 const out_scale = (temperature * EIGHT_LN2) * inv_scale;
 		u16 *dq_row = d_q + (row_base + qi) * Q_STRIDE + (size_t)head * HD;
 		X17_UNROLL for (u32 db = 0; db < D_BLOCKS; ++db) {
 			X17_UNROLL for (int g = 0; g < 4; ++g) {

@@ -73,11 +73,13 @@ def _specs():
 	# ---- tests/test_gpu_attn_bwd.py
 	for h, hd in ((8, 64), (2, 128), (4, 32), (2, 64)):
 		add(("attn_d_q", h, hd, True))
-	add(("attn_d_q", 8, 64, False))
+	for h, hd in ((8, 64), (2, 128), (4, 32), (2, 64)):
+		add(("attn_d_q", h, hd, False))
 	add(("attn_d_q", 16, 128, False))                    # bench.py
 	for h, hd in ((8, 64), (2, 128), (4, 32), (2, 64)):
 		add(("attn_d_kv", h, hd, True))
-	add(("attn_d_kv", 8, 64, False))
+	for h, hd in ((8, 64), (2, 128), (4, 32), (2, 64)):
+		add(("attn_d_kv", h, hd, False))
 	add(("attn_d_kv", 16, 128, False))                   # bench.py
 	add(("attn_d_q", 4, 128, False))
 	add(("attn_d_kv", 4, 128, False))
