@@ -68,12 +68,12 @@ constexpr u32 GROUP_BYTES = BLOCKS * (gt::WAVES_K - 1) * BLOCK_BYTES;
 X17_DEV u32 exchange_offset(int j, u32 from) { return (j * (gt::WAVES_K - 1) + (from < owner(j) ? from : from - 1)) * BLOCK_BYTES; }
 static_assert(gt::WAVES / gt::WAVES_K * GROUP_BYTES <= gt::SMEM_BYTES, "the exchange fits the ring");
 
-// The barrier of a K step of the widening form, behind this wavefront's LDS reads and writes
+// The barrier of a K step, behind this wavefront's LDS reads and writes.  (The builtins order no memory access for the compiler:
+// the clobbers keep the step's reads behind the barrier and the last one's in front of it.)
 X17_DEV void step_barrier() {
 	asm volatile("" ::: "memory");
 	__builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0)
 	__builtin_amdgcn_s_barrier();
-	__builtin_amdgcn_sched_barrier(0);
 	asm volatile("" ::: "memory");
 }
 
@@ -117,6 +117,7 @@ X17_DEV void step_barrier() {
 		X17_UNROLL for (u32 j = 0; j < gt::WIDENER_DEPTH; ++j) {
 			if (base + j < K_STEPS) {
 				step_barrier();
+				__builtin_amdgcn_sched_barrier(0);
 				store((j + 1) % gt::WIDE_TILES);
 				widen((j + 2) % gt::WIDENER_DEPTH);
 				load(base + j + 2 + gt::WIDENER_DEPTH, (j + 2) % gt::WIDENER_DEPTH);
@@ -230,6 +231,7 @@ void kernel(
 					// so are everybody's, the step's weights are widened, and the slot of the token tile before is free
 					wait_vmcnt<(gt::STAGES - 2) * gt::X_UNITS>();
 					step_barrier();
+					__builtin_amdgcn_sched_barrier(0);
 					v4i raw[SLICES];
 					v8h wide[SLICES][2];
 					X17_UNROLL for (u32 s = 0; s < SLICES; ++s) {
@@ -255,8 +257,7 @@ void kernel(
 		// this wavefront's requests of step ks have landed and its reads of step ks - 1 are done; behind the barrier so
 		// are everybody's, and the slot of step ks - 1 takes the requests of step ks + STAGES - 1
 		wait_vmcnt<(gt::STAGES - 2) * LOADS_PER_STAGE>();
-		__builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0)
-		__builtin_amdgcn_s_barrier();
+		step_barrier();
 		u8 const *stage = smem + slot * gt::STAGE_BYTES;
 		Frags frags[SLICES_PER_WAVE];
 		auto read = [&](u32 s) __attribute__((always_inline)) {
