@@ -1085,7 +1085,9 @@ Status GemmKernel::launch(GemmArgs const &args) {
 // below 4096 rows with weights that no cache holds (the next layer's: the two-stage 128 x 128 form, ahead with weights in
 // L2, loses to four stages there: 256 rows, K = 2048, 8.4 / 8.7 us and 16 / 12).  A fit is 3-10 % off in the mean of a curve
 // and up to 40 % at single points; over those launches the form taken is 0.3 % slower than the best one in the mean (16 % at
-// most), over 460 of other widths 0.6 % (36 %).  us measured at 4096 columns:
+// most), over 460 of other widths 0.6 % (36 %).  The four-stage forms have become 0-10 % faster since: over 535 launches of
+// the present code (256 .. 4096 rows, K = 512 .. 16384, ten writers, weights from memory) the form taken is 0.2 % slower than
+// the best one (18 % at most), so the curves stand.  us measured at 4096 columns:
 //                        rows:  256    512   1024   2048   4096   8192
 //   int8, K = 2048   64 x 64    8.1   14.1   27.1   56.2    107    215
 //           128 x 128, 4 / 2   12/16  12/16  13/16  26/22  48/41  95/78

@@ -54,9 +54,13 @@ static_assert(SLICES_PER_WAVE * gt::WAVES_K == SLICES, "K steps divide evenly ov
 static_assert(N_RAW % gt::N_PER_BLOCK == 0, "raw output columns are whole tiles");
 // One workgroup of one or two wavefronts per SIMD fills a compute unit in the four-stage forms, and nothing runs beside a
 // step's start: there the fragment reads go out in front of the requests' instructions, and all before anything waits for
-// one (int8, 128 x 128, K = 8192, 4096 columns, 512 rows: 30.4 -> 27.7 us; e4m3, K = 16384, 8192 columns, 320 rows: 61 -> 56;
-// the first slice's reads alone 30.5 -> 29.4 and no gain).  In the two-stage form the other workgroup does, and a request
-// that goes out later is waited for (int8, 512 rows x 16384 columns: 18.7 and 20.1 us).
+// one.  What it gives depends on where the weights come from.  us, requests first / reads first, from L2 or the memory-side
+// cache | from memory (128 x 128, 4096 columns unless said):
+//   int8, K = 8192, 512 rows              28.7 / 26.1 | 37.5 / 36.9      int8, K = 2048, 256 rows   8.9 / 8.5 | 8.9 / 8.5
+//   int8 GeGLU, 16384 columns, K = 2048, 256 rows (256 workgroups)       12.0 / 11.7 | 14.9 / 14.6
+//   e4m3, K = 16384, 8192 columns, 320 rows            61 / 56 | 72.6 / 71.6: a pair whose weights no cache holds gains 1 %
+// No launch of 58 lost.  (The first slice's reads alone: half of it.)  In the two-stage form the other workgroup runs beside a
+// step's start, and a request that goes out later is waited for (int8, 512 rows x 16384 columns: 18.7 and 20.1 us).
 constexpr bool READS_FIRST = gt::STAGES >= 4;
 
 // the exchange: blocks of 32 x 32 outputs, 16 registers per lane; block j belongs to wavefront owner(j) of the WAVES_K
