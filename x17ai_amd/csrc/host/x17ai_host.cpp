@@ -1359,17 +1359,20 @@ bool AttnKernel::narrow_for(size_t seq_len, size_t batch, size_t window) const {
 
 // Heads a workgroup takes one behind the other (a power of two up to 128 / head_dim, the reference's group,
 // src/device/cuda/attn.rs:60-66).  One head each fills the chip in a small launch; in a large launch of short walks a
-// group saves its workgroup's start.  Estimated per choice, in key steps (32 keys; dK / dV: query tiles): rounds of the
-// workgroups a compute unit holds, a partly filled last round counting more than its share, each round `start` plus the
-// group's walks, plus the tail of the longest walk.  Fitted to 870 launches of 8 .. 64 heads of 32 and 64, 1024 .. 32768
-// rows, windows of 64 .. 4096 and none: 0.1-0.8 % behind the best choice in the mean.  us, one head / the whole group:
+// group saves its workgroup's start.  Estimated per choice, in key steps (32 keys; dK / dV: query tiles): rounds of
+// `resident` workgroups per compute unit, a partly filled last round counting more than its share, each round `start` plus the
+// group's walks, plus the tail of the longest walk.  All four are fitted, `resident` too (registers hold three workgroups of
+// the forward, two of dQ, four of dK / dV): the forward and dQ to 870 launches of 8 .. 64 heads of 32 and 64, 1024 .. 32768
+// rows, windows of 64 .. 4096 and none, dK / dV to 144 and 99 later ones.  Behind the best choice, in the mean and at most: the
+// forward 0.1-0.8 %; over 99 launches each of the present code dQ 0.3 and 9 % (head_dim 32), 0.5 and 9 % (64), dK / dV 1.1 and 22 %,
+// 0.5 and 10 % (always one head: 4.1, 2.1, 4.8 and 1.0 % in the mean).  us, one head / the whole group:
 //   forward, 8 heads of 64:    1024 rows, no window 23 / 42    16384 rows in sequences of 128 16.2 / 14.7
 //   dQ, 64 heads of 32:        8192 rows, window 64, 8 sequences 73 / 66
 //   dK / dV, 64 heads of 32:   1024 rows, no window 24 / 70    16384 rows in sequences of 128 103 / 94
 size_t AttnKernel::heads_per_workgroup(size_t seq_len, size_t batch, size_t window) const {
 	struct Fit { double resident, start, last_round, tail; };
 	static constexpr Fit FITS[3][2] = {       // forward, dQ, dK / dV; head_dim 32 and 64
-		{{3, 2.5, 0, 0.5}, {3, 1.5, 0.5, 0.25}}, {{3, 8, 0, 0.75}, {3, 4, 0, 0.75}}, {{3, 2, 0, 0.25}, {5, 1, 0.5, 0.1}},
+		{{3, 2.5, 0, 0.5}, {3, 1.5, 0.5, 0.25}}, {{3, 8, 0, 0.75}, {3, 4, 0, 0.75}}, {{3, 2, 0, 0.25}, {4, 0.5, 0, 0.1}},
 	};
 	Fit const &f = FITS[config.backward_q ? 1 : config.backward_kv ? 2 : 0][config.head_dim == 32 ? 0 : 1];
 	size_t const own_rows = metadata.rows_per_workgroup();
