@@ -390,3 +390,35 @@ def test_decode_row_scaled_bit_exact(dev, h, hd, cap, w, out_dtype):
 		kern.launch(X.Tensor.from_numpy(dev, qd, X.INT8), X.Tensor.from_numpy(dev, cache, X.INT8),
 		            X.Tensor.from_numpy(dev, lens.view(np.float32), X.F32), X.Tensor.from_numpy(dev, sk, X.INT8),
 		            X.Tensor.from_numpy(dev, sv, X.INT8), f32(temp), out, l, w)
+
+
+@pytest.mark.parametrize("t,h,hd,w,batch,heads_per_workgroup", [
+	(1088, 8, 64, 64, 6, 1), (192, 8, 64, 16, 64, 2), (1088, 4, 32, 48, 12, 1), (128, 4, 32, 0, 256, 2), (1088, 2, 128, 112, 24, 1), (576, 2, 128, 0, 48, 1)])
+@pytest.mark.parametrize("rows", [False, True])
+def test_attn_fast_thirty_two_queries_per_wavefront(dev, t, h, hd, w, batch, heads_per_workgroup, rows):
+	"""The speed build's form of large launches against the strict definition, at every head_dim, one head and several per workgroup, with
+	one scale and with a scale per row: odd multiples of 64 tokens, short windows and none, a negative and a zero head temperature.
+	Sequences are independent: the oracle recomputes the first and the last."""
+	rng = rng_for("attn-wide", t, h, hd, w, batch)
+	if rows:
+		q, kv, qs, ks, vs, sk, sv, temp = _row_scaled_inputs(rng, t * batch, h, hd)
+	else:
+		q, kv, sk, sv, temp = _attn_inputs(rng, t * batch, h, hd)
+	temp[0], temp[1] = -temp[0], 0.0
+	if rows:
+		vw, sw, osc = recipes.attn_row_scale_operands(vs, X.INT8)
+		kern = recipes.attn_row_scaled_kernel(dev, h, hd, X.INT8, False)
+		got, got_l = _run_row_scaled(dev, kern, q, kv, sk, sv, temp, w, qs, ks, vw, sw, osc, batch=batch)
+	else:
+		kern = recipes.attn_kernel(dev, h, hd, False)
+		got, got_l = _run_attn(dev, kern, q, kv, sk, sv, temp, w, batch=batch)
+	assert kern.queries_per_wavefront(t, batch, w) == 32 and kern.heads_per_workgroup(t, batch, w) == heads_per_workgroup
+	for i in (0, batch - 1):
+		r = slice(i * t, (i + 1) * t)
+		if rows:
+			want, want_l = S.attn_fwd_i8_row_scaled(q[r], kv[r], sk, sv, temp, h, hd, w, *(np.ascontiguousarray(a[:, r]) for a in (qs, ks, vw)), sw, osc)
+		else:
+			want, want_l = S.attn_fwd_i8(q[r], kv[r], sk, sv, temp, h, hd, w)
+		d = np.abs(got[r].astype(np.int32) - want.astype(np.int32))
+		assert d.max() <= 1 and np.mean(d > 0) < 0.02, (d.max(), np.mean(d > 0))
+		assert np.max(np.abs(got_l[:, r] - want_l)) < 1e-4
