@@ -1,6 +1,6 @@
 """The kernels' hand-written tile requests (global -> LDS, 16 bytes per lane, addresses formed from scalar bases and
 lane offsets outside the compiler's view) are audited on the CPU: the index arithmetic lives in gemm_tile.h /
-gemm_small_tile.h / attn_tile.h, the kernels call it, and the audit programs beside them (gemm_requests_audit.cpp,
+gemm_small_tile.h / attn_tile.h / attn_narrow_tile.h / attn_bwd_tile.h / attn_bwd_kv_tile.h, the kernels call it, and the audit programs beside them (gemm_requests_audit.cpp,
 gemm_small_requests_audit.cpp, attn_requests_audit.cpp) are compiled here with a kernel's own generated common.h and enumerate every request of a
 launch -- every tile of the persistent walk and K step, every (sequence, head, query block) and step of the request
 schedule, overhanging tiles and past-the-end repeats included.  Each must stay inside its operand and each tile's
@@ -141,4 +141,27 @@ def test_attention_backward_kv_requests_and_lds_layouts(tmp_path, label, make, s
 	rep, rc = _audit(tmp_path, kern, "attn_bwd_kv_requests_audit.cpp", seq_len, batch, window, seq_len * batch - 1)
 	assert rc != 0 and not rep["ok"] and "past the end" in rep["error"], rep
 	rep, rc = _audit(tmp_path, kern, "attn_bwd_kv_requests_audit.cpp", 64, 1, 0)
+	assert rc != 0 and not rep["ok"]
+
+
+D_QS = [
+	("config 4", lambda: recipes.attn_d_q_kernel(None, 16, 128, False), ((1024, 4, 512), (128, 1, 0), (192, 3, 16), (320, 2, 4096))),
+	("head_dim 64 (two staging wavefronts)", lambda: recipes.attn_d_q_kernel(None, 8, 64, True), ((1024, 1, 256), (192, 2, 0), (128, 1, 16))),
+	("head_dim 32 (one staging wavefront)", lambda: recipes.attn_d_q_kernel(None, 4, 32, True), ((768, 1, 64), (256, 3, 16))),
+]
+
+
+@pytest.mark.parametrize("label,make,shapes", D_QS, ids=[a[0] for a in D_QS])
+def test_attention_backward_q_requests_and_lds_layouts(tmp_path, label, make, shapes):
+	"""attn_bwd_tile.h: reads name what requests and widening wrote; every tile a step reads or widens has landed under the
+	kernel's waits, no request overwrites a slot that is read, and the runs without a mask see no hidden key."""
+	kern = make()
+	for seq_len, batch, window in shapes:
+		rep, rc = _audit(tmp_path, kern, "attn_bwd_requests_audit.cpp", seq_len, batch, window)
+		assert rc == 0 and rep["ok"], (label, seq_len, batch, window, rep)
+		assert rep["q_extent"] == rep["q_bytes"] and rep["o_extent"] == rep["o_bytes"] and rep["row_extent"] == rep["rows"], rep
+	seq_len, batch, window = shapes[0]
+	rep, rc = _audit(tmp_path, kern, "attn_bwd_requests_audit.cpp", seq_len, batch, window, seq_len * batch - 1)
+	assert rc != 0 and not rep["ok"] and "past the end" in rep["error"], rep
+	rep, rc = _audit(tmp_path, kern, "attn_bwd_requests_audit.cpp", 64, 1, 0)
 	assert rc != 0 and not rep["ok"]

@@ -72,30 +72,6 @@ X17_DEV i32 partner_i32(i32 x, u32 half) {
 	return (i32)(half == 0 ? r[1] : r[0]);
 }
 
-// Raw K tile, as in the forward: linear 16-byte chunk n = key * CPR + c lives in 128-byte line n / 8 at position
-// (n % 8) ^ ((line >> 1) & 7), so that the sixteen keys a ds_read_b128 serves at a time land in sixteen slots.
-X17_DEV u32 k_chunk_offset(u32 key, u32 c) {
-	u32 n = key * CPR + c;
-	u32 line = n >> 3;
-	return (line << 7) | (((n & 7) ^ ((line >> 1) & 7)) << 4);
-}
-// f16 K tile, the forward's f16 V layout: 32-byte granule n = key * CPR + c (16 dims) lives in 256-byte line n / 8 at
-// position (n % 8) ^ ((line & 3) << 1); the transposed 8-byte reads of 32 lanes then cover all banks once.
-X17_DEV u32 granule_offset(u32 key, u32 c) {
-	u32 n = key * CPR + c;
-	u32 line = n >> 3;
-	return (line << 8) | (((n & 7) ^ ((line & 3) << 1)) << 5);
-}
-// f16 V tile, read by rows: a key row is HD / 8 chunks of 16 bytes (8 dims); 16 / (HD / 8) keys share a 256-byte
-// line, and chunk c16 of a key is stored at position c16 ^ line inside its key's part of the line: the sixteen keys
-// a ds_read_b128 serves at a time (same c16) land in sixteen different slots for head_dim 32, 64 and 128.
-X17_DEV u32 vrow_offset(u32 key, u32 c16) {
-	constexpr u32 R = HD / 8, KPL = 16 / R;
-	u32 const line = key / KPL;
-	u32 const slot = (key % KPL) * R + (c16 ^ (line & (R - 1)));
-	return line * 256 + slot * 16;
-}
-
 // sixteen int8 (four words) -> sixteen f16 (eight words), exact: flip the sign bit (b + 128 as an unsigned byte u),
 // splice u under the f16 exponent of 1024 (0x6400 | u == 1024 + u), subtract 1152; or (EIGHTHS) an eighth of each code, its real
 // value: under the exponent of 128, whose last place is an eighth, less 144
@@ -175,12 +151,9 @@ void kernel(
 		if (stager) {
 			stage_k_src = at::stage_k_offset(tid, KV_STRIDE);
 			stage_v_src = at::stage_v_offset(tid, KV_STRIDE);
-			// stored chunk `tid` of the raw K tile holds logical chunk n: key n / CPR, dims 16 * (n % CPR) .. + 15
-			u32 const line = tid >> 3;
-			u32 const n = (line << 3) | ((tid & 7) ^ ((line >> 1) & 7));
-			k_f16_dst = granule_offset(n / CPR, n % CPR);
-			v_f16_dst0 = vrow_offset(tid / CPR, 2 * (tid % CPR));
-			v_f16_dst1 = vrow_offset(tid / CPR, 2 * (tid % CPR) + 1);
+			k_f16_dst = bt::k_widened_offset(tid);
+			v_f16_dst0 = bt::v_widened_offset(tid, 0);
+			v_f16_dst1 = bt::v_widened_offset(tid, 1);
 		}
 		auto widen = [&](u32 slot, u32 buf) __attribute__((always_inline)) {
 			if (CPR == 8 || stager) {          // (head_dim 128: every thread stages)
@@ -278,8 +251,8 @@ void kernel(
 		{
 			u32 const t = lane % 16, dh = (lane / 16) % 2;
 			X17_UNROLL for (u32 db = 0; db < D_BLOCKS; ++db) {
-				kt_lane_off[db] = granule_offset(4 * half + (t >> 2), 2 * db + dh) + 8 * (t & 3);
-				kt_lane_off8[db] = granule_offset(8 + 4 * half + (t >> 2), 2 * db + dh) + 8 * (t & 3);
+				kt_lane_off[db] = bt::granule_offset(4 * half + (t >> 2), 2 * db + dh) + 8 * (t & 3);
+				kt_lane_off8[db] = bt::granule_offset(8 + 4 * half + (t >> 2), 2 * db + dh) + 8 * (t & 3);
 			}
 		}
 
@@ -305,8 +278,8 @@ void kernel(
 		}
 		f32 const d1 = d8 * 0.125f;           // D in the units of dO . v (real v)
 		u32 k_lane_off[K_SLICES], v_lane_off[D_SLICES];
-		X17_UNROLL for (u32 sl = 0; sl < K_SLICES; ++sl) k_lane_off[sl] = k_chunk_offset(qlane, 2 * sl + half);
-		X17_UNROLL for (u32 sl = 0; sl < D_SLICES; ++sl) v_lane_off[sl] = vrow_offset(qlane, 2 * sl + half);
+		X17_UNROLL for (u32 sl = 0; sl < K_SLICES; ++sl) k_lane_off[sl] = bt::k_chunk_offset(qlane, 2 * sl + half);
+		X17_UNROLL for (u32 sl = 0; sl < D_SLICES; ++sl) v_lane_off[sl] = bt::vrow_offset(qlane, 2 * sl + half);
 
 		// SLOT: the step's position in the rings (s % RING) as a compile-time number, or -1 for "compute it"; SLOT >= 0 also
 		// says that tile s + 4 exists (the caller's loop bound)
