@@ -1725,7 +1725,7 @@ std::unique_ptr<AttnDecodeKernel> AttnDecodeKernel::create(std::shared_ptr<HipDe
 
 // Threads per workgroup, by the number of workgroups and by the key bytes each may have to stream (figures in
 // attn_decode_i8.hip; 1062 launches of 8 .. 64 heads of 32, 64 and 128, windows 128 .. 16384, full and ragged caches: 1-2 %
-// behind the best width in the mean).  At most one workgroup per compute unit: as many wavefronts as the window keeps
+// behind the best width in the mean; 380 of the present kernel, 1 .. 64 sequences from memory: 0.9 %, 11 % at most).  At most one workgroup per compute unit: as many wavefronts as the window keeps
 // busy.  More: a long window streams best from 512 threads whatever their number; below that the width that keeps the
 // workgroups resident, two wavefronts for many short windows.  At head_dim 64 two wavefronts already stream at the
 // memory's rate from three workgroups per compute unit on (48 sequences x 16 heads x 1024 keys, every probability

@@ -15,11 +15,10 @@
 // are and how many key bytes each streams: few workgroups have to keep enough loads in flight by themselves, many
 // short ones want to be resident together.  Measured at 32 heads of 128, capacity 4096, normal keys and queries (us,
 // 128 / 256 / 512 / 1024 threads; in parentheses 512 threads and 128 where every probability counts):
-//    3 sequences x 4096 keys  112 / 41 / 27 / 24    16 x 4096  126 / 60 / 55 / 62    16 x 512   21 / 12 / 11 / 17
-//   32 x 1024                  43 / 31 / 32 / 46    32 x 4096  141 / 103 / 97 / 109  32 x 128  9.1 / 8.7 / 16 / 28
-//   48 x 1024                  50 / 46 / 46 / 67    48 x 4096  158 / 148 / 137 / 157 (266, 271)
-//   64 x 128                 10.9 / 17 / 31 / 57    64 x 4096  193 / 192 / 184 / 206 (349, 343)
-// (the table was measured before phases 3 and 4 took their present form, which took 0.5 to 4 us off a launch at every width.)
+//    3 sequences x 4096 keys  112 / 40 / 26 / 22    16 x 4096  123 / 62 / 57 / 58    16 x 512   22 / 13 / 13 / 18
+//   32 x 1024                  40 / 33 / 32 / 42    32 x 4096  134 / 105 / 95 / 105  32 x 128  9.9 / 9.5 / 16 / 28
+//   48 x 1024                  47 / 44 / 43 / 60    48 x 4096  154 / 148 / 135 / 152 (251, 266)
+//   64 x 128                  12 / 16 / 29 / 53     64 x 4096  185 / 188 / 177 / 199 (331, 334)
 // What the tail behind the scores costs counts where few workgroups run: the slowest heads, with 100 to 180 listed tiles of 240,
 // spent 9 to 13 of their 22 us in phases 3 and 4.  Four keys per dot product, the partial sums beside the O chain and the
 // listed tiles' factors in a list of their own: 3 ragged caches 22.0 -> 19.3 us, 8 31.9 -> 27.5, 64 full ones 185.8 -> 183.5.
