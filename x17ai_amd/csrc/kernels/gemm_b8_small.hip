@@ -14,8 +14,8 @@
 // e4m3 x int8 in 64 x 64 tiles is bound by the instructions around the f16 matrix instructions, which one wavefront per SIMD
 // issues at one in about ten clocks.  Of 34 per 32 bytes of K twenty widened a weight fragment, the same one in two
 // wavefronts; four further wavefronts now do that once, from memory through registers, and leave f16 in LDS (gemm_small_tile.h:
-// WIDEN_ONCE).  256 rows, 4096 columns, K = 8192: 34.8 -> 30.7 us (39.1 -> 34 with weights from memory; vector ALU 29 %, matrix
-// cores 21 %, LDS 38 % busy: the step's chain barrier - reads - widening - multiplications bounds it); 320 rows, two
+// WIDEN_ONCE).  256 rows, 4096 columns, K = 8192: 34.8 -> 30.7 us (39.1 -> 34 with weights from memory; vector ALU 28 %, matrix
+// cores 21 %, LDS 37 % busy: the step's chain barrier - reads - widening - multiplications bounds it); 320 rows, two
 // workgroups per compute unit: 61 -> 44 us.  Tried: token tiles through the same registers 34.6 / 49.7 us, half a step's
 // fragments read across the barrier from a third widened tile 32.2 / 45.5 us.
 
