@@ -21,7 +21,10 @@ def test_forms_of_a_kernel_pass_the_code_object_scans(tmp_path):
 	assert all(os.path.exists(f) for f in forms)
 	for k in (1536, 2048, 2176):          # loops the compiler would unroll altogether, beyond a wavefront's 128 registers
 		recipes.dequant_gemm_kernel(None, k, 256, X.E4M3, X.E4M3, False, True)
-	for path in glob.glob(os.path.join(objects.KERNELS, "*", "*", "kernel.hsaco")):
+	names = {f: recipe().name for f, recipe in (("q16", lambda: recipes.attn_kernel(None, 2, 64, False)), ("s64x4", lambda: recipes.ffn_y_kernel(None, 128, 512, True, X.E4M3, X.INT8)))}
+	scanned = glob.glob(os.path.join(objects.KERNELS, "*", "*", "kernel.hsaco"))
+	assert all(os.path.join(objects.KERNELS, name, f, "kernel.hsaco") in scanned for f, name in names.items())      # 16 queries; weights widened once
+	for path in scanned:
 		ins = scan._instructions(path, str(tmp_path))
 		assert scan._hazards(ins) == [] and scan._m0_hazards(ins) == [], path
 		assert [line for line in ins if scan.PACKED_F32.match(line)] == [], path

@@ -67,7 +67,7 @@ int main(int argc, char **argv) {
 	for (unsigned lane = 0; lane < 64; ++lane) {
 		unsigned const half = lane / 32, qlane = lane % 32, t = lane % 16, dh = (lane / 16) % 2;
 		for (unsigned s = 0; s < HD / 32; ++s) {
-			unsigned const off = bt::k_chunk_offset(qlane, 2 * s + half);
+			unsigned const off = at::k_chunk_offset(qlane, 2 * s + half);
 			if (off % 16 != 0 || off + 16 > bt::RAW_TILE_BYTES || raw_k[off / 16] != qlane * HD + 32 * s + 16 * half + 1) return fail("a raw K read finds another chunk", off, lane);
 		}
 		for (unsigned sl = 0; sl < HD / 16; ++sl) {

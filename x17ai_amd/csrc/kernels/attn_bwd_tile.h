@@ -32,12 +32,6 @@ constexpr unsigned SMEM_BYTES = V_F16_OFFSET + 2 * F16_TILE_BYTES;
 
 constexpr unsigned CPR = at::CHUNKS_PER_ROW;                 // 16-byte chunks of an int8 row of the head
 
-// Raw K tile, as in the forward: linear 16-byte chunk n = key * CPR + c lives in 128-byte line n / 8 at position
-// (n % 8) ^ ((line >> 1) & 7), so that the sixteen keys a ds_read_b128 serves at a time land in sixteen slots.
-constexpr unsigned k_chunk_offset(unsigned key, unsigned c) {
-	unsigned const n = key * CPR + c, line = n >> 3;
-	return (line << 7) | (((n & 7) ^ ((line >> 1) & 7)) << 4);
-}
 // f16 K tile, the forward's f16 V layout: 32-byte granule n = key * CPR + c (16 dims) lives in 256-byte line n / 8 at
 // position (n % 8) ^ ((line & 3) << 1); the transposed 8-byte reads of 32 lanes then cover all banks once.
 constexpr unsigned granule_offset(unsigned key, unsigned c) {

@@ -32,10 +32,12 @@
 #include "common.h"
 #include "x17_device.h"
 #include "attn_bwd_tile.h"
+#include "attn_parts.h"
 
 using namespace x17;
 namespace at = x17::attn_tile;
 namespace bt = x17::attn_bwd_tile;
+using namespace x17::attn_parts;
 
 namespace {
 
@@ -53,7 +55,6 @@ constexpr u32 CPR = at::CHUNKS_PER_ROW;
 static_assert(HD == 32 || HD == 64 || HD == 128, "head_dim must be 32, 64 or 128");
 static_assert(N_HEADS % HPK == 0, "n_heads must be divisible by heads_per_kernel");
 
-constexpr f32 LOG2_PROB_SCALE = 7.9943534368588578f;                       // lg2(255): the forward's L carries it
 constexpr f32 BASE_TEMPERATURE = f32(constexpr_inv_sqrt(f64(HD)) / 64.0);  // for dots of codes (8 q . 8 k)
 // dq = t_real * ln 2 * sum_j w_j k_j with t_real = 64 * temperature (the temperature below is for dots of codes)
 // and k = code / 8: 64 * ln 2 / 8
@@ -61,33 +62,6 @@ constexpr f32 EIGHT_LN2 = 5.5451774444795625f;
 
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef short v8s __attribute__((ext_vector_type(8)));
-
-X17_DEV f32 partner_f32(f32 x, u32 half) {
-	u32 u = f2u(x);
-	auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-	return u2f(half == 0 ? r[1] : r[0]);
-}
-X17_DEV i32 partner_i32(i32 x, u32 half) {
-	auto r = __builtin_amdgcn_permlane32_swap((u32)x, (u32)x, false, false);
-	return (i32)(half == 0 ? r[1] : r[0]);
-}
-
-// sixteen int8 (four words) -> sixteen f16 (eight words), exact: flip the sign bit (b + 128 as an unsigned byte u),
-// splice u under the f16 exponent of 1024 (0x6400 | u == 1024 + u), subtract 1152; or (EIGHTHS) an eighth of each code, its real
-// value: under the exponent of 128, whose last place is an eighth, less 144
-template <bool EIGHTHS>
-X17_DEV void widen16(v4u raw, u32 (&w)[8]) {
-	_Float16 const less = (_Float16)(EIGHTHS ? -144.0f : -1152.0f);
-	u32 const exponent = EIGHTHS ? 0x58585858u : 0x64646464u;
-	v2h const bias = {less, less};
-	X17_UNROLL for (int i = 0; i < 4; ++i) {
-		u32 word = raw[i] ^ 0x80808080u;
-		u32 lo = __builtin_amdgcn_perm(exponent, word, 0x04010400u);
-		u32 hi = __builtin_amdgcn_perm(exponent, word, 0x04030402u);
-		w[2 * i] = __builtin_bit_cast(u32, __builtin_bit_cast(v2h, lo) + bias);
-		w[2 * i + 1] = __builtin_bit_cast(u32, __builtin_bit_cast(v2h, hi) + bias);
-	}
-}
 
 X17_DEV f32 i8_of(u32 word, int b) { return f32((i32)(i8)((word >> (8 * b)) & 0xFFu)); }
 
@@ -278,7 +252,7 @@ void kernel(
 		}
 		f32 const d1 = d8 * 0.125f;           // D in the units of dO . v (real v)
 		u32 k_lane_off[K_SLICES], v_lane_off[D_SLICES];
-		X17_UNROLL for (u32 sl = 0; sl < K_SLICES; ++sl) k_lane_off[sl] = bt::k_chunk_offset(qlane, 2 * sl + half);
+		X17_UNROLL for (u32 sl = 0; sl < K_SLICES; ++sl) k_lane_off[sl] = at::k_chunk_offset(qlane, 2 * sl + half);
 		X17_UNROLL for (u32 sl = 0; sl < D_SLICES; ++sl) v_lane_off[sl] = bt::vrow_offset(qlane, 2 * sl + half);
 
 		// SLOT: the step's position in the rings (s % RING) as a compile-time number, or -1 for "compute it"; SLOT >= 0 also

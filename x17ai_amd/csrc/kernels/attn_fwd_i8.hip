@@ -56,9 +56,11 @@
 #include "common.h"
 #include "x17_device.h"
 #include "attn_tile.h"
+#include "attn_parts.h"
 
 using namespace x17;
 namespace at = x17::attn_tile;
+using namespace x17::attn_parts;
 
 namespace {
 
@@ -79,34 +81,10 @@ static_assert(ROW_SCALES || !OUT_BF16, "the bf16 output needs the row-scaled bui
 static_assert(HD == 32 || HD == 64 || HD == 128, "head_dim must be 32, 64 or 128");
 static_assert(N_HEADS % HPK == 0, "n_heads must be divisible by heads_per_kernel");
 
-constexpr f32 PROB_SCALE = 255.0f;                                  // cuda/attn_fwd_i8.cuh:206
-constexpr f32 LOG2_PROB_SCALE = 7.9943534368588578f;                // lg2(255)
-constexpr f32 MAX_LIFT = 32.0f;                                     // (1024 + 255) * 32 stays inside f16
 constexpr f32 BASE_TEMPERATURE = ROW_SCALES ? f32(constexpr_inv_sqrt(f64(HD)))
                                             : f32(constexpr_inv_sqrt(f64(HD)) / 64.0);   // :47, :447-449
 
 typedef short v4s __attribute__((ext_vector_type(4)));
-
-// value of lane ^ 32
-X17_DEV f32 partner_f32(f32 x, u32 half) {
-	u32 u = f2u(x);
-	auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-	return u2f(half == 0 ? r[1] : r[0]);
-}
-X17_DEV i32 partner_i32(i32 x, u32 half) {
-	auto r = __builtin_amdgcn_permlane32_swap((u32)x, (u32)x, false, false);
-	return (i32)(half == 0 ? r[1] : r[0]);
-}
-
-// K tile: linear 16-byte chunk n = key * CPR + c lives in 128-byte line n / 8 at position
-// (n % 8) ^ ((line >> 1) & 7).  The LDS serves a ds_read_b128 sixteen lanes at a time out of 64
-// four-byte banks; with this mapping the sixteen keys of such a group land in sixteen different
-// 16-byte slots for every supported head_dim.
-X17_DEV u32 k_chunk_offset(u32 key, u32 c) {
-	u32 n = key * CPR + c;
-	u32 line = n >> 3;
-	return (line << 7) | (((n & 7) ^ ((line >> 1) & 7)) << 4);
-}
 
 // V tile (f16): linear 32-byte granule n = key * CPR + c (16 dims) lives in 256-byte line n / 8
 // at position (n % 8) ^ ((line & 3) << 1): the 4 keys x 2 granules that 32 lanes of a transposed
@@ -133,11 +111,6 @@ X17_DEV void load_to_lds_16(u8 *lds_uniform, i8 const *src_uniform, u32 lane_off
 	asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
 	             :: "s"(lds), "v"(lane_offset), "s"(src_uniform) : "memory", "m0");
 }
-
-// Speed build: p + PACK_MAGIC rounds p in [0, 256) to the nearest integer P (ties to even, as rintf) and leaves
-// the f16 bit pattern of 1024 + P in the low half of the sum: 12582912 = 1.5 * 2^23 has an ulp of 1 and the bits
-// 0x4B400000; adding 0x6400 = 25600 puts the f16 exponent of 1024 above the eight integer bits.
-constexpr f32 PACK_MAGIC = 12582912.0f + 25600.0f;
 
 } // namespace
 
@@ -224,16 +197,8 @@ void kernel(
 		auto widen_v = [&](u32 slot, u32 tile) {
 			if (CPR == 8 || stager) {          // (head_dim 128: every thread stages)
 				v4u raw = *reinterpret_cast<v4u const *>(smem + at::RAW_V_RING_OFFSET + slot * at::RAW_V_TILE_BYTES + tid * 16);
-				// int8 -> f16: b + 128 as an unsigned byte u, 0x6400 | u == 1024 + u, minus 1152
-				v2h const bias = {(_Float16)-1152.0f, (_Float16)-1152.0f};
 				u32 w[8];
-				X17_UNROLL for (int i = 0; i < 4; ++i) {
-					u32 word = raw[i] ^ 0x80808080u;
-					u32 l = __builtin_amdgcn_perm(0x64646464u, word, 0x04010400u);
-					u32 h = __builtin_amdgcn_perm(0x64646464u, word, 0x04030402u);
-					w[2 * i] = __builtin_bit_cast(u32, __builtin_bit_cast(v2h, l) + bias);
-					w[2 * i + 1] = __builtin_bit_cast(u32, __builtin_bit_cast(v2h, h) + bias);
-				}
+				widen16(raw, w);
 				u8 *dst = smem + at::V_TILES_OFFSET + tile * at::V_TILE_BYTES + widen_dst;
 				*reinterpret_cast<v4u *>(dst) = v4u{w[0], w[1], w[2], w[3]};
 				*reinterpret_cast<v4u *>(dst + 16) = v4u{w[4], w[5], w[6], w[7]};
@@ -340,7 +305,6 @@ void kernel(
 		//    scales and 32 value weights with the K tile (one more load in flight per prefetched step: its waits count
 		//    three loads per step).  Scales are taken to be non-negative (absmax / 127): the sign of a query's
 		//    temperature is then the head's.
-		constexpr f32 HEADROOM = 12.0f, LIFT0 = 1.0f / 4096.0f, DOT_BIAS = 12582912.0f;
 		v16i s_bias;
 		X17_UNROLL for (int r = 0; r < 16; ++r) s_bias[r] = ROW_SCALES || STRICT ? 0 : 0x4B400000;
 		if constexpr (!ROW_SCALES && !STRICT) {
@@ -350,23 +314,11 @@ void kernel(
 		f32 const sgn = positive_temperature ? 1.0f : -1.0f;
 		f32 ext = ROW_SCALES ? (f32(sink_dot) * 0.125f) * sgn : (f32(sink_dot) + DOT_BIAS) * sgn;
 		[[maybe_unused]] f32 mb = 0.0f, fine = 1.0f;
-		auto set_subtrahend = [&]() {
-			if constexpr (ROW_SCALES) {
-				mb = fmaf32(ext, abs_t, -LOG2_PROB_SCALE);
-				fine = 1.0f;
-			} else {
-				// ext * |t| as a rounded product and its exact remainder; prod - mb is exact (neighbouring floats)
-				f32 const prod = ext * abs_t;
-				f32 const low = fmaf32(ext, abs_t, -prod);
-				mb = prod - LOG2_PROB_SCALE;
-				fine = hw::ex2(-(((prod - mb) - LOG2_PROB_SCALE) + low));          // 2^-(what mb leaves over): close to 1
-			}
-		};
 		f32 ext_ref = ext;                        // O and the sums refer to the maximum HEADROOM above this extreme's score
 		[[maybe_unused]] f32 sum_lift = 1.0f;
 		[[maybe_unused]] v2h neg_bias2 = {(_Float16)(-1024.0f * LIFT0), (_Float16)(-1024.0f * LIFT0)};      // -1024 * lift2
 		if constexpr (!STRICT) {
-			set_subtrahend();
+			set_subtrahend<ROW_SCALES>(ext, abs_t, mb, fine);
 			lift = LIFT0;
 			sum_lift = LIFT0 * fine;
 			lift2 = v2h{(_Float16)LIFT0, (_Float16)LIFT0};
@@ -550,7 +502,7 @@ void kernel(
 			}
 		};
 		u32 k_lane_off[K_SLICES];
-		X17_UNROLL for (u32 sl = 0; sl < K_SLICES; ++sl) k_lane_off[sl] = k_chunk_offset(qlane, 2 * sl + half);
+		X17_UNROLL for (u32 sl = 0; sl < K_SLICES; ++sl) k_lane_off[sl] = at::k_chunk_offset(qlane, 2 * sl + half);
 
 		auto compute = [&]<bool MASKED, int SLOT>(u32 i) __attribute__((always_inline)) {
 			u32 const k_slot = SLOT >= 0 ? (u32)SLOT : i % at::RING;
@@ -616,7 +568,7 @@ void kernel(
 						tmax = __builtin_fmaxf(tmax, partner_f32(tmax, half));
 					}
 					ext = tmax > ext ? tmax : ext;
-					set_subtrahend();
+					set_subtrahend<ROW_SCALES>(ext, abs_t, mb, fine);
 					lift = hw::ex2(fmaf32(ext - ext_ref, abs_t, -HEADROOM));      // (the difference is exact)
 					if (__any(lift > MAX_LIFT)) {
 						// O and the partial sums come down to the scale of the new maximum
@@ -757,14 +709,7 @@ void kernel(
 					word[g] = pack4_fixedi8(o_acc[db][4 * g] * inv, o_acc[db][4 * g + 1] * inv,
 					                        o_acc[db][4 * g + 2] * inv, o_acc[db][4 * g + 3] * inv);
 				} else {
-					// the scaling rides in the rounding addition; clamping the rounded value gives what rounding the
-					// clamped one gives
-					constexpr f32 MAGIC = 12582912.0f;
-					u32 u[4];
-					X17_UNROLL for (int e = 0; e < 4; ++e) {
-						u[e] = f2u(__builtin_amdgcn_fmed3f(fmaf32(o_acc[db][4 * g + e], inv, MAGIC), MAGIC - 127.0f, MAGIC + 127.0f));
-					}
-					word[g] = __builtin_amdgcn_perm(u[1], u[0], 0x0c0c0400u) | __builtin_amdgcn_perm(u[3], u[2], 0x04000c0cu);
+					word[g] = scaled_codes(o_acc[db][4 * g], o_acc[db][4 * g + 1], o_acc[db][4 * g + 2], o_acc[db][4 * g + 3], inv);
 				}
 			}
 			// The lane pair (lane, lane + 32) holds the 32 bytes of this block interleaved word by word; two

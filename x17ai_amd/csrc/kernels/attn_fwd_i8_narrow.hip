@@ -28,10 +28,12 @@
 #include "common.h"
 #include "x17_device.h"
 #include "attn_narrow_tile.h"
+#include "attn_parts.h"
 
 using namespace x17;
 namespace at = x17::attn_tile;
 namespace nt = x17::attn_narrow_tile;
+using namespace x17::attn_parts;
 
 namespace {
 
@@ -48,11 +50,6 @@ static_assert(X17_STRICT_MATH == 0, "the strict build has one order of operation
 static_assert(ROW_SCALES || !OUT_BF16, "the bf16 output needs the row-scaled build (it supplies out_scale)");
 static_assert(HD == 32 || HD == 64 || HD == 128, "head_dim must be 32, 64 or 128");
 
-constexpr f32 PROB_SCALE = 255.0f;                                  // cuda/attn_fwd_i8.cuh:206
-constexpr f32 LOG2_PROB_SCALE = 7.9943534368588578f;                // lg2(255)
-constexpr f32 MAX_LIFT = 32.0f;
-constexpr f32 HEADROOM = 12.0f, LIFT0 = 1.0f / 4096.0f, DOT_BIAS = 12582912.0f;
-constexpr f32 PACK_MAGIC = 12582912.0f + 25600.0f;
 constexpr f32 BASE_TEMPERATURE = ROW_SCALES ? f32(constexpr_inv_sqrt(f64(HD)))
                                             : f32(constexpr_inv_sqrt(f64(HD)) / 64.0);   // :47, :447-449
 
@@ -195,19 +192,7 @@ void kernel(
 	f32 ext = sink_extreme(sink_dot);
 	f32 twin_ext = sink_extreme(twin_sink_dot), twin_ext_ref = twin_ext;      // (twin_ext: of this lane's keys and the sink)
 	f32 mb, fine;
-	auto set_subtrahend = [&]() {
-		if constexpr (ROW_SCALES) {
-			mb = fmaf32(ext, abs_t, -LOG2_PROB_SCALE);
-			fine = 1.0f;
-		} else {
-			// ext * |t| as a rounded product and its exact remainder; prod - mb is exact (neighbouring floats)
-			f32 const prod = ext * abs_t;
-			f32 const low = fmaf32(ext, abs_t, -prod);
-			mb = prod - LOG2_PROB_SCALE;
-			fine = hw::ex2(-(((prod - mb) - LOG2_PROB_SCALE) + low));
-		}
-	};
-	set_subtrahend();
+	set_subtrahend<ROW_SCALES>(ext, abs_t, mb, fine);
 	f32 ext_ref = ext;                       // O and the sum refer to the maximum HEADROOM above this extreme's score
 	f32 lift = LIFT0, sum_lift = LIFT0 * fine;
 	v2h lift2 = {(_Float16)LIFT0, (_Float16)LIFT0}, neg_bias2 = {(_Float16)(-1024.0f * LIFT0), (_Float16)(-1024.0f * LIFT0)};
@@ -232,22 +217,15 @@ void kernel(
 	// ---- lane offsets of the operand reads and of the widening
 	u32 k_lane_off[2][K_SLICES], v_lane_off[D_TILES];
 	X17_UNROLL for (u32 tile = 0; tile < 2; ++tile) {
-		X17_UNROLL for (u32 s = 0; s < K_SLICES; ++s) k_lane_off[tile][s] = nt::k_chunk_offset(16 * tile + nt::key_of_row(qlane), group_in_row ? 4 * s + group : 0);
+		X17_UNROLL for (u32 s = 0; s < K_SLICES; ++s) k_lane_off[tile][s] = at::k_chunk_offset(16 * tile + nt::key_of_row(qlane), group_in_row ? 4 * s + group : 0);
 	}
 	X17_UNROLL for (u32 dt = 0; dt < D_TILES; ++dt) v_lane_off[dt] = nt::v_granule_offset(4 * group + (qlane >> 2), dt) + 8 * (qlane & 3);
 	u32 const widen_dst = stager ? nt::widened_offset(tid) : 0;
 	auto widen_v = [&](u32 slot, u32 buf) __attribute__((always_inline)) {
 		if (CPR == 8 || stager) {
 			v4u const raw = *reinterpret_cast<v4u const *>(smem + nt::RAW_V_RING_OFFSET + slot * at::RAW_V_TILE_BYTES + tid * 16);
-			// int8 -> f16: b + 128 as an unsigned byte u, 0x6400 | u == 1024 + u, minus 1152
-			v2h const bias = {(_Float16)-1152.0f, (_Float16)-1152.0f};
 			u32 w[8];
-			X17_UNROLL for (int i = 0; i < 4; ++i) {
-				u32 const word = raw[i] ^ 0x80808080u;
-				u32 const l = __builtin_amdgcn_perm(0x64646464u, word, 0x04010400u), h = __builtin_amdgcn_perm(0x64646464u, word, 0x04030402u);
-				w[2 * i] = __builtin_bit_cast(u32, __builtin_bit_cast(v2h, l) + bias);
-				w[2 * i + 1] = __builtin_bit_cast(u32, __builtin_bit_cast(v2h, h) + bias);
-			}
+			widen16(raw, w);
 			u8 *dst = smem + nt::V_TILES_OFFSET + buf * at::V_TILE_BYTES + widen_dst;
 			*reinterpret_cast<v4u *>(dst) = v4u{w[0], w[1], w[2], w[3]};
 			*reinterpret_cast<v4u *>(dst + 16) = v4u{w[4], w[5], w[6], w[7]};
@@ -328,7 +306,7 @@ void kernel(
 			if (__any(tmax > ext) || twin_asks) {
 				tmax = u2f(over_groups(f2u(tmax), larger));
 				ext = tmax > ext ? tmax : ext;
-				set_subtrahend();
+				set_subtrahend<ROW_SCALES>(ext, abs_t, mb, fine);
 				lift = hw::ex2(fmaf32(ext - ext_ref, abs_t, -HEADROOM));      // (the difference is exact)
 				if (__any(lift > MAX_LIFT) || twin_asks) {
 					// O and the partial sum come down to the scale of the new maximum
@@ -435,10 +413,6 @@ void kernel(
 #endif
 	i8 *o_row = out + (row_base + qi) * O_STRIDE + (size_t)head * HD;
 	X17_UNROLL for (u32 dt = 0; dt < D_TILES; ++dt) {
-		// the scaling rides in the rounding addition; clamping the rounded value gives what rounding the clamped one gives
-		constexpr f32 MAGIC = 12582912.0f;
-		u32 u[4];
-		X17_UNROLL for (int e = 0; e < 4; ++e) u[e] = f2u(__builtin_amdgcn_fmed3f(fmaf32(o_acc[dt][e], inv, MAGIC), MAGIC - 127.0f, MAGIC + 127.0f));
-		*reinterpret_cast<u32 *>(o_row + 16 * dt + 4 * group) = __builtin_amdgcn_perm(u[1], u[0], 0x0c0c0400u) | __builtin_amdgcn_perm(u[3], u[2], 0x04000c0cu);
+		*reinterpret_cast<u32 *>(o_row + 16 * dt + 4 * group) = scaled_codes(o_acc[dt][0], o_acc[dt][1], o_acc[dt][2], o_acc[dt][3], inv);
 	}
 }

@@ -35,7 +35,7 @@ int main(int argc, char **argv) {
 
 	// ---- K: thread t's request lands in stored chunk t; a read of (key, chunk) must name the thread that asked for it
 	for (unsigned key = 0; key < KEYS; ++key) for (unsigned c = 0; c < CPR; ++c) {
-		unsigned const off = nt::k_chunk_offset(key, c);
+		unsigned const off = at::k_chunk_offset(key, c);
 		if (off + 16 > at::K_TILE_BYTES || !at::is_stager(off / 16)) return fail("a K read leaves the tile", off + 16, at::K_TILE_BYTES);
 		if (at::stage_k_offset(off / 16, KV_STRIDE) != key * KV_STRIDE + 16 * c) return fail("a K read names a chunk that holds another key", key, c);
 	}

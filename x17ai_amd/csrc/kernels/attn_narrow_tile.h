@@ -34,11 +34,6 @@ constexpr unsigned first_inside_block(unsigned q_pair0, unsigned wr) {
 // inverse; the keys of a lane group of four stay neighbours.)
 constexpr unsigned key_of_row(unsigned r) { return (r & 3) | ((r & 4) << 1) | ((r & 8) >> 1); }
 
-// K tile: as requested (attn_tile.h: linear 16-byte chunk n = key * CPR + c in 128-byte line n / 8 at position (n % 8) ^ ((line / 2) % 8))
-constexpr unsigned k_chunk_offset(unsigned key, unsigned c) {
-	unsigned const n = key * at::CHUNKS_PER_ROW + c, line = n >> 3;
-	return (line << 7) | (((n & 7) ^ ((line >> 1) & 7)) << 4);
-}
 // f16 V tile, by matrix rows (row r of key block 16 * t: r = 16 t + row of the tile), read transposed: 32-byte granule n = r * CPR + c
 // (16 dims) in 256-byte line n / 8 at position (n % 8) ^ (line % CPR): the 32 lanes a ds_read_b64_tr_b16 serves at a time ask for
 // one granule of eight consecutive rows, which then lie in eight different 32-byte columns

@@ -70,6 +70,14 @@ constexpr unsigned stage_k_offset(unsigned tid, unsigned kv_stride) {
 	unsigned const n = (line << 3) | ((tid & 7) ^ ((line >> 1) & 7));
 	return (n / CHUNKS_PER_ROW) * kv_stride + (n % CHUNKS_PER_ROW) * 16;
 }
+// Where a reader finds chunk c of a key in the K tile: linear 16-byte chunk n = key * CHUNKS_PER_ROW + c lives in 128-byte line
+// n / 8 at position (n % 8) ^ ((line >> 1) & 7).  The LDS serves a ds_read_b128 sixteen lanes at a time out of 64
+// four-byte banks; with this mapping the sixteen keys of such a group land in sixteen different
+// 16-byte slots for every supported head_dim.
+constexpr unsigned k_chunk_offset(unsigned key, unsigned c) {
+	unsigned const n = key * CHUNKS_PER_ROW + c, line = n >> 3;
+	return (line << 7) | (((n & 7) ^ ((line >> 1) & 7)) << 4);
+}
 constexpr unsigned stage_v_offset(unsigned tid, unsigned kv_stride) {
 	return (tid / CHUNKS_PER_ROW) * kv_stride + HEAD_DIM + (tid % CHUNKS_PER_ROW) * 16;
 }
