@@ -65,6 +65,22 @@ def test_attn_strict_bit_exact(dev, t, h, hd, w):
 	assert np.array_equal(got_l.view(np.uint32), want_l.view(np.uint32))
 
 
+@pytest.mark.parametrize("t,h,hd,w", [(512, 4, 32, 0), (384, 2, 64, 128), (320, 2, 128, 0)])
+@pytest.mark.parametrize("scale", [1.0, 12.0, 45.0, 400.0, -45.0, 1e13, 2.0 ** -41, 2.0 ** 40, 0.0])
+def test_attn_strict_bit_exact_at_any_temperature(dev, t, h, hd, w, scale):
+	"""Scores up to hundreds and thousands below their row's maximum: around ex2's last kept argument (-125), around -128 and far
+	beyond, at temperatures inside and outside the range the scaled steps are for.  Bit for bit."""
+	rng = rng_for("attn-temperature", t, h, hd, w, scale)
+	q, kv, sk, sv, temp = _attn_inputs(rng, t, h, hd)
+	q[::7] = np.where(q[::7] < 0, -127, 127)               # the largest dot products, of both signs
+	kv[5::11] = np.where(kv[5::11] < 0, -127, 127)
+	temp = (temp * scale).astype(np.float32)
+	got, got_l = _run_attn(dev, recipes.attn_kernel(dev, h, hd, True), q, kv, sk, sv, temp, w)
+	want, want_l = S.attn_fwd_i8(q, kv, sk, sv, temp, h, hd, w)
+	assert np.array_equal(got, want)
+	assert np.array_equal(got_l.view(np.uint32), want_l.view(np.uint32))
+
+
 @pytest.mark.parametrize("t,h,hd,w", [(512, 2, 64, 128), (640, 2, 128, 256), (1024, 8, 64, 256), (1536, 4, 32, 512), (1024, 2, 128, 0)])
 def test_attn_fast_within_one_code(dev, t, h, hd, w):
 	rng = rng_for("attn", t, h, hd, w)

@@ -95,6 +95,62 @@ X17_DEV u32 v_granule_offset(u32 key, u32 c) {
 	return (line << 8) | (((n & 7) ^ ((line & 3) << 1)) << 5);
 }
 
+// Strict build without row scales.  The reference's numbers at powers of two of its own scale, so that a score of a fully visible tile
+// takes 17 vector instructions instead of 19 and the slow ones of them (conversion, comparison and select, rounding) go:
+//  * Score accumulators start at the bits of DOT_START = 1 / 2 pi, which the matrix instruction takes as an inline constant: read as a
+//    float the sum is DOT_START + dot * 2^-26 exactly (0x3E22F983 has 2 290 051 steps of 2^-26 below it in its binade and
+//    more above, |dot| <= 128 * 128 * 128), one exact subtraction away from the dot product.
+//  * Scores, and the maximum their probabilities refer to, at 2^-7: maximum - score is what ex2 takes, and the subtraction's own
+//    clamp to [0, 1] keeps its argument above -128.
+//  * ex2's polynomial at one half: a result below 2^-125, which the reference's ex2 flushes, then has an exponent field of 0 (an f32
+//    denormal) or a negative one (a set sign bit).  The key loop runs with f32 denormals flushed, so that the multiplication by 255
+//    takes the former for 0; its clamp makes 0 of the latter.  The clamp wants probabilities below 1: they and the partial sums
+//    are at 2^-8.  (What else could be denormal there has no bearing on the output: O and the sums, decayed by 2^-100 and
+//    more, next to a sum of at least 63.)
+//  * Adding 1.5 * 2^15 rounds p / 256 to the integer P and leaves it in the low half of the sum, where it is the f16 denormal
+//    P * 2^-24: the matrix instructions multiply those exactly, O is at 2^-24.
+// Powers of two change no rounding, so the bits are the reference's.  A head whose temperature is zero, not finite or outside
+// 2^-40 .. 2^40 takes the masked steps throughout.  Bound by vector issue (2.5 clocks an instruction, by the counters):
+// 64 heads of 32, 16384 tokens, no window 3168 -> 3009 us; 32 heads of 128, 8192 tokens 869 -> 822.
+constexpr bool SCALED_SUMS = STRICT && !ROW_SCALES;
+constexpr u32 DOT_START_BITS = 0x3E22F983u;
+constexpr f32 DOT_START = __builtin_bit_cast(f32, DOT_START_BITS);
+constexpr f32 SUM_SCALE = SCALED_SUMS ? 0.00390625f : 1.0f;                        // 2^-8
+constexpr f32 SUM_PROB_SCALE = PROB_SCALE * SUM_SCALE;
+constexpr f32 O_SCALE = SCALED_SUMS ? 5.9604644775390625e-08f : 1.0f;              // 2^-24
+constexpr f32 ROUND_MAGIC = 49152.0f;                                               // 1.5 * 2^15: last place 2^-8
+constexpr f32 EX2_MAGIC = 98304.0f;                                                 // 1.5 * 2^16: last place 2^-7
+constexpr int F32_DENORMALS = 1 | 4 << 6 | 1 << 11;                                 // the register MODE, its bits 4 and 5
+X17_DEV bool regular_temperature(f32 t) { return ((f2u(t) >> 23) & 0xFFu) - 87u <= 80u; }
+X17_DEV f32 dot_of(i32 sum) {
+	if constexpr (SCALED_SUMS) return fmaf32(u2f((u32)sum), 67108864.0f, -67108864.0f * DOT_START);      // exact
+	else return f32(sum);
+}
+
+// Constants of the fully visible step, kept in scalar registers (an addition then is four bytes of code, not eight)
+struct StepConstants {
+	f32 dot_start = DOT_START, ex2_magic = EX2_MAGIC, minus_ex2_magic = -EX2_MAGIC, round_magic = ROUND_MAGIC;
+	X17_DEV void keep() { asm volatile("" : "+s"(dot_start), "+s"(ex2_magic), "+s"(minus_ex2_magic), "+s"(round_magic)); }
+};
+
+// 255 / 256 * strict::ex2(-128 * below), with f32 denormals flushed
+X17_DEV f32 scaled_probability(f32 below, StepConstants const &c) {
+	f32 const x = __builtin_amdgcn_fmed3f(below, 0.0f, 1.0f);      // (becomes the subtraction's clamp)
+	f32 const t = c.ex2_magic - x;
+	f32 const g = (t + c.minus_ex2_magic) + x;                      // -f / 128
+	// strict::ex2's coefficients in powers of g, halved
+	constexpr auto of_g = [](f32 coefficient, int power) { f32 v = 0.5f * coefficient; for (int i = 0; i < power; ++i) v *= -128.0f; return v; };
+	f32 p = of_g(0.00015453163359779865f, 6);
+	p = fmaf32(p, g, of_g(0.0013390863314270973f, 5));
+	p = fmaf32(p, g, of_g(0.009618083015084267f, 4));
+	p = fmaf32(p, g, of_g(0.055503569543361664f, 3));
+	p = fmaf32(p, g, of_g(0.24022650718688965f, 2));
+	p = fmaf32(p, g, of_g(0.6931471824645996f, 1));
+	p = fmaf32(p, g, of_g(1.0f, 0));
+	f32 const r = u2f(f2u(p) + (f2u(t) << 23));                     // (the bits of EX2_MAGIC above the integer leave in the shift)
+	return __builtin_amdgcn_fmed3f(r * (2.0f * SUM_PROB_SCALE), 0.0f, 1.0f);      // (the multiplication's clamp)
+}
+
 X17_DEV u32 pack_f16(f32 lo, f32 hi) {
 	// both values are integers below 2048: exact in f16 whatever the rounding mode
 	return __builtin_bit_cast(u32, __builtin_amdgcn_cvt_pkrtz(lo, hi));
@@ -230,8 +286,8 @@ void kernel(
 		f32 m = ROW_SCALES ? f32(sink_dot) * (temperature * 0.125f) : f32(sink_dot) * temperature;
 		f32 lift = 1.0f;                     // speed build: 2^(m - the maximum O's scale refers to)
 		v2h lift2 = {(_Float16)1.0f, (_Float16)1.0f};
-		f32 sum_lo = 0.25f * PROB_SCALE;     // partial sum of key quad `half` of every tile
-		f32 sum_hi = 0.25f * PROB_SCALE;     // partial sum of key quad `2 + half`
+		f32 sum_lo = 0.25f * SUM_PROB_SCALE;     // partial sum of key quad `half` of every tile
+		f32 sum_hi = 0.25f * SUM_PROB_SCALE;     // partial sum of key quad `2 + half`
 		// (the lane pair holds the reference's four partial sums two-and-two; each starts at 63.75)
 		v16f o_acc[D_BLOCKS];                // O^T: lane = query, register r = dim 32*db + 8*(r/4) + 4*half + r%4
 		if constexpr (!STRICT && !ROW_SCALES) {
@@ -257,7 +313,7 @@ void kernel(
 				// 255 * v for the int8 byte v, through the unsigned byte v + 128 (one conversion and one fma per value, all exact)
 				u32 const word = *reinterpret_cast<u32 const *>(sink_v + (size_t)head * HD + 32 * db + 8 * r4 + 4 * half) ^ 0x80808080u;
 				X17_UNROLL for (int b = 0; b < 4; ++b) {
-					o_acc[db][4 * r4 + b] = fmaf32(f32((word >> (8 * b)) & 0xFFu), 255.0f, -32640.0f);
+					o_acc[db][4 * r4 + b] = fmaf32(f32((word >> (8 * b)) & 0xFFu), 255.0f * O_SCALE, -32640.0f * O_SCALE);
 				}
 			}
 		}
@@ -306,11 +362,15 @@ void kernel(
 		//    three loads per step).  Scales are taken to be non-negative (absmax / 127): the sign of a query's
 		//    temperature is then the head's.
 		v16i s_bias;
-		X17_UNROLL for (int r = 0; r < 16; ++r) s_bias[r] = ROW_SCALES || STRICT ? 0 : 0x4B400000;
+		X17_UNROLL for (int r = 0; r < 16; ++r) s_bias[r] = SCALED_SUMS ? (i32)DOT_START_BITS : ROW_SCALES || STRICT ? 0 : 0x4B400000;
 		if constexpr (!ROW_SCALES && !STRICT) {
 			asm volatile("" : "+v"(s_bias));      // (kept in registers: rebuilding it per step would cost what it saves)
 		}
 		f32 const abs_t = __builtin_fabsf(temperature);
+		// strict build, fully visible steps: what takes dot * 2^-26 to a score at 2^-7, and the maximum at 2^-7
+		[[maybe_unused]] f32 const scaled_temperature = temperature * 524288.0f;
+		[[maybe_unused]] f32 scaled_m = m * 0.0078125f;
+		[[maybe_unused]] bool const regular = SCALED_SUMS && regular_temperature(u2f(__builtin_amdgcn_readfirstlane(f2u(attn_temperature[head]))));
 		f32 const sgn = positive_temperature ? 1.0f : -1.0f;
 		f32 ext = ROW_SCALES ? (f32(sink_dot) * 0.125f) * sgn : (f32(sink_dot) + DOT_BIAS) * sgn;
 		[[maybe_unused]] f32 mb = 0.0f, fine = 1.0f;
@@ -336,8 +396,9 @@ void kernel(
 		u32 const inside_kb = q_wave0 + 31 > wr ? (q_wave0 + 62 - wr) / 32 : 0;
 		u32 const inside_clamped = inside_kb < wave_kb_first ? wave_kb_first : (inside_kb > wave_kb_last ? wave_kb_last : inside_kb);
 		// (the speed build's fully visible steps take the row maximum over the scores' bits, which needs a positive
-		// temperature; with any other temperature every step goes the way of the masked ones)
-		u32 const first_full = (STRICT || positive_temperature ? inside_clamped : wave_kb_last) - kb_begin;
+		// temperature, the strict build's scaled ones a regular one; with any other temperature every step goes the way of the masked ones)
+		bool const all_masked = STRICT ? SCALED_SUMS && !regular : !positive_temperature;
+		u32 const first_full = (all_masked ? wave_kb_last : inside_clamped) - kb_begin;
 
 		// Tile requests.  Step s asks for K tile s + 3 and raw V tile s + 4, into the ring slots that K tile s - 1 and raw
 		// V tile s have just left (a V tile is widened -- by the thread that fetched it -- during the step before its
@@ -445,17 +506,22 @@ void kernel(
 			v8s const both = {lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], hi4[2], hi4[3]};
 			return __builtin_bit_cast(v8h, both);
 		};
+		[[maybe_unused]] StepConstants step_constants;
+		if constexpr (SCALED_SUMS) step_constants.keep();
 		// Strict build, one 16-key tile: the reference's operations one by one.
 		auto strict_tile = [&]<bool MASKED>(u32 i, u32 tile, v16i const &s_acc, u32 k_slot, u8 const *v_tile) __attribute__((always_inline)) {
+			constexpr bool SCALED = !MASKED && SCALED_SUMS;      // scores at 2^-7
 			f32 s[8];
 			// row-scaled build: this lane's 8 keys of the tile are 4 * half + {0..3} and 8 + 4 * half + {0..3}
 			[[maybe_unused]] f32 const *sc = nullptr;
 			if constexpr (ROW_SCALES) {
 				sc = reinterpret_cast<f32 const *>(smem + at::SCALE_RING_OFFSET + k_slot * at::SCALE_TILE_BYTES) + 16 * tile + 4 * half;
 				v4f const k0 = *reinterpret_cast<v4f const *>(sc), k1 = *reinterpret_cast<v4f const *>(sc + 8);
-				X17_UNROLL for (u32 r = 0; r < 8; ++r) s[r] = (f32(s_acc[8 * tile + r]) * (r < 4 ? k0[r % 4] : k1[r % 4])) * temperature;
+				X17_UNROLL for (u32 r = 0; r < 8; ++r) s[r] = (dot_of(s_acc[8 * tile + r]) * (r < 4 ? k0[r % 4] : k1[r % 4])) * temperature;
+			} else if constexpr (SCALED) {
+				X17_UNROLL for (u32 r = 0; r < 8; ++r) s[r] = (u2f((u32)s_acc[8 * tile + r]) - step_constants.dot_start) * scaled_temperature;
 			} else {
-				X17_UNROLL for (u32 r = 0; r < 8; ++r) s[r] = f32(s_acc[8 * tile + r]) * temperature;
+				X17_UNROLL for (u32 r = 0; r < 8; ++r) s[r] = dot_of(s_acc[8 * tile + r]) * temperature;
 			}
 			if constexpr (MASKED) {
 				// key j is visible iff j < qi and qi - j <= wr, i.e. iff the distance qi - 1 - j, taken as an
@@ -472,29 +538,38 @@ void kernel(
 			// cuda/attn_fwd_i8.cuh:233-256 -- rescale only when some row's max grew (both lanes of a pair hold the same m:
 			// the tile's maximum exceeds it exactly when one of the two halves does)
 			f32 resc = 1.0f;
-			if (__any(tmax > m)) {
+			if (__any(tmax > (SCALED ? scaled_m : m))) {
 				tmax = __builtin_fmaxf(tmax, partner_f32(tmax, half));
-				f32 const new_m = __builtin_fmaxf(tmax, m);
+				f32 const new_m = SCALED ? __builtin_fmaxf(tmax, scaled_m) * 128.0f : __builtin_fmaxf(tmax, m);
 				resc = strict::ex2<true>(m - new_m);      // exactly 1 for rows whose max did not move
 				m = new_m;
+				if constexpr (SCALED_SUMS) scaled_m = m * 0.0078125f;
 				X17_UNROLL for (u32 db = 0; db < D_BLOCKS; ++db) {
 					X17_UNROLL for (int r = 0; r < 16; ++r) o_acc[db][r] = o_acc[db][r] * resc;
 				}
 			}
-			// :265-290 -- p = ex2(s - max) * 255; partial sums over key quads; P = rne(p)
+			// :265-290 -- p = ex2(s - max) * 255 (without row scales: at 2^-8); partial sums over key quads; P = rne(p)
 			f32 p[8];
-			X17_UNROLL for (u32 r = 0; r < 8; ++r) p[r] = strict::ex2<true>(s[r] - m) * PROB_SCALE;
+			if constexpr (SCALED) {
+				X17_UNROLL for (u32 r = 0; r < 8; ++r) p[r] = scaled_probability(scaled_m - s[r], step_constants);
+			} else {
+				X17_UNROLL for (u32 r = 0; r < 8; ++r) p[r] = strict::ex2<true>(s[r] - m) * SUM_PROB_SCALE;
+			}
 			sum_lo = fmaf32(sum_lo, resc, (p[0] + p[1]) + (p[2] + p[3]));
 			sum_hi = fmaf32(sum_hi, resc, (p[4] + p[5]) + (p[6] + p[7]));
+			v4u pp;
 			if constexpr (ROW_SCALES) {
 				// the numerator takes the probabilities at the value rows' relative scales
 				v4f const w0 = *reinterpret_cast<v4f const *>(sc + 32), w1 = *reinterpret_cast<v4f const *>(sc + 40);
 				X17_UNROLL for (u32 r = 0; r < 8; ++r) p[r] = p[r] * (r < 4 ? w0[r % 4] : w1[r % 4]);
+				X17_UNROLL for (int w = 0; w < 4; ++w) pp[w] = pack_f16(__builtin_rintf(p[2 * w]), __builtin_rintf(p[2 * w + 1]));
+			} else {
+				X17_UNROLL for (int w = 0; w < 4; ++w) {
+					pp[w] = __builtin_amdgcn_perm(f2u(p[2 * w + 1] + step_constants.round_magic), f2u(p[2 * w] + step_constants.round_magic), 0x05040100u);
+				}
 			}
-			v4u pp;
-			X17_UNROLL for (int w = 0; w < 4; ++w) pp[w] = pack_f16(__builtin_rintf(p[2 * w]), __builtin_rintf(p[2 * w + 1]));
 			v8h const pfrag = __builtin_bit_cast(v8h, pp);
-			// :588-605 -- O += f32(P . V) for this 16-key tile
+			// :588-605 -- O += f32(P . V) for this 16-key tile (without row scales: at 2^-24)
 			X17_UNROLL for (u32 db = 0; db < D_BLOCKS; ++db) {
 				v16f const zero = {0};
 				v16f const pv = __builtin_amdgcn_mfma_f32_32x32x16_f16(v_fragment(v_tile, tile, db), pfrag, zero, 0, 0, 0);
@@ -643,6 +718,7 @@ void kernel(
 			__builtin_amdgcn_s_waitcnt(0x0F76);   // vmcnt(6): raw V tile 0 has landed
 		}
 		widen_v(0, 0);
+		if (regular) __builtin_amdgcn_s_setreg(F32_DENORMALS, 0);      // flushed
 		u32 i = 0;
 		for (; i < first_active; ++i) idle_step(i);
 		for (; i < first_full; ++i) step.template operator()<true, -1>(i);
@@ -662,6 +738,7 @@ void kernel(
 		for (; i < diagonal; ++i) step.template operator()<false, -1>(i);
 		step.template operator()<true, -1>(i);
 		for (++i; i < n_steps; ++i) idle_step(i);
+		if constexpr (SCALED_SUMS) __builtin_amdgcn_s_setreg(F32_DENORMALS, 3);      // kept
 		__builtin_amdgcn_s_waitcnt(0x0F70);   // the last requests write LDS: they land before the tiles are reused
 		// speed build: the partial sums are at the scale of the maximum HEADROOM above ext_ref's score: the common ending below
 		// takes them as if that were the maximum (sgn * ext_ref - 12582912 is that extreme's dot product, exactly)
@@ -676,11 +753,11 @@ void kernel(
 		f32 s1 = half == 0 ? other_lo : sum_lo;
 		f32 s2 = half == 0 ? sum_hi : other_hi;
 		f32 s3 = half == 0 ? other_hi : sum_hi;
-		f32 total = (s0 + s1) + (s2 + s3);
+		f32 total = ((s0 + s1) + (s2 + s3)) * (1.0f / SUM_SCALE);
 		if (l_out != nullptr && half == 0) {
 			l_out[(size_t)head * ((size_t)gridDim.z * seq_len) + row_base + qi] = sfu::lg2(total) + m;
 		}
-		f32 inv = sfu::rcp(total);
+		f32 inv = sfu::rcp(total) * (1.0f / O_SCALE);
 #if X17_ATTN_ROW_SCALES
 		f32 const head_out_scale = out_scale[head];
 		if constexpr (OUT_BF16) {
