@@ -111,7 +111,7 @@ X17_DEV u32 v_granule_offset(u32 key, u32 c) {
 //    P * 2^-24: the matrix instructions multiply those exactly, O is at 2^-24.
 // Powers of two change no rounding, so the bits are the reference's.  A head whose temperature is zero, not finite or outside
 // 2^-40 .. 2^40 takes the masked steps throughout.  Bound by vector issue (2.5 clocks an instruction, by the counters):
-// 64 heads of 32, 16384 tokens, no window 3168 -> 3009 us; 32 heads of 128, 8192 tokens 869 -> 822.
+// 64 heads of 32, 16384 tokens, no window 3165 -> 2977 us; 32 heads of 128, 8192 tokens 868 -> 826.
 constexpr bool SCALED_SUMS = STRICT && !ROW_SCALES;
 constexpr u32 DOT_START_BITS = 0x3E22F983u;
 constexpr f32 DOT_START = __builtin_bit_cast(f32, DOT_START_BITS);
@@ -122,14 +122,10 @@ constexpr f32 ROUND_MAGIC = 49152.0f;                                           
 constexpr f32 EX2_MAGIC = 98304.0f;                                                 // 1.5 * 2^16: last place 2^-7
 constexpr int F32_DENORMALS = 1 | 4 << 6 | 1 << 11;                                 // the register MODE, its bits 4 and 5
 X17_DEV bool regular_temperature(f32 t) { return ((f2u(t) >> 23) & 0xFFu) - 87u <= 80u; }
-X17_DEV f32 dot_of(i32 sum) {
-	if constexpr (SCALED_SUMS) return fmaf32(u2f((u32)sum), 67108864.0f, -67108864.0f * DOT_START);      // exact
-	else return f32(sum);
-}
-
 // Constants of the fully visible step, kept in scalar registers (an addition then is four bytes of code, not eight)
 struct StepConstants {
 	f32 dot_start = DOT_START, ex2_magic = EX2_MAGIC, minus_ex2_magic = -EX2_MAGIC, round_magic = ROUND_MAGIC;
+	X17_DEV f32 dot(i32 sum) const { return (u2f((u32)sum) - dot_start) * 67108864.0f; }      // exact
 	X17_DEV void keep() { asm volatile("" : "+s"(dot_start), "+s"(ex2_magic), "+s"(minus_ex2_magic), "+s"(round_magic)); }
 };
 
@@ -193,11 +189,7 @@ void kernel(
 ) {
 	extern __shared__ __attribute__((aligned(1024))) u8 smem[];
 
-	u32 const tid = threadIdx.x;
-	u32 const lane = tid % 64;
-	u32 const wave = __builtin_amdgcn_readfirstlane(tid / 64);
-	u32 const half = lane / 32;
-	u32 const qlane = lane % 32;
+	u32 const wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
 
 	// Which (sequence, head group, query block) this workgroup takes.  The hardware starts workgroups in the order of
 	// their linear index (and deals them round-robin to the 8 XCDs).  The query block is the slowest index of that
@@ -221,7 +213,6 @@ void kernel(
 	// src/device/cuda/attn.rs:398-404) starts earlier and recomputes some of its neighbour's queries
 	u32 const q_block0 = at::block_first_query(q_block_index, seq_len);
 	u32 const q_wave0 = q_block0 + wave * at::Q_PER_WAVE;
-	u32 const qi = q_wave0 + qlane;                         // this lane's query position
 
 	// cuda/attn_fwd_i8.cuh:408-412 -- window 0 means "no window"; otherwise rounded up to 16
 	u32 const wr = at::rounded_window(window_size);
@@ -235,6 +226,13 @@ void kernel(
 
 	for (u32 hh = 0; hh < heads_here; ++hh) {
 		u32 const head = head_group * heads_here + hh;
+		// (opaque: what a head derives from it is derived anew for the next one, not kept in registers from here on)
+		u32 tid = threadIdx.x;
+		if constexpr (STRICT) asm volatile("" : "+v"(tid));
+		u32 const lane = tid % 64;
+		u32 const half = lane / 32;
+		u32 const qlane = lane % 32;
+		u32 const qi = q_wave0 + qlane;                     // this lane's query position
 		i8 const *q_head = q + row_base * Q_STRIDE + (size_t)head * HD;
 		i8 const *kv_head = kv + row_base * KV_STRIDE + (size_t)head * 2 * HD;
 
@@ -517,11 +515,11 @@ void kernel(
 			if constexpr (ROW_SCALES) {
 				sc = reinterpret_cast<f32 const *>(smem + at::SCALE_RING_OFFSET + k_slot * at::SCALE_TILE_BYTES) + 16 * tile + 4 * half;
 				v4f const k0 = *reinterpret_cast<v4f const *>(sc), k1 = *reinterpret_cast<v4f const *>(sc + 8);
-				X17_UNROLL for (u32 r = 0; r < 8; ++r) s[r] = (dot_of(s_acc[8 * tile + r]) * (r < 4 ? k0[r % 4] : k1[r % 4])) * temperature;
+				X17_UNROLL for (u32 r = 0; r < 8; ++r) s[r] = (f32(s_acc[8 * tile + r]) * (r < 4 ? k0[r % 4] : k1[r % 4])) * temperature;
 			} else if constexpr (SCALED) {
 				X17_UNROLL for (u32 r = 0; r < 8; ++r) s[r] = (u2f((u32)s_acc[8 * tile + r]) - step_constants.dot_start) * scaled_temperature;
 			} else {
-				X17_UNROLL for (u32 r = 0; r < 8; ++r) s[r] = dot_of(s_acc[8 * tile + r]) * temperature;
+				X17_UNROLL for (u32 r = 0; r < 8; ++r) s[r] = step_constants.dot(s_acc[8 * tile + r]) * temperature;
 			}
 			if constexpr (MASKED) {
 				// key j is visible iff j < qi and qi - j <= wr, i.e. iff the distance qi - 1 - j, taken as an
