@@ -8,11 +8,10 @@
 // Design, MI355X-first (nothing here is derived from the SM80 kernel):
 //   * One workgroup = a 256 (tokens) x 256 (raw columns) output tile, by default 8 wavefronts of
 //     64 x 128 (two per SIMD); gemm_tile.h can also build 8 wavefronts of 128 x 64 or 4 wavefronts of 128 x 128
-//     (a 4 x 4 grid of 32x32 MFMA blocks, 256 accumulator registers per lane, one wavefront per SIMD: what the
-//     host picks whenever an operand is e4m3).
+//     (256 accumulator registers per lane, one wavefront per SIMD: what the host picks whenever an operand is e4m3).
 //   * The WEIGHTS are the MFMA "A" operand and the TOKENS the "B" operand, i.e. the matrix
-//     cores compute C^T.  A lane then owns one token and, per MFMA block, 16 output columns;
-//     weight rows are permuted on their way into LDS so that those are 64 (32 for 64-column waves)
+//     cores compute C^T.  A lane then owns one token and, per MFMA block, 4 output columns (16 of a 32 x 32 block);
+//     weight rows are permuted on their way into LDS so that those are 32 (64)
 //     CONSECUTIVE columns across the blocks.  Gate/value pairs, whole K|V heads and 16-byte output
 //     vectors all live inside one lane: the epilogues need no cross-lane shuffles (the SM80
 //     code needs a 4x4 shuffle transpose per 32x32 tile, cuda/gemm_b8.cuh:411, 570, 592).
@@ -22,7 +21,8 @@
 //     16-byte chunks are XOR-swizzled so that ds_read_b128 is conflict-free.  In the int8 and e4m3 kernels the
 //     issue order of a K step is pinned: each MFMA is followed by its share of the LDS reads and tile requests
 //     (and, in the mixed arithmetic, of the next round's conversions to f16).
-//   * int8: v_mfma_i32_32x32x32_i8.  e4m3 x e4m3: v_mfma_f32_32x32x64_f8f6f4.  Mixed
+//   * int8: v_mfma_i32_16x16x64_i8.  e4m3 x e4m3: v_mfma_f32_16x16x128_f8f6f4 (with the head-normalising writers and with
+//     fewer than three K steps the 32 x 32 forms of both).  Mixed
 //     e4m3 x int8: both widened exactly to f16 in registers, v_mfma_f32_32x32x16_f16
 //     (int8 codes need 7 significand bits, e4m3 has 4; every e4m3 value is a normal f16).
 //   * Workgroup ids are remapped so that each XCD (own L2) works on a compact block of tiles.
@@ -49,7 +49,7 @@
 using namespace x17;
 namespace gt = x17::gemm_tile;
 namespace {
-constexpr int LANE_COLS = gt::WAVE_N / 2;                   // consecutive raw columns a lane ends up with
+constexpr int LANE_COLS = gt::WAVE_N / gt::GROUPS;          // consecutive raw columns a lane ends up with
 }
 #include "gemm_parts.h"
 
@@ -75,15 +75,16 @@ constexpr u32 K_STEPS = K_TOTAL / gt::K_STEP;
 
 constexpr u32 WAVES = gt::WAVES_M * gt::WAVES_N;
 
+constexpr bool BLOCKS16 = gt::BLOCKS16;
+constexpr int XB = gt::WAVE_M / 16, WB = gt::WAVE_N / 16, WH = WB / 2;      // blocks of 16 tokens, of 16 columns, of half the columns
+constexpr u32 CH = MMA == 1 ? 2 : 1;                         // 16-byte chunks a lane fetches per operand row
+constexpr u32 SLICES16 = gt::K_STEP / (64 * CH);             // slices of a K step
+
 // ------------------------------------------------------------------ tile loads
 
-// LDS rows hold K_STEP bytes = CHUNKS chunks of 16; logical chunk c of row r is stored at position
-// c ^ ((r >> SWZ_SHIFT) & (CHUNKS - 1)).  The LDS has 64 four-byte banks (256 bytes per bank line)
-// and serves a ds_read_b128 sixteen lanes at a time, so sixteen consecutive rows must land in sixteen
-// different 16-byte slots of the bank line: with 128-byte rows two rows share a bank line and the row
-// PAIR index has to be mixed in, with 64-byte rows the row QUAD index.
+// LDS rows hold K_STEP bytes = CHUNKS chunks of 16; logical chunk c of row r is stored at position c ^ gt::swizzle(r): with 128-byte
+// rows two rows share a line of the 64 four-byte banks, so the row PAIR is what has to be mixed in, with 64-byte rows the row QUAD.
 constexpr u32 CHUNKS = gt::CHUNKS;
-constexpr u32 SWZ_SHIFT = gt::SWZ_SHIFT;
 constexpr u32 UNIT_ROWS = gt::UNIT_ROWS;                    // rows one 64-lane x 16-byte direct-to-LDS load fills
 // With eight waves, two per SIMD, only the first of each pair (waves 0 .. 3) requests tiles.  The arbiter serves
 // that wave first: with the loads shared evenly it ended its step early and sat at the barrier while its partner,
@@ -107,8 +108,8 @@ X17_DEV constexpr u32 w_unit_row(u32 r0) {   // weight row that LDS weight row r
 struct LaneOffsets {
 	u32 x_src[X_OFFSETS];   // per-lane byte offset into A for a direct-to-LDS load (even / odd load unit, or per unit)
 	u32 w_src[W_OFFSETS];   // per-lane byte offset into B
-	u32 frag_row;   // (lane % 32) * ROW_BYTES
-	u32 half;       // lane / 32
+	u32 frag_row;   // (lane % BLOCK) * ROW_BYTES
+	u32 half;       // lane / BLOCK
 	u32 swz;        // swizzle key of the fragment row this lane reads
 };
 
@@ -355,6 +356,110 @@ X17_DEV void mixed_round(Wide const &cur, Wide &nxt, Frags const &raw, Frags &rd
 	}
 }
 
+// ---- 16 x 16 blocks (int8 x int8 and e4m3 x e4m3).  What bounds these kernels is the power the chip may draw: it lowers the clock
+// until they fit, and per product the 16 x 16 instructions cost less of it than the 32 x 32 ones (half the accumulator traffic).  Loops
+// of nothing but matrix instructions on Gaussian operands: int8 3.56 -> 4.16 POP/s, e4m3 4.04 -> 4.42.  us, blocks of 32 / of 16:
+//   int8, K = 2048, 16384 columns with the GeGLU writer, 32768 rows 866 / 806 (clock 1.68 -> 1.88 GHz, as many cycles)
+//   int8, run-time scales, K = 8192, 2048 columns, 8192 rows 115 / 105     e4m3, K = 16384, 8192 columns, 16384 rows 1469 / 1402
+// The bytes are those of the 32 x 32 instructions.  int32 sums are exact; a 16x16x128 instruction adds sixteen products of every lane
+// group at a time, in the groups' order, and so goes through K as two 32x32x64 instructions do if group g takes the chunks
+// chunk16 names (no difference in 400 thousand sums of 2048 products each).
+struct Frags16 {
+	v4i x[XB][CH];
+	v4i w[2][WH][CH];          // the wavefront's columns in two halves
+};
+// 16-byte chunk of a K step that is chunk c of slice s in lane group `group`'s fragments
+X17_DEV u32 chunk16(u32 s, u32 c, u32 group) {
+	return MMA == 0 ? 4 * s + group : 4 * c + ((group & 1) << 1 | group >> 1);
+}
+// chunk C of token block B, of slice s; chunk I of a half's column blocks
+template <int B, u32 C>
+X17_DEV void read_x16(Frags16 &f, u8 const *x_tile, u32 s, LaneOffsets const &lo) {
+	f.x[B][C] = lds_chunk(x_tile, B * 16 * ROW_BYTES, chunk16(s, C, lo.half), lo.swz);
+}
+template <int HALF, int I>
+X17_DEV void read_w16(Frags16 &f, u8 const *w_tile, u32 s, LaneOffsets const &lo) {
+	f.w[HALF][I / CH][I % CH] = lds_chunk(w_tile, (HALF * WH + I / CH) * 16 * ROW_BYTES, chunk16(s, I % CH, lo.half), lo.swz);
+}
+template <int I>
+X17_DEV void read_first16(Frags16 &f, u8 const *w_tile, u8 const *x_tile, LaneOffsets const &lo) {
+	if constexpr (I < XB * (int)CH) {
+		if constexpr (I < WH * (int)CH) read_w16<0, I>(f, w_tile, 0, lo);
+		read_x16<I / (int)CH, I % (int)CH>(f, x_tile, 0, lo);
+		read_first16<I + 1>(f, w_tile, x_tile, lo);
+	}
+}
+X17_DEV v4i mma16(v4i const (&w)[CH], v4i const (&x)[CH], v4i acc) {
+	if constexpr (MMA == 0) {
+		return __builtin_amdgcn_mfma_i32_16x16x64_i8(w[0], x[0], acc, 0, 0, 0);
+	} else {
+		v4i const w1 = w[CH - 1], x1 = x[CH - 1];
+		v8i const wf = {w[0][0], w[0][1], w[0][2], w[0][3], w1[0], w1[1], w1[2], w1[3]};
+		v8i const xf = {x[0][0], x[0][1], x[0][2], x[0][3], x1[0], x1[1], x1[2], x1[3]};
+		return __builtin_bit_cast(v4i, __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, xf, __builtin_bit_cast(v4f, acc), 0, 0, 0, 0, 0, 0));
+	}
+}
+constexpr bool w_units_alike() {
+	for (u32 wave = 0; wave < LOADER_WAVES; ++wave) {
+		for (u32 u = 0; u < W_UNITS; ++u) {
+			if (w_unit_row((wave * W_UNITS + u) * UNIT_ROWS) - w_unit_row(wave * W_UNITS * UNIT_ROWS) != w_unit_row(u * UNIT_ROWS)) return false;
+		}
+	}
+	return true;
+}
+static_assert(w_units_alike(), "a loading wave's weight rows lie alike whichever wave it is");
+// (a pointer that is the same in every lane; reading it from the first one tells the compiler so)
+X17_DEV u8 const *uniform(u8 const *p) {
+	u64 const a = (u64)p;
+	return (u8 const *)((u64)(u32)__builtin_amdgcn_readfirstlane((u32)(a >> 32)) << 32 | (u32)__builtin_amdgcn_readfirstlane((u32)a));
+}
+// Tile request U of a loading wave: a buffer load (base of the step's rows, lane offset, the unit's rows as a scalar offset) to the
+// unit's part of `lds`.  (A scalar write of M0 needs one wait state before a direct-to-LDS load reads it.)
+template <bool WEIGHTS, u32 U>
+X17_DEV void request16(v4u rows, u32 lds, LaneOffsets const &lo) {
+	constexpr u32 row = LANE_UNIT_OFFSETS ? 0 : WEIGHTS ? w_unit_row(U * UNIT_ROWS) : U * UNIT_ROWS;
+	u32 const lane_offset = WEIGHTS ? lo.w_src[LANE_UNIT_OFFSETS ? U : U & 1] : lo.x_src[LANE_UNIT_OFFSETS ? U : U & 1];
+	asm volatile("s_add_i32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds"
+	             :: "s"(lds), "i"(U * UNIT_ROWS * ROW_BYTES), "v"(lane_offset), "s"(rows), "s"(row * K_TOTAL) : "memory", "m0", "scc");
+}
+X17_DEV v4u rows_resource(u8 const *p) {
+	return v4u{(u32)(u64)p, (u32)((u64)p >> 32), 256 * K_TOTAL, 0x00020000u};
+}
+// One part of a step: slice Q / 2 of K, all tokens, half Q % 2 of the columns.  Its reads are the other half's columns (of `w_tile`) and,
+// behind a slice's last use of a token block, that block of the next slice (of `x_tile`), into the same registers.  Behind a matrix instruction
+// comes one read, one request or a piece of the next step's addresses (`between`), not several: a wavefront issues an
+// instruction in about nine clocks, a matrix instruction takes 16 (int8) or 32.
+template <int Q, int I, bool READS, int KIND, u32 FIRST, u32 COUNT, class Between>
+X17_DEV void paced16(Frags16 &f, u8 const *w_tile, u8 const *x_tile, LaneOffsets const &lo, v4i (&acc)[WB][XB], v4u rows, u32 lds, Between const &between) {
+	constexpr int MFMAS = XB * WH, HALF = Q % 2, NEXT = HALF == 0 ? Q / 2 : (Q / 2 + 1) % (int)SLICES16;
+	if constexpr (I < MFMAS) {
+		constexpr int b = I / WH, j = I % WH;
+		constexpr int EVERY = MFMAS / (int)COUNT, SLOT = HALF == 0 ? I - 1 : I;
+		static_assert(MFMAS % COUNT == 0, "requests at even distances");
+		acc[HALF * WH + j][b] = mma16(f.w[HALF][j], f.x[b], acc[HALF * WH + j][b]);
+		__builtin_amdgcn_sched_barrier(0);      // (a token block's read stays behind the instruction above: it takes its operand's registers)
+		if constexpr (READS) {
+			// columns: behind every other instruction from the first one; in a slice's second half behind the second and (two chunks) third
+			// of a token block's four
+			constexpr int W_READS = WH * (int)CH;
+			constexpr int W = HALF == 0 ? (I % 2 == 0 ? I / 2 : W_READS) : j == 1 ? b * (int)CH : j == 2 && CH == 2 ? b * 2 + 1 : W_READS;
+			if constexpr (W < W_READS) read_w16<1 - HALF, W>(f, w_tile, NEXT, lo);
+			if constexpr (HALF == 1) {
+				// tokens: first chunks behind the block's last instruction, second ones where the columns' reads were
+				if constexpr (j == WH - 1) read_x16<b, 0>(f, x_tile, NEXT, lo);
+				constexpr int LATE = CH == 1 ? XB : b >= XB / 2 && (j == 1 || j == 2) ? 2 * (b - XB / 2) + j - 1 : I == MFMAS - 1 ? XB - 1 : XB;
+				if constexpr (LATE < (I == MFMAS - 1 ? XB : XB - 1)) read_x16<LATE, CH - 1>(f, x_tile, NEXT, lo);
+			}
+		}
+		if constexpr (KIND != 0) {
+			if constexpr (SLOT >= 0 && SLOT % EVERY == 0) request16<KIND == 2, FIRST + SLOT / EVERY>(rows, lds, lo);
+		}
+		between.template operator()<I>();
+		__builtin_amdgcn_sched_barrier(0);
+		paced16<Q, I + 1, READS, KIND, FIRST, COUNT>(f, w_tile, x_tile, lo, acc, rows, lds, between);
+	}
+}
+
 } // namespace
 
 extern "C" __global__ __launch_bounds__(gt::THREADS_PER_BLOCK)
@@ -429,9 +534,9 @@ void kernel(
 				lo.w_src[odd] = even_odd_w[odd];
 			}
 		}
-		lo.frag_row = (lane % 32) * ROW_BYTES;
-		lo.half = lane / 32;
-		lo.swz = ((lane % 32) >> SWZ_SHIFT) & (CHUNKS - 1);
+		lo.frag_row = (lane % gt::BLOCK) * ROW_BYTES;
+		lo.half = lane / gt::BLOCK;
+		lo.swz = gt::swizzle(lane % gt::BLOCK);
 	}
 
 	// ---- main loop.  Rings of XS token tiles and WS weight tiles in LDS; step ks consumes ring positions
@@ -506,7 +611,114 @@ void kernel(
 			}
 		}
 
-		Acc acc[BN][BM];   // [bn][bm]
+		[[maybe_unused]] v4i acc16[WB][XB];
+		if constexpr (BLOCKS16) {
+			X17_UNROLL for (int bn = 0; bn < WB; ++bn) {
+				X17_UNROLL for (int bm = 0; bm < XB; ++bm) acc16[bn][bm] = v4i{0, 0, 0, 0};
+			}
+			Frags16 f;
+			read_first16<0>(f, smem + wb * W_TILE_BYTES + w_off, smem + xb * X_TILE_BYTES + x_off, lo);
+			auto k_loop = [&]<bool LOADER>() __attribute__((always_inline)) {
+				constexpr u32 PARTS = 2 * SLICES16, X_PARTS = PARTS / 2;        // parts of a step; those that carry token requests
+				size_t const x_wave = (size_t)(wave * X_UNITS * UNIT_ROWS) * K_TOTAL, w_wave = (size_t)w_unit_row(wave * W_UNITS * UNIT_ROWS) * K_TOTAL;
+				u8 const *const a_rows_here = uniform(a_tile + x_wave), *const a_rows_next = uniform(a_next + x_wave);
+				u8 const *const b_rows_here = uniform(b_tile + w_wave), *const b_rows_next = uniform(b_next + w_wave);
+				u32 const lds0 = (u32)(size_t)X17_LDS_PTR(smem);
+				u32 const lds_wave_x = lds0 + wave * X_UNITS * UNIT_ROWS * ROW_BYTES, lds_wave_w = lds0 + W_RING_OFFSET + wave * W_UNITS * UNIT_ROWS * ROW_BYTES;
+				bool const hn = has_next;
+				// a step's tiles, the rows its requests take and where they go; the next step's are computed a piece at a time in this one
+				struct Step { u8 const *w_tile, *x_tile, *lx, *lw; u32 x_lds, w_lds; } now, next;
+				u32 next_xb = xb, next_wb = wb;
+				auto tiles = [&](Step &s) __attribute__((always_inline)) {
+					s.w_tile = smem + next_wb * W_TILE_BYTES + w_off;
+					s.x_tile = smem + next_xb * X_TILE_BYTES + x_off;
+				};
+				u32 x_k0 = 0, w_k0 = 0;
+				auto offsets = [&](u32 ks) __attribute__((always_inline)) {
+					u32 const x_step = ks + XS - 1, w_step = ks + WS;
+					x_k0 = (x_step < K_STEPS ? x_step : (hn ? x_step - K_STEPS : 0)) * gt::K_STEP;
+					w_k0 = (w_step < K_STEPS ? w_step : (hn ? w_step - K_STEPS : 0)) * gt::K_STEP;
+				};
+				// (values, not the captured variables: a choice between two captured pointers would keep them in memory)
+				auto token_rows = [&](Step &s, u32 ks) __attribute__((always_inline)) {
+					u8 const *const here = a_rows_here, *const after = a_rows_next;
+					s.lx = (ks + XS - 1 < K_STEPS || !hn ? here : after) + x_k0;
+				};
+				auto weight_rows = [&](Step &s, u32 ks) __attribute__((always_inline)) {
+					u8 const *const here = b_rows_here, *const after = b_rows_next;
+					s.lw = (ks + WS < K_STEPS || !hn ? here : after) + w_k0;
+				};
+				auto token_destination = [&](Step &s) __attribute__((always_inline)) {
+					s.x_lds = __builtin_amdgcn_readfirstlane(lds_wave_x + (next_xb == 0 ? XS - 1 : next_xb - 1) * X_TILE_BYTES);
+				};
+				auto weight_destination = [&](Step &s) __attribute__((always_inline)) {
+					s.w_lds = __builtin_amdgcn_readfirstlane(lds_wave_w + next_wb * W_TILE_BYTES);
+				};
+				tiles(now);
+				offsets(0);
+				token_rows(now, 0);
+				weight_rows(now, 0);
+				token_destination(now);
+				weight_destination(now);
+				auto const nothing = [&]<int I>() __attribute__((always_inline)) {};
+				auto step = [&]<bool LAST_STEP>(u32 ks) __attribute__((always_inline)) {
+					auto const addresses = [&]<int I>() __attribute__((always_inline)) {
+						constexpr int FROM = XB * WH / 2;      // behind the part's reads
+						if constexpr (I == FROM) {
+							next_xb = next_xb + 1 == XS ? 0 : next_xb + 1;
+							next_wb = next_wb + 1 == WS ? 0 : next_wb + 1;
+						} else if constexpr (I == FROM + 1 && !LAST_STEP) {
+							tiles(next);
+						} else if constexpr (I == FROM + 2 && !LAST_STEP) {
+							offsets(ks + 1);
+						} else if constexpr (I == FROM + 3 && !LAST_STEP) {
+							token_rows(next, ks + 1);
+						} else if constexpr (I == FROM + 4 && !LAST_STEP) {
+							weight_rows(next, ks + 1);
+						} else if constexpr (I == FROM + 5 && !LAST_STEP) {
+							token_destination(next);
+						} else if constexpr (I == FROM + 6 && !LAST_STEP) {
+							weight_destination(next);
+						}
+					};
+					v4u const x_rows = rows_resource(now.lx), w_rows = rows_resource(now.lw);
+					auto parts = [&]<u32 Q>(auto &&self) __attribute__((always_inline)) {
+						if constexpr (Q + 1 < PARTS) {
+							constexpr u32 FIRST = (Q < X_PARTS ? Q : X_PARTS) * X_UNITS / X_PARTS, LAST = (Q + 1 < X_PARTS ? Q + 1 : X_PARTS) * X_UNITS / X_PARTS;
+							constexpr int KIND = LOADER && Q < X_PARTS ? 1 : 0;
+							constexpr u32 COUNT = KIND != 0 ? LAST - FIRST : 1;
+							if constexpr (Q + 2 < PARTS) paced16<Q, 0, true, KIND, FIRST, COUNT>(f, now.w_tile, now.x_tile, lo, acc16, x_rows, now.x_lds, nothing);
+							else paced16<Q, 0, true, KIND, FIRST, COUNT>(f, now.w_tile, now.x_tile, lo, acc16, x_rows, now.x_lds, addresses);
+							self.template operator()<Q + 1>(self);
+						} else {
+							// the next step's tiles have landed once all but the token tile just requested have; this wave is done
+							// reading this step's tiles
+							wait_vmcnt<X_UNITS>();
+							__builtin_amdgcn_s_waitcnt(0xC07F);
+							__builtin_amdgcn_s_barrier();
+							paced16<Q, 0, !LAST_STEP, LOADER ? 2 : 0, 0, W_UNITS>(f, next.w_tile, next.x_tile, lo, acc16, w_rows, now.w_lds, nothing);
+						}
+					};
+					parts.template operator()<0>(parts);
+				};
+				// (the last step, which reads nothing ahead, behind the loop: a choice inside makes copies of the accumulators)
+				_Pragma("clang loop unroll(disable)")
+				for (u32 ks = 0; ks + 1 < K_STEPS; ++ks) {
+					step.template operator()<false>(ks);
+					now = next;
+				}
+				step.template operator()<true>(K_STEPS - 1);
+				xb = next_xb;
+				wb = next_wb;
+			};
+			if (WAVES == LOADER_WAVES || wave < LOADER_WAVES) {
+				k_loop.template operator()<true>();
+			} else {
+				k_loop.template operator()<false>();
+			}
+		}
+		[[maybe_unused]] Acc acc[BN][BM];   // [bn][bm]
+		if constexpr (!BLOCKS16) {
 		X17_UNROLL for (int bn = 0; bn < BN; ++bn) {
 			X17_UNROLL for (int bm = 0; bm < BM; ++bm) {
 				X17_UNROLL for (int r = 0; r < 16; ++r) acc[bn][bm][r] = 0;
@@ -661,22 +873,32 @@ void kernel(
 		}
 		}
 
-	// ---- epilogue.  Lane owns token (32*bm + lane%32) of its wave and raw columns
-	// LANE_COLS*(lane/32) + 16*bn + r of its wave, r = accumulator register index.
-	u32 const row0 = tile_m + wm * gt::WAVE_M + lane % 32;
+		}
+	// ---- epilogue.  Lane owns token (BLOCK*bm + lane%BLOCK) of its wave and raw columns LANE_COLS*(lane/BLOCK) + 16*bn + r
+	// (blocks of 16: 4*bn + r) of its wave, r = accumulator register index.
+	u32 const row0 = tile_m + wm * gt::WAVE_M + lane % gt::BLOCK;
 	u32 const n0 = tile_n + wn * gt::WAVE_N + LANE_COLS * lo.half;
 
-	X17_UNROLL for (int bm = 0; bm < BM; ++bm) {
+	X17_UNROLL for (int bm = 0; bm < (BLOCKS16 ? XB : BM); ++bm) {
 		if constexpr (gt::WAVES_PER_SIMD == 1) {
 			// Accumulators in the second half of the register file (where the vector ALU cannot read them) are copied
 			// out row by row: pinning the later rows where they are keeps the register allocator from copying all
 			// 256 out at once behind the K loop, which leaves no register for anything else.
-			X17_UNROLL for (int later = bm + 1; later < BM; ++later) {
-				X17_UNROLL for (int bn = 0; bn < BN; ++bn) asm volatile("" : "+a"(acc[bn][later]));
+			X17_UNROLL for (int later = bm + 1; later < (BLOCKS16 ? XB : BM); ++later) {
+				X17_UNROLL for (int bn = 0; bn < (BLOCKS16 ? WB : BN); ++bn) {
+					if constexpr (BLOCKS16) asm volatile("" : "+a"(acc16[bn][later]));
+					else asm volatile("" : "+a"(acc[bn][later]));
+				}
 			}
 		}
-		u32 row = row0 + 32 * bm;
+		u32 row = row0 + gt::BLOCK * bm;
 		f32 x[LANE_COLS];
+		if constexpr (BLOCKS16) {
+			X17_UNROLL for (int bn = 0; bn < WB; ++bn) {
+				v4f const as_f32 = __builtin_bit_cast(v4f, acc16[bn][bm]);
+				X17_UNROLL for (int r = 0; r < 4; ++r) x[4 * bn + r] = ACC_F32 ? as_f32[r] : f32(acc16[bn][bm][r]);
+			}
+		} else
 		X17_UNROLL for (int bn = 0; bn < BN; ++bn) {
 			// (bit-casting a single vector element in place reads element 0; cast the whole vector first)
 			v16f const as_f32 = __builtin_bit_cast(v16f, acc[bn][bm]);

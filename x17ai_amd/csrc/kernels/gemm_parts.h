@@ -51,11 +51,14 @@ struct ScaleEpilogue {
 	static constexpr u32 OUT_COLS = N_RAW;
 	X17_DEV static void run(f32 const (&x)[LANE_COLS], u8 *c, u32 row, u32 n, void const *) {
 		u8 *dst = c + (size_t)row * OUT_COLS + n;
+		// (a value of its own: a factor of 1 that folds away lets the compiler start on several rows at once, and it spills)
+		f32 scale = f32(SCALE);
+		asm("" : "+s"(scale));
 		X17_UNROLL for (int v = 0; v < LANE_COLS / 16; ++v) {
 			v4u pack;
 			X17_UNROLL for (int w = 0; w < 4; ++w) {
 				f32 y[4];
-				X17_UNROLL for (int b = 0; b < 4; ++b) y[b] = x[16 * v + 4 * w + b] * f32(SCALE);
+				X17_UNROLL for (int b = 0; b < 4; ++b) y[b] = x[16 * v + 4 * w + b] * scale;
 				pack[w] = pack4_store<STORE>(y[0], y[1], y[2], y[3]);
 			}
 			*reinterpret_cast<v4u *>(dst + 16 * v) = pack;

@@ -63,6 +63,12 @@ constexpr unsigned MAX_BLOCKS = 256;
 // (two workgroups per compute unit when a workgroup has four waves); 128 x 128 waves need all 512.
 constexpr unsigned WAVES_PER_SIMD = (WAVE_M / 32) * (WAVE_N / 32) <= 8 ? 2 : 1;
 
+// Rows of an operand per matrix instruction.  The writers that normalise whole heads (NATURAL) keep the weight rows in order.
+constexpr bool NATURAL = X17_EPILOGUE == 3 || X17_EPILOGUE == 5 || X17_EPILOGUE == 6;
+constexpr bool BLOCKS16 = X17_A_KIND == X17_B_KIND && !NATURAL && STAGES == 2 && X_STAGES == 3 && (X17_A_COLS) / K_STEP >= X_STAGES
+	&& WAVE_N == 128 && (WAVE_M == 64 || WAVE_M == 128) && (X17_A_KIND == 0 || WAVES_PER_SIMD == 1);
+constexpr unsigned BLOCK = BLOCKS16 ? 16 : 32;
+
 // ---- index arithmetic of the tile requests (global -> LDS, 16 bytes per lane).  The kernel calls these; so does the
 // host-side audit (gemm_requests_audit.cpp), which enumerates every request of a launch on the CPU and checks that it
 // stays inside its operand.
@@ -70,26 +76,38 @@ constexpr unsigned WAVES_PER_SIMD = (WAVE_M / 32) * (WAVE_N / 32) <= 8 ? 2 : 1;
 constexpr unsigned CHUNKS = K_STEP / 16;
 constexpr unsigned SWZ_SHIFT = K_STEP == 128 ? 1 : 2;
 constexpr unsigned UNIT_ROWS = 64 / CHUNKS;
+// Chunk c of an LDS row is stored at position c ^ swizzle(row).  The LDS serves a ds_read_b128 sixteen lanes at a time, lanes 0 .. 3,
+// 12 .. 15, 20 .. 23 and 24 .. 27 together (and so on); with blocks of 16 rows the last eight ask for another chunk than
+// the first.  With 128-byte rows the map of a row pair's number keeps their sixteen 16-byte positions apart whichever chunk that is:
+// pairs 0, 1, 6, 7 take keys 0 .. 3, pairs 2 .. 5 keys 4 .. 7.
+constexpr unsigned swizzle(unsigned row) {
+	unsigned const t = (row >> SWZ_SHIFT) & (CHUNKS - 1);
+	return CHUNKS == 8 ? (t & 1) | (t >> 2) << 1 | ((t >> 1 ^ t >> 2) & 1) << 2 : t;
+}
 // With eight waves, two per SIMD, only the first of each pair (waves 0 .. 3) requests tiles.
 constexpr unsigned LOADER_WAVES = WAVES_M * WAVES_N == 8 ? 4 : WAVES_M * WAVES_N;
 constexpr unsigned X_UNITS = M_PER_BLOCK / UNIT_ROWS / LOADER_WAVES;   // load units per loading wave, step and tile
 constexpr unsigned W_UNITS = N_PER_BLOCK / UNIT_ROWS / LOADER_WAVES;
-// The weight row that LDS weight row r0 (a multiple of UNIT_ROWS) starts from.  With WN = WAVE_N columns per wave, LDS
-// weight row R = WN*wn + 32*bn + i holds weight row WN*wn + (WN/2)*((i/4)%2) + 16*bn + 4*(i/8) + i%4 (so that a lane
-// collects consecutive output columns); the head-normalising writers keep the natural order.
+// The weight row that LDS weight row r0 (a multiple of UNIT_ROWS) starts from.  With WN = WAVE_N columns per wave, a lane collects
+// WN / GROUPS consecutive output columns: LDS weight row R = WN*wn + BLOCK*bn + i holds weight row
+//   blocks of 32 (GROUPS = 2: lanes 32 apart)    WN*wn + (WN/2)*((i/4)%2) + 16*bn + 4*(i/8) + i%4
+//   blocks of 16 (GROUPS = 4: lanes 16 apart)    WN*wn + (WN/4)*(i/4) + 4*bn + i%4
+// the head-normalising writers keep the natural order.
+constexpr unsigned GROUPS = 64 / BLOCK;
 constexpr unsigned w_unit_row(unsigned r0, bool natural) {
-	return natural ? r0 : WAVE_N * (r0 / WAVE_N) + 16 * ((r0 % WAVE_N) / 32) + 4 * ((r0 % 32) / 8);
+	return natural ? r0 : WAVE_N * (r0 / WAVE_N) + (BLOCK * BLOCK / 64) * ((r0 % WAVE_N) / BLOCK)
+	                      + (BLOCKS16 ? (WAVE_N / 4) * ((r0 % 16) / 4) : 4 * ((r0 % 32) / 8));
 }
 // Row inside its load unit, as an operand row offset, and 16-byte chunk of the K step that lane `lane` fetches
 // (`odd`: parity of the unit, which shifts the swizzle phase).
 constexpr unsigned x_lane_row(unsigned lane) { return lane / CHUNKS; }
 constexpr unsigned w_lane_row(unsigned lane, bool natural) {
 	unsigned const j = lane / CHUNKS;
-	return natural ? j : (WAVE_N / 2) * ((j >> 2) & 1) + 4 * (j >> 3) + (j & 3);
+	return natural ? j : BLOCKS16 ? (WAVE_N / 4) * (j >> 2) + (j & 3) : (WAVE_N / 2) * ((j >> 2) & 1) + 4 * (j >> 3) + (j & 3);
 }
 constexpr unsigned lane_chunk(unsigned lane, unsigned odd) {
 	unsigned const j = lane / CHUNKS, p = lane % CHUNKS;
-	return p ^ (((odd * UNIT_ROWS + j) >> SWZ_SHIFT) & (CHUNKS - 1));
+	return p ^ swizzle(odd * UNIT_ROWS + j);
 }
 // First token row and first raw column of tile `lin` of the persistent walk: each XCD (the hardware deals workgroups
 // round-robin to 8 of them) gets a contiguous run of tiles, walked in bands of `band` token tiles; a last tile that
