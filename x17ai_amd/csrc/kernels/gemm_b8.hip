@@ -21,8 +21,8 @@
 //     16-byte chunks are XOR-swizzled so that ds_read_b128 is conflict-free.  In the int8 and e4m3 kernels the
 //     issue order of a K step is pinned: each MFMA is followed by its share of the LDS reads and tile requests
 //     (and, in the mixed arithmetic, of the next round's conversions to f16).
-//   * int8: v_mfma_i32_16x16x64_i8.  e4m3 x e4m3: v_mfma_f32_16x16x128_f8f6f4 (with the head-normalising writers and with
-//     fewer than three K steps the 32 x 32 forms of both).  Mixed
+//   * int8: v_mfma_i32_16x16x64_i8.  e4m3 x e4m3: v_mfma_f32_16x16x128_f8f6f4 (with the head-normalising writers, with
+//     fewer than three K steps and for e4m3 below K = 2048 the 32 x 32 forms of both).  Mixed
 //     e4m3 x int8: both widened exactly to f16 in registers, v_mfma_f32_32x32x16_f16
 //     (int8 codes need 7 significand bits, e4m3 has 4; every e4m3 value is a normal f16).
 //   * Workgroup ids are remapped so that each XCD (own L2) works on a compact block of tiles.

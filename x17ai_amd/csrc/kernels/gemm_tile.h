@@ -64,9 +64,12 @@ constexpr unsigned MAX_BLOCKS = 256;
 constexpr unsigned WAVES_PER_SIMD = (WAVE_M / 32) * (WAVE_N / 32) <= 8 ? 2 : 1;
 
 // Rows of an operand per matrix instruction.  The writers that normalise whole heads (NATURAL) keep the weight rows in order.
+// e4m3 takes blocks of 16 from K = 2048 on: below, the accumulators' way to the writer costs more than the K loop gains (GeGLU writer,
+// 4096 columns, 16384 rows, us, blocks of 32 / of 16: K = 384 37.4 / 39.9, 512 41.6 / 44.4, 1024 66.0 / 66.7, 2048 111.3 / 108.9).
+// int8 gains at every K (scale writer: K = 384 41.0 / 34.9, 1024 77 / 63; GeGLU, K = 512 42.2 / 41.9, 1024 69.9 / 63.7).
 constexpr bool NATURAL = X17_EPILOGUE == 3 || X17_EPILOGUE == 5 || X17_EPILOGUE == 6;
 constexpr bool BLOCKS16 = X17_A_KIND == X17_B_KIND && !NATURAL && STAGES == 2 && X_STAGES == 3 && (X17_A_COLS) / K_STEP >= X_STAGES
-	&& WAVE_N == 128 && (WAVE_M == 64 || WAVE_M == 128) && (X17_A_KIND == 0 || WAVES_PER_SIMD == 1);
+	&& WAVE_N == 128 && (WAVE_M == 64 || WAVE_M == 128) && (X17_A_KIND == 0 || (WAVES_PER_SIMD == 1 && (X17_A_COLS) >= 2048));
 constexpr unsigned BLOCK = BLOCKS16 ? 16 : 32;
 
 // ---- index arithmetic of the tile requests (global -> LDS, 16 bytes per lane).  The kernel calls these; so does the
