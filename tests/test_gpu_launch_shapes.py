@@ -123,6 +123,8 @@ GEMM_FORMS = [
 	("mixed", lambda: recipes.mixed_gemm_kernel(None, 512, 384, False), 512, 384),
 	("mixed_residual", lambda: recipes.ffn_y_kernel(None, 128, 512, True, X.E4M3, X.INT8), 512, 256),
 	("e4m3", lambda: recipes.ffn_f_f8_kernel(None, 512, 256, True), 512, 256),
+	# (the least K whose 256 x 256 tiles are blocks of 16 x 16, and an overhanging column tile)
+	("e4m3", lambda: recipes.ffn_f_f8_kernel(None, 2048, 384, True), 2048, 384),
 	("one_step", lambda: recipes.attn_q_kernel(None, 128, 256), 128, 256),
 ]
 

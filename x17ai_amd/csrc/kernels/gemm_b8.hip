@@ -76,6 +76,11 @@ constexpr u32 K_STEPS = K_TOTAL / gt::K_STEP;
 constexpr u32 WAVES = gt::WAVES_M * gt::WAVES_N;
 
 constexpr bool BLOCKS16 = gt::BLOCKS16;
+#if X17_EPILOGUE == 3 || X17_EPILOGUE == 5 || X17_EPILOGUE == 6
+template <bool> struct NaturalOf { using Writers = NaturalWriters; };
+template <> struct NaturalOf<true> { using Writers = NaturalWriters16; };
+using Natural = NaturalOf<BLOCKS16>::Writers;
+#endif
 constexpr int XB = gt::WAVE_M / 16, WB = gt::WAVE_N / 16, WH = WB / 2;      // blocks of 16 tokens, of 16 columns, of half the columns
 constexpr u32 CH = MMA == 1 ? 2 : 1;                         // 16-byte chunks a lane fetches per operand row
 constexpr u32 SLICES16 = gt::K_STEP / (64 * CH);             // slices of a K step
@@ -876,8 +881,16 @@ void kernel(
 		}
 	// ---- epilogue.  Lane owns token (BLOCK*bm + lane%BLOCK) of its wave and raw columns LANE_COLS*(lane/BLOCK) + 16*bn + r
 	// (blocks of 16: 4*bn + r) of its wave, r = accumulator register index.
-	u32 const row0 = tile_m + wm * gt::WAVE_M + lane % gt::BLOCK;
-	u32 const n0 = tile_n + wn * gt::WAVE_N + LANE_COLS * lo.half;
+	u32 here = lane;
+	if constexpr (BLOCKS16 && gt::NATURAL) {
+		// (asked for anew: what these writers derive from the lane would live through the K loop, and spills)
+		u32 every = ~0u;
+		asm volatile("" : "+s"(every));
+		here = __builtin_amdgcn_mbcnt_hi(every, __builtin_amdgcn_mbcnt_lo(every, 0));
+	}
+	u32 const part = here / gt::BLOCK;
+	u32 const row0 = tile_m + wm * gt::WAVE_M + here % gt::BLOCK;
+	u32 const n0 = tile_n + wn * gt::WAVE_N + LANE_COLS * part;
 
 	X17_UNROLL for (int bm = 0; bm < (BLOCKS16 ? XB : BM); ++bm) {
 		if constexpr (gt::WAVES_PER_SIMD == 1) {
@@ -919,19 +932,11 @@ void kernel(
 #elif X17_EPILOGUE == 4
 		DequantEpilogue::run(x, c, row, n0, row_scale, col_scale);
 #elif X17_EPILOGUE == 3
-		NaturalWriters::l2norm_row(x, c, rrms, row, tile_n + wn * gt::WAVE_N, N_RAW, lo.half);
+		Natural::l2norm_row(x, c, rrms, row, tile_n + wn * gt::WAVE_N, N_RAW, part);
 #elif X17_EPILOGUE == 5
-		NaturalWriters::qnorm_row(x, c, q_norm_scales, row, tile_n + wn * gt::WAVE_N, lo.half);
+		Natural::qnorm_row(x, c, q_norm_scales, row, tile_n + wn * gt::WAVE_N, part);
 #else
-		{
-			constexpr u32 Q_COLS = X17_Q_COLS;
-			u32 const col0 = tile_n + wn * gt::WAVE_N;
-			if (col0 < Q_COLS) {
-				NaturalWriters::scale_row(x, c, row, col0, Q_COLS, lo.half);
-			} else {
-				NaturalWriters::l2norm_row(x, c_kv, rrms, row, col0 - Q_COLS, N_RAW - Q_COLS, lo.half);
-			}
-		}
+		Natural::qkv_row(x, c, c_kv, rrms, row, tile_n + wn * gt::WAVE_N, part);
 #endif
 	}
 

@@ -14,8 +14,8 @@ constexpr int A_KIND = X17_A_KIND;
 constexpr int B_KIND = X17_B_KIND;
 constexpr int STORE = X17_STORE;
 
-// The writers that normalise whole heads (and the fused q + kv kernel, which contains one) keep the weight rows in
-// their natural order: a lane then owns, of every 32-column block, the columns whose (column % 8) / 4 equals
+// The writers that normalise whole heads (and the fused q + kv kernel, which contains one) keep the weight rows, in blocks
+// of 32, in their natural order (blocks of 16: NaturalWriters16): a lane then owns, of every 32-column block, the columns whose (column % 8) / 4 equals
 // lane / 32 -- exactly two of the reference's four partial sums of squares (cuda/gemm_b8.cuh:789-801), so a head's
 // sum needs one exchange between the lanes of a pair whatever its width.  Every other writer takes 64 consecutive
 // columns per lane (pairs and 16-byte output vectors stay inside a lane).
@@ -221,7 +221,7 @@ struct DequantEpilogue {
 // For ONE token row a lane holds x[16 * b + r] = raw column 32 * b + 8 * (r / 4) + 4 * (lane / 32) + r % 4 of its
 // wave's 128 columns (b = 32-column block, r = accumulator register).
 #if X17_EPILOGUE == 3 || X17_EPILOGUE == 5 || X17_EPILOGUE == 6
-static_assert(LANE_COLS == 64, "the head-normalising writers are written for 128-column waves");
+static_assert(LANE_COLS == 64 || LANE_COLS == 32, "the head-normalising writers are written for 128-column waves");
 constexpr u32 HEAD_DIM = X17_HEAD_DIM;
 static_assert(HEAD_DIM == 32 || HEAD_DIM == 64 || HEAD_DIM == 128, "head_dim must be 32, 64 or 128");
 struct NaturalWriters {
@@ -344,6 +344,123 @@ struct NaturalWriters {
 	X17_DEV static void scale_row(f32 const (&x)[64], u8 *c, u32 row, u32 col0, u32 q_cols, u32 half) {
 		u8 *dst = c + (size_t)row * q_cols + col0;
 		X17_UNROLL for (int b = 0; b < 4; ++b) emit_block<false>(x, b, f32(f64(X17_Q_SCALE)), dst, nullptr, half);
+	}
+	X17_DEV static void qkv_row(f32 const (&x)[64], u8 *c, u8 *c_kv, f32 *rrms, u32 row, u32 col0, u32 half) {
+		constexpr u32 Q_COLS = X17_Q_COLS;
+		if (col0 < Q_COLS) {
+			scale_row(x, c, row, col0, Q_COLS, half);
+		} else {
+			l2norm_row(x, c_kv, rrms, row, col0 - Q_COLS, N_RAW - Q_COLS, half);
+		}
+	}
+#endif
+};
+
+// The same writers for blocks of 16 x 16: lane group g (lane / 16) holds x[4 * bn + r] = raw column 16 * bn + 8 * (r / 2) + 2 * g + r % 2 of
+// its token row, which is the reference's partial sum g of every head, in its order.
+struct NaturalWriters16 {
+	static constexpr int HB = HEAD_DIM / 32;
+	// (a scale in a register of its own: see ScaleEpilogue)
+	X17_DEV static f32 opaque(f32 v) {
+		asm("" : "+s"(v));
+		return v;
+	}
+	// the sum over the four lanes of a row: (0 + 1) + (2 + 3)
+	X17_DEV static f32 over_groups(f32 v) {
+		auto const a = __builtin_amdgcn_permlane16_swap(f2u(v), f2u(v), false, false);
+		f32 const pair = u2f(a[0]) + u2f(a[1]);
+		auto const b = __builtin_amdgcn_permlane32_swap(f2u(pair), f2u(pair), false, false);
+		return u2f(b[0]) + u2f(b[1]);
+	}
+	// kv_helpers::l2_norm, cuda/gemm_b8.cuh:767-830, of the head made of 32-column blocks [B0, B0 + HB)
+	template <int B0>
+	X17_DEV static f32 head_scale(f32 const (&x)[32]) {
+		f32 p = 0.0f;
+		X17_UNROLL for (int i = 8 * B0; i < 8 * (B0 + HB); ++i) p = fmaf32(x[i], x[i], p);
+		return strict::rsq(over_groups(p) + NaturalWriters::EPS) * NaturalWriters::HEAD_SCALE;
+	}
+	// The row times `scale` per 32-column block (and, with learned scales, as in NaturalWriters::emit_block) -> FixedI8.  A lane's words hold
+	// two columns of every eight: an exchange of words between the four lanes gives each the 32 bytes of one block.
+	template <bool DYN>
+	X17_DEV static void emit(f32 const (&x)[32], f32 const (&scale)[4], u8 *dst, u16 const *dyn, u32 group) {
+		u32 w[8];
+		X17_UNROLL for (int bn = 0; bn < 8; ++bn) {
+			f32 y[4];
+			X17_UNROLL for (int e = 0; e < 4; ++e) y[e] = x[4 * bn + e] * scale[bn / 2];
+			if constexpr (DYN) {
+				X17_UNROLL for (int h = 0; h < 2; ++h) {
+					u32 const d = *reinterpret_cast<u32 const *>(dyn + 16 * bn + 8 * h + 2 * group);
+					y[2 * h] = y[2 * h] * u2f(d << 16);
+					y[2 * h + 1] = y[2 * h + 1] * u2f(d & 0xFFFF0000u);
+				}
+				if constexpr (f32(f64(X17_INP_SCALE)) != 1.0f) {
+					X17_UNROLL for (int e = 0; e < 4; ++e) y[e] = y[e] * f32(f64(X17_INP_SCALE));
+				}
+			}
+			w[bn] = pack4_fixedi8(y[0], y[1], y[2], y[3]);
+		}
+		X17_UNROLL for (int e = 0; e < 2; ++e) {
+			auto const even = __builtin_amdgcn_permlane32_swap(w[e], w[4 + e], false, false);
+			auto const odd = __builtin_amdgcn_permlane32_swap(w[2 + e], w[6 + e], false, false);
+			auto const t01 = __builtin_amdgcn_permlane16_swap(even[0], odd[0], false, false);      // word 2 * group + e of lane groups 0, 1
+			auto const t23 = __builtin_amdgcn_permlane16_swap(even[1], odd[1], false, false);      // of lane groups 2, 3
+			*reinterpret_cast<v4u *>(dst + 32 * group + 16 * e) = v4u{
+				__builtin_amdgcn_perm(t01[1], t01[0], 0x05040100u), __builtin_amdgcn_perm(t23[1], t23[0], 0x05040100u),
+				__builtin_amdgcn_perm(t01[1], t01[0], 0x07060302u), __builtin_amdgcn_perm(t23[1], t23[0], 0x07060302u)};
+		}
+	}
+#if X17_EPILOGUE == 3 || X17_EPILOGUE == 6
+	// the scales of the K heads among the columns, whose first is column col0 of the kv matrix
+	X17_DEV static void key_scales(f32 const (&x)[32], f32 (&scale)[4], f32 *rrms, u32 row, u32 col0, u32 kv_cols, u32 group) {
+		f32 *rr = rrms + (size_t)row * (kv_cols / (2 * HEAD_DIM));
+		if constexpr (HEAD_DIM == 32) {
+			scale[0] = head_scale<0>(x);
+			scale[2] = head_scale<2>(x);
+			if (group == 0) {
+				rr[col0 / 64] = scale[0];
+				rr[col0 / 64 + 1] = scale[2];
+			}
+		} else if (HEAD_DIM == 64 || (col0 / 128) % 2 == 0) {       // (head_dim 128: the wave's columns are K or V of one head)
+			scale[0] = head_scale<0>(x);
+			X17_UNROLL for (int b = 1; b < HB; ++b) scale[b] = scale[0];
+			if (group == 0) rr[col0 / (2 * HEAD_DIM)] = scale[0];
+		}
+	}
+	X17_DEV static void l2norm_row(f32 const (&x)[32], u8 *c, f32 *rrms, u32 row, u32 col0, u32 kv_cols, u32 group) {
+		f32 const sep = opaque(NaturalWriters::SEP_SCALE);
+		f32 scale[4] = {sep, sep, sep, sep};
+		key_scales(x, scale, rrms, row, col0, kv_cols, group);
+		emit<false>(x, scale, c + (size_t)row * kv_cols + col0, nullptr, group);
+	}
+#endif
+#if X17_EPILOGUE == 5
+	X17_DEV static void qnorm_row(f32 const (&x)[32], u8 *c, u16 const *dyn, u32 row, u32 col0, u32 group) {
+		f32 scale[4];
+		scale[0] = head_scale<0>(x);
+		if constexpr (HB == 4) {
+			scale[1] = scale[2] = scale[3] = scale[0];
+		} else {
+			scale[2] = head_scale<2>(x);
+			if constexpr (HB == 2) {
+				scale[1] = scale[0];
+				scale[3] = scale[2];
+			} else {
+				scale[1] = head_scale<1>(x);
+				scale[3] = head_scale<3>(x);
+			}
+		}
+		emit<true>(x, scale, c + (size_t)row * N_RAW + col0, dyn + col0, group);
+	}
+#endif
+#if X17_EPILOGUE == 6
+	// q columns or kv columns of the fused kernel: one copy of the writer (two spill)
+	X17_DEV static void qkv_row(f32 const (&x)[32], u8 *c, u8 *c_kv, f32 *rrms, u32 row, u32 col0, u32 group) {
+		constexpr u32 Q_COLS = X17_Q_COLS, KV_COLS = N_RAW - Q_COLS;
+		bool const q = col0 < Q_COLS;
+		f32 const all = opaque(q ? f32(f64(X17_Q_SCALE)) : NaturalWriters::SEP_SCALE);
+		f32 scale[4] = {all, all, all, all};
+		if (!q) key_scales(x, scale, rrms, row, col0 - Q_COLS, KV_COLS, group);
+		emit<false>(x, scale, q ? c + (size_t)row * Q_COLS + col0 : c_kv + (size_t)row * KV_COLS + (col0 - Q_COLS), nullptr, group);
 	}
 #endif
 };

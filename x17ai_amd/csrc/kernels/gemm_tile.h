@@ -63,12 +63,19 @@ constexpr unsigned MAX_BLOCKS = 256;
 // (two workgroups per compute unit when a workgroup has four waves); 128 x 128 waves need all 512.
 constexpr unsigned WAVES_PER_SIMD = (WAVE_M / 32) * (WAVE_N / 32) <= 8 ? 2 : 1;
 
-// Rows of an operand per matrix instruction.  The writers that normalise whole heads (NATURAL) keep the weight rows in order.
+// Rows of an operand per matrix instruction.  NATURAL: the writers that normalise whole heads, with an order of the weight rows of their own.
 // e4m3 takes blocks of 16 from K = 2048 on: below, the accumulators' way to the writer costs more than the K loop gains (GeGLU writer,
 // 4096 columns, 16384 rows, us, blocks of 32 / of 16: K = 384 37.4 / 39.9, 512 41.6 / 44.4, 1024 66.0 / 66.7, 2048 111.3 / 108.9).
-// int8 gains at every K (scale writer: K = 384 41.0 / 34.9, 1024 77 / 63; GeGLU, K = 512 42.2 / 41.9, 1024 69.9 / 63.7).
+// The kv writer with heads of 32 columns keeps blocks of 32: with blocks of 16 one or two of its registers spill.
+// int8 gains at every K (scale writer: K = 384 41.0 / 34.9, 1024 77 / 63; GeGLU, K = 512 42.2 / 41.9, 1024 69.9 / 63.7;
+// q + kv, K = 2048, 6144 columns, 3264 rows 48.6 / 46.4, 32768 rows 325 / 304; kv alone, 4096 columns, K = 512 43.5 / 42.8, 2048 118 / 111).
 constexpr bool NATURAL = X17_EPILOGUE == 3 || X17_EPILOGUE == 5 || X17_EPILOGUE == 6;
-constexpr bool BLOCKS16 = X17_A_KIND == X17_B_KIND && !NATURAL && STAGES == 2 && X_STAGES == 3 && (X17_A_COLS) / K_STEP >= X_STAGES
+#if X17_EPILOGUE == 3
+constexpr bool SPILLS16 = X17_HEAD_DIM == 32;
+#else
+constexpr bool SPILLS16 = false;
+#endif
+constexpr bool BLOCKS16 = X17_A_KIND == X17_B_KIND && !SPILLS16 && STAGES == 2 && X_STAGES == 3 && (X17_A_COLS) / K_STEP >= X_STAGES
 	&& WAVE_N == 128 && (WAVE_M == 64 || WAVE_M == 128) && (X17_A_KIND == 0 || (WAVES_PER_SIMD == 1 && (X17_A_COLS) >= 2048));
 constexpr unsigned BLOCK = BLOCKS16 ? 16 : 32;
 
@@ -95,9 +102,11 @@ constexpr unsigned W_UNITS = N_PER_BLOCK / UNIT_ROWS / LOADER_WAVES;
 // WN / GROUPS consecutive output columns: LDS weight row R = WN*wn + BLOCK*bn + i holds weight row
 //   blocks of 32 (GROUPS = 2: lanes 32 apart)    WN*wn + (WN/2)*((i/4)%2) + 16*bn + 4*(i/8) + i%4
 //   blocks of 16 (GROUPS = 4: lanes 16 apart)    WN*wn + (WN/4)*(i/4) + 4*bn + i%4
-// the head-normalising writers keep the natural order.
+// The head-normalising writers keep the natural order in blocks of 32, and in blocks of 16 take
+//   16*bn + 8*((i%4)/2) + 2*(i/4) + i%2     of a wave's columns: lane group i/4 holds those with (column % 8) / 2 == i / 4.
 constexpr unsigned GROUPS = 64 / BLOCK;
 constexpr unsigned w_unit_row(unsigned r0, bool natural) {
+	if (natural && BLOCKS16) return r0 / 16 * 16 + 2 * (r0 % 16 / 4);
 	return natural ? r0 : WAVE_N * (r0 / WAVE_N) + (BLOCK * BLOCK / 64) * ((r0 % WAVE_N) / BLOCK)
 	                      + (BLOCKS16 ? (WAVE_N / 4) * ((r0 % 16) / 4) : 4 * ((r0 % 32) / 8));
 }
@@ -106,6 +115,7 @@ constexpr unsigned w_unit_row(unsigned r0, bool natural) {
 constexpr unsigned x_lane_row(unsigned lane) { return lane / CHUNKS; }
 constexpr unsigned w_lane_row(unsigned lane, bool natural) {
 	unsigned const j = lane / CHUNKS;
+	if (natural && BLOCKS16) return 8 * ((j & 3) / 2) + 2 * (j >> 2) + (j & 1);
 	return natural ? j : BLOCKS16 ? (WAVE_N / 4) * (j >> 2) + (j & 3) : (WAVE_N / 2) * ((j >> 2) & 1) + 4 * (j >> 3) + (j & 3);
 }
 constexpr unsigned lane_chunk(unsigned lane, unsigned odd) {
