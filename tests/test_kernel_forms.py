@@ -47,7 +47,10 @@ def test_forms_of_a_kernel_pass_the_code_object_scans(tmp_path):
 	(lambda: recipes.attn_kv_kernel(None, 256, 2048, 64), {256: "s64x4", 8192: "", 262144: ""}),
 	# (a short product of e4m3 operands is faster in small tiles at any size: 16384 x 4096, K = 256: 46 us and 63)
 	(lambda: recipes.ffn_f_f8_kernel(None, 384, 512, True), {256: "s128x2", 131072: "s128x2"}),
-], ids=["int8", "int8, past a round", "e4m3 x int8", "e4m3", "int8, short K", "L2 norm, short K", "e4m3, short K"])
+	# behind the first round of 256 x 256 tiles
+	(lambda: recipes.ffn_f_f8_kernel(None, 4096, 32768, False), {320: "", 640: ""}),
+	(lambda: recipes.ffn_f_kernel(None, 2048, 16384, False, X.E4M3), {1088: "", 2048: ""}),
+], ids=["int8", "int8, past a round", "e4m3 x int8", "e4m3", "int8, short K", "L2 norm, short K", "e4m3, short K", "e4m3, second round", "int8, second round"])
 def test_the_form_a_launch_takes(make, picks):
 	kernel = make()
 	assert {rows: kernel.form(rows) for rows in picks} == picks

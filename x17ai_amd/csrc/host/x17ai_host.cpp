@@ -1080,14 +1080,17 @@ Status GemmKernel::launch(GemmArgs const &args) {
 // Estimated microseconds of a launch: measured curves over the number of its tiles, in units of the 256 compute units,
 // each point fixed + per_k * K / 1024 (K in bytes) and straight lines between them.  Two points close behind each other
 // (1 and 1.02 rounds) are the step where one tile more begins another round: the 256 x 256 kernel at K = 2048 and 4096
-// columns takes 35 us at 4096 rows and 48 at 4160, the two-stage 128 x 128 one 41 and 48.  Fitted on an MI355X to 1721
+// columns takes 30 us at 4096 rows and 45 at 4160, the two-stage 128 x 128 one 41 and 48.  Fitted on an MI355X to 1721
 // launches of 256 .. 65536 token rows, 1024 .. 32768 columns and K = 128 .. 16384, row counts just past a round among them,
 // below 4096 rows with weights that no cache holds (the next layer's: the two-stage 128 x 128 form, ahead with weights in
 // L2, loses to four stages there: 256 rows, K = 2048, 8.4 / 8.7 us and 16 / 12).  A fit is 3-10 % off in the mean of a curve
 // and up to 40 % at single points; over those launches the form taken is 0.3 % slower than the best one in the mean (16 % at
 // most), over 460 of other widths 0.6 % (36 %).  The four-stage forms have become 0-10 % faster since: over 535 launches of
-// the present code (256 .. 4096 rows, K = 512 .. 16384, ten writers, weights from memory) the form taken is 0.2 % slower than
-// the best one (18 % at most), so the curves stand.  us measured at 4096 columns:
+// that code (256 .. 4096 rows, K = 512 .. 16384, ten writers, weights from memory) the form taken is 0.2 % slower than
+// the best one (18 % at most).  The 256 x 256 kernel of int8 and of e4m3 has become 3-18 % faster since (blocks of 16 x 16): from the second
+// round on its curves are 6 % lower than the fits.  Over 59 launches of the present code near the lines (512 .. 12288 rows, weights from memory) the form taken is 0.2 % slower than
+// the best one (5 % at most; the fits 0.9 %, 13 %), over 44 others 0.5 % (12 %; 1.5 %, 17 %): e4m3, K = 4096, 32768 columns, 640 rows 107 -> 95 us,
+// int8 GeGLU, 16384 columns, 1088 rows 56 -> 50.  us measured at 4096 columns, 256 x 256 by the fitted code:
 //                        rows:  256    512   1024   2048   4096   8192
 //   int8, K = 2048   64 x 64    8.1   14.1   27.1   56.2    107    215
 //           128 x 128, 4 / 2   12/16  12/16  13/16  26/22  48/41  95/78
@@ -1115,7 +1118,7 @@ namespace gemm_cost {
 	struct Curves { Curve large, tile64, tile128_deep, tile128; };   // 256 x 256 | 64 x 64 | 128 x 128, four stages | two
 	static Curves const CURVES[5] = {
 		{   // int8
-			{{{0.125, 4.9, 7.5}, {0.5, 6.6, 8.3}, {1, 8.7, 12.5}, {1.02, 10.5, 18.2}, {2, 13.9, 23.5}, {2.02, 15.4, 30.0}, {3, 16.6, 35.7}}, 0.3},
+			{{{0.125, 4.9, 7.5}, {0.5, 6.6, 8.3}, {1, 8.7, 12.5}, {1.02, 10.5, 18.2}, {2, 13.1, 22.1}, {2.02, 14.5, 28.2}, {3, 15.6, 33.6}}, 0.3},
 			{{{0.25, 3.5, 1.1}, {1, 3.5, 1.6}, {1.02, 5.3, 2.7}, {2, 5.7, 4.6}, {4, 7.9, 8.6}}},
 			{{{0.25, 3.6, 2.7}, {1, 3.7, 4.2}, {1.02, 6.0, 6.3}, {2, 6.0, 9.1}, {2.02, 8.2, 10.1}, {4, 10.3, 17.0}, {4.02, 12.8, 17.4}, {6, 14.2, 25.1}}},
 			{{{0.25, 3.0, 4.3}, {1, 3.3, 5.7}, {1.02, 4.3, 5.1}, {2, 4.2, 8.3}, {2.02, 5.7, 10.9}, {4, 7.1, 15.3}, {4.02, 8.2, 18.1}, {6, 8.6, 23.5}}},
@@ -1127,7 +1130,7 @@ namespace gemm_cost {
 			{{{0.25, 4.2, 4.2}, {1, 3.9, 6.6}, {1.02, 5.2, 5.4}, {2, 5.1, 8.5}, {2.02, 7.4, 11.1}, {4, 7.5, 17.2}, {4.02, 10.4, 18.1}, {6, 11.3, 24.2}}},
 		},
 		{   // e4m3 x e4m3
-			{{{0.125, 9.7, 7.7}, {0.5, 12.5, 8.2}, {1, 18.7, 10.5}, {1.02, 23.6, 17.1}, {2, 28.6, 21.0}, {2.02, 36.9, 27.4}, {3, 36.0, 33.9}}, 0.3},
+			{{{0.125, 9.7, 7.7}, {0.5, 12.5, 8.2}, {1, 18.7, 10.5}, {1.02, 23.6, 17.1}, {2, 26.9, 19.7}, {2.02, 34.7, 25.8}, {3, 33.8, 31.9}}, 0.3},
 			{{{0.25, 3.7, 1.1}, {1, 3.6, 1.6}, {1.02, 4.5, 3.0}, {2, 5.0, 4.7}, {4, 6.3, 9.0}}},
 			{{{0.25, 3.9, 3.0}, {1, 4.3, 4.6}, {1.02, 6.9, 6.6}, {2, 6.5, 8.9}, {2.02, 9.4, 10.5}, {4, 11.5, 17.2}, {4.02, 14.1, 18.5}, {6, 17.2, 26.4}}},
 			{{{0.25, 3.3, 4.5}, {1, 3.5, 6.6}, {1.02, 5.0, 5.7}, {2, 5.8, 8.1}, {2.02, 6.8, 11.1}, {4, 8.7, 16.2}, {4.02, 10.4, 18.3}, {6, 12.0, 24.6}}},
