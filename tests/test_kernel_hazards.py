@@ -90,3 +90,19 @@ def test_the_scan_sees_a_hazard_when_there_is_one():
 	assert len(_m0_hazards(["s_mov_b32 m0, s8", "global_load_lds_dwordx4 v122, s[20:21]"])) == 1
 	assert _m0_hazards(["s_mov_b32 m0, s8", "s_nop 0", "global_load_lds_dwordx4 v122, s[20:21]"]) == []
 	assert _m0_hazards(["s_add_i32 m0, s8, 0x1000", "v_add_u32_e32 v1, v2, v3", "global_load_lds_dwordx4 v122, s[20:21]"]) == []
+
+
+def test_every_barrier_is_a_compiler_fence():
+	"""__builtin_amdgcn_s_barrier orders no memory access for the compiler: it stands between clobbers in step_barrier, and
+	nowhere else (__syncthreads brings fences of its own)."""
+	kernels = os.path.join(os.path.dirname(os.path.abspath(recipes.__file__)), "csrc", "kernels")
+	barriers = {}
+	for path in glob.glob(os.path.join(kernels, "*.h")) + glob.glob(os.path.join(kernels, "*.hip")):
+		with open(path) as f:
+			text = f.read()
+		if "amdgcn_s_barrier" in text:
+			barriers[os.path.basename(path)] = text
+	assert list(barriers) == ["x17_device.h"]
+	clobber = r'asm volatile\("" ::: "memory"\);\n'
+	fenced = re.compile(r"void step_barrier\(\) \{\n\t" + clobber + r"\t__builtin_amdgcn_s_waitcnt\(0xC07F\);[^\n]*\n\t__builtin_amdgcn_s_barrier\(\);\n\t" + clobber)
+	assert len(fenced.findall(barriers["x17_device.h"])) == 1 and barriers["x17_device.h"].count("amdgcn_s_barrier") == 1

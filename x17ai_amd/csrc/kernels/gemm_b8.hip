@@ -591,7 +591,7 @@ void kernel(
 			issue_x_loads(a_tile, smem + WS * X_TILE_BYTES, WS * gt::K_STEP, wave, lo);
 		}
 		wait_vmcnt<0>();
-		__builtin_amdgcn_s_barrier();
+		step_barrier();
 	};
 	prologue();
 
@@ -608,8 +608,7 @@ void kernel(
 		u8 const *b_next = weight_tile(next_n);
 		if constexpr (!CROSS_TILE) {
 			if (!first_tile) {
-				__builtin_amdgcn_s_waitcnt(0xC07F);        // lgkmcnt(0)
-				__builtin_amdgcn_s_barrier();              // nobody still reads the previous tile's buffers
+				step_barrier();      // nobody still reads the previous tile's buffers
 				xb = 0;
 				wb = 0;
 				prologue();
@@ -699,8 +698,7 @@ void kernel(
 							// the next step's tiles have landed once all but the token tile just requested have; this wave is done
 							// reading this step's tiles
 							wait_vmcnt<X_UNITS>();
-							__builtin_amdgcn_s_waitcnt(0xC07F);
-							__builtin_amdgcn_s_barrier();
+							step_barrier();
 							paced16<Q, 0, !LAST_STEP, LOADER ? 2 : 0, 0, W_UNITS>(f, next.w_tile, next.x_tile, lo, acc16, w_rows, now.w_lds, nothing);
 						}
 					};
@@ -713,6 +711,13 @@ void kernel(
 					now = next;
 				}
 				step.template operator()<true>(K_STEPS - 1);
+				if constexpr (gt::NATURAL) {
+					// (one register each where the loading wavefronts' loop and the others' meet: with places of their own in either, up to
+					// eight spill in the q + kv writer at head_dim 64)
+					X17_UNROLL for (int bn = 0; bn < WB; ++bn) {
+						X17_UNROLL for (int bm = 0; bm < XB; ++bm) asm volatile("" : "+v"(acc16[bn][bm]));
+					}
+				}
 				xb = next_xb;
 				wb = next_wb;
 			};
@@ -775,8 +780,7 @@ void kernel(
 						u32 const k0 = LAST ? w_k0 : x_k0;
 						if constexpr (LAST) {
 							wait_vmcnt<X_UNITS>();
-							__builtin_amdgcn_s_waitcnt(0xC07F);
-							__builtin_amdgcn_s_barrier();
+							step_barrier();
 							// (the same code in a tile's last step, where what it reads and widens is never used: two
 							// copies of the rounds would have to agree on where 256 accumulators live when they meet)
 							mixed_round<0, 1, true, 0, 0, 0>(wide[0], wide[1], frags[S & 1], frags[(S + 1) & 1], nw_tile, nx_tile, 0, lo, acc, src, dst, k0, wave);
@@ -795,8 +799,7 @@ void kernel(
 						// the next step's tiles have landed once all but the token tile just requested have;
 						// this wave is done reading this step's tiles
 						wait_vmcnt<X_UNITS>();
-						__builtin_amdgcn_s_waitcnt(0xC07F);
-						__builtin_amdgcn_s_barrier();
+						step_barrier();
 						constexpr int KIND = LOADER ? 2 : 0;
 						if (ks + 1 < K_STEPS) {
 							paced_slice<0, true, KIND, 0, W_UNITS>(
@@ -850,8 +853,7 @@ void kernel(
 					} else {
 						wait_step(later_steps, token_tile_behind);
 					}
-					__builtin_amdgcn_s_waitcnt(0xC07F);    // lgkmcnt(0): this wave is done reading this step's tiles
-					__builtin_amdgcn_s_barrier();
+					step_barrier();      // this wave is done reading this step's tiles
 					if (w_here || has_next) {
 						issue_w_loads(lw, smem + W_RING_OFFSET + wb * W_TILE_BYTES, w_k0, wave, lo);
 					}

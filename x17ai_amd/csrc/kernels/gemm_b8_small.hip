@@ -72,15 +72,6 @@ constexpr u32 GROUP_BYTES = BLOCKS * (gt::WAVES_K - 1) * BLOCK_BYTES;
 X17_DEV u32 exchange_offset(int j, u32 from) { return (j * (gt::WAVES_K - 1) + (from < owner(j) ? from : from - 1)) * BLOCK_BYTES; }
 static_assert(gt::WAVES / gt::WAVES_K * GROUP_BYTES <= gt::SMEM_BYTES, "the exchange fits the ring");
 
-// The barrier of a K step, behind this wavefront's LDS reads and writes.  (The builtins order no memory access for the compiler:
-// the clobbers keep the step's reads behind the barrier and the last one's in front of it.)
-X17_DEV void step_barrier() {
-	asm volatile("" ::: "memory");
-	__builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0)
-	__builtin_amdgcn_s_barrier();
-	asm volatile("" ::: "memory");
-}
-
 // The widening form's second half of a workgroup: weights from memory into registers, WIDENER_DEPTH K steps ahead, and from
 // there as f16 into the tile behind the one the matrix wavefronts are at, widened one step before that.  Past the
 // end the last step is loaded again, into tiles nobody reads any more.
@@ -285,8 +276,7 @@ void kernel(
 	wait_vmcnt<0>();
 	u8 *const exchange = smem + (wave / gt::WAVES_K) * GROUP_BYTES + lane * 16;
 	if constexpr (gt::WAVES_K > 1) {
-		__builtin_amdgcn_s_waitcnt(0xC07F);
-		__builtin_amdgcn_s_barrier();
+		step_barrier();
 		X17_UNROLL for (int j = 0; j < BLOCKS; ++j) {
 			if (owner(j) != wk) {
 				X17_UNROLL for (int q = 0; q < 4; ++q) {

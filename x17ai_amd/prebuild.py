@@ -57,6 +57,7 @@ def _specs():
 		add(("dequant", 512, 384, INT8, INT8, geglu, True))
 	add(("attn_q_norm", 512, 384, 64, 0.0))
 	add(("attn_qkv", 512, 256, 384, 64, True))
+	add(("attn_qkv", 384, 256, 384, 64, True))       # (the fullest registers of its kernel's forms: scanned for spills)
 	add(("attn_q", 384, 1024))           # the shortest K with the deeper token ring, more tiles than workgroups
 	add(("ffn_f_f8", 384, 512, True))
 	# ---- tests/test_gpu_attn.py
