@@ -978,6 +978,7 @@ std::unique_ptr<GemmKernel> GemmKernel::create(std::shared_ptr<HipDevice> device
 	out->name = kernel_name;
 	out->files = *built;
 	out->epilogue_kind = kind;
+	out->blocks_of_16 = get("BLOCK") == 16;
 	out->a_cols = g.a.cols;
 	out->b_rows = g.b.rows;
 	out->a_dtype = g.a.dtype;
@@ -1080,17 +1081,14 @@ Status GemmKernel::launch(GemmArgs const &args) {
 // Estimated microseconds of a launch: measured curves over the number of its tiles, in units of the 256 compute units,
 // each point fixed + per_k * K / 1024 (K in bytes) and straight lines between them.  Two points close behind each other
 // (1 and 1.02 rounds) are the step where one tile more begins another round: the 256 x 256 kernel at K = 2048 and 4096
-// columns takes 30 us at 4096 rows and 45 at 4160, the two-stage 128 x 128 one 41 and 48.  Fitted on an MI355X to 1721
+// columns takes 35 us at 4096 rows and 48 at 4160, the two-stage 128 x 128 one 41 and 48.  Fitted on an MI355X to 1721
 // launches of 256 .. 65536 token rows, 1024 .. 32768 columns and K = 128 .. 16384, row counts just past a round among them,
 // below 4096 rows with weights that no cache holds (the next layer's: the two-stage 128 x 128 form, ahead with weights in
 // L2, loses to four stages there: 256 rows, K = 2048, 8.4 / 8.7 us and 16 / 12).  A fit is 3-10 % off in the mean of a curve
 // and up to 40 % at single points; over those launches the form taken is 0.3 % slower than the best one in the mean (16 % at
 // most), over 460 of other widths 0.6 % (36 %).  The four-stage forms have become 0-10 % faster since: over 535 launches of
 // that code (256 .. 4096 rows, K = 512 .. 16384, ten writers, weights from memory) the form taken is 0.2 % slower than
-// the best one (18 % at most).  The 256 x 256 kernel of int8 and of e4m3 has become 3-18 % faster since (blocks of 16 x 16): from the second
-// round on its curves are 6 % lower than the fits.  Over 59 launches of the present code near the lines (512 .. 12288 rows, weights from memory) the form taken is 0.2 % slower than
-// the best one (5 % at most; the fits 0.9 %, 13 %), over 44 others 0.5 % (12 %; 1.5 %, 17 %): e4m3, K = 4096, 32768 columns, 640 rows 107 -> 95 us,
-// int8 GeGLU, 16384 columns, 1088 rows 56 -> 50.  us measured at 4096 columns, 256 x 256 by the fitted code:
+// the best one (18 % at most), so the curves stand.  us measured at 4096 columns, 256 x 256 by the fitted code:
 //                        rows:  256    512   1024   2048   4096   8192
 //   int8, K = 2048   64 x 64    8.1   14.1   27.1   56.2    107    215
 //           128 x 128, 4 / 2   12/16  12/16  13/16  26/22  48/41  95/78
@@ -1101,14 +1099,14 @@ Status GemmKernel::launch(GemmArgs const &args) {
 namespace gemm_cost {
 	struct Point { double tiles, fixed, per_k; };          // tiles / 256
 	struct Curve {
-		Point points[8];                                    // (unused ones at the end are zero)
+		Point points[9];                                    // (unused ones at the end are zero)
 		double rounds = 0.0;                                      // past the last point: the share of the time that goes with rounds begun
 		double us(size_t tiles, double k) const {
 			double const n = double(tiles) / double(COMPUTE_UNITS);
 			auto at = [&](Point const &p) { return p.fixed + p.per_k * (k / 1024.0); };
 			if (n <= points[0].tiles) return at(points[0]);
 			size_t i = 1;
-			for (; i < 8 && points[i].tiles != 0.0; ++i) {
+			for (; i < 9 && points[i].tiles != 0.0; ++i) {
 				Point const &a = points[i - 1], &b = points[i];
 				if (n <= b.tiles) return at(a) + (at(b) - at(a)) * (n - a.tiles) / (b.tiles - a.tiles);
 			}
@@ -1118,7 +1116,7 @@ namespace gemm_cost {
 	struct Curves { Curve large, tile64, tile128_deep, tile128; };   // 256 x 256 | 64 x 64 | 128 x 128, four stages | two
 	static Curves const CURVES[5] = {
 		{   // int8
-			{{{0.125, 4.9, 7.5}, {0.5, 6.6, 8.3}, {1, 8.7, 12.5}, {1.02, 10.5, 18.2}, {2, 13.1, 22.1}, {2.02, 14.5, 28.2}, {3, 15.6, 33.6}}, 0.3},
+			{{{0.125, 4.9, 7.5}, {0.5, 6.6, 8.3}, {1, 8.7, 12.5}, {1.02, 10.5, 18.2}, {2, 13.9, 23.5}, {2.02, 15.4, 30.0}, {3, 16.6, 35.7}}, 0.3},
 			{{{0.25, 3.5, 1.1}, {1, 3.5, 1.6}, {1.02, 5.3, 2.7}, {2, 5.7, 4.6}, {4, 7.9, 8.6}}},
 			{{{0.25, 3.6, 2.7}, {1, 3.7, 4.2}, {1.02, 6.0, 6.3}, {2, 6.0, 9.1}, {2.02, 8.2, 10.1}, {4, 10.3, 17.0}, {4.02, 12.8, 17.4}, {6, 14.2, 25.1}}},
 			{{{0.25, 3.0, 4.3}, {1, 3.3, 5.7}, {1.02, 4.3, 5.1}, {2, 4.2, 8.3}, {2.02, 5.7, 10.9}, {4, 7.1, 15.3}, {4.02, 8.2, 18.1}, {6, 8.6, 23.5}}},
@@ -1130,7 +1128,7 @@ namespace gemm_cost {
 			{{{0.25, 4.2, 4.2}, {1, 3.9, 6.6}, {1.02, 5.2, 5.4}, {2, 5.1, 8.5}, {2.02, 7.4, 11.1}, {4, 7.5, 17.2}, {4.02, 10.4, 18.1}, {6, 11.3, 24.2}}},
 		},
 		{   // e4m3 x e4m3
-			{{{0.125, 9.7, 7.7}, {0.5, 12.5, 8.2}, {1, 18.7, 10.5}, {1.02, 23.6, 17.1}, {2, 26.9, 19.7}, {2.02, 34.7, 25.8}, {3, 33.8, 31.9}}, 0.3},
+			{{{0.125, 9.7, 7.7}, {0.5, 12.5, 8.2}, {1, 18.7, 10.5}, {1.02, 23.6, 17.1}, {2, 28.6, 21.0}, {2.02, 36.9, 27.4}, {3, 36.0, 33.9}}, 0.3},
 			{{{0.25, 3.7, 1.1}, {1, 3.6, 1.6}, {1.02, 4.5, 3.0}, {2, 5.0, 4.7}, {4, 6.3, 9.0}}},
 			{{{0.25, 3.9, 3.0}, {1, 4.3, 4.6}, {1.02, 6.9, 6.6}, {2, 6.5, 8.9}, {2.02, 9.4, 10.5}, {4, 11.5, 17.2}, {4.02, 14.1, 18.5}, {6, 17.2, 26.4}}},
 			{{{0.25, 3.3, 4.5}, {1, 3.5, 6.6}, {1.02, 5.0, 5.7}, {2, 5.8, 8.1}, {2.02, 6.8, 11.1}, {4, 8.7, 16.2}, {4.02, 10.4, 18.3}, {6, 12.0, 24.6}}},
@@ -1150,6 +1148,17 @@ namespace gemm_cost {
 			{{{0.25, 3.1, 7.1}, {1, 3.4, 7.7}, {1.02, 3.9, 11.4}, {2, 3.7, 14.1}, {2.02, 4.3, 19.0}, {4, 5.3, 28.2}, {4.02, 5.7, 32.4}, {6, 5.7, 43.8}}},
 		},
 	};
+	// The 256 x 256 kernel where it is ahead of its fit: the GeGLU writer to eight bits, and of int8 with blocks of 16 x 16 (from K = 384
+	// on) the Scale writer and the dequantising GeGLU.  6 % below the fits from the second round on; between, up to 1.2 rounds, the fit.
+	// The launches that change form by it, us of the 256 x 256 kernel over the form taken before (three launches for each K and
+	// 2048 .. 16384 columns): int8 GeGLU, K = 128 0.76-0.87, 256 0.86-0.99, 384 and 512 0.85-0.95, 1024 0.87-1.07 (32.8 -> 29.4 us
+	// at 1216 rows, 16384 columns; 26.7 -> 28.7 at 2496 rows, 8192), 2048 0.88 (53.5 -> 47.1 at 1088 rows); Scale, K = 384 and 512 0.79-0.90, 1024
+	// 0.91-0.99; dequantising GeGLU, K = 384 and 512 0.86-0.98, 1024 0.96-1.06; e4m3 GeGLU, K = 512 0.70-0.90, 768 0.80-1.0, 1024 0.82-1.03,
+	// 1280 .. 2048 0.80-1.0, 4096 1.01-1.02.  The other writers lose by the lower line: plain dequantising, e4m3, K = 768, 2048 columns,
+	// 16192 rows 41 -> 63 us, int8, K = 128, 8192 columns, 4800 rows 35 -> 47; residual, K = 1024, 2048 columns, 9664 rows 31 -> 34; Scale,
+	// K = 256, 8192 columns, 3968 rows 20.3 -> 22.8.
+	static Curve const AHEAD_INT8 = {{{0.125, 4.9, 7.5}, {0.5, 6.6, 8.3}, {1, 8.7, 12.5}, {1.02, 10.5, 18.2}, {1.2, 11.1, 19.2}, {1.25, 11.1, 19.1}, {2, 13.1, 22.1}, {2.02, 14.5, 28.2}, {3, 15.6, 33.6}}, 0.3};
+	static Curve const AHEAD_E4M3 = {{{0.125, 9.7, 7.7}, {0.5, 12.5, 8.2}, {1, 18.7, 10.5}, {1.02, 23.6, 17.1}, {2, 26.9, 19.7}, {2.02, 34.7, 25.8}, {3, 33.8, 31.9}}, 0.3};
 	// What a small form has to gain by the estimate: the curves' spread.  Without it 23 of the 1721 launches take a form
 	// slower than the 256 x 256 kernel by more than 2 %, one by a fifth; with it 12 do, by 9 % at most.
 	static constexpr double MARGIN = 1.05;
@@ -1162,7 +1171,10 @@ GemmKernel::Small const *GemmKernel::form_for(size_t a_rows) const {
 	};
 	bool const natural = epilogue_kind == 3 || epilogue_kind == 5 || epilogue_kind == 6;
 	gemm_cost::Curves const &c = gemm_cost::CURVES[a_dtype != b_dtype ? (a_dtype == DType::E4m3 && !natural ? 3 : 4) : a_dtype == DType::E4m3 ? 2 : natural ? 1 : 0];
-	double best = c.large.us(tiles_of(metadata), double(a_cols));
+	bool const int8 = a_dtype == DType::Int8 && b_dtype == DType::Int8, e4m3 = a_dtype == DType::E4m3 && b_dtype == DType::E4m3;
+	bool const ahead = epilogue_kind == 1 || (int8 && blocks_of_16 && (epilogue_kind == 0 || dequant_geglu));
+	gemm_cost::Curve const &large = ahead && int8 ? gemm_cost::AHEAD_INT8 : ahead && e4m3 ? gemm_cost::AHEAD_E4M3 : c.large;
+	double best = large.us(tiles_of(metadata), double(a_cols));
 	Small const *chosen = nullptr;
 	for (Small const &s : small) {
 		gemm_cost::Curve const &curve = s.tile == 64 ? c.tile64 : s.stages == 4 ? c.tile128_deep : c.tile128;

@@ -241,6 +241,7 @@ struct GemmKernel {
 	DType a_dtype, b_dtype, c_dtype;
 	size_t head_dim = 0, sep_dim = 0;
 	bool dequant_geglu = false;
+	bool blocks_of_16 = false;            // the 256 x 256 kernel's matrix instructions: 16 x 16 or 32 x 32
 	GemmLauncherMetadata metadata{};
 	std::shared_ptr<HipDevice> device;    // null for a build-only kernel
 	std::unique_ptr<HipKernel> kernel;

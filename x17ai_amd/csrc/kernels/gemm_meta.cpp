@@ -11,6 +11,7 @@ int main() {
 	std::printf("\t\"SMEM_BYTES\": %u,\n", gt::SMEM_BYTES);
 	std::printf("\t\"M_PER_BLOCK\": %u,\n", gt::M_PER_BLOCK);
 	std::printf("\t\"N_PER_BLOCK\": %u,\n", gt::N_PER_BLOCK);
-	std::printf("\t\"MAX_BLOCKS\": %u\n", gt::MAX_BLOCKS);
+	std::printf("\t\"MAX_BLOCKS\": %u,\n", gt::MAX_BLOCKS);
+	std::printf("\t\"BLOCK\": %u\n", gt::BLOCK);
 	std::printf("}\n");
 }
