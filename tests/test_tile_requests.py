@@ -60,6 +60,16 @@ def test_gemm_tile_requests_stay_inside_their_operands(tmp_path, label, make, ro
 	assert rc != 0 and not rep["ok"]
 
 
+@pytest.mark.parametrize("k,block", [((1 << 24) - 128, 16), (1 << 24, 32)])
+def test_gemm_tile_requests_fit_their_buffer_resource(tmp_path, k, block):
+	"""A buffer resource has 32 bits for its size, and a request beyond it reads zeros: a tile of 4 GiB takes another kind of load."""
+	kern = recipes.dequant_gemm_kernel(None, k, 256, X.E4M3, X.E4M3, False, False)
+	with open(os.path.join(_ffi.kernel_cache_dir(), kern.name, "meta.json")) as f:
+		assert json.load(f)["BLOCK"] == block
+	rep, rc = _audit(tmp_path, kern, "gemm_requests_audit.cpp", 256)
+	assert rc == 0 and rep["ok"] and rep["a_extent"] == rep["a_bytes"], rep
+
+
 @pytest.mark.parametrize("form", ["s64x4", "s128x4", "s128x2"])
 @pytest.mark.parametrize("label,make,row_counts", GEMMS, ids=[g[0] for g in GEMMS])
 def test_small_tile_gemm_requests_stay_inside_their_operands(tmp_path, label, make, row_counts, form):

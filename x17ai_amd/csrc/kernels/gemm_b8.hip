@@ -64,6 +64,7 @@ constexpr int LANE_COLS = gt::WAVE_N / gt::GROUPS;          // consecutive raw c
 namespace {
 
 static_assert(K_TOTAL % gt::K_STEP == 0, "K must be a multiple of 128");
+static_assert(128ull * K_TOTAL <= 1ull << 32, "a wave's share of a tile lies within 32-bit lane offsets");
 static_assert(N_RAW % 128 == 0 && N_RAW >= gt::N_PER_BLOCK, "raw output columns: a multiple of 128, at least one tile");
 
 constexpr u32 X_TILE_BYTES = gt::M_PER_BLOCK * ROW_BYTES;   // tokens
@@ -428,7 +429,7 @@ X17_DEV void request16(v4u rows, u32 lds, LaneOffsets const &lo) {
 	             :: "s"(lds), "i"(U * UNIT_ROWS * ROW_BYTES), "v"(lane_offset), "s"(rows), "s"(row * K_TOTAL) : "memory", "m0", "scc");
 }
 X17_DEV v4u rows_resource(u8 const *p) {
-	return v4u{(u32)(u64)p, (u32)((u64)p >> 32), 256 * K_TOTAL, 0x00020000u};
+	return v4u{(u32)(u64)p, (u32)((u64)p >> 32), (u32)gt::RESOURCE_BYTES, 0x00020000u};
 }
 // One part of a step: slice Q / 2 of K, all tokens, half Q % 2 of the columns.  Its reads are the other half's columns (of `w_tile`) and,
 // behind a slice's last use of a token block, that block of the next slice (of `x_tile`), into the same registers.  Behind a matrix instruction

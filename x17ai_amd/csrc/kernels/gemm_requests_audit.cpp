@@ -1,7 +1,7 @@
 // Host-side audit of the GEMM kernel's tile requests.  Compiled with the kernel's own common.h and gemm_tile.h -- the
 // index arithmetic below IS the kernel's (gemm_b8.hip calls the same functions) -- it enumerates, on the CPU, every
 // 16-byte direct-to-LDS request a launch with `a_rows` token rows makes: every tile of the persistent walk, every K
-// step, every loading wave, load unit and lane.  It checks that each request stays inside its operand and that the
+// step, every loading wave, load unit and lane.  It checks that each request stays inside its operand (and its buffer resource) and that the
 // requests of one tile and step cover the tile's 16-byte chunks exactly once, and prints the extents as JSON.
 //
 //     gemm_requests_audit <a_rows> [rows the token operand really has, default a_rows]
@@ -45,6 +45,8 @@ int main(int argc, char **argv) {
 	std::vector<unsigned> x_seen(gt::M_PER_BLOCK * gt::CHUNKS, 0), w_seen(gt::N_PER_BLOCK * gt::CHUNKS, 0);
 	unsigned x_max_row = 0, w_max_row = 0, max_chunk = 0;
 	unsigned long long per_step = 0;
+	// a request's bytes, from the first row of the wave's share on: inside the buffer resource (blocks of 16), which has 32 bits for its size
+	unsigned long long const resource = gt::BLOCKS16 ? (unsigned)gt::RESOURCE_BYTES : 1ull << 32;
 	for (unsigned wave = 0; wave < gt::LOADER_WAVES; ++wave) {
 		for (unsigned u = 0; u < gt::X_UNITS; ++u) {
 			for (unsigned lane = 0; lane < 64; ++lane) {
@@ -52,6 +54,8 @@ int main(int argc, char **argv) {
 				unsigned const chunk = gt::lane_chunk(lane, u & 1);
 				if (row >= gt::M_PER_BLOCK) return fail("token row of a request outside its tile", row, gt::M_PER_BLOCK);
 				if (chunk >= gt::CHUNKS) return fail("chunk of a request outside the K step", chunk, gt::CHUNKS);
+				unsigned long long const end = (unsigned long long)(u * gt::UNIT_ROWS + gt::x_lane_row(lane)) * K + 16 * chunk + 16;
+				if (end > resource) return fail("token request past its buffer resource", end, resource);
 				++x_seen[row * gt::CHUNKS + chunk];
 				x_max_row = row > x_max_row ? row : x_max_row;
 				max_chunk = chunk > max_chunk ? chunk : max_chunk;
@@ -65,6 +69,9 @@ int main(int argc, char **argv) {
 				unsigned const chunk = gt::lane_chunk(lane, u & 1);
 				if (row >= gt::N_PER_BLOCK) return fail("weight row of a request outside its tile", row, gt::N_PER_BLOCK);
 				if (chunk >= gt::CHUNKS) return fail("chunk of a request outside the K step", chunk, gt::CHUNKS);
+				unsigned const share = gt::w_unit_row(wave * gt::W_UNITS * gt::UNIT_ROWS, NATURAL);
+				unsigned long long const end = (unsigned long long)(row - share) * K + 16 * chunk + 16;
+				if (end > resource) return fail("weight request past its buffer resource", end, resource);
 				++w_seen[row * gt::CHUNKS + chunk];
 				w_max_row = row > w_max_row ? row : w_max_row;
 				++per_step;

@@ -75,8 +75,10 @@ constexpr bool SPILLS16 = X17_HEAD_DIM == 32;
 #else
 constexpr bool SPILLS16 = false;
 #endif
+// (their tile requests are buffer loads, whose resource has 32 bits for a tile's bytes: from K = 2^24 on, blocks of 32)
+constexpr unsigned long long RESOURCE_BYTES = 256ull * (X17_A_COLS);
 constexpr bool BLOCKS16 = X17_A_KIND == X17_B_KIND && !SPILLS16 && STAGES == 2 && X_STAGES == 3 && (X17_A_COLS) / K_STEP >= X_STAGES
-	&& WAVE_N == 128 && (WAVE_M == 64 || WAVE_M == 128) && (X17_A_KIND == 0 || (WAVES_PER_SIMD == 1 && (X17_A_COLS) >= 2048));
+	&& WAVE_N == 128 && (WAVE_M == 64 || WAVE_M == 128) && (X17_A_KIND == 0 || (WAVES_PER_SIMD == 1 && (X17_A_COLS) >= 2048)) && RESOURCE_BYTES < 1ull << 32;
 constexpr unsigned BLOCK = BLOCKS16 ? 16 : 32;
 
 // ---- index arithmetic of the tile requests (global -> LDS, 16 bytes per lane).  The kernel calls these; so does the
