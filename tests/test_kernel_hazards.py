@@ -22,7 +22,7 @@ BUNDLER = "/opt/rocm/llvm/bin/clang-offload-bundler"
 OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
 MEMORY = re.compile(r"(global|buffer|flat|scratch)_(load|store|atomic)")
 SCALAR_WRITE = re.compile(r"(v_readfirstlane_b32|v_readlane_b32)\s+s(\d+)")
-SCALAR_PAIR = re.compile(r"s\[(\d+):(\d+)\]")
+SCALAR_OPERAND = re.compile(r"\bs(?:\[(\d+):(\d+)\]|(\d+)\b)")
 M0_WRITE = re.compile(r"s_\w+\s+m0\s*,")
 LDS_DMA = re.compile(r"(global|buffer)_load_lds_\w+|buffer_load_\w+.*\blds\b")
 PACKED_F32 = re.compile(r"v_pk_(add|mul|fma)_f32")
@@ -41,13 +41,11 @@ def _hazards(ins):
 	for i, line in enumerate(ins):
 		if not MEMORY.match(line):
 			continue
-		pair = SCALAR_PAIR.search(line)
-		if not pair:
-			continue
-		lo, hi = int(pair.group(1)), int(pair.group(2))
+		# (a buffer load reads two: its resource and its scalar offset)
+		operands = [(int(m.group(1) or m.group(3)), int(m.group(2) or m.group(3))) for m in SCALAR_OPERAND.finditer(line)]
 		for j in range(max(0, i - 5), i):
 			w = SCALAR_WRITE.match(ins[j])
-			if w and lo <= int(w.group(2)) <= hi:
+			if w and any(lo <= int(w.group(2)) <= hi for lo, hi in operands):
 				found.append((ins[j], line, i - j))
 	return found
 
@@ -84,6 +82,9 @@ def test_no_memory_instruction_reads_a_scalar_register_the_vector_unit_has_just_
 def test_the_scan_sees_a_hazard_when_there_is_one():
 	ins = ["v_readfirstlane_b32 s21, v117", "v_readfirstlane_b32 s20, v116", "s_mov_b32 m0, s8", "global_load_lds_dwordx4 v122, s[20:21]"]
 	assert len(_hazards(ins)) == 2
+	request = "buffer_load_dwordx4 v195, s[20:23], s36 offen lds"
+	assert len(_hazards(["v_readfirstlane_b32 s36, v116", "s_nop 0", request])) == len(_hazards(["v_readfirstlane_b32 s23, v116", "s_nop 0", request])) == 1
+	assert _hazards(["v_readfirstlane_b32 s36, v116"] + ["s_nop 0"] * 5 + [request]) == _hazards(["v_readfirstlane_b32 s3, v116", request]) == []
 	ins = ["v_readfirstlane_b32 s20, v116"] + ["s_nop 0"] * 5 + ["global_load_lds_dwordx4 v122, s[20:21]"]
 	assert _hazards(ins) == []
 	assert len(_m0_hazards(["s_add_i32 m0, s8, 0x1000", "global_load_lds_dwordx4 v122, s[20:21]"])) == 1
