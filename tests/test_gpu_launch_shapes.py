@@ -119,7 +119,12 @@ GEMM_FORMS = [
 	("dequant", lambda: recipes.dequant_gemm_kernel(None, 512, 384, X.INT8, X.INT8, False, True), 512, 384),
 	("dequant_geglu", lambda: recipes.dequant_gemm_kernel(None, 512, 384, X.INT8, X.INT8, True, True), 512, 384),
 	("qnorm", lambda: recipes.attn_q_norm_kernel(None, 512, 384, 64, 0.0), 512, 384),
+	("qnorm_32", lambda: recipes.attn_q_norm_kernel(None, 512, 512, 32, 0.0), 512, 512),
+	("qnorm_128", lambda: recipes.attn_q_norm_kernel(None, 512, 512, 128, 0.0), 512, 512),
+	("qnorm_post", lambda: recipes.attn_q_norm_kernel(None, 512, 512, 64, 0.0, True, 1.0 / math.sqrt(512)), 512, 512),
 	("qkv", lambda: recipes.attn_qkv_kernel(None, 512, 256, 384, 64), 512, 640),
+	("qkv_32", lambda: recipes.attn_qkv_kernel(None, 512, 256, 512, 32), 512, 768),
+	("qkv_128", lambda: recipes.attn_qkv_kernel(None, 512, 256, 512, 128), 512, 768),
 	("mixed", lambda: recipes.mixed_gemm_kernel(None, 512, 384, False), 512, 384),
 	("mixed_residual", lambda: recipes.ffn_y_kernel(None, 128, 512, True, X.E4M3, X.INT8), 512, 256),
 	("e4m3", lambda: recipes.ffn_f_f8_kernel(None, 512, 256, True), 512, 256),
@@ -127,6 +132,11 @@ GEMM_FORMS = [
 	("e4m3", lambda: recipes.ffn_f_f8_kernel(None, 2048, 384, True), 2048, 384),
 	("one_step", lambda: recipes.attn_q_kernel(None, 128, 256), 128, 256),
 ]
+
+
+def _head_dim(name):
+	"""The width of a head where the writer has any: "l2norm_32", "qkv_128"; 64 where the name has no number."""
+	return next((int(part) for part in name.split("_") if part.isdigit()), 64)
 
 
 def _oracle(name, k, n, q_cols, a, b, b_kv, residual, scales, learned):
@@ -148,12 +158,12 @@ def _oracle(name, k, n, q_cols, a, b, b_kv, residual, scales, learned):
 	if name == "residual":
 		return [S.epilogue_residual(acc, residual, inp, 1.0, S.STORE_E4M3)]
 	if name.startswith("l2norm"):
-		return list(S.epilogue_l2norm(acc, int(name.split("_")[1]), recipes.L2_NORM_EPS, inp, 8.0))
+		return list(S.epilogue_l2norm(acc, _head_dim(name), recipes.L2_NORM_EPS, inp, 8.0))
 	if name.startswith("dequant"):
 		return [S.epilogue_dequant(acc, *scales, name == "dequant_geglu")]
-	if name == "qnorm":
-		return [S.epilogue_qnorm(acc, 64, 0.0, 8.0, learned)]
-	kv, rrms = S.epilogue_l2norm(S.gemm_i32(a, b_kv), 64, recipes.L2_NORM_EPS, inp, 8.0)
+	if name.startswith("qnorm"):
+		return [S.epilogue_qnorm(acc, _head_dim(name), 0.0, 8.0, learned, post_scale=1.0 / math.sqrt(k) if name == "qnorm_post" else 1.0)]
+	kv, rrms = S.epilogue_l2norm(S.gemm_i32(a, b_kv), _head_dim(name), recipes.L2_NORM_EPS, inp, 8.0)
 	return [S.epilogue_scale(acc, inp, 8.0), rrms, kv]
 
 
@@ -175,10 +185,12 @@ def test_every_tile_size_gives_the_same_product(shim, name, make, k, n, rows):  
 	out_cols, out_type = n // 2 if pairs else n, X.BF16 if "dequant" in name else X.E4M3 if pairs and name != "geglu_i8_fast" else X.INT8
 	residual = i8_codes(rng, (rows, out_cols))
 	scales = (0.01 + 0.01 * rng.random(rows)).astype(np.float32), (0.01 + 0.01 * rng.random(n)).astype(np.float32)
-	learned = (rng.standard_normal(n).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
-	q_cols = 256 if name == "qkv" else n
+	learned = (16.0 * rng.standard_normal(n) if name == "qnorm_post" else rng.standard_normal(n)).astype(np.float32)
+	learned = (learned.view(np.uint32) >> 16).astype(np.uint16)
+	qkv = name.startswith("qkv")
+	q_cols = 256 if qkv else n
 	b, b_kv = weights(q_cols), weights(max(n - q_cols, 128))
-	heads = (n - q_cols if name == "qkv" else n) // (2 * int(name.split("_")[1]) if name.startswith("l2norm") else 128)
+	heads = (n - q_cols if qkv else n) // (2 * _head_dim(name))
 	ta, tb, tb_kv = t(a, X.E4M3 if e4 else X.INT8), *(t(w, X.E4M3 if name == "e4m3" else X.INT8) for w in (b, b_kv))
 	extras = t(residual, X.INT8), [t(v, X.F32) for v in scales], t(learned, X.BF16)
 	results = {}
@@ -192,7 +204,7 @@ def test_every_tile_size_gives_the_same_product(shim, name, make, k, n, rows):  
 		def poisoned(shape, dtype):
 			size = {X.INT8: 1, X.E4M3: 1, X.BF16: 2, X.F32: 4}[dtype]
 			return t(np.full(shape[:-1] + (shape[-1] * size,), pattern, np.uint8).view({1: np.uint8, 2: np.uint16, 4: np.float32}[size]), dtype)
-		c = poisoned((rows, q_cols if name == "qkv" else out_cols), out_type)
+		c = poisoned((rows, q_cols if qkv else out_cols), out_type)
 		c_kv, rrms = poisoned((rows, max(n - q_cols, 128)), X.INT8), poisoned((rows, max(heads, 1)), X.F32)
 		outputs = [c]
 		slots = [ta, rows, tb, n, c]
@@ -203,9 +215,9 @@ def test_every_tile_size_gives_the_same_product(shim, name, make, k, n, rows):  
 			slots.append(extras[0])
 		elif "dequant" in name:
 			slots.extend(extras[1])
-		elif name == "qnorm":
+		elif name.startswith("qnorm"):
 			slots.append(extras[2])
-		elif name == "qkv":
+		elif qkv:
 			slots.extend([rrms, tb_kv, c_kv])
 			outputs.extend([rrms, c_kv])
 		dev.synchronize()
@@ -229,7 +241,8 @@ def test_every_tile_size_gives_the_same_product(shim, name, make, k, n, rows):  
 def test_the_persistent_walk_over_more_tiles_than_workgroups(shim):  # noqa: F811
 	"""The 256 x 256 kernel alone, whatever launch() takes at these sizes: 256 workgroups walk 260 tiles of K = 384 (three
 	steps: every request of a tile's last two belongs to the workgroup's next tile), int8 and in the four-wavefront e4m3
-	form, and 264 tiles through the L2-norm writer, whose rrms stores are in flight next to the next tile's loads."""
+	form, and 264 tiles through the L2-norm writer, whose rrms stores are in flight next to the next tile's loads.  e4m3 at K = 384 and
+	the L2-norm writer at K = 256 are blocks of 32 x 32; at K = 2048 and 384 they are blocks of 16."""
 	from oracle import strict as S
 	dev = X.Device(0)
 	t = lambda a, dtype: X.Tensor.from_numpy(dev, np.ascontiguousarray(a), dtype)
@@ -247,20 +260,22 @@ def test_the_persistent_walk_over_more_tiles_than_workgroups(shim):  # noqa: F81
 	assert np.array_equal(c.download(), S.epilogue_scale(S.gemm_i32(a, b), 1.0 / math.sqrt(k) / 64.0, 8.0))
 
 	m, n = 256 * 130, 512
-	a8, b8 = e4m3_bytes(rng, (m, k)), e4m3_bytes(rng, (n, k))
-	c = t(np.full((m, n // 2), 0x5A, np.uint8), X.E4M3)
-	launch(recipes.ffn_f_f8_kernel(None, k, n, True), m, n, [t(a8, X.E4M3), m, t(b8, X.E4M3), n, c])
-	want = S.epilogue_geglu(S.gemm_f32_seq(a8, True, b8, True), 1.0 / math.sqrt(k), 1.0, S.STORE_E4M3)
-	differ, beyond = e4m3_compare(c.download(), want)
-	assert differ < 5e-3 and beyond == 0.0, (differ, beyond)
+	for k, every in ((384, 1), (2048, 5)):      # (the oracle's rows: all, or some of every tile)
+		a8, b8 = e4m3_bytes(rng, (m, k)), e4m3_bytes(rng, (n, k))
+		c = t(np.full((m, n // 2), 0x5A, np.uint8), X.E4M3)
+		launch(recipes.ffn_f_f8_kernel(None, k, n, True), m, n, [t(a8, X.E4M3), m, t(b8, X.E4M3), n, c])
+		want = S.epilogue_geglu(S.gemm_f32_seq(np.ascontiguousarray(a8[::every]), True, b8, True), 1.0 / math.sqrt(k), 1.0, S.STORE_E4M3)
+		differ, beyond = e4m3_compare(c.download()[::every], want)
+		assert differ < 5e-3 and beyond == 0.0, (k, differ, beyond)
 
-	m, k, n = 256 * 33, 256, 2048
-	a, b = i8_codes(rng, (m, k)), i8_codes(rng, (n, k))
-	for hd in (64, 128):
-		c, rrms = t(np.full((m, n), 0x5A, np.int8), X.INT8), t(np.full((m, n // (2 * hd)), 7.5, np.float32), X.F32)
-		launch(recipes.attn_kv_kernel(None, k, n, hd), m, n, [t(a, X.INT8), m, t(b, X.INT8), n, c, rrms])
-		want_c, want_r = S.epilogue_l2norm(S.gemm_i32(a, b), hd, recipes.L2_NORM_EPS, 1.0 / math.sqrt(k) / 64.0, 8.0)
-		assert np.array_equal(c.download(), want_c) and np.array_equal(rrms.download().view(np.uint32), want_r.view(np.uint32)), hd
+	m, n = 256 * 33, 2048
+	for k in (256, 384):
+		a, b = i8_codes(rng, (m, k)), i8_codes(rng, (n, k))
+		for hd in (64, 128):
+			c, rrms = t(np.full((m, n), 0x5A, np.int8), X.INT8), t(np.full((m, n // (2 * hd)), 7.5, np.float32), X.F32)
+			launch(recipes.attn_kv_kernel(None, k, n, hd), m, n, [t(a, X.INT8), m, t(b, X.INT8), n, c, rrms])
+			want_c, want_r = S.epilogue_l2norm(S.gemm_i32(a, b), hd, recipes.L2_NORM_EPS, 1.0 / math.sqrt(k) / 64.0, 8.0)
+			assert np.array_equal(c.download(), want_c) and np.array_equal(rrms.download().view(np.uint32), want_r.view(np.uint32)), (k, hd)
 
 
 @pytest.mark.parametrize("name,make,out_type", [

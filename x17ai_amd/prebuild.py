@@ -136,6 +136,9 @@ def _specs():
 		add(("dequant", 8192, 2048, INT8, INT8, False, strict))
 	# ---- tests/test_gpu_launch_shapes.py: e4m3 products with inexact float32 sums
 	add(("ffn_f_f8", 2048, 384, True))
+	add(("ffn_f_f8", 2048, 512, True))
+	for hd in (64, 128):
+		add(("attn_kv", 384, 2048, hd))
 	add(("dequant", 4096, 384, E4M3, E4M3, False, True))
 	add(("dequant", 4096, 384, E4M3, INT8, False, True))
 	add(("ffn_y", 256, 4096, True, E4M3, INT8))
