@@ -98,22 +98,23 @@ X17_DEV u32 v_granule_offset(u32 key, u32 c) {
 // Strict build without row scales.  The reference's numbers at powers of two of its own scale, so that a score of a fully visible tile
 // takes 17 vector instructions instead of 19 and the slow ones of them (conversion, comparison and select, rounding) go:
 //  * Score accumulators start at the bits of DOT_START = 1 / 2 pi, which the matrix instruction takes as an inline constant: read as a
-//    float the sum is DOT_START + dot * 2^-26 exactly (0x3E22F983 has 2 290 051 steps of 2^-26 below it in its binade and
+//    float the sum is DOT_START + dot * 2^-26 exactly (0x3E22F983 has 2 292 099 steps of 2^-26 below it in its binade and
 //    more above, |dot| <= 128 * 128 * 128), one exact subtraction away from the dot product.
 //  * Scores, and the maximum their probabilities refer to, at 2^-7: maximum - score is what ex2 takes, and the subtraction's own
 //    clamp to [0, 1] keeps its argument above -128.
 //  * ex2's polynomial at one half: a result below 2^-125, which the reference's ex2 flushes, then has an exponent field of 0 (an f32
-//    denormal) or a negative one (a set sign bit).  The key loop runs with f32 denormals flushed, so that the multiplication by 255
-//    takes the former for 0; its clamp makes 0 of the latter.  The clamp wants probabilities below 1: they and the partial sums
+//    denormal) or a negative one (a set sign bit, or a NaN).  The key loop runs with f32 denormals flushed, so that the multiplication by 255
+//    takes the former for 0; its clamp makes 0 of the latter, of NaNs too.  The clamp wants probabilities below 1: they and the partial sums
 //    are at 2^-8.  (What else could be denormal there has no bearing on the output: O and the sums, decayed by 2^-100 and
 //    more, next to a sum of at least 63.)
 //  * Adding 1.5 * 2^15 rounds p / 256 to the integer P and leaves it in the low half of the sum, where it is the f16 denormal
 //    P * 2^-24: the matrix instructions multiply those exactly, O is at 2^-24.
 // Powers of two change no rounding, so the bits are the reference's.  A head whose temperature is zero, not finite or outside
 // 2^-40 .. 2^40 takes the masked steps throughout.  Bound by vector issue (2.5 clocks an instruction, by the counters):
-// 64 heads of 32, 16384 tokens, no window 3165 -> 2977 us; 32 heads of 128, 8192 tokens 868 -> 826.
+// 64 heads of 32, 16384 tokens, no window 3219 -> 3047 us; 32 heads of 128, 8192 tokens 868 -> 831 (in turn, three times each).
 constexpr bool SCALED_SUMS = STRICT && !ROW_SCALES;
 constexpr u32 DOT_START_BITS = 0x3E22F983u;
+static_assert((DOT_START_BITS & 0x7FFFFFu) >= 128 * 128 * HD && 0x7FFFFFu - (DOT_START_BITS & 0x7FFFFFu) >= 128 * 128 * HD, "every dot product stays in DOT_START's binade");
 constexpr f32 DOT_START = __builtin_bit_cast(f32, DOT_START_BITS);
 constexpr f32 SUM_SCALE = SCALED_SUMS ? 0.00390625f : 1.0f;                        // 2^-8
 constexpr f32 SUM_PROB_SCALE = PROB_SCALE * SUM_SCALE;

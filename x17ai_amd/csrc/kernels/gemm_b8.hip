@@ -21,8 +21,8 @@
 //     16-byte chunks are XOR-swizzled so that ds_read_b128 is conflict-free.  In the int8 and e4m3 kernels the
 //     issue order of a K step is pinned: each MFMA is followed by its share of the LDS reads and tile requests
 //     (and, in the mixed arithmetic, of the next round's conversions to f16).
-//   * int8: v_mfma_i32_16x16x64_i8.  e4m3 x e4m3: v_mfma_f32_16x16x128_f8f6f4 (with the head-normalising writers, with
-//     fewer than three K steps and for e4m3 below K = 2048 the 32 x 32 forms of both).  Mixed
+//   * int8: v_mfma_i32_16x16x64_i8.  e4m3 x e4m3: v_mfma_f32_16x16x128_f8f6f4 (the 32 x 32 forms of both with fewer than three
+//     K steps, for e4m3 below K = 2048 and in the kv writer at head_dim 32: gemm_tile.h).  Mixed
 //     e4m3 x int8: both widened exactly to f16 in registers, v_mfma_f32_32x32x16_f16
 //     (int8 codes need 7 significand bits, e4m3 has 4; every e4m3 value is a normal f16).
 //   * Workgroup ids are remapped so that each XCD (own L2) works on a compact block of tiles.
@@ -121,10 +121,10 @@ struct LaneOffsets {
 
 // Direct-to-LDS loads of a loading wave's share of one token tile / one weight tile: loading wave w copies
 // token rows [X_UNITS * UNIT_ROWS * w, +X_UNITS * UNIT_ROWS) and as many LDS weight rows.
-// With WN = WAVE_N columns per wave, LDS weight row R = WN*wn + 32*bn + i holds weight row
-// WN*wn + (WN/2)*((i/4)%2) + 16*bn + 4*(i/8) + i%4: the MFMA hands output row i = 8*(r/4) + 4*(lane/32) + r%4
-// to register r, so a lane collects columns (WN/2)*(lane/32) + 16*bn + r.  For the rows of one load unit the
-// lane-dependent part is constant.
+// Which weight row an LDS weight row holds: gt::w_unit_row.  A 32 x 32 matrix instruction hands output row
+// i = 8*(r/4) + 4*(lane/32) + r%4 to register r, so with WN = WAVE_N columns per wave a lane collects columns
+// (WN/2)*(lane/32) + 16*bn + r; a 16 x 16 one row i = 4*(lane/16) + r, and columns (WN/4)*(lane/16) + 4*bn + r.  For the
+// rows of one load unit the lane-dependent part is constant.
 template <u32 U>
 X17_DEV void issue_x_load(u8 const *a_tile, u8 *x_tile, u32 k0, u32 wave, LaneOffsets const &lo) {
 	u8 *x_lds = x_tile + (wave * X_UNITS + U) * UNIT_ROWS * ROW_BYTES;
@@ -364,9 +364,10 @@ X17_DEV void mixed_round(Wide const &cur, Wide &nxt, Frags const &raw, Frags &rd
 
 // ---- 16 x 16 blocks (int8 x int8 and e4m3 x e4m3).  What bounds these kernels is the power the chip may draw: it lowers the clock
 // until they fit, and per product the 16 x 16 instructions cost less of it than the 32 x 32 ones (half the accumulator traffic).  Loops
-// of nothing but matrix instructions on Gaussian operands: int8 3.56 -> 4.16 POP/s, e4m3 4.04 -> 4.42.  us, blocks of 32 / of 16:
-//   int8, K = 2048, 16384 columns with the GeGLU writer, 32768 rows 866 / 806 (clock 1.68 -> 1.88 GHz, as many cycles)
-//   int8, run-time scales, K = 8192, 2048 columns, 8192 rows 115 / 105     e4m3, K = 16384, 8192 columns, 16384 rows 1469 / 1402
+// of nothing but matrix instructions on Gaussian operands: int8 3.71 -> 4.29 POP/s, e4m3 4.16 -> 4.46.  us in turn, blocks of 32 / of 16:
+//   int8, K = 2048, 16384 columns with the GeGLU writer, 32768 rows 865 / 795 (by the counters 1.69 -> 1.80 GHz and 1.5 % more cycles)
+//   int8, run-time scales, K = 8192, 2048 columns, 8192 rows 115 / 104     e4m3, K = 16384, 8192 columns, 16384 rows 1485 / 1471,
+//   4096 rows 358 / 345; K = 4096, 32768 columns, 16384 rows 1463 / 1442 (ten of eleven e4m3 products 1-4 % faster, one equal)
 // The bytes are those of the 32 x 32 instructions.  int32 sums are exact; a 16x16x128 instruction adds sixteen products of every lane
 // group at a time, in the groups' order, and so goes through K as two 32x32x64 instructions do if group g takes the chunks
 // chunk16 names (no difference in 400 thousand sums of 2048 products each).

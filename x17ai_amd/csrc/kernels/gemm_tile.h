@@ -65,10 +65,10 @@ constexpr unsigned WAVES_PER_SIMD = (WAVE_M / 32) * (WAVE_N / 32) <= 8 ? 2 : 1;
 
 // Rows of an operand per matrix instruction.  NATURAL: the writers that normalise whole heads, with an order of the weight rows of their own.
 // e4m3 takes blocks of 16 from K = 2048 on: below, the accumulators' way to the writer costs more than the K loop gains (GeGLU writer,
-// 4096 columns, 16384 rows, us, blocks of 32 / of 16: K = 384 37.4 / 39.9, 512 41.6 / 44.4, 1024 66.0 / 66.7, 2048 111.3 / 108.9).
+// 4096 columns, 16384 rows, us, blocks of 32 / of 16: K = 384 37.4 / 39.9, 512 41.6 / 44.4, 1024 66.0 / 66.7, 2048 104.1 / 102.7).
 // The kv writer with heads of 32 columns keeps blocks of 32: with blocks of 16 one or two of its registers spill.
 // int8 gains at every K (scale writer: K = 384 41.0 / 34.9, 1024 77 / 63; GeGLU, K = 512 42.2 / 41.9, 1024 69.9 / 63.7;
-// q + kv, K = 2048, 6144 columns, 3264 rows 48.6 / 46.4, 32768 rows 325 / 304; kv alone, 4096 columns, K = 512 43.5 / 42.8, 2048 118 / 111).
+// q + kv, K = 2048, 6144 columns, 3264 rows 46.4 / 44.8, 32768 rows 323 / 301; kv alone, 4096 columns, K = 2048 110 / 103, and K = 512 41.5 both).
 constexpr bool NATURAL = X17_EPILOGUE == 3 || X17_EPILOGUE == 5 || X17_EPILOGUE == 6;
 #if X17_EPILOGUE == 3
 constexpr bool SPILLS16 = X17_HEAD_DIM == 32;
