@@ -93,17 +93,37 @@ def test_the_scan_sees_a_hazard_when_there_is_one():
 	assert _m0_hazards(["s_add_i32 m0, s8, 0x1000", "v_add_u32_e32 v1, v2, v3", "global_load_lds_dwordx4 v122, s[20:21]"]) == []
 
 
-def test_every_barrier_is_a_compiler_fence():
-	"""__builtin_amdgcn_s_barrier orders no memory access for the compiler: it stands between clobbers in step_barrier, and
-	nowhere else (__syncthreads brings fences of its own)."""
+def test_the_barriers_of_the_gemm_order_memory_accesses():
+	"""A K step's barrier stands between clobbers in step_barrier, and nowhere else in the 256 x 256 kernel, whose
+	wavefronts in part request no tiles: there nothing else would keep a step's reads behind it."""
 	kernels = os.path.join(os.path.dirname(os.path.abspath(recipes.__file__)), "csrc", "kernels")
-	barriers = {}
-	for path in glob.glob(os.path.join(kernels, "*.h")) + glob.glob(os.path.join(kernels, "*.hip")):
-		with open(path) as f:
-			text = f.read()
-		if "amdgcn_s_barrier" in text:
-			barriers[os.path.basename(path)] = text
-	assert list(barriers) == ["x17_device.h"]
+	text = {}
+	for name in ("x17_device.h", "gemm_b8.hip", "gemm_parts.h"):
+		with open(os.path.join(kernels, name)) as f:
+			text[name] = f.read()
 	clobber = r'asm volatile\("" ::: "memory"\);\n'
 	fenced = re.compile(r"void step_barrier\(\) \{\n\t" + clobber + r"\t__builtin_amdgcn_s_waitcnt\(0xC07F\);[^\n]*\n\t__builtin_amdgcn_s_barrier\(\);\n\t" + clobber)
-	assert len(fenced.findall(barriers["x17_device.h"])) == 1 and barriers["x17_device.h"].count("amdgcn_s_barrier") == 1
+	assert len(fenced.findall(text["x17_device.h"])) == 1 and text["x17_device.h"].count("amdgcn_s_barrier") == 1
+	assert "amdgcn_s_barrier" not in text["gemm_b8.hip"] + text["gemm_parts.h"] and "step_barrier()" in text["gemm_b8.hip"]
+
+
+@pytest.mark.skipif(not (os.path.exists(BUNDLER) and os.path.exists(OBJDUMP) and shutil.which("hipcc")), reason="needs the ROCm LLVM tools")
+def test_the_compiler_takes_the_barrier_and_the_wait_for_memory_accesses(tmp_path):
+	"""What the barriers outside step_barrier stand on: three reads of one LDS word, a barrier and a wait between them, stay three,
+	each where it was written."""
+	source, code_object = tmp_path / "reads.hip", tmp_path / "reads.hsaco"
+	source.write_text("""#include <hip/hip_runtime.h>
+extern "C" __global__ void kernel(int *out) {
+	extern __shared__ int words[];
+	int const a = words[threadIdx.x];
+	__builtin_amdgcn_s_barrier();
+	int const b = words[threadIdx.x];
+	__builtin_amdgcn_s_waitcnt(0xC07F);
+	int const c = words[threadIdx.x];
+	out[threadIdx.x] = a + 3 * b + 5 * c;
+}
+""")
+	subprocess.run(["hipcc", "-O3", "--offload-arch=gfx950", "--genco", str(source), "-o", str(code_object)], check=True, capture_output=True)
+	kinds = [line.split()[0] for line in _instructions(str(code_object), str(tmp_path)) if line.startswith(("ds_read", "s_barrier", "s_waitcnt lgkmcnt(0)"))]
+	assert [k for k in kinds if k != "s_waitcnt"] == ["ds_read_b32", "s_barrier", "ds_read_b32", "ds_read_b32"]
+	assert kinds[3] == "s_waitcnt" and kinds[4] == "ds_read_b32", kinds

@@ -259,7 +259,8 @@ void kernel(
 			} else {
 				__builtin_amdgcn_s_waitcnt(kt::Q_STAGERS == kt::THREADS_PER_BLOCK ? 0x0F71 : 0x0F70);      // (wavefronts that request no Q: all of dO)
 			}
-			step_barrier();
+			__builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
+			__builtin_amdgcn_s_barrier();
 			request_do((slot + 1) & 1, SLOT >= 0 || i + 2 < n_steps);
 			request_q((slot + 3) % kt::RING, SLOT >= 0 || i + 4 < n_steps);
 		};

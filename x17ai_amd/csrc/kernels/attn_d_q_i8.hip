@@ -259,7 +259,8 @@ void kernel(
 		// says that tile s + 4 exists (the caller's loop bound)
 		auto stage = [&]<int SLOT>(u32 s) __attribute__((always_inline)) {
 			__builtin_amdgcn_s_waitcnt(0x0F72);          // vmcnt(2): tile s + 1 has landed (this thread's chunks), s + 2 may be in flight
-			step_barrier();      // own LDS traffic of step s - 1 is complete, behind it so is everybody else's: tiles s are visible
+			__builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0): own LDS traffic of step s - 1 is complete
+			__builtin_amdgcn_s_barrier();                // ... and so is everybody else's: tiles s are visible
 			// step s requests tile min(s + 3, last) into the slot of tile s - 1, which nobody reads any more
 			request(SLOT >= 0 ? (SLOT + 3) % bt::RING : (s + 3) % bt::RING);
 			if (SLOT >= 0 || at::further_tile_exists(s, n_steps)) {

@@ -463,7 +463,8 @@ void kernel(
 			} else {
 				__builtin_amdgcn_s_waitcnt(0x0F74);      // vmcnt(4): K tile i and raw V tile i + 1 have landed
 			}
-			step_barrier();      // own LDS traffic of step i - 1 is complete, behind it so is everybody else's: tiles i are visible
+			__builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0): own LDS traffic of step i-1 is complete
+			__builtin_amdgcn_s_barrier();                // ... and so is everybody else's: tiles i are visible
 			request_tiles.template operator()<SLOT>(i);
 		};
 		// raw V tile of step i + 1 -> f16 tile (i + 1) % 2

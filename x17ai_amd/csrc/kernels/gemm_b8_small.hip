@@ -276,7 +276,8 @@ void kernel(
 	wait_vmcnt<0>();
 	u8 *const exchange = smem + (wave / gt::WAVES_K) * GROUP_BYTES + lane * 16;
 	if constexpr (gt::WAVES_K > 1) {
-		step_barrier();
+		__builtin_amdgcn_s_waitcnt(0xC07F);
+		__builtin_amdgcn_s_barrier();
 		X17_UNROLL for (int j = 0; j < BLOCKS; ++j) {
 			if (owner(j) != wk) {
 				X17_UNROLL for (int q = 0; q < 4; ++q) {

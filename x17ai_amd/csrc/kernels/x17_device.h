@@ -56,9 +56,9 @@ X17_DEV u32 f2u(f32 f) { return __builtin_bit_cast(u32, f); }
 X17_DEV f32 u2f(u32 u) { return __builtin_bit_cast(f32, u); }
 X17_DEV f32 fmaf32(f32 a, f32 b, f32 c) { return __builtin_fmaf(a, b, c); }
 
-// The barrier of a workgroup's pipeline step, behind this wavefront's LDS reads and writes.  The builtins order no memory access for the
-// compiler: the clobbers keep the next step's reads behind the barrier and the last one's in front of it, also in wavefronts that
-// request no tiles.
+// The barrier of a GEMM's K step, behind this wavefront's LDS reads and writes.  The clobbers keep the next step's reads behind the barrier and
+// the last one's in front of it, also in wavefronts that request no tiles, whatever the compiler takes the builtins for.  (The one at
+// hand takes both for accesses to any memory, and a test holds it to that: elsewhere they stand alone.)
 X17_DEV void step_barrier() {
 	asm volatile("" ::: "memory");
 	__builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0)
