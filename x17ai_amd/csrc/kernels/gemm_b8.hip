@@ -64,7 +64,7 @@ constexpr int LANE_COLS = gt::WAVE_N / gt::GROUPS;          // consecutive raw c
 namespace {
 
 static_assert(K_TOTAL % gt::K_STEP == 0, "K must be a multiple of 128");
-static_assert(128ull * K_TOTAL <= 1ull << 32, "a wave's share of a tile lies within 32-bit lane offsets");
+static_assert((gt::max_offset_row(NATURAL_COLS) + 1ull) * K_TOTAL <= 1ull << 32, "a lane's operand offsets fit 32 bits");
 static_assert(N_RAW % 128 == 0 && N_RAW >= gt::N_PER_BLOCK, "raw output columns: a multiple of 128, at least one tile");
 
 constexpr u32 X_TILE_BYTES = gt::M_PER_BLOCK * ROW_BYTES;   // tokens

@@ -124,6 +124,22 @@ constexpr unsigned lane_chunk(unsigned lane, unsigned odd) {
 	unsigned const j = lane / CHUNKS, p = lane % CHUNKS;
 	return p ^ swizzle(odd * UNIT_ROWS + j);
 }
+// The largest row that a lane's 32-bit operand offset holds: of its load unit, and with one wavefront per SIMD, which keeps an offset per unit,
+// of its wave's share.
+constexpr unsigned max_offset_row(bool natural) {
+	unsigned most = 0;
+	for (unsigned wave = 0; wave < LOADER_WAVES; ++wave) {
+		for (unsigned u = 0; u < (WAVES_PER_SIMD == 1 ? W_UNITS : 1); ++u) {
+			for (unsigned lane = 0; lane < 64; ++lane) {
+				unsigned const first = wave * W_UNITS * UNIT_ROWS;
+				unsigned const row = w_unit_row(first + u * UNIT_ROWS, natural) - w_unit_row(first, natural) + w_lane_row(lane, natural);
+				most = row > most ? row : most;
+			}
+		}
+	}
+	unsigned const x = (WAVES_PER_SIMD == 1 ? X_UNITS : 1) * UNIT_ROWS - 1;
+	return x > most ? x : most;
+}
 // First token row and first raw column of tile `lin` of the persistent walk: each XCD (the hardware deals workgroups
 // round-robin to 8 of them) gets a contiguous run of tiles, walked in bands of `band` token tiles; a last tile that
 // would overhang the matrix is moved back to end at its edge.
